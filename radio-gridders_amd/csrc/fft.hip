@@ -1,8 +1,12 @@
-// fft.hip -- batched 2-D FFTs, fft-shift and transposes.
+// fft.hip -- batched 2-D FFTs and fft-shift.
 //
-// n <= 512: row pass (B rows per block, padded LDS) then column pass
-// (CB columns per block, each row segment of the block is one 128-byte line).
-// n > 512: row pass, tiled transpose, row pass, transpose back.
+// A row pass, then a column pass, both in place: every array is read and
+// written twice and nothing else.  A quadrant swap before and after the
+// transform is an index offset of n / 2 in the loads and stores of both passes
+// (sh: 0 or n / 2, applied as idx ^ sh, n being a power of two).
+// n <= 512: lines in LDS (B rows per block, padded; CB columns per block, each
+// row segment of the block is one 128-byte line).
+// n > 512: lines in registers, 16 values per thread (fft16_line).
 #include "fft_core.hpp"
 
 namespace rg {
@@ -17,7 +21,8 @@ template <typename T2, int LOGN, int B, bool INV>
 __global__ __launch_bounds__(B *((1 << LOGN) / 8)) void k_fft_rows(T2 *data, int64_t nrows,
                                                                    const T2 *__restrict__ twg,
                                                                    const uint32_t *row_flags,
-                                                                   const int32_t *dev_batch)
+                                                                   const int32_t *dev_batch,
+                                                                   int sh)
 {
     constexpr int n = 1 << LOGN;
     constexpr int NT = B * (n / 8);
@@ -55,7 +60,7 @@ __global__ __launch_bounds__(B *((1 << LOGN) / 8)) void k_fft_rows(T2 *data, int
         val.x = 0;
         val.y = 0;
         if (r < nrows)
-            val = data[r * n + idx];
+            val = data[r * n + (idx ^ sh)];
         lds[idx * LS + line] = val;
     }
     __syncthreads();
@@ -65,7 +70,7 @@ __global__ __launch_bounds__(B *((1 << LOGN) / 8)) void k_fft_rows(T2 *data, int
         const int64_t r = row0 + line;
         if (r < nrows) {
             if (!row_flags || ((row_flags[r >> 5] >> (r & 31)) & 1u))
-                data[r * n + idx] = lds[idx * LS + line];
+                data[r * n + (idx ^ sh)] = lds[idx * LS + line];
         }
     }
 }
@@ -76,7 +81,8 @@ __global__ __launch_bounds__(B *((1 << LOGN) / 8)) void k_fft_rows(T2 *data, int
 template <typename T2, int LOGN, int CB, bool INV>
 __global__ __launch_bounds__(CB *((1 << LOGN) / 8)) void k_fft_cols(T2 *data,
                                                                     const T2 *__restrict__ twg,
-                                                                    const int32_t *dev_batch)
+                                                                    const int32_t *dev_batch,
+                                                                    int sh)
 {
     if (dev_batch && (int)blockIdx.y >= *dev_batch)
         return;
@@ -89,32 +95,87 @@ __global__ __launch_bounds__(CB *((1 << LOGN) / 8)) void k_fft_cols(T2 *data,
     T2 *a = data + (size_t)blockIdx.y * n * n + (size_t)blockIdx.x * CB;
     for (int e = threadIdx.x; e < n * CB; e += NT) {
         const int row = e / CB, col = e - row * CB;
-        lds[e] = a[(size_t)row * n + col];
+        lds[e] = a[(size_t)(row ^ sh) * n + col];
     }
     __syncthreads();
     fft_block<T2, LOGN, CB, CB, INV>(lds, tw);
     for (int e = threadIdx.x; e < n * CB; e += NT) {
         const int row = e / CB, col = e - row * CB;
-        a[(size_t)row * n + col] = lds[e];
+        a[(size_t)(row ^ sh) * n + col] = lds[e];
     }
 }
 
-// ---- transpose -------------------------------------------------------------------
-template <typename T2>
-__global__ __launch_bounds__(256) void k_transpose(const T2 *__restrict__ in, T2 *__restrict__ out,
-                                                   int n, const int32_t *dev_batch)
+// ---- long lines (n > 512) ----------------------------------------------------------
+// Bound by HBM: 2 n^2 values moved per pass.  A 4096^2 FP64 array: rows 124 us (4.3
+// TB/s), columns 125 us; the image of a grid (shift, transform, shift) 660 -> 250
+// us, where two shift passes, two row passes through LDS and two transposes
+// moved the array six times.  2048^2 FP64: 152 -> 63 us, FP32 35 us.
+// Rows [blockIdx.x NL, +NL) of nrows contiguous rows; arguments as k_fft_rows.
+template <typename T2, int LOGN, int NL, bool INV>
+__global__ __launch_bounds__(NL *((1 << LOGN) / 16)) void k_fft_rows16(
+    T2 *data, int64_t nrows, const T2 *__restrict__ tw, const uint32_t *row_flags,
+    const int32_t *dev_batch, int sh)
 {
-    if (dev_batch && (int)blockIdx.z >= *dev_batch)
+    using T = decltype(T2().x);
+    using L = typename std::conditional<sizeof(T2) == 16, T, T2>::type; // FP64: split
+    constexpr int n = 1 << LOGN, TPL = n / 16, LW = pad16(n);
+    __shared__ L lds[NL * LW];
+    const int line = threadIdx.x / TPL, lt = threadIdx.x % TPL;
+    const int64_t row = (int64_t)blockIdx.x * NL + line;
+    if (dev_batch && (int64_t)blockIdx.x * NL >= (int64_t)*dev_batch * n)
+        return; // the block's rows (NL divides n) lie in an inactive array
+    const bool on =
+        row < nrows && (!row_flags || ((row_flags[row >> 5] >> (row & 31)) & 1u));
+    if (row_flags && !__syncthreads_or(on))
+        return; // every row of the block is empty
+    T2 *a = data + (on ? row : 0) * n + lt;
+    L *mine = lds + line * LW;
+    const int shm = sh / TPL; // 8 or 0: positions lt + m TPL to lt + (m ^ 8) TPL
+    fft16_line<T2, LOGN, INV>(
+        tw, lt, [&](int i) { return mine + i; },
+        [&](int m) {
+            T2 v;
+            v.x = v.y = 0;
+            if (on)
+                v = a[(m ^ shm) * TPL];
+            return v;
+        },
+        [&](int m, const T2 &v) {
+            if (on)
+                a[(m ^ shm) * TPL] = v;
+        });
+}
+
+// Columns [cb CB, +CB) of array blockIdx.y, CB columns side by side in LDS.
+// A row segment of the block is 64 bytes (32 for FP32 at 4096), a part of a
+// cache line, since 1024 threads or the LDS hold no more, so the G workgroups that share
+// lines run on one XCD next to each other: workgroup b lies on XCD b mod 8.
+template <typename T2, int LOGN, int CB, bool INV>
+__global__ __launch_bounds__(CB *((1 << LOGN) / 16)) void k_fft_cols16(
+    T2 *data, const T2 *__restrict__ tw, const int32_t *dev_batch, int sh)
+{
+    using T = decltype(T2().x);
+    using L = typename std::conditional<sizeof(T2) == 16, T, T2>::type;
+    constexpr int n = 1 << LOGN;
+    constexpr int G = 128 / (CB * (int)sizeof(T2)) > 1 ? 128 / (CB * (int)sizeof(T2)) : 1;
+    static_assert((n / CB) % (8 * G) == 0, "whole rounds of 8 XCDs");
+    __shared__ L lds[pad16(n) * CB];
+    if (dev_batch && (int)blockIdx.y >= *dev_batch)
         return;
-    __shared__ T2 tile[32][33];
-    const size_t off = (size_t)blockIdx.z * n * n;
-    const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
-    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
-    for (int j = ty; j < 32; j += 8)
-        tile[j][tx] = in[off + (size_t)(y0 + j) * n + x0 + tx];
-    __syncthreads();
-    for (int j = ty; j < 32; j += 8)
-        out[off + (size_t)(x0 + j) * n + y0 + tx] = tile[tx][j];
+    const int b = blockIdx.x;
+    const int cb = ((b / (8 * G)) * 8 + b % 8) * G + (b / 8) % G;
+    constexpr int TPL = n / 16;
+    const int line = threadIdx.x % CB, lt = threadIdx.x / CB;
+    // uniform address of row group m plus the thread's 32-bit offset
+    char *a = reinterpret_cast<char *>(data + (size_t)blockIdx.y * n * n + cb * CB);
+    const uint32_t off = (uint32_t)((lt * n + line) * sizeof(T2));
+    const int shm = sh / TPL;
+    auto at = [&](int m) {
+        return reinterpret_cast<T2 *>(a + (size_t)(m ^ shm) * (TPL * n * sizeof(T2)) + off);
+    };
+    fft16_line<T2, LOGN, INV>(
+        tw, lt, [&](int i) { return lds + i * CB + line; }, [&](int m) { return *at(m); },
+        [&](int m, const T2 &v) { *at(m) = v; });
 }
 
 // ---- fft shift (fft_shift_kernel, common_kernels.cuh:17-32) ------------------------
@@ -237,108 +298,97 @@ int get_stage_twiddles(rg_context *ctx, int n, int type, int sign, const void **
 
 template <typename T2, int LOGN, bool INV>
 static int rows_t(T2 *data, int64_t nrows, const T2 *tw, const uint32_t *flags,
-                  const int32_t *dev_batch, hipStream_t s)
+                  const int32_t *dev_batch, int sh, hipStream_t s)
 {
     constexpr int n = 1 << LOGN;
-    constexpr int TPL = n / 8;
-    constexpr int B = TPL >= 256 ? 1 : 256 / TPL;
-    const int64_t blocks = (nrows + B - 1) / B;
-    hipLaunchKernelGGL((k_fft_rows<T2, LOGN, B, INV>), dim3((unsigned)blocks), dim3(B * TPL), 0, s,
-                       data, nrows, tw, flags, dev_batch);
+    if constexpr (n > 512) {
+        constexpr int TPL = n / 16, NL = TPL >= 256 ? 1 : 256 / TPL;
+        hipLaunchKernelGGL((k_fft_rows16<T2, LOGN, NL, INV>),
+                           dim3((unsigned)((nrows + NL - 1) / NL)), dim3(NL * TPL), 0, s, data,
+                           nrows, tw, flags, dev_batch, sh);
+    } else {
+        constexpr int TPL = n / 8;
+        constexpr int B = 256 / TPL;
+        hipLaunchKernelGGL((k_fft_rows<T2, LOGN, B, INV>), dim3((unsigned)((nrows + B - 1) / B)),
+                           dim3(B * TPL), 0, s, data, nrows, tw, flags, dev_batch, sh);
+    }
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
 
 template <typename T2, int LOGN, bool INV>
-static int cols_t(T2 *data, int batch, const T2 *tw, const int32_t *dev_batch, hipStream_t s)
+static int cols_t(T2 *data, int batch, const T2 *tw, const int32_t *dev_batch, int sh,
+                  hipStream_t s)
 {
     constexpr int n = 1 << LOGN;
-    constexpr int CB = sizeof(T2) == 8 ? 16 : 8;
-    constexpr int cb = CB > n ? n : CB;
-    hipLaunchKernelGGL((k_fft_cols<T2, LOGN, cb, INV>), dim3(n / cb, batch), dim3(cb * (n / 8)), 0,
-                       s, data, tw, dev_batch);
+    if constexpr (n > 512) {
+        constexpr int CBW = 64 / (int)sizeof(T2);
+        constexpr int CB = CBW * (n / 16) > 1024 ? 1024 / (n / 16) : CBW;
+        hipLaunchKernelGGL((k_fft_cols16<T2, LOGN, CB, INV>), dim3(n / CB, batch),
+                           dim3(CB * (n / 16)), 0, s, data, tw, dev_batch, sh);
+    } else {
+        constexpr int CB = sizeof(T2) == 8 ? 16 : 8;
+        constexpr int cb = CB > n ? n : CB;
+        hipLaunchKernelGGL((k_fft_cols<T2, LOGN, cb, INV>), dim3(n / cb, batch),
+                           dim3(cb * (n / 8)), 0, s, data, tw, dev_batch, sh);
+    }
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
 
 template <typename T2, bool INV>
-int fft_rows_dispatch(T2 *data, int n, int64_t nrows, const T2 *tw, const uint32_t *flags,
-                      const int32_t *dev_batch, hipStream_t s)
+static int fft_rows_dispatch(T2 *data, int n, int64_t nrows, const T2 *tw, const uint32_t *flags,
+                      const int32_t *dev_batch, int sh, hipStream_t s)
 {
     switch (n) {
-    case 8: return rows_t<T2, 3, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 16: return rows_t<T2, 4, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 32: return rows_t<T2, 5, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 64: return rows_t<T2, 6, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 128: return rows_t<T2, 7, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 256: return rows_t<T2, 8, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 512: return rows_t<T2, 9, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 1024: return rows_t<T2, 10, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 2048: return rows_t<T2, 11, INV>(data, nrows, tw, flags, dev_batch, s);
-    case 4096: return rows_t<T2, 12, INV>(data, nrows, tw, flags, dev_batch, s);
+    case 8: return rows_t<T2, 3, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 16: return rows_t<T2, 4, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 32: return rows_t<T2, 5, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 64: return rows_t<T2, 6, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 128: return rows_t<T2, 7, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 256: return rows_t<T2, 8, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 512: return rows_t<T2, 9, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 1024: return rows_t<T2, 10, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 2048: return rows_t<T2, 11, INV>(data, nrows, tw, flags, dev_batch, sh, s);
+    case 4096: return rows_t<T2, 12, INV>(data, nrows, tw, flags, dev_batch, sh, s);
     default: return fail(RG_ERR_PARAM, "FFT size %d unsupported (power of two 8..4096)", n);
     }
 }
 
 template <typename T2, bool INV>
 static int fft_cols_dispatch(T2 *data, int n, int batch, const T2 *tw, const int32_t *dev_batch,
-                             hipStream_t s)
+                             int sh, hipStream_t s)
 {
     switch (n) {
-    case 8: return cols_t<T2, 3, INV>(data, batch, tw, dev_batch, s);
-    case 16: return cols_t<T2, 4, INV>(data, batch, tw, dev_batch, s);
-    case 32: return cols_t<T2, 5, INV>(data, batch, tw, dev_batch, s);
-    case 64: return cols_t<T2, 6, INV>(data, batch, tw, dev_batch, s);
-    case 128: return cols_t<T2, 7, INV>(data, batch, tw, dev_batch, s);
-    case 256: return cols_t<T2, 8, INV>(data, batch, tw, dev_batch, s);
-    case 512: return cols_t<T2, 9, INV>(data, batch, tw, dev_batch, s);
+    case 8: return cols_t<T2, 3, INV>(data, batch, tw, dev_batch, sh, s);
+    case 16: return cols_t<T2, 4, INV>(data, batch, tw, dev_batch, sh, s);
+    case 32: return cols_t<T2, 5, INV>(data, batch, tw, dev_batch, sh, s);
+    case 64: return cols_t<T2, 6, INV>(data, batch, tw, dev_batch, sh, s);
+    case 128: return cols_t<T2, 7, INV>(data, batch, tw, dev_batch, sh, s);
+    case 256: return cols_t<T2, 8, INV>(data, batch, tw, dev_batch, sh, s);
+    case 512: return cols_t<T2, 9, INV>(data, batch, tw, dev_batch, sh, s);
+    case 1024: return cols_t<T2, 10, INV>(data, batch, tw, dev_batch, sh, s);
+    case 2048: return cols_t<T2, 11, INV>(data, batch, tw, dev_batch, sh, s);
+    case 4096: return cols_t<T2, 12, INV>(data, batch, tw, dev_batch, sh, s);
     default: return fail(RG_ERR_PARAM, "column pass size %d unsupported", n);
     }
 }
 
-template int fft_rows_dispatch<float2, true>(float2 *, int, int64_t, const float2 *,
-                                             const uint32_t *, const int32_t *, hipStream_t);
-template int fft_rows_dispatch<double2, true>(double2 *, int, int64_t, const double2 *,
-                                             const uint32_t *, const int32_t *, hipStream_t);
-template int fft_rows_dispatch<float2, false>(float2 *, int, int64_t, const float2 *,
-                                             const uint32_t *, const int32_t *, hipStream_t);
-template int fft_rows_dispatch<double2, false>(double2 *, int, int64_t, const double2 *,
-                                             const uint32_t *, const int32_t *, hipStream_t);
-
 template <typename T2>
 static int fft2d_t(rg_context *ctx, T2 *data, int type, int n, int batch, int sign,
-                   const uint32_t *row_flags, const int32_t *dev_batch, hipStream_t s)
+                   const uint32_t *row_flags, const int32_t *dev_batch, bool shift, hipStream_t s)
 {
     const void *twv = nullptr;
     RG_TRY(get_twiddles(ctx, n, type, sign, &twv));
     const T2 *tw = (const T2 *)twv;
-    const bool inv = sign > 0;
     const int64_t nrows = (int64_t)n * batch;
-    if (n <= 512) {
-        if (inv) {
-            RG_TRY((fft_rows_dispatch<T2, true>(data, n, nrows, tw, row_flags, dev_batch, s)));
-            return fft_cols_dispatch<T2, true>(data, n, batch, tw, dev_batch, s);
-        }
-        RG_TRY((fft_rows_dispatch<T2, false>(data, n, nrows, tw, row_flags, dev_batch, s)));
-        return fft_cols_dispatch<T2, false>(data, n, batch, tw, dev_batch, s);
+    const int sh = shift ? n / 2 : 0;
+    if (sign > 0) {
+        RG_TRY((fft_rows_dispatch<T2, true>(data, n, nrows, tw, row_flags, dev_batch, sh, s)));
+        return fft_cols_dispatch<T2, true>(data, n, batch, tw, dev_batch, sh, s);
     }
-    // rows, transpose, rows, transpose back
-    RG_TRY(ctx->scratch[11].ensure(sizeof(T2) * (size_t)n * n * batch));
-    T2 *tmp = ctx->scratch[11].as<T2>();
-    dim3 tg(n / 32, n / 32, batch);
-    for (int pass = 0; pass < 2; ++pass) {
-        const uint32_t *flags = pass == 0 ? row_flags : nullptr;
-        if (inv)
-            RG_TRY((fft_rows_dispatch<T2, true>(data, n, nrows, tw, flags, dev_batch, s)));
-        else
-            RG_TRY((fft_rows_dispatch<T2, false>(data, n, nrows, tw, flags, dev_batch, s)));
-        hipLaunchKernelGGL(k_transpose<T2>, tg, dim3(256), 0, s, (const T2 *)data, tmp, n,
-                           dev_batch);
-        RG_HIP(hipGetLastError());
-        std::swap(data, tmp);
-    }
-    // two transposes leave the result in the original array
-    return RG_OK;
+    RG_TRY((fft_rows_dispatch<T2, false>(data, n, nrows, tw, row_flags, dev_batch, sh, s)));
+    return fft_cols_dispatch<T2, false>(data, n, batch, tw, dev_batch, sh, s);
 }
 
 int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int sign, hipStream_t s)
@@ -351,18 +401,19 @@ int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int si
     RG_TRY(get_twiddles(ctx, n, type, sign, &tw));
     if (type == RG_C128)
         return sign > 0 ? fft_rows_dispatch<double2, true>((double2 *)data, n, nrows,
-                                                           (const double2 *)tw, nullptr, nullptr, s)
+                                                           (const double2 *)tw, nullptr, nullptr, 0, s)
                         : fft_rows_dispatch<double2, false>((double2 *)data, n, nrows,
                                                             (const double2 *)tw, nullptr, nullptr,
-                                                            s);
+                                                            0, s);
     return sign > 0 ? fft_rows_dispatch<float2, true>((float2 *)data, n, nrows, (const float2 *)tw,
-                                                      nullptr, nullptr, s)
+                                                      nullptr, nullptr, 0, s)
                     : fft_rows_dispatch<float2, false>((float2 *)data, n, nrows,
-                                                       (const float2 *)tw, nullptr, nullptr, s);
+                                                       (const float2 *)tw, nullptr, nullptr, 0,
+                                                       s);
 }
 
 int fft2d(rg_context *ctx, void *data, int type, int n, int batch, int sign, hipStream_t s,
-          const uint32_t *row_flags, const int32_t *dev_batch)
+          const uint32_t *row_flags, const int32_t *dev_batch, bool shift)
 {
     if (n < 8 || n > 4096 || (n & (n - 1)))
         return fail(RG_ERR_PARAM, "FFT size %d unsupported (power of two 8..4096)", n);
@@ -370,8 +421,9 @@ int fft2d(rg_context *ctx, void *data, int type, int n, int batch, int sign, hip
         return fail(RG_ERR_PARAM, "invalid FFT batch/sign");
     if (type == RG_C128)
         return fft2d_t<double2>(ctx, (double2 *)data, type, n, batch, sign, row_flags, dev_batch,
-                                s);
-    return fft2d_t<float2>(ctx, (float2 *)data, type, n, batch, sign, row_flags, dev_batch, s);
+                                shift, s);
+    return fft2d_t<float2>(ctx, (float2 *)data, type, n, batch, sign, row_flags, dev_batch, shift,
+                          s);
 }
 
 } // namespace rg

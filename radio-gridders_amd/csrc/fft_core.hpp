@@ -129,6 +129,45 @@ template <bool INV, typename T2> __device__ inline void dft8(T2 *x)
     x[7] = csub(e3, t3);
 }
 
+// logical index -> LDS index with one pad element after every 16
+__host__ __device__ constexpr int pad16(int x) { return x + (x >> 4); }
+
+// x[0..15] -> its 16-point transform, as 4 x 4: four transforms over elements
+// 4 apart, the twiddles w16^(i k), four transforms over neighbours.  Output
+// k1 + 4 k2 is left in x[4 k1 + k2] (dft16_slot).
+constexpr int dft16_slot(int k) { return 4 * (k & 3) + (k >> 2); }
+
+template <bool INV, typename T2> __device__ inline void dft16(T2 *x)
+{
+    using T = decltype(x[0].x);
+    constexpr T c = (T)0.92387953251128675612818318939678828682241662586364; // cos(pi/8)
+    constexpr T s = (T)0.38268343236508977172845998403039886676134456248563; // sin(pi/8)
+    constexpr T h = (T)0.70710678118654752440084436210484903928483593768847;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        dft4<INV>(x[i], x[i + 4], x[i + 8], x[i + 12]); // k1 in x[i + 4 k1]
+    auto mul = [](T2 a, T re, T im) { // a (re + sign i im)
+        T2 r;
+        const T m = INV ? im : -im;
+        r.x = a.x * re - a.y * m;
+        r.y = a.x * m + a.y * re;
+        return r;
+    };
+    // w16^(i k1) at x[i + 4 k1]
+    x[5] = mul(x[5], c, s);
+    x[6] = mul(x[6], h, h);
+    x[7] = mul(x[7], s, c);
+    x[9] = mul(x[9], h, h);
+    x[10] = mul_si<INV>(x[10]);
+    x[11] = mul(x[11], -h, h);
+    x[13] = mul(x[13], s, c);
+    x[14] = mul(x[14], -h, h);
+    x[15] = mul(x[15], -c, -s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        dft4<INV>(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]); // k2 in x[4 k1 + k2]
+}
+
 // radix of the stage with current sub-transform size Ns
 template <int LOGN> __host__ __device__ constexpr int stage_radix(int logns)
 {
@@ -272,6 +311,122 @@ __device__ inline void fft_block_io(T2 *lds, const T2 *tw, Load &&load, Emit &&e
     fft_stage_io<T2, LOGN, B, LS, last_radix<LOGN, RMAX>(), INV, 2>(lds, tw, logns, load, emit);
 }
 
+// ---- 16 values per thread -----------------------------------------------------------
+// A line of n = 2^LOGN (n >= 256) by n / 16 threads, lt = 0 .. n / 16 - 1, 16 values each,
+// that stay in registers: the first stage takes its inputs from load(m), the
+// last hands its outputs to store(m, value), m = 0 .. 15 (compile-time) standing
+// for position lt + m n / 16, and between stages the values change threads
+// through LDS at at(pad16(position)).  Radix-16 stages, the last one
+// takes what is left of LOGN (16, 8, 4 or 2; 16 / R butterflies per thread).  A
+// line of FP64 values passes through LDS one component at a time (SPLIT): half the
+// space, so that twice the lines fit a workgroup.  Every thread of the workgroup takes
+// part; the caller synchronises before LDS is used again.
+template <int LOGN> __host__ __device__ constexpr int last_radix16()
+{
+    return LOGN % 4 == 0 ? 16 : (1 << (LOGN % 4));
+}
+
+template <typename T2, int LOGN, int R, bool INV>
+__device__ inline void fft16_stage(T2 *v, const T2 *__restrict__ tw, int logns, int lt)
+{
+    constexpr int n = 1 << LOGN, TPL = n / 16;
+    constexpr int LOGR = R == 16 ? 4 : R == 8 ? 3 : R == 4 ? 2 : 1;
+#pragma unroll
+    for (int q = 0; q < 16 / R; ++q) {
+        T2 *x = v + q * R;
+        if (logns > 0) {
+            const int k = (lt + q * TPL) & ((1 << logns) - 1);
+            // byte offsets below 2^32 from the table's address
+            const uint32_t tstep = (uint32_t)(k << (LOGN - logns - LOGR)) * sizeof(T2);
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                x[r] = cmul(x[r], *reinterpret_cast<const T2 *>(
+                                      reinterpret_cast<const char *>(tw) + (uint32_t)r * tstep));
+                // two twiddles at a time: more would spill in the 4096-row FP64
+                // column pass, whose 1024 threads have 128 registers (241 -> 125 us)
+                if (sizeof(T2) == 16 && r % 2 == 0)
+                    __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (R == 16)
+            dft16<INV>(x);
+        else if (R == 8)
+            dft8<INV>(x);
+        else if (R == 4)
+            dft4<INV>(x[0], x[1], x[2], x[3]);
+        else
+            dft2<INV>(x[0], x[1]);
+    }
+}
+
+template <typename T2, int LOGN, bool INV, typename At, typename Load, typename Store>
+__device__ inline void fft16_line(const T2 *__restrict__ tw, int lt, At &&at, Load &&load,
+                                  Store &&store)
+{
+    static_assert(LOGN >= 8, "at least two stages");
+    constexpr int n = 1 << LOGN, TPL = n / 16;
+    constexpr bool SPLIT = sizeof(T2) == 16;
+    constexpr int RL = last_radix16<LOGN>(), NST = LOGN / 4 + (RL < 16 ? 1 : 0);
+    T2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        v[r] = load(r);
+    fft16_stage<T2, LOGN, 16, INV>(v, tw, 0, lt);
+#pragma unroll
+    for (int st = 1; st < NST; ++st) {
+        // outputs of the radix-16 stage st - 1 to the inputs of stage st
+        const int logns = 4 * (st - 1), Ns = 1 << logns;
+        const int d = ((lt >> logns) << (logns + 4)) + (lt & (Ns - 1));
+        const bool last = st == NST - 1;
+        const int R = last ? RL : 16;
+        auto in = [&](int e) { // input index of value e of the stage
+            return lt + (e / R) * TPL + (e % R) * (n / R);
+        };
+        T2 nv[16];
+        if (st > 1)
+            __syncthreads(); // the previous exchange has been read
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                *at(pad16(d + r * Ns)) = v[dft16_slot(r)].x;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                nv[e].x = *at(pad16(in(e)));
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                *at(pad16(d + r * Ns)) = v[dft16_slot(r)].y;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                nv[e].y = *at(pad16(in(e)));
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                *at(pad16(d + r * Ns)) = v[dft16_slot(r)];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                nv[e] = *at(pad16(in(e)));
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            v[e] = nv[e];
+        if (last)
+            fft16_stage<T2, LOGN, RL, INV>(v, tw, 4 * st, lt);
+        else
+            fft16_stage<T2, LOGN, 16, INV>(v, tw, 4 * st, lt);
+    }
+    // the last stage has n / RL = Ns butterflies, 16 / RL of them this thread's:
+    // output r of butterfly lt + q n / 16 lies at lt + (q + r 16 / RL) n / 16
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int q = e / RL, r = e % RL;
+        store(q + r * (16 / RL), v[RL == 16 ? dft16_slot(r) : e]);
+    }
+}
+
 // ---- line-major variant ---------------------------------------------------------
 // Lines stored contiguously (line l at base + l * LSTR); thread t of a round
 // works on line t / TPL, position t % TPL.  `active` threads do the work, all
@@ -404,8 +559,6 @@ __device__ inline void fft_block(T2 *lds, const T2 *tw)
 // radix R holds w^(r k n / (Ns R)) for r = 1..R-1, k < Ns at
 // tws[Ns - 1 + (r - 1) Ns + k], so the lanes of a wavefront read consecutive
 // words (a plain table read at r k conflicts for even r).
-__host__ __device__ constexpr int pad16(int x) { return x + (x >> 4); }
-
 // One stage: reads src (padded, or with SRC_PAD false the row's logical
 // layout), writes row (padded); every read precedes every write (barrier).
 template <typename T2, int LOGN, int R, bool INV, bool SRC_PAD = true>

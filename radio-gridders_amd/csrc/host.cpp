@@ -447,10 +447,7 @@ int rg_grid_to_image(rg_context *ctx, void *grid, int32_t type, int32_t n, void 
     if (type != RG_C128 && type != RG_C64)
         return fail(RG_ERR_PARAM, "unknown grid type %d", type);
     RG_HIP(hipSetDevice(ctx->device));
-    hipStream_t s = (hipStream_t)stream;
-    RG_TRY(fft_shift(grid, type, n, 1, s));
-    RG_TRY(fft2d(ctx, grid, type, n, 1, +1, s));
-    return fft_shift(grid, type, n, 1, s);
+    return fft2d(ctx, grid, type, n, 1, +1, (hipStream_t)stream, nullptr, nullptr, true);
 }
 
 int rg_fft2d(rg_context *ctx, void *data, int32_t type, int32_t n, int32_t batch, int32_t sign,

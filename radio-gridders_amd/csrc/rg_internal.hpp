@@ -133,8 +133,8 @@ struct rg_context {
     // context run one after another on their stream):
     //   0-6, 15  visibility sort (binning.hpp; W-stack sort: 0-5, 7, 8, 15)
     //   7-12     W-towers batch buffers (12: the padded kernel table); 9-10
-    //            also the W-stack build's row flags / row buffer, 11 the FFT
-    //            transposes
+    //            also the W-stack build's row flags / row buffer, 11 the band
+    //            records
     //   13       channel offsets, 14 DFT, 16 uniform-weighting counts
     //   17       the W-stack, kept between calls
     //   8        W-towers floor range; 18 W-towers task tables, 19 band masks
@@ -212,9 +212,11 @@ int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int si
 // row_flags (optional): bit r set for every row r (of the n * batch rows) that
 // may be nonzero on input; the first row pass skips the others, which must be 0.
 // dev_batch (optional, device int): only the first *dev_batch <= batch arrays
-// are transformed (the launch is sized for batch).
+// are transformed (the launch is sized for batch).  shift: quadrants swapped
+// before and after the transform.
 int fft2d(rg_context *ctx, void *data, int type, int n, int batch, int sign, hipStream_t s,
-          const uint32_t *row_flags = nullptr, const int32_t *dev_batch = nullptr);
+          const uint32_t *row_flags = nullptr, const int32_t *dev_batch = nullptr,
+          bool shift = false);
 int fft_shift(void *data, int type, int n, int batch, hipStream_t s);
 int zero_fill(void *p, size_t bytes, hipStream_t s);
 int weight_vis(rg_context *ctx, const double *u, const double *v, int64_t n, void *vis,

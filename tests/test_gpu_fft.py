@@ -45,3 +45,28 @@ def test_bad_sizes_rejected(ctx):
     with pytest.raises(rgamd.RGError) as e:
         ctx.fft2d(t, 1)
     assert e.value.code == rgamd.RG_ERR_PARAM
+
+
+@pytest.mark.parametrize("n", [8, 64, 512, 1024, 2048, 4096])
+def test_grid_to_image_shift_in_the_passes(ctx, n):
+    """Quadrant swaps as index offsets of the row and column passes, in both
+    precisions, against numpy (same tolerances as the transform alone)."""
+    rng = np.random.default_rng(n + 1)
+    a = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    ref = np.fft.fftshift(np.fft.ifft2(np.fft.fftshift(a)) * n * n)
+    for dt, tol in ((torch.complex128, 1e-13 * np.log2(n) * 4), (torch.complex64,
+                                                                 2e-6 * np.log2(n))):
+        t = dev(a).to(dt)
+        ctx.grid_to_image(t)
+        torch.cuda.synchronize()
+        assert rel_max(t.cpu().numpy(), ref) < tol
+
+
+def test_batch_of_long_transforms(ctx):
+    n, batch = 1024, 3
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((batch, n, n)) + 1j * rng.standard_normal((batch, n, n))
+    t = dev(a)
+    ctx.fft2d(t, -1)
+    torch.cuda.synchronize()
+    assert rel_max(t.cpu().numpy(), np.fft.fft2(a)) < 1e-13 * 40

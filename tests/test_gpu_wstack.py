@@ -253,3 +253,22 @@ def test_empty_and_all_dropped_streams(ctx, kernels):
     assert torch.all(out == 0)
     st = ctx.stats()
     assert st.n_vis == nv and st.n_dropped == nv and st.n_gridded == 0
+
+
+@pytest.mark.parametrize("lam", [5120.0, 10240.0])
+def test_dense_sky_with_long_rows(ctx, kernels, lam):
+    """More sources than the sparse form takes, on planes of 1024 and 2048: the
+    row pass of long lines skips the rows without a source."""
+    theta = 0.1
+    h, d = kernels["host"], kernels["desc"]
+    rng = np.random.default_rng(31)
+    ns = 90
+    l = rng.uniform(-0.45 * theta, 0.45 * theta, ns)
+    m = rng.uniform(-0.1 * theta, 0.1 * theta, ns)
+    flux = rng.uniform(0.1, 1.0, ns)
+    stack, _ = orc.wstack_build(theta, lam, l, m, flux, h["uv"].du, h["w"].dw, h["w"].size,
+                                h["lm"].x0, h["lm"].data, h["n"].data)
+    og, wp, _ = ctx.wstack_build(params(kernels, theta, lam), dev(l), dev(m), dev(flux), d["lm"],
+                                 d["n"])
+    assert (og, wp) == (stack.shape[1], stack.shape[0])
+    assert np.abs(ctx.wstack_stack(og, wp) - stack).max() < 1e-11 * np.abs(stack).max()
