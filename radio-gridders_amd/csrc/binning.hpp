@@ -5,10 +5,9 @@
 //   count   : wave-aggregated atomics on count[rep][key]; each visibility
 //             keeps the counter value it got (its rank inside the replica's
 //             share of the key) with its key, position and tap index
-//   scan    : three-phase exclusive scan of (count, ceil(count / K)), where
-//             count[key] is the sum over the replicas, then the start of
-//             every replica's share of every key
-//   items   : one work item per K records of a key
+//   scan    : exclusive scan of (count, ceil(count / K)), where count[key] is
+//             the sum over the replicas, then the start of every replica's
+//             share of every key and one work item per K records of a key
 //   scatter : record i written at start[rep][key] + rank (no atomics)
 // Chunk c of BIN_CHUNK visibilities uses counter replica rep = c mod NREP.
 // Device-scope atomics on one address serialise, and a few keys (the
@@ -20,14 +19,14 @@
 // the W-projection Romein accumulation relies on).
 #pragma once
 
+#include <algorithm>
+
 #include "rg_internal.hpp"
 
 namespace rg {
 
 constexpr int SCAN_BLOCK = 256;
-constexpr int SCAN_PER_THREAD = 4; // 1024 keys per block: W-towers key spaces of ~1 M keys
-                                   // give ~1000 blocks, enough to fill the CUs
-constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_PER_THREAD; // keys per scan block
+constexpr int SCAN_DIRECT = 2048; // scan blocks that add up the totals before them themselves
 
 struct Item {
     uint32_t key;
@@ -185,20 +184,132 @@ __global__ __launch_bounds__(BIN_TB) void k_bin_scatter(Keyer kf, int64_t n,
     }
 }
 
-// Phase 1: per-block totals of (count, items).
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const uint32_t *count, Replicas rp,
-                                                            int64_t nkeys, uint32_t per_item,
-                                                            uint2 *block_sums);
-// Phase 2: exclusive scan of block totals (single block), totals to stats.
-__global__ __launch_bounds__(1024) void k_scan_blocks(uint2 *block_sums, int nblocks,
-                                                      unsigned long long *stats);
-// Phase 3: per-key starts, work items and the scatter cursors of every replica.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(const uint32_t *count, Replicas rp,
-                                                          int64_t nkeys, uint32_t per_item,
-                                                          const uint2 *block_sums,
-                                                          uint32_t *vis_start,
-                                                          uint32_t *item_start, uint32_t *cursor,
-                                                          Item *items);
+// ---- short streams -------------------------------------------------------------------
+// Up to BIN_SMALL visibilities over at most BIN_SMALL_KEYS keys are sorted by
+// one workgroup with its counters in LDS: one launch instead of a clear, a
+// count, two scans and a scatter, whose latencies are all there is to a short
+// call (448 visibilities, 25 keys: 31 us -> one launch of about 8 us).
+constexpr int BIN_SMALL_VPT = 4;
+constexpr int BIN_SMALL_KPT = 8;
+constexpr int BIN_SMALL = 1024 * BIN_SMALL_VPT;
+constexpr int BIN_SMALL_KEYS = 1024 * BIN_SMALL_KPT;
+
+template <typename Keyer, typename T>
+__global__ __launch_bounds__(1024) void k_bin_small(Keyer kf, int n, int nkeys, uint32_t per_item,
+                                                    uint32_t *vis_start, uint32_t *item_start,
+                                                    Item *items, Rec<T> *recs,
+                                                    unsigned long long *stats)
+{
+    __shared__ uint32_t cnt[BIN_SMALL_KEYS];
+    __shared__ uint2 wtot[16];
+    __shared__ uint32_t s_stat[3];
+    for (int k = threadIdx.x; k < nkeys; k += 1024)
+        cnt[k] = 0;
+    if (threadIdx.x < 3)
+        s_stat[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t key[BIN_SMALL_VPT], rank[BIN_SMALL_VPT];
+    Rec<T> rec[BIN_SMALL_VPT];
+#pragma unroll
+    for (int q = 0; q < BIN_SMALL_VPT; ++q) {
+        const int i = q * 1024 + (int)threadIdx.x;
+        key[q] = KEY_NONE;
+        if (i < n) {
+            uint32_t k = 0, pos = 0, kidx = 0;
+            const int st = kf.classify(i, k, pos, kidx);
+            if (st == VIS_OK) {
+                key[q] = k;
+                rank[q] = atomicAdd(&cnt[k], 1u);
+                rec[q].pos = pos;
+                rec[q].kidx = kidx;
+                rec[q].vis = kf.template vis_value<T>(i);
+            } else {
+                atomicAdd(&s_stat[st == VIS_BAD_PLANE ? 1 : 0], 1u);
+                if (st == VIS_OVERFLOW)
+                    atomicAdd(&s_stat[2], 1u);
+            }
+        }
+    }
+    __syncthreads();
+    // exclusive scan of (records, items) over the keys, BIN_SMALL_KPT per thread
+    const int k0 = (int)threadIdx.x * BIN_SMALL_KPT;
+    const int lane = __lane_id(), wv = threadIdx.x / 64;
+    uint2 acc = make_uint2(0, 0);
+    uint32_t c[BIN_SMALL_KPT];
+#pragma unroll
+    for (int j = 0; j < BIN_SMALL_KPT; ++j) {
+        c[j] = k0 + j < nkeys ? cnt[k0 + j] : 0u;
+        acc.x += c[j];
+        acc.y += (c[j] + per_item - 1) / per_item;
+    }
+    uint2 inc = acc;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t x = (uint32_t)__shfl_up((int)inc.x, o);
+        const uint32_t y = (uint32_t)__shfl_up((int)inc.y, o);
+        if (lane >= o) {
+            inc.x += x;
+            inc.y += y;
+        }
+    }
+    if (lane == 63)
+        wtot[wv] = inc;
+    __syncthreads();
+    uint2 run = make_uint2(inc.x - acc.x, inc.y - acc.y), total = make_uint2(0, 0);
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const uint2 t = wtot[w];
+        if (w < wv) {
+            run.x += t.x;
+            run.y += t.y;
+        }
+        total.x += t.x;
+        total.y += t.y;
+    }
+#pragma unroll
+    for (int j = 0; j < BIN_SMALL_KPT; ++j) {
+        const int k = k0 + j;
+        if (k < nkeys) {
+            cnt[k] = run.x;
+            vis_start[k] = run.x;
+            item_start[k] = run.y;
+            for (uint32_t b = 0; b < c[j]; b += per_item) {
+                Item it;
+                it.key = (uint32_t)k;
+                it.start = run.x + b;
+                it.count = min(per_item, c[j] - b);
+                items[run.y++] = it;
+            }
+            run.x += c[j];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < BIN_SMALL_VPT; ++q)
+        if (key[q] != KEY_NONE)
+            recs[cnt[key[q]] + rank[q]] = rec[q];
+    if (threadIdx.x == 0) {
+        vis_start[nkeys] = total.x;
+        item_start[nkeys] = total.y;
+        stats[CNT_RECORDS] = total.x;
+        stats[CNT_ITEMS] = total.y;
+        stats[CNT_DROPPED] = s_stat[0];
+        stats[CNT_BAD_PLANE] = s_stat[1];
+        stats[CNT_OVERFLOW] += s_stat[2];
+    }
+}
+
+// Starts, items and (cursor not NULL) the replicas' scatter cursors of the
+// counted keys; totals to the call counters.  bsums holds scan_blocks(nkeys) + 1
+// entries.
+int64_t scan_blocks(int64_t nkeys);
+// Space for the scan blocks' sums of any call with up to nkeys keys (their
+// number drops where a thread takes more keys): scratch that a captured graph
+// holds then serves every smaller call.
+size_t scan_sums_bytes(int64_t nkeys);
+int scan_keys(const uint32_t *count, Replicas rp, int64_t nkeys, uint32_t per_item, uint2 *bsums,
+              uint32_t *vis_start, uint32_t *item_start, uint32_t *cursor, Item *items,
+              unsigned long long *stats, hipStream_t s);
 
 // Host driver for count + scan + items + scatter.
 struct BinResult {
@@ -224,7 +335,7 @@ enum BinArray {
 
 struct BinPlan {
     Replicas rp;
-    int64_t nblocks_scan, max_items;
+    int64_t max_items;
     size_t bytes[BIN__N];
 };
 
@@ -241,14 +352,17 @@ struct BinBufs {
 int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, size_t rec_bytes,
              BinPlan &pl);
 // The sort into caller-provided arrays of the plan's sizes; timer_ctx (may be
-// NULL) receives the RG_TIMER_BINNING events.
+// NULL) receives the RG_TIMER_BINNING events.  The areas of `zero` are cleared
+// before the sort, in one launch with the counters it needs cleared.
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, rg_context *timer_ctx, hipStream_t s, BinResult &out);
+            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s,
+            BinResult &out);
 // bin_run into the context's scratch slots 0-6 and 15.
 template <typename Keyer, typename T>
 int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
-                     hipStream_t s, BinResult &out, int64_t max_counters = (int64_t)1 << 22);
+                     ZeroList &zero, hipStream_t s, BinResult &out,
+                     int64_t max_counters = (int64_t)1 << 22);
 
 // Work items over per-key lengths len[0..nkeys): prefix[k] = exclusive sum of
 // len, item_start[k] = first item of key k (both nkeys + 1 entries), items of

@@ -2,54 +2,65 @@
 // per translation unit that instantiates bin_visibilities).
 #pragma once
 
+#include <algorithm>
+
 #include "binning.hpp"
 
 namespace rg {
 
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, rg_context *timer_ctx, hipStream_t s, BinResult &out)
+            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s, BinResult &out)
 {
     const Replicas rp = pl.rp;
+    out.vis_start = b.vis_start;
+    out.item_start = b.item_start;
+    out.items = b.items;
+    out.recs = b.recs;
+    out.max_items = pl.max_items;
+    const bool small = n <= BIN_SMALL && nkeys <= BIN_SMALL_KEYS;
+    if (!small)
+        RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
+    RG_TRY(zero.launch(s));
     KernelTimer kt(timer_ctx, RG_TIMER_BINNING, s);
-    RG_TRY(zero_fill(b.count, pl.bytes[BIN_COUNT], s));
+    if (small) {
+        hipLaunchKernelGGL((k_bin_small<Keyer, T>), dim3(1), dim3(1024), 0, s, kf, (int)n,
+                           (int)nkeys, per_item, b.vis_start, b.item_start, b.items,
+                           (Rec<T> *)b.recs, b.stats);
+        RG_HIP(hipGetLastError());
+        return RG_OK;
+    }
 
     const int64_t nb = (n + BIN_CHUNK - 1) / BIN_CHUNK;
     if (nb > 0)
         hipLaunchKernelGGL((k_bin_count<Keyer>), dim3((unsigned)nb), dim3(BIN_TB), 0, s, kf, n,
                            b.count, rp, b.krp, b.stats);
     RG_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)pl.nblocks_scan), dim3(SCAN_BLOCK), 0, s,
-                       (const uint32_t *)b.count, rp, nkeys, per_item, b.bsums);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, b.bsums, (int)pl.nblocks_scan,
-                       b.stats);
-    hipLaunchKernelGGL(k_scan_down, dim3((unsigned)pl.nblocks_scan), dim3(SCAN_BLOCK), 0, s,
-                       (const uint32_t *)b.count, rp, nkeys, per_item, (const uint2 *)b.bsums,
-                       b.vis_start, b.item_start, b.cursor, b.items);
-    RG_HIP(hipGetLastError());
+    RG_TRY(scan_keys(b.count, rp, nkeys, per_item, b.bsums, b.vis_start, b.item_start, b.cursor,
+                     b.items, b.stats, s));
     if (nb > 0)
         hipLaunchKernelGGL((k_bin_scatter<Keyer, T>), dim3((unsigned)nb), dim3(BIN_TB), 0, s, kf, n,
                            (const uint32_t *)b.cursor, rp, (const uint4 *)b.krp,
                            (Rec<T> *)b.recs);
     RG_HIP(hipGetLastError());
-
-    out.vis_start = b.vis_start;
-    out.item_start = b.item_start;
-    out.items = b.items;
-    out.recs = b.recs;
-    out.max_items = pl.max_items;
     return RG_OK;
 }
 
 template <typename Keyer, typename T>
 int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
-                     hipStream_t s, BinResult &out, int64_t max_counters)
+                     ZeroList &zero, hipStream_t s, BinResult &out, int64_t max_counters)
 {
     BinPlan pl;
     RG_TRY(bin_plan(n, nkeys, per_item, max_counters, sizeof(Rec<T>), pl));
     RG_TRY(ensure_counters(ctx));
     // context scratch slots of the sort (rg_internal.hpp)
     static const int slot[BIN__N] = {0, 1, 2, 3, 4, 5, 6, 15};
+    // items and scan sums: room for every call of up to this many visibilities
+    // and keys, whatever item size it picks (scratch that a captured graph holds
+    // cannot grow)
+    const int64_t room = nkeys + std::max<int64_t>(n / per_item, std::max<int64_t>(700, n / 512)) + 1;
+    pl.bytes[BIN_ITEMS] = std::max(pl.bytes[BIN_ITEMS], sizeof(Item) * (size_t)room);
+    pl.bytes[BIN_BSUMS] = scan_sums_bytes(nkeys);
     for (int k = 0; k < BIN__N; ++k)
         RG_TRY(ctx->scratch[slot[k]].ensure(pl.bytes[k]));
     BinBufs b;
@@ -62,7 +73,7 @@ int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys,
     b.bsums = ctx->scratch[slot[BIN_BSUMS]].as<uint2>();
     b.krp = ctx->scratch[slot[BIN_KRP]].as<uint4>();
     b.stats = ctx->counters.as<unsigned long long>();
-    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, ctx, s, out);
+    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, zero, ctx, s, out);
 }
 
 } // namespace rg

@@ -378,21 +378,31 @@ static int grid_common(rg_context *ctx, const rg_grid_params *p, const rg_flat_v
     const bool capturing = cap == hipStreamCaptureStatusActive;
     if (capturing)
         ctx->frozen = true; // the graph will hold this context's scratch addresses
-    RG_TRY(zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s));
+    // batched W-projection clears the counters with its grids
+    const bool counters_later = p->subgrid_size == 0 && p->mode == RG_MODE_BATCHED;
+    if (!counters_later)
+        RG_TRY(zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s));
     ctx->last_stream = s;
     ctx->last_nvis = vis->n;
     if (p->mode == RG_MODE_PLAIN && n_chan != 1)
         return fail(RG_ERR_UNSUPPORTED, "plain mode grids one channel per call");
     const int64_t *d_off = nullptr;
-    RG_TRY(channel_offsets(ctx, offsets, n_chan, s, &d_off));
+    int st = channel_offsets(ctx, offsets, n_chan, s, &d_off);
+    if (st == RG_OK && counters_later) {
+        ctx->last_kind = 1;
+        st = wproj_batched(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s);
+    }
+    if (counters_later) {
+        if (st != RG_OK) // a refused call leaves cleared counters
+            (void)zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s);
+        return st;
+    }
+    RG_TRY(st);
     if (p->subgrid_size == 0) {
         ctx->last_kind = 1;
-        if (p->mode == RG_MODE_PLAIN) {
-            if (grid_type != RG_C128)
-                return fail(RG_ERR_PARAM, "plain mode writes an RG_C128 grid");
-            return wproj_plain(ctx, p, vis, wk, grid, s);
-        }
-        return wproj_batched(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s);
+        if (grid_type != RG_C128)
+            return fail(RG_ERR_PARAM, "plain mode writes an RG_C128 grid");
+        return wproj_plain(ctx, p, vis, wk, grid, s);
     }
     ctx->last_kind = 2;
     return wtowers_run(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s, capturing);

@@ -219,6 +219,16 @@ int fft2d(rg_context *ctx, void *data, int type, int n, int batch, int sign, hip
           bool shift = false);
 int fft_shift(void *data, int type, int n, int batch, hipStream_t s);
 int zero_fill(void *p, size_t bytes, hipStream_t s);
+// Areas (16-byte aligned) cleared by one kernel launch: graph-capturable, no
+// memset nodes.  launch() empties the list.
+struct ZeroList {
+    static constexpr int MAX = 6;
+    void *p[MAX];
+    size_t bytes[MAX];
+    int n = 0;
+    int add(void *q, size_t nbytes);
+    int launch(hipStream_t s);
+};
 int weight_vis(rg_context *ctx, const double *u, const double *v, int64_t n, void *vis,
                int vis_type, int N, double theta, uint32_t *counts, hipStream_t s);
 int make_hermitian(void *grid, int type, int n, hipStream_t s);

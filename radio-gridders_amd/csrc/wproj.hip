@@ -20,31 +20,52 @@ namespace rg {
 
 // ---- zero fill (graph-capturable, no memset nodes) ---------------------------
 
-__global__ void k_zero(uint4 *p, size_t n16, unsigned char *tail, size_t ntail)
+// Every workgroup takes its share of each area, 16 bytes per store.
+__global__ __launch_bounds__(256) void k_zero(ZeroList z)
 {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride)
-        p[i] = make_uint4(0, 0, 0, 0);
-    if (blockIdx.x == 0 && threadIdx.x < ntail)
-        tail[threadIdx.x] = 0;
+    for (int k = 0; k < z.n; ++k) {
+        uint4 *p = reinterpret_cast<uint4 *>(z.p[k]);
+        const size_t n16 = z.bytes[k] / 16, tail = z.bytes[k] % 16;
+        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride)
+            p[i] = make_uint4(0, 0, 0, 0);
+        if (blockIdx.x == 0 && threadIdx.x < tail)
+            reinterpret_cast<unsigned char *>(p + n16)[threadIdx.x] = 0;
+    }
+}
+
+int ZeroList::add(void *q, size_t nbytes)
+{
+    if (nbytes == 0)
+        return RG_OK;
+    if (((uintptr_t)q & 15) != 0)
+        return fail(RG_ERR_PARAM, "zero_fill: pointer not 16-byte aligned");
+    if (n == MAX)
+        return fail(RG_ERR_PARAM, "zero_fill: too many areas");
+    p[n] = q;
+    bytes[n++] = nbytes;
+    return RG_OK;
+}
+
+int ZeroList::launch(hipStream_t s)
+{
+    size_t most = 0;
+    for (int k = 0; k < n; ++k)
+        most = std::max(most, bytes[k]);
+    if (most == 0)
+        return RG_OK;
+    const size_t blocks = std::max<size_t>(1, std::min<size_t>((most / 16 + 255) / 256, 8192));
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)blocks), dim3(256), 0, s, *this);
+    RG_HIP(hipGetLastError());
+    n = 0;
+    return RG_OK;
 }
 
 int zero_fill(void *p, size_t bytes, hipStream_t s)
 {
-    if (bytes == 0)
-        return RG_OK;
-    if (((uintptr_t)p & 15) != 0)
-        return fail(RG_ERR_PARAM, "zero_fill: pointer not 16-byte aligned");
-    const size_t n16 = bytes / 16, ntail = bytes % 16;
-    size_t blocks = (n16 + 255) / 256;
-    if (blocks > 8192)
-        blocks = 8192;
-    if (blocks == 0)
-        blocks = 1;
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)blocks), dim3(256), 0, s, (uint4 *)p, n16,
-                       (unsigned char *)p + n16 * 16, ntail);
-    RG_HIP(hipGetLastError());
-    return RG_OK;
+    ZeroList z;
+    RG_TRY(z.add(p, bytes));
+    return z.launch(s);
 }
 
 // ---- plain FP64 Romein (reference launch structure) ---------------------------
@@ -265,7 +286,26 @@ struct WprojShape {
     uint32_t per_item;
 };
 
-static int wproj_shape(const rg_grid_params *p, const rg_wkern *wk, WprojShape &sh)
+// Records per work item when the caller leaves it open.  A workgroup walks its
+// item's records one after another (about 0.1 us each), so a stream is cut
+// into about 350 to 700 items, which fills the CUs without flushing a tile for a
+// handful of records; long streams take larger items, up to the size at which
+// the longest item still hides behind the others.  Tile time, FP64, 32-cell tiles:
+// 448 visibilities 32 us in items of 2048, 10 us in items of 32; 90 k 167 -> 53
+// us (2048 -> 256; 64: 61); 520 k, FP32, 186 -> 117 us (2048 -> 1024; 256: 135);
+// 64 channels, 4.2 M: 907 -> 845 us (2048 -> 512; 256: 968); 48-cell tiles, 8.4 M: 1539
+// us at 2048, 1689 at 1024.
+static uint32_t default_item(int64_t nvis, int n_chan, int tile)
+{
+    const uint32_t cap = n_chan > 1 ? 512 : tile == 48 ? 2048 : 1024;
+    uint32_t k = 32;
+    while (k < cap && (int64_t)k * 700 <= nvis)
+        k *= 2;
+    return k;
+}
+
+static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const rg_wkern *wk,
+                       WprojShape &sh)
 {
     const int S = wk->size;
     sh.tile = p->tile > 0 ? p->tile : 32;
@@ -275,7 +315,8 @@ static int wproj_shape(const rg_grid_params *p, const rg_wkern *wk, WprojShape &
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection supports kernel sizes 8 and 16 (got %d)", S);
     sh.ntx = (p->grid_size + S + sh.tile - 1) / sh.tile;
     sh.ntiles = sh.ntx * sh.ntx;
-    sh.per_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item : 2048u;
+    sh.per_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item
+                                      : default_item(nvis, n_chan, sh.tile);
     return RG_OK;
 }
 
@@ -312,16 +353,19 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
 {
     const int N = p->grid_size;
     WprojShape sh;
-    RG_TRY(wproj_shape(p, wk, sh));
+    RG_TRY(wproj_shape(p, vis->n, n_chan, wk, sh));
 
+    // the call's counters, the grids and the sort's counters in one launch
     const size_t gbytes = (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N * n_chan;
-    RG_TRY(zero_fill(grid, gbytes, s));
+    ZeroList zero;
+    RG_TRY(zero.add(ctx->counters.p, sizeof(unsigned long long) * CNT__N));
+    RG_TRY(zero.add(grid, gbytes));
 
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
     RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, (int64_t)sh.ntiles * n_chan,
-                                            sh.per_item, s, br)));
+                                            sh.per_item, zero, s, br)));
     return dispatch_tiles<T>(br, ctx, ctx->counters.as<unsigned long long>(), wk, grid, grid_type,
                              p->compensated != 0, N, sh.tile, sh.ntx, sh.ntiles, s);
 }
@@ -376,22 +420,36 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
 {
     const int N = p->grid_size;
     WprojShape sh;
-    RG_TRY(wproj_shape(p, wk, sh));
+    RG_TRY(wproj_shape(p, vis->n, 1, wk, sh));
     BinPlan pl;
     RG_TRY(bin_plan(vis->n, sh.ntiles, sh.per_item, (int64_t)1 << 22, sizeof(Rec<T>), pl));
-    // carve the arrays from the static scratch, 256-byte aligned
-    size_t off[BIN__N + 1];
-    size_t at = (sizeof(unsigned long long) * CNT__N + 255) / 256 * 256; // call counters first
+    // Carve the arrays from the static scratch, 256-byte aligned.  The scatter
+    // cursors take the place of the counters they are made from; the space this leaves
+    // covers the shorter default work items and scan blocks of small calls, so
+    // the limit on the stream is that of separate cursors, items of 2048
+    // records and scan blocks of 1024 keys.
+    auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t head = aligned(sizeof(unsigned long long) * CNT__N); // call counters first
+    const int64_t limit_item = p->vis_per_item > 0 ? p->vis_per_item : 2048;
+    size_t off[BIN__N];
+    size_t at = head, want = head;
     for (int k = 0; k < BIN__N; ++k) {
-        off[k] = at;
-        at += (pl.bytes[k] + 255) / 256 * 256;
+        if (k == BIN_CURSOR) {
+            off[k] = off[BIN_COUNT];
+        } else {
+            off[k] = at;
+            at += aligned(pl.bytes[k]);
+        }
+        want += aligned(
+            k == BIN_ITEMS ? sizeof(Item) * (size_t)(sh.ntiles + vis->n / limit_item + 1)
+            : k == BIN_BSUMS ? sizeof(uint2) * (size_t)((sh.ntiles + 1023) / 1024 + 1)
+                             : pl.bytes[k]);
     }
-    off[BIN__N] = at;
-    if (at > NOALLOC_SCRATCH_BYTES)
+    if (want > NOALLOC_SCRATCH_BYTES || at > NOALLOC_SCRATCH_BYTES)
         return fail(RG_ERR_PARAM,
                     "rg_grid_noalloc: %lld visibilities on a %d^2 grid need %zu bytes of scratch; "
                     "the static scratch holds %zu: split the stream over calls with accumulate = 1",
-                    (long long)vis->n, N, at, NOALLOC_SCRATCH_BYTES);
+                    (long long)vis->n, N, want, NOALLOC_SCRATCH_BYTES);
     void *base = nullptr;
     RG_TRY(noalloc_scratch(&base));
     char *b0 = static_cast<char *>(base);
@@ -406,15 +464,17 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     b.bsums = reinterpret_cast<uint2 *>(b0 + off[BIN_BSUMS]);
     b.krp = reinterpret_cast<uint4 *>(b0 + off[BIN_KRP]);
     // the previous call's counters are still there: start from zero
-    RG_TRY(zero_fill(b.stats, sizeof(unsigned long long) * CNT__N, s));
+    ZeroList zero;
+    RG_TRY(zero.add(b.stats, sizeof(unsigned long long) * CNT__N));
     if (!accumulate)
-        RG_TRY(zero_fill(grid, (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N, s));
+        RG_TRY(zero.add(grid, (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N));
     if (vis->n == 0)
-        return RG_OK;
+        return zero.launch(s);
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
-    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.ntiles, sh.per_item, pl, b, nullptr, s, br)));
+    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.ntiles, sh.per_item, pl, b, zero, nullptr, s,
+                                   br)));
     return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N,
                              sh.tile, sh.ntx, sh.ntiles, s);
 }

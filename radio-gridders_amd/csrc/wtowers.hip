@@ -1651,7 +1651,8 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
     const TowerKeyer kf = wt_keyer(p, vis, wk, g, d_range, nwp, nullptr);
     const int64_t nslots = (int64_t)cc * cc * nwp;
     BinResult br;
-    RG_TRY((bin_visibilities<TowerKeyer, double>(ctx, kf, vis->n, nslots, 0x40000000u, s, br,
+    ZeroList zero;
+    RG_TRY((bin_visibilities<TowerKeyer, double>(ctx, kf, vis->n, nslots, 0x40000000u, zero, s, br,
                                                  (int64_t)1 << 20)));
     RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (2 * nslots + 1)));
     uint32_t *d_nvis = ctx->scratch[9].as<uint32_t>();
@@ -1829,7 +1830,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     BinResult br;
     // (task, band) keys: 4 counter replicas at the reference's workload (the
     // scans read every replica; 16 were slower, 1 << 20 counters in all)
-    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, 0x40000000u, s, br,
+    ZeroList zero;
+    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, 0x40000000u, zero, s, br,
                                             (int64_t)1 << 20)));
 
     // capacities: tables by the slot count, buffers by the plan (or, measuring,

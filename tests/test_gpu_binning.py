@@ -1,0 +1,124 @@
+"""The visibility sort at the edges of its forms: the one-workgroup sort of
+short streams, scan blocks of one and four keys per thread, the two- and
+three-launch scans, hot keys with many work items."""
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as orc
+import rgamd
+from gpu_util import dev, kern, rel_max, stage
+
+pytestmark = pytest.mark.gpu
+
+THETA, S, R = 0.1, 8, 4
+
+
+@pytest.fixture(scope="module")
+def table():
+    return rgamd.make_wkernels(11, R, S, THETA, -5.0, 1.0)
+
+
+def stream(n, half, wmax, seed):
+    rng = np.random.default_rng(seed)
+    return (rng.uniform(-half, half, n), rng.uniform(-half, half, n), rng.uniform(-wmax, wmax, n),
+            rng.standard_normal(n) + 1j * rng.standard_normal(n))
+
+
+@pytest.mark.parametrize("n", [0, 1, 31, 33, 1025, 4095, 4096, 4097, 23_000])
+@pytest.mark.parametrize("per_item", [0, 5])
+def test_wprojection_hot_tile(ctx, table, n, per_item):
+    """Visibilities of a few tiles, some outside the table's planes: FP64 sums
+    of at most 23 000 terms of order 0.1 against the oracle's."""
+    N = 128
+    u, v, w, vis = stream(n, 60.0, 6.0, n + 1)
+    ref, _, bad = orc.grid_wprojection(N, THETA, u, v, w, vis, table, -5.0, 1.0)
+    _, fv = stage(u, v, w, vis)
+    _, wk = kern(table, -5.0, 1.0)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    p = rgamd.params(N, THETA, vis_per_item=per_item)
+    ctx.grid(p, fv, wk, g)
+    st = ctx.stats()
+    assert st.n_bad_plane == bad and st.n_gridded == n - bad and st.n_dropped == 0
+    assert st.n_records == n - bad
+    assert np.abs(g.cpu().numpy() - ref).max() <= 1e-12 * max(np.abs(ref).max(), 1e-300)
+    g2 = torch.zeros_like(g)
+    rgamd.grid_noalloc(p, fv, wk, g2)
+    torch.cuda.synchronize()
+    assert rel_max(g2.cpu().numpy(), ref) <= 1e-12 or n == 0
+
+
+@pytest.mark.parametrize("nchan", [3, 60, 70])
+def test_channels_across_scan_forms(ctx, table, nchan):
+    """1089 keys per channel: below and above the 65 536 keys at which a scan
+    thread takes four."""
+    N = 1024
+    counts = np.random.default_rng(nchan).integers(0, 300, nchan)
+    counts[1] = 0
+    counts[2] = 5000
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    u, v, w, vis = stream(off[-1], 4500.0, 5.0, 9)
+    (du, dv, dw, dvis), fv = stage(u, v, w, vis)
+    _, wk = kern(table, -5.0, 1.0)
+    p = rgamd.params(N, THETA)
+    g = torch.empty((nchan, N, N), dtype=torch.complex128, device="cuda")
+    ctx.grid_channels(p, fv, off, wk, g)
+    assert ctx.stats().n_gridded == off[-1]
+    one = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    for c in (0, 1, 2, nchan - 1):
+        a, b = off[c], off[c + 1]
+        fc = rgamd.flat_vis(du[a:b].clone(), dv[a:b].clone(), dw[a:b].clone(), dvis[a:b].clone())
+        ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN), fc, wk, one)
+        torch.cuda.synchronize()
+        scale = max(float(one.abs().max()), 1e-300)
+        assert float((g[c] - one).abs().max()) <= 1e-12 * scale
+
+
+def test_wtowers_with_millions_of_keys(ctx, table):
+    """2500 floors of 121 towers: over 2048 scan blocks, whose totals a launch
+    of their own scans."""
+    N = 512
+    u, v, w, vis = stream(300, 2400.0, 12_000.0, 5)
+    _, fv = stage(u, v, w, vis)
+    _, wk = kern(table, -5.0, 1.0)
+    kw = dict(subgrid=64, margin=16, winc=10.0)
+    ref = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    g = torch.empty_like(ref)
+    ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN, **kw), fv, wk, ref)
+    for _ in range(2):  # the measuring call, then one by its plan
+        ctx.grid(rgamd.params(N, THETA, **kw), fv, wk, g)
+        torch.cuda.synchronize()
+        assert float((g - ref).abs().max()) <= 1e-11 * float(ref.abs().max())
+
+
+def test_short_call_on_a_frozen_context(table):
+    """Scratch held by a captured graph serves shorter calls, which pick other
+    item sizes."""
+    c = rgamd.Context(0)
+    N = 128
+    _, wk = kern(table, -5.0, 1.0)
+    keep = [stage(*stream(n, 60.0, 4.0, n)) for n in (60_000, 30_000, 4096, 10)]
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    p = rgamd.params(N, THETA)
+    c.grid(p, keep[0][1], wk, g)
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        c.grid(p, keep[0][1], wk, g)
+    want = torch.empty_like(g)
+    for _, fv in keep:
+        c.grid(p, fv, wk, g)
+        ctx2 = rgamd.Context(0)
+        ctx2.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN), fv, wk, want)
+        torch.cuda.synchronize()
+        assert float((g - want).abs().max()) <= 1e-12 * float(want.abs().max())
+        ctx2.close()
+    c.grid(p, keep[0][1], wk, want)
+    for _ in range(3):
+        g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((g - want).abs().max()) <= 1e-12 * float(want.abs().max())
+    del graph
+    c.close()
