@@ -193,11 +193,16 @@ constexpr int BIN_SMALL_VPT = 4;
 constexpr int BIN_SMALL_KPT = 8;
 constexpr int BIN_SMALL = 1024 * BIN_SMALL_VPT;
 constexpr int BIN_SMALL_KEYS = 1024 * BIN_SMALL_KPT;
+inline bool bin_small(int64_t n, int64_t nkeys)
+{
+    return n <= BIN_SMALL && nkeys <= BIN_SMALL_KEYS;
+}
 
 template <typename Keyer, typename T>
 __global__ __launch_bounds__(1024) void k_bin_small(Keyer kf, int n, int nkeys, uint32_t per_item,
                                                     uint32_t *vis_start, uint32_t *item_start,
                                                     Item *items, Rec<T> *recs,
+                                                    uint32_t *group_start, int group_keys,
                                                     unsigned long long *stats)
 {
     __shared__ uint32_t cnt[BIN_SMALL_KEYS];
@@ -271,6 +276,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(Keyer kf, int n, int nkeys, 
         const int k = k0 + j;
         if (k < nkeys) {
             cnt[k] = run.x;
+            if (group_start && (k & (group_keys - 1)) == 0)
+                group_start[k / group_keys] = run.x;
             vis_start[k] = run.x;
             item_start[k] = run.y;
             for (uint32_t b = 0; b < c[j]; b += per_item) {
@@ -290,6 +297,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(Keyer kf, int n, int nkeys, 
             recs[cnt[key[q]] + rank[q]] = rec[q];
     if (threadIdx.x == 0) {
         vis_start[nkeys] = total.x;
+        if (group_start)
+            group_start[nkeys / group_keys] = total.x;
         item_start[nkeys] = total.y;
         stats[CNT_RECORDS] = total.x;
         stats[CNT_ITEMS] = total.y;
@@ -302,14 +311,17 @@ __global__ __launch_bounds__(1024) void k_bin_small(Keyer kf, int n, int nkeys, 
 // Starts, items and (cursor not NULL) the replicas' scatter cursors of the
 // counted keys; totals to the call counters.  bsums holds scan_blocks(nkeys) + 1
 // entries.
+int scan_per_thread(int64_t nkeys);
 int64_t scan_blocks(int64_t nkeys);
+int launch_scan_blocks(uint2 *bsums, int64_t nb, hipStream_t s);
 // Space for the scan blocks' sums of any call with up to nkeys keys (their
 // number drops where a thread takes more keys): scratch that a captured graph
 // holds then serves every smaller call.
 size_t scan_sums_bytes(int64_t nkeys);
 int scan_keys(const uint32_t *count, Replicas rp, int64_t nkeys, uint32_t per_item, uint2 *bsums,
               uint32_t *vis_start, uint32_t *item_start, uint32_t *cursor, Item *items,
-              unsigned long long *stats, hipStream_t s);
+              unsigned long long *stats, hipStream_t s, uint32_t *group_start = nullptr,
+              int group_keys = 0);
 
 // Host driver for count + scan + items + scatter.
 struct BinResult {
@@ -318,6 +330,10 @@ struct BinResult {
     Item *items;          // [max_items]
     void *recs;           // Rec<T>[n]
     int64_t max_items;
+    // optional, set by the caller: [nkeys / group_keys + 1] first record of every
+    // group of group_keys (a power of two) consecutive keys
+    uint32_t *group_start = nullptr;
+    int group_keys = 0;
 };
 
 // Device arrays of one sort and their sizes (bin_plan).
@@ -353,16 +369,23 @@ int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, 
              BinPlan &pl);
 // The sort into caller-provided arrays of the plan's sizes; timer_ctx (may be
 // NULL) receives the RG_TIMER_BINNING events.  The areas of `zero` are cleared
-// before the sort, in one launch with the counters it needs cleared.
+// before the sort, in one launch with the counters it needs cleared (`cleared`:
+// those are clear already).
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s,
-            BinResult &out);
-// bin_run into the context's scratch slots 0-6 and 15.
+            const BinBufs &b, ZeroList &zero, bool cleared, rg_context *timer_ctx,
+            hipStream_t s, BinResult &out);
+// Plan and scratch (the context's slots 0-6 and 15) of a sort, and what it needs
+// cleared added to `zero`: for a caller that clears more in the same launch.
+template <typename T>
+int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters,
+                ZeroList &zero, BinPlan &pl);
+// bin_run into the context's scratch; ready: the plan of a bin_prepare whose
+// areas have been cleared (NULL: none).
 template <typename Keyer, typename T>
 int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
                      ZeroList &zero, hipStream_t s, BinResult &out,
-                     int64_t max_counters = (int64_t)1 << 22);
+                     int64_t max_counters = (int64_t)1 << 22, const BinPlan *ready = nullptr);
 
 // Work items over per-key lengths len[0..nkeys): prefix[k] = exclusive sum of
 // len, item_start[k] = first item of key k (both nkeys + 1 entries), items of

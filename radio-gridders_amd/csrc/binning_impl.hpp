@@ -10,7 +10,8 @@ namespace rg {
 
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s, BinResult &out)
+            const BinBufs &b, ZeroList &zero, bool cleared, rg_context *timer_ctx,
+            hipStream_t s, BinResult &out)
 {
     const Replicas rp = pl.rp;
     out.vis_start = b.vis_start;
@@ -18,15 +19,15 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
     out.items = b.items;
     out.recs = b.recs;
     out.max_items = pl.max_items;
-    const bool small = n <= BIN_SMALL && nkeys <= BIN_SMALL_KEYS;
-    if (!small)
+    const bool small = bin_small(n, nkeys);
+    if (!small && !cleared)
         RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
     RG_TRY(zero.launch(s));
     KernelTimer kt(timer_ctx, RG_TIMER_BINNING, s);
     if (small) {
         hipLaunchKernelGGL((k_bin_small<Keyer, T>), dim3(1), dim3(1024), 0, s, kf, (int)n,
                            (int)nkeys, per_item, b.vis_start, b.item_start, b.items,
-                           (Rec<T> *)b.recs, b.stats);
+                           (Rec<T> *)b.recs, out.group_start, out.group_keys, b.stats);
         RG_HIP(hipGetLastError());
         return RG_OK;
     }
@@ -37,7 +38,7 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
                            b.count, rp, b.krp, b.stats);
     RG_HIP(hipGetLastError());
     RG_TRY(scan_keys(b.count, rp, nkeys, per_item, b.bsums, b.vis_start, b.item_start, b.cursor,
-                     b.items, b.stats, s));
+                     b.items, b.stats, s, out.group_start, out.group_keys));
     if (nb > 0)
         hipLaunchKernelGGL((k_bin_scatter<Keyer, T>), dim3((unsigned)nb), dim3(BIN_TB), 0, s, kf, n,
                            (const uint32_t *)b.cursor, rp, (const uint4 *)b.krp,
@@ -46,23 +47,40 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
     return RG_OK;
 }
 
-template <typename Keyer, typename T>
-int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
-                     ZeroList &zero, hipStream_t s, BinResult &out, int64_t max_counters)
+// context scratch slots of the sort (rg_internal.hpp)
+static const int bin_slot[BIN__N] = {0, 1, 2, 3, 4, 5, 6, 15};
+
+template <typename T>
+int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters,
+                ZeroList &zero, BinPlan &pl)
 {
-    BinPlan pl;
     RG_TRY(bin_plan(n, nkeys, per_item, max_counters, sizeof(Rec<T>), pl));
     RG_TRY(ensure_counters(ctx));
-    // context scratch slots of the sort (rg_internal.hpp)
-    static const int slot[BIN__N] = {0, 1, 2, 3, 4, 5, 6, 15};
     // items and scan sums: room for every call of up to this many visibilities
     // and keys, whatever item size it picks (scratch that a captured graph holds
     // cannot grow)
     const int64_t room = nkeys + std::max<int64_t>(n / per_item, std::max<int64_t>(700, n / 512)) + 1;
+    const size_t count_bytes = pl.bytes[BIN_COUNT];
     pl.bytes[BIN_ITEMS] = std::max(pl.bytes[BIN_ITEMS], sizeof(Item) * (size_t)room);
     pl.bytes[BIN_BSUMS] = scan_sums_bytes(nkeys);
     for (int k = 0; k < BIN__N; ++k)
-        RG_TRY(ctx->scratch[slot[k]].ensure(pl.bytes[k]));
+        RG_TRY(ctx->scratch[bin_slot[k]].ensure(pl.bytes[k]));
+    if (!bin_small(n, nkeys))
+        RG_TRY(zero.add(ctx->scratch[bin_slot[BIN_COUNT]].p, count_bytes));
+    return RG_OK;
+}
+
+template <typename Keyer, typename T>
+int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
+                     ZeroList &zero, hipStream_t s, BinResult &out, int64_t max_counters,
+                     const BinPlan *ready)
+{
+    BinPlan pl;
+    if (ready)
+        pl = *ready;
+    else
+        RG_TRY(bin_prepare<T>(ctx, n, nkeys, per_item, max_counters, zero, pl));
+    const int *slot = bin_slot;
     BinBufs b;
     b.count = ctx->scratch[slot[BIN_COUNT]].as<uint32_t>();
     b.vis_start = ctx->scratch[slot[BIN_VIS_START]].as<uint32_t>();
@@ -73,7 +91,7 @@ int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys,
     b.bsums = ctx->scratch[slot[BIN_BSUMS]].as<uint2>();
     b.krp = ctx->scratch[slot[BIN_KRP]].as<uint4>();
     b.stats = ctx->counters.as<unsigned long long>();
-    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, zero, ctx, s, out);
+    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, zero, true, ctx, s, out);
 }
 
 } // namespace rg

@@ -391,7 +391,8 @@ static int fft2d_t(rg_context *ctx, T2 *data, int type, int n, int batch, int si
     return fft_cols_dispatch<T2, false>(data, n, batch, tw, dev_batch, sh, s);
 }
 
-int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int sign, hipStream_t s)
+int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int sign, hipStream_t s,
+             const int32_t *dev_batch)
 {
     if (n < 8 || n > 4096 || (n & (n - 1)) || (sign != 1 && sign != -1))
         return fail(RG_ERR_PARAM, "FFT size %d / sign %d unsupported", n, sign);
@@ -401,15 +402,31 @@ int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int si
     RG_TRY(get_twiddles(ctx, n, type, sign, &tw));
     if (type == RG_C128)
         return sign > 0 ? fft_rows_dispatch<double2, true>((double2 *)data, n, nrows,
-                                                           (const double2 *)tw, nullptr, nullptr, 0, s)
+                                                           (const double2 *)tw, nullptr, dev_batch, 0, s)
                         : fft_rows_dispatch<double2, false>((double2 *)data, n, nrows,
-                                                            (const double2 *)tw, nullptr, nullptr,
+                                                            (const double2 *)tw, nullptr, dev_batch,
                                                             0, s);
     return sign > 0 ? fft_rows_dispatch<float2, true>((float2 *)data, n, nrows, (const float2 *)tw,
-                                                      nullptr, nullptr, 0, s)
+                                                      nullptr, dev_batch, 0, s)
                     : fft_rows_dispatch<float2, false>((float2 *)data, n, nrows,
-                                                       (const float2 *)tw, nullptr, nullptr, 0,
+                                                       (const float2 *)tw, nullptr, dev_batch, 0,
                                                        s);
+}
+
+int fft_cols(rg_context *ctx, void *data, int type, int n, int batch, int sign, hipStream_t s,
+             const int32_t *dev_batch)
+{
+    const void *tw = nullptr;
+    RG_TRY(get_twiddles(ctx, n, type, sign, &tw));
+    if (type == RG_C128)
+        return sign > 0 ? fft_cols_dispatch<double2, true>((double2 *)data, n, batch,
+                                                           (const double2 *)tw, dev_batch, 0, s)
+                        : fft_cols_dispatch<double2, false>((double2 *)data, n, batch,
+                                                            (const double2 *)tw, dev_batch, 0, s);
+    return sign > 0 ? fft_cols_dispatch<float2, true>((float2 *)data, n, batch, (const float2 *)tw,
+                                                      dev_batch, 0, s)
+                    : fft_cols_dispatch<float2, false>((float2 *)data, n, batch,
+                                                       (const float2 *)tw, dev_batch, 0, s);
 }
 
 int fft2d(rg_context *ctx, void *data, int type, int n, int batch, int sign, hipStream_t s,

@@ -92,8 +92,18 @@ void PinnedBuf::release()
 
 int ensure_counters(rg_context *ctx)
 {
-    RG_TRY(ctx->counters.ensure(sizeof(unsigned long long) * CNT__N));
+    RG_TRY(ctx->counters.ensure(COUNTER_BYTES));
     RG_TRY(ctx->counters_host.ensure(sizeof(unsigned long long) * CNT__N));
+    return RG_OK;
+}
+
+int range_done_counter(rg_context *ctx, uint32_t **done, hipStream_t s)
+{
+    *done = reinterpret_cast<uint32_t *>(ctx->counters.as<char>() + COUNTER_BYTES - 64);
+    if (!ctx->range_ready) {
+        RG_TRY(zero_fill(*done, 64, s));
+        ctx->range_ready = true;
+    }
     return RG_OK;
 }
 
@@ -378,8 +388,8 @@ static int grid_common(rg_context *ctx, const rg_grid_params *p, const rg_flat_v
     const bool capturing = cap == hipStreamCaptureStatusActive;
     if (capturing)
         ctx->frozen = true; // the graph will hold this context's scratch addresses
-    // batched W-projection clears the counters with its grids
-    const bool counters_later = p->subgrid_size == 0 && p->mode == RG_MODE_BATCHED;
+    // the batched paths clear the counters in a launch of their own work
+    const bool counters_later = p->mode == RG_MODE_BATCHED;
     if (!counters_later)
         RG_TRY(zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s));
     ctx->last_stream = s;
@@ -387,25 +397,19 @@ static int grid_common(rg_context *ctx, const rg_grid_params *p, const rg_flat_v
     if (p->mode == RG_MODE_PLAIN && n_chan != 1)
         return fail(RG_ERR_UNSUPPORTED, "plain mode grids one channel per call");
     const int64_t *d_off = nullptr;
+    ctx->last_kind = p->subgrid_size == 0 ? 1 : 2;
     int st = channel_offsets(ctx, offsets, n_chan, s, &d_off);
-    if (st == RG_OK && counters_later) {
-        ctx->last_kind = 1;
+    if (st == RG_OK && p->subgrid_size != 0)
+        st = wtowers_run(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s, capturing);
+    else if (st == RG_OK && p->mode == RG_MODE_BATCHED)
         st = wproj_batched(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s);
-    }
-    if (counters_later) {
-        if (st != RG_OK) // a refused call leaves cleared counters
-            (void)zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s);
-        return st;
-    }
-    RG_TRY(st);
-    if (p->subgrid_size == 0) {
-        ctx->last_kind = 1;
-        if (grid_type != RG_C128)
-            return fail(RG_ERR_PARAM, "plain mode writes an RG_C128 grid");
-        return wproj_plain(ctx, p, vis, wk, grid, s);
-    }
-    ctx->last_kind = 2;
-    return wtowers_run(ctx, p, vis, d_off, n_chan, wk, grid, grid_type, s, capturing);
+    else if (st == RG_OK && grid_type != RG_C128)
+        st = fail(RG_ERR_PARAM, "plain mode writes an RG_C128 grid");
+    else if (st == RG_OK)
+        st = wproj_plain(ctx, p, vis, wk, grid, s);
+    if (st != RG_OK && counters_later) // a refused call leaves cleared counters
+        (void)zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s);
+    return st;
 }
 
 int rg_grid(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk,

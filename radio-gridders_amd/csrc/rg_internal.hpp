@@ -108,6 +108,8 @@ struct WtPlan {
     bool valid = false;
     int N = 0, n = 0, M = 0, S = 0, R = 0, P = 0, H = 0, type = 0, nchan = 0;
     uint32_t K = 0;
+    bool k_auto = false; // K chosen by the stream's length (vis_per_item 0)
+    int tpc = 32;        // tasks per column-pass chunk
     int floor_batch = 0;
     double theta = 0, winc = 0, w_min = 0, w_step = 0;
     int64_t nvis = 0;   // longest stream the plan was made for
@@ -124,6 +126,7 @@ struct rg_context {
     // counters[0..7] written by kernels (int64): see Counter enum in gridding code
     rg::DevBuf counters;
     rg::PinnedBuf counters_host;
+    bool range_ready = false; // range_done_counter's word has been cleared
     hipStream_t last_stream = nullptr;
     int last_kind = 0; // 0 none, 1 wproj, 2 wtowers
     int64_t last_nvis = 0;
@@ -172,7 +175,13 @@ enum Counter {
     CNT__N = 11
 };
 
+// the counters and, in the last 64 bytes, the word of range_done_counter
+constexpr size_t COUNTER_BYTES = 256;
+static_assert(sizeof(unsigned long long) * CNT__N <= COUNTER_BYTES - 64, "counter space");
 int ensure_counters(rg_context *ctx);
+// a device word that is 0 between launches (behind the counters; cleared on s
+// the first time)
+int range_done_counter(rg_context *ctx, uint32_t **done, hipStream_t s);
 
 // Records a (start, stop) event pair around the launches issued while it is
 // alive, when the context's timing is enabled.
@@ -208,7 +217,12 @@ int wtowers_run(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis
 int channel_offsets(rg_context *ctx, const int64_t *offsets, int n_chan, hipStream_t s,
                     const int64_t **d_off);
 // in-place FFT of nrows contiguous rows of length n (power of two 8..4096)
-int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int sign, hipStream_t s);
+// (dev_batch, optional, device int: only the first *dev_batch arrays of n rows)
+int fft_rows(rg_context *ctx, void *data, int type, int n, int64_t nrows, int sign, hipStream_t s,
+             const int32_t *dev_batch = nullptr);
+// the column pass alone
+int fft_cols(rg_context *ctx, void *data, int type, int n, int batch, int sign, hipStream_t s,
+             const int32_t *dev_batch = nullptr);
 // row_flags (optional): bit r set for every row r (of the n * batch rows) that
 // may be nonzero on input; the first row pass skips the others, which must be 0.
 // dev_batch (optional, device int): only the first *dev_batch <= batch arrays
@@ -228,6 +242,28 @@ struct ZeroList {
     int n = 0;
     int add(void *q, size_t nbytes);
     int launch(hipStream_t s);
+    // workgroups of 256 threads worth launching (0: nothing to clear)
+    unsigned blocks() const
+    {
+        size_t most = 0;
+        for (int k = 0; k < n; ++k)
+            most = bytes[k] > most ? bytes[k] : most;
+        const size_t b = (most / 16 + 255) / 256;
+        return most == 0 ? 0u : (unsigned)(b < 1 ? 1 : b > 8192 ? 8192 : b);
+    }
+    // workgroup b's share of nb: every area in turn, 16 bytes per store
+    __device__ void clear(unsigned b, unsigned nb) const
+    {
+        const size_t stride = (size_t)nb * 256;
+        for (int k = 0; k < n; ++k) {
+            uint4 *q = reinterpret_cast<uint4 *>(p[k]);
+            const size_t n16 = bytes[k] / 16, tail = bytes[k] % 16;
+            for (size_t i = (size_t)b * 256 + threadIdx.x; i < n16; i += stride)
+                q[i] = make_uint4(0, 0, 0, 0);
+            if (b == 0 && threadIdx.x < tail)
+                reinterpret_cast<unsigned char *>(q + n16)[threadIdx.x] = 0;
+        }
+    }
 };
 int weight_vis(rg_context *ctx, const double *u, const double *v, int64_t n, void *vis,
                int vis_type, int N, double theta, uint32_t *counts, hipStream_t s);

@@ -20,19 +20,7 @@ namespace rg {
 
 // ---- zero fill (graph-capturable, no memset nodes) ---------------------------
 
-// Every workgroup takes its share of each area, 16 bytes per store.
-__global__ __launch_bounds__(256) void k_zero(ZeroList z)
-{
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (int k = 0; k < z.n; ++k) {
-        uint4 *p = reinterpret_cast<uint4 *>(z.p[k]);
-        const size_t n16 = z.bytes[k] / 16, tail = z.bytes[k] % 16;
-        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride)
-            p[i] = make_uint4(0, 0, 0, 0);
-        if (blockIdx.x == 0 && threadIdx.x < tail)
-            reinterpret_cast<unsigned char *>(p + n16)[threadIdx.x] = 0;
-    }
-}
+__global__ __launch_bounds__(256) void k_zero(ZeroList z) { z.clear(blockIdx.x, gridDim.x); }
 
 int ZeroList::add(void *q, size_t nbytes)
 {
@@ -49,13 +37,8 @@ int ZeroList::add(void *q, size_t nbytes)
 
 int ZeroList::launch(hipStream_t s)
 {
-    size_t most = 0;
-    for (int k = 0; k < n; ++k)
-        most = std::max(most, bytes[k]);
-    if (most == 0)
-        return RG_OK;
-    const size_t blocks = std::max<size_t>(1, std::min<size_t>((most / 16 + 255) / 256, 8192));
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)blocks), dim3(256), 0, s, *this);
+    if (const unsigned nb = blocks())
+        hipLaunchKernelGGL(k_zero, dim3(nb), dim3(256), 0, s, *this);
     RG_HIP(hipGetLastError());
     n = 0;
     return RG_OK;
@@ -473,8 +456,8 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
-    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.ntiles, sh.per_item, pl, b, zero, nullptr, s,
-                                   br)));
+    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.ntiles, sh.per_item, pl, b, zero, false, nullptr,
+                                   s, br)));
     return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N,
                              sh.tile, sh.ntx, sh.ntiles, s);
 }

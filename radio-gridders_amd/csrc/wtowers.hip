@@ -24,6 +24,7 @@
 #include "binning_impl.hpp"
 #include "fft_core.hpp"
 #include "romein.hpp"
+#include "scan.hpp"
 #include "tiles.hpp"
 
 namespace rg {
@@ -113,89 +114,105 @@ struct TowerKeyer {
     }
 };
 
-// min / max floor index over visibilities that fall in the tower set; four
-// visibilities per thread and pass (their loads issued together), wavefront
-// then workgroup reduction into part[workgroup]; k_range_finish reduces the
-// parts (atomics on the same two words serialise: ~10 ns each)
+// ---- floor range and preparation -----------------------------------------------------------
+// min / max floor index over visibilities that fall in the tower set: each
+// workgroup of the range part reduces its share (four visibilities per thread
+// and pass, their loads issued together) into part[workgroup], and the last one
+// to finish (a counter that it sets back to 0) reduces the parts into range[0..1]
+// (INT_MAX / INT_MIN if there are none).  Atomics on the two words instead
+// serialise: about 10 ns each.
 constexpr int RANGE_VPT = 4;
-constexpr int RANGE_BLOCKS = 2048;
+constexpr int RANGE_BLOCKS = 1024;
 // the range (2 ints) and the workgroups' parts in one buffer
 constexpr size_t RANGE_BYTES = 256 + sizeof(int2) * RANGE_BLOCKS;
 
-__global__ __launch_bounds__(256) void k_floor_range(const double *u, const double *v,
-                                                     const double *w, int64_t n, double theta,
-                                                     int N, int chunk, int cc, double winc,
-                                                     int2 *part)
+struct RangeJob {
+    const double *u, *v, *w;
+    int64_t n;
+    double theta, winc;
+    int N, chunk, cc;
+    int *range;            // [2]
+    unsigned long long *part;
+    uint32_t *done;
+    unsigned blocks;       // the first workgroups of the launch
+};
+
+__device__ inline void minmax_block(int &lo, int &hi, int (&smin)[4], int (&smax)[4])
 {
-    __shared__ int smin[4], smax[4];
-    int lo = INT_MAX, hi = INT_MIN;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n;
-         i0 += RANGE_VPT * stride) {
-        double uu[RANGE_VPT], vv[RANGE_VPT], ww[RANGE_VPT];
-#pragma unroll
-        for (int q = 0; q < RANGE_VPT; ++q) {
-            const int64_t i = i0 + q * stride < n ? i0 + q * stride : i0;
-            uu[q] = u[i];
-            vv[q] = v[i];
-            ww[q] = w[i];
-        }
-#pragma unroll
-        for (int q = 0; q < RANGE_VPT; ++q) {
-            const int cx = tower_index(uu[q], theta, N, chunk);
-            const int cy = tower_index(vv[q], theta, N, chunk);
-            if (cx < 0 || cx >= cc || cy < 0 || cy >= cc)
-                continue;
-            const int wp = floor_index(ww[q], winc);
-            lo = min(lo, wp);
-            hi = max(hi, wp);
-        }
-    }
     for (int o = 32; o > 0; o >>= 1) {
         lo = min(lo, __shfl_xor(lo, o));
         hi = max(hi, __shfl_xor(hi, o));
-    }
-    const int wv = threadIdx.x / 64;
-    if (__lane_id() == 0) {
-        smin[wv] = lo;
-        smax[wv] = hi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < (int)blockDim.x / 64; ++k) {
-            lo = min(lo, smin[k]);
-            hi = max(hi, smax[k]);
-        }
-        part[blockIdx.x] = make_int2(lo, hi);
-    }
-}
-
-// range[0..1] = min / max over the nparts parts (INT_MAX / INT_MIN if none)
-__global__ __launch_bounds__(1024) void k_range_finish(const int2 *part, int nparts, int *range)
-{
-    __shared__ int smin[16], smax[16];
-    int lo = INT_MAX, hi = INT_MIN;
-    for (int k = threadIdx.x; k < nparts; k += blockDim.x) {
-        const int2 v = part[k];
-        lo = min(lo, v.x);
-        hi = max(hi, v.y);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        lo = min(lo, __shfl_xor(lo, o));
-        hi = max(hi, __shfl_xor(hi, o));
-    }
     if (__lane_id() == 0) {
         smin[threadIdx.x / 64] = lo;
         smax[threadIdx.x / 64] = hi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < (int)blockDim.x / 64; ++k) {
-            lo = min(lo, smin[k]);
-            hi = max(hi, smax[k]);
+    for (int k = 0; k < 4; ++k) {
+        lo = min(lo, smin[k]);
+        hi = max(hi, smax[k]);
+    }
+}
+
+__device__ inline void floor_range_block(const RangeJob &r)
+{
+    __shared__ int smin[4], smax[4];
+    __shared__ uint32_t s_last;
+    int lo = INT_MAX, hi = INT_MIN;
+    const int64_t stride = (int64_t)r.blocks * 256;
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < r.n;
+         i0 += RANGE_VPT * stride) {
+        double uu[RANGE_VPT], vv[RANGE_VPT], ww[RANGE_VPT];
+#pragma unroll
+        for (int q = 0; q < RANGE_VPT; ++q) {
+            const int64_t i = i0 + q * stride < r.n ? i0 + q * stride : i0;
+            uu[q] = r.u[i];
+            vv[q] = r.v[i];
+            ww[q] = r.w[i];
         }
-        range[0] = lo;
-        range[1] = hi;
+#pragma unroll
+        for (int q = 0; q < RANGE_VPT; ++q) {
+            const int cx = tower_index(uu[q], r.theta, r.N, r.chunk);
+            const int cy = tower_index(vv[q], r.theta, r.N, r.chunk);
+            if (cx < 0 || cx >= r.cc || cy < 0 || cy >= r.cc)
+                continue;
+            const int wp = floor_index(ww[q], r.winc);
+            lo = min(lo, wp);
+            hi = max(hi, wp);
+        }
+    }
+    minmax_block(lo, hi, smin, smax);
+    if (threadIdx.x == 0) {
+        const unsigned long long v =
+            (unsigned long long)(uint32_t)lo | (unsigned long long)(uint32_t)hi << 32;
+        // Device-scope exchange, then the count: the exchange's result goes
+        // into the count's operand, so the part is in place before the
+        // workgroup is counted.  (Release ordering instead would write back an
+        // XCD's L2 per workgroup: 142 us for the launch at 8.4 M visibilities.)
+        const unsigned long long old = __hip_atomic_exchange(
+            &r.part[blockIdx.x], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t one = 1u;
+        asm volatile("" : "+v"(one) : "v"((uint32_t)old), "v"((uint32_t)(old >> 32)));
+        s_last = __hip_atomic_fetch_add(r.done, one, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT) == r.blocks - 1;
+    }
+    __syncthreads();
+    if (!s_last)
+        return;
+    lo = INT_MAX;
+    hi = INT_MIN;
+    for (unsigned k = threadIdx.x; k < r.blocks; k += 256) {
+        const unsigned long long v =
+            __hip_atomic_load(&r.part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lo = min(lo, (int)(uint32_t)v);
+        hi = max(hi, (int)(uint32_t)(v >> 32));
+    }
+    minmax_block(lo, hi, smin, smax);
+    if (threadIdx.x == 0) {
+        r.range[0] = lo;
+        r.range[1] = hi;
+        *r.done = 0;
     }
 }
 
@@ -214,44 +231,56 @@ __global__ __launch_bounds__(256) void k_task_info(const uint32_t *vis_start,
 // ---- task tables (batched mode, built on the device) ---------------------------------------
 // Tasks are the non-empty slots in slot order (tower id, then floor), so the
 // tasks of a tower are consecutive.  Each tower's run of tasks is cut into
-// chunks of at most TASKS_PER_CHUNK (one column-pass partial image each);
-// active towers are ranked in tower-id order (the subimage index).
-constexpr int TASKS_PER_CHUNK = 32;
+// chunks of at most tpc (one column-pass partial image each); active towers
+// are ranked in tower-id order (the subimage index).
+constexpr int TASKS_PER_CHUNK_MIN = 8, TASKS_PER_CHUNK_MAX = 32;
+
+// Tasks per chunk.  A column-pass workgroup takes its chunk's floors one after
+// another, so chunks are short enough for about 2048 workgroups (n / 8 column
+// blocks per chunk), while every chunk costs a partial image to write and add up.
+// Column pass, chunks of 32 against shorter: 945 tasks of 128^2 FP32 68 -> 32 us
+// (8), 665 of 256^2 FP64 164 -> 152 us (8), 1568 of 512^2 FP32 607 -> 650 us (16).
+static int tasks_per_chunk(int64_t ntasks, int n)
+{
+    int tpc = TASKS_PER_CHUNK_MAX;
+    while (tpc > TASKS_PER_CHUNK_MIN && ntasks / tpc * (n / 8) < 2048)
+        tpc /= 2;
+    return tpc;
+}
 
 struct TaskTables {
     int32_t *tower_ntasks;   // [ntw]
     int32_t *tower_task_off; // [ntw]
     int32_t *tower_chunk_off; // [ntw]
     int32_t *rank_of_tower;  // [ntw], -1 inactive
-    int32_t *tower_of_rank;  // [ntw]
     int32_t *rank_chunk0;    // [ntw] first chunk of rank r
     int32_t *rank_nchunk;    // [ntw]
     int32_t *task_slot;      // [ntasks_cap]
     int32_t *task_wp;        // [ntasks_cap]
-    int32_t *task_rank;      // [ntasks_cap] tower rank of the task
     int32_t *chunk_first;    // [nchunks_cap]
     int32_t *chunk_count;    // [nchunks_cap]
     int32_t *rank_of_slot;   // [nslots] task index of a non-empty slot
     // totals[0] tasks, [1] towers, [2] chunks (each clipped to its capacity)
     int32_t *totals;
-    int ntw, nwp, nk; // tower ids, floors per tower, keys per task
+    int ntw, nwp;     // tower ids, floors per tower
+    int tpc;          // tasks per chunk
     int ntasks_cap, nchunks_cap, ntowers_cap;
 };
 
-__device__ inline bool slot_nonempty(const uint32_t *key_start, int64_t s, int nk)
+__device__ inline bool slot_nonempty(const uint32_t *slot_start, int64_t s)
 {
-    return key_start[(s + 1) * nk] > key_start[s * nk];
+    return slot_start[s + 1] > slot_start[s];
 }
 
 // block t: number of non-empty slots of tower t
-__global__ __launch_bounds__(256) void k_tower_count(const uint32_t *__restrict__ key_start,
+__global__ __launch_bounds__(256) void k_tower_count(const uint32_t *__restrict__ slot_start,
                                                      TaskTables tt)
 {
     __shared__ int wsum[4];
     const int t = blockIdx.x;
     int c = 0;
     for (int f = threadIdx.x; f < tt.nwp; f += 256)
-        c += slot_nonempty(key_start, (int64_t)t * tt.nwp + f, tt.nk) ? 1 : 0;
+        c += slot_nonempty(slot_start, (int64_t)t * tt.nwp + f) ? 1 : 0;
     for (int o = 32; o > 0; o >>= 1)
         c += __shfl_xor(c, o);
     if (__lane_id() == 0)
@@ -269,7 +298,7 @@ __global__ __launch_bounds__(1024) void k_tower_scan(TaskTables tt, unsigned lon
     for (int base = 0; base < tt.ntw; base += 1024) {
         const int t = base + (int)threadIdx.x;
         const int nt = t < tt.ntw ? tt.tower_ntasks[t] : 0;
-        const int nc = (nt + TASKS_PER_CHUNK - 1) / TASKS_PER_CHUNK;
+        const int nc = (nt + tt.tpc - 1) / tt.tpc;
         const int act = nt > 0 ? 1 : 0;
         s_task[threadIdx.x] = nt;
         s_chunk[threadIdx.x] = nc;
@@ -299,7 +328,6 @@ __global__ __launch_bounds__(1024) void k_tower_scan(TaskTables tt, unsigned lon
             tt.tower_chunk_off[t] = coff;
             tt.rank_of_tower[t] = keep ? rk : -1;
             if (keep) {
-                tt.tower_of_rank[rk] = t;
                 tt.rank_chunk0[rk] = coff;
                 tt.rank_nchunk[rk] = nc;
             }
@@ -324,7 +352,7 @@ __global__ __launch_bounds__(1024) void k_tower_scan(TaskTables tt, unsigned lon
 }
 
 // block t: the task entries and chunks of tower t (block scan over its slots)
-__global__ __launch_bounds__(256) void k_tower_tasks(const uint32_t *__restrict__ key_start,
+__global__ __launch_bounds__(256) void k_tower_tasks(const uint32_t *__restrict__ slot_start,
                                                      TaskTables tt,
                                                      const int *__restrict__ range)
 {
@@ -333,13 +361,13 @@ __global__ __launch_bounds__(256) void k_tower_tasks(const uint32_t *__restrict_
     const int nt = tt.tower_ntasks[t];
     if (nt == 0)
         return;
-    const int toff = tt.tower_task_off[t], rk = tt.rank_of_tower[t];
+    const int toff = tt.tower_task_off[t];
     const int wp_min = range[0];
     int run = 0;
     for (int base = 0; base < tt.nwp; base += 256) {
         const int f = base + (int)threadIdx.x;
         const int64_t s = (int64_t)t * tt.nwp + f;
-        const bool ne = f < tt.nwp && slot_nonempty(key_start, s, tt.nk);
+        const bool ne = f < tt.nwp && slot_nonempty(slot_start, s);
         const unsigned long long m = __ballot(ne);
         const int lane = __lane_id(), wv = threadIdx.x / 64;
         const int in_wave = __popcll(m & ((1ull << lane) - 1ull));
@@ -354,7 +382,6 @@ __global__ __launch_bounds__(256) void k_tower_tasks(const uint32_t *__restrict_
             if (k < tt.ntasks_cap) {
                 tt.task_slot[k] = (int32_t)s;
                 tt.task_wp[k] = wp_min + f;
-                tt.task_rank[k] = rk;
                 tt.rank_of_slot[s] = k;
             }
         }
@@ -362,35 +389,131 @@ __global__ __launch_bounds__(256) void k_tower_tasks(const uint32_t *__restrict_
         __syncthreads();
     }
     const int coff = tt.tower_chunk_off[t];
-    const int nc = (nt + TASKS_PER_CHUNK - 1) / TASKS_PER_CHUNK;
+    const int nc = (nt + tt.tpc - 1) / tt.tpc;
     for (int c = threadIdx.x; c < nc; c += 256) {
         if (coff + c < tt.nchunks_cap) {
-            const int first = toff + c * TASKS_PER_CHUNK;
+            const int first = toff + c * tt.tpc;
             tt.chunk_first[coff + c] = first;
             tt.chunk_count[coff + c] =
-                max(0, min(min(TASKS_PER_CHUNK, nt - c * TASKS_PER_CHUNK), tt.ntasks_cap - first));
+                max(0, min(min(tt.tpc, nt - c * tt.tpc), tt.ntasks_cap - first));
         }
     }
 }
 
-// Per task: bit b of word b / 32 set when band b has work items (the band was
-// written); MW = NB / 32 words per task (rounded up).
-__global__ __launch_bounds__(256) void k_band_masks(const uint32_t *__restrict__ item_start,
-                                                    const int32_t *__restrict__ task_slot,
-                                                    const int32_t *__restrict__ totals, int nb,
-                                                    int mw, uint32_t *masks)
+// All tables of a call of few slots and towers by one workgroup: the tables of
+// a small call are all latency, one launch instead of three.  Thread t takes
+// the slots [t SPT, (t + 1) SPT).
+constexpr int TABLE_SPT = 32;
+constexpr int TABLE_SLOTS = 1024 * TABLE_SPT;
+constexpr int TABLE_TOWERS = 1024;
+
+// exclusive scan over 1024 threads of (x, y) pairs
+__device__ inline int2 scan_pairs(int2 v, int2 &total, int2 (&wtot)[16])
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // (task, word)
-    const int k = (int)(e / mw), wd = (int)(e - (int64_t)k * mw);
-    if (k >= totals[0])
-        return;
-    const uint32_t *f = item_start + (size_t)task_slot[k] * nb;
-    uint32_t m = 0;
-    for (int q = 0; q < 32 && wd * 32 + q < nb; ++q) {
-        const int bnd = wd * 32 + q;
-        m |= (f[bnd + 1] > f[bnd] ? 1u : 0u) << q;
+    const int lane = __lane_id(), wv = threadIdx.x / 64;
+    int2 inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(inc.x, o), y = __shfl_up(inc.y, o);
+        if (lane >= o) {
+            inc.x += x;
+            inc.y += y;
+        }
     }
-    masks[e] = m;
+    __syncthreads();
+    if (lane == 63)
+        wtot[wv] = inc;
+    __syncthreads();
+    int2 run = make_int2(inc.x - v.x, inc.y - v.y);
+    total = make_int2(0, 0);
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const int2 t = wtot[w];
+        if (w < wv) {
+            run.x += t.x;
+            run.y += t.y;
+        }
+        total.x += t.x;
+        total.y += t.y;
+    }
+    return run;
+}
+
+__global__ __launch_bounds__(1024) void k_tower_tables(const uint32_t *__restrict__ slot_start,
+                                                       TaskTables tt, int nslots,
+                                                       const int *__restrict__ range,
+                                                       unsigned long long *stats)
+{
+    __shared__ int2 wtot[16];
+    __shared__ int s_toff[TABLE_TOWERS + 1];
+    const int spt = (nslots + 1023) / 1024; // slots per thread, at most TABLE_SPT
+    const int s0 = (int)threadIdx.x * spt, s1 = min(nslots, s0 + spt);
+    uint32_t m = 0; // non-empty slots of the thread
+    uint32_t prev = s0 < nslots ? slot_start[s0] : 0u;
+#pragma unroll
+    for (int j = 0; j < TABLE_SPT; ++j) {
+        if (j >= spt)
+            break;
+        const uint32_t next = slot_start[min(s0 + j + 1, nslots)];
+        m |= (next > prev && s0 + j < nslots ? 1u : 0u) << j;
+        prev = next;
+    }
+    int2 total;
+    const int off = scan_pairs(make_int2(__popc(m), 0), total, wtot).x;
+    const int wp_min = range[0];
+    int k = off;
+    int tower = s0 / tt.nwp, f = s0 - tower * tt.nwp;
+    for (int sl = s0; sl < s1; ++sl, ++f) {
+        if (f == tt.nwp) {
+            f = 0;
+            ++tower;
+        }
+        if (f == 0)
+            s_toff[tower] = k;
+        if ((m >> (sl - s0)) & 1u) {
+            if (k < tt.ntasks_cap) {
+                tt.task_slot[k] = sl;
+                tt.task_wp[k] = wp_min + f;
+                tt.rank_of_slot[sl] = k;
+            }
+            ++k;
+        }
+    }
+    if (threadIdx.x == 0)
+        s_toff[tt.ntw] = total.x;
+    const int ntasks = total.x;
+    __syncthreads();
+    const int t = threadIdx.x;
+    const int toff = t < tt.ntw ? s_toff[t] : 0;
+    const int nt = t < tt.ntw ? s_toff[t + 1] - toff : 0;
+    const int nc = (nt + tt.tpc - 1) / tt.tpc;
+    const int2 run = scan_pairs(make_int2(nc, nt > 0 ? 1 : 0), total, wtot);
+    if (t < tt.ntw) {
+        // a tower ranked beyond the subimage capacity is left out (the call
+        // reports an overrun)
+        const bool keep = nt > 0 && run.y < tt.ntowers_cap;
+        tt.rank_of_tower[t] = keep ? run.y : -1;
+        if (keep) {
+            tt.rank_chunk0[run.y] = run.x;
+            tt.rank_nchunk[run.y] = nc;
+        }
+        for (int c = 0; c < nc && run.x + c < tt.nchunks_cap; ++c) {
+            const int first = toff + c * tt.tpc;
+            tt.chunk_first[run.x + c] = first;
+            tt.chunk_count[run.x + c] =
+                max(0, min(min(tt.tpc, nt - c * tt.tpc), tt.ntasks_cap - first));
+        }
+    }
+    if (threadIdx.x == 0) {
+        stats[CNT_TASKS] = (unsigned long long)ntasks;
+        stats[CNT_TOWERS] = (unsigned long long)total.y;
+        stats[CNT_CHUNKS] = (unsigned long long)total.x;
+        if (ntasks > tt.ntasks_cap || total.x > tt.nchunks_cap || total.y > tt.ntowers_cap)
+            atomicAdd(&stats[CNT_OVERFLOW], 1ull);
+        tt.totals[0] = min(ntasks, tt.ntasks_cap);
+        tt.totals[1] = min(total.y, tt.ntowers_cap);
+        tt.totals[2] = min(total.x, tt.nchunks_cap);
+    }
 }
 
 // Tasks [t0, t1) of batch b (Q tasks per batch); false when the batch is empty.
@@ -503,14 +626,19 @@ __device__ inline BandRec<T> band_record(const Rec<T> &r, int S, int H, int Hb, 
 
 // Kernel table for the band pass: H zero rows, then sub-kernel k (S x S) at
 // row H + k PS followed by H zero rows (PS = S + H); (H + nsub PS) S taps.
-template <typename T2>
-__global__ __launch_bounds__(256) void k_pad_kernels(const T2 *__restrict__ src, T2 *dst,
-                                                     int64_t nsub, int S, int H)
+template <typename T2> struct PadJob {
+    const T2 *src;
+    T2 *dst;
+    int64_t nsub;
+    int S, H;
+    unsigned blocks;
+};
+
+template <typename T2> __device__ inline void pad_kernels_block(const PadJob<T2> &p, unsigned b)
 {
-    const int PS = padded_rows(S, H);
-    const int64_t total = ((int64_t)H + nsub * PS) * S;
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * 256) {
+    const int S = p.S, H = p.H, PS = padded_rows(S, H);
+    const int64_t total = ((int64_t)H + p.nsub * PS) * S;
+    for (int64_t e = (int64_t)b * 256 + threadIdx.x; e < total; e += (int64_t)p.blocks * 256) {
         const int64_t prow = e / S - H; // row counted from the first sub-kernel
         const int col = (int)(e % S);
         T2 v;
@@ -520,12 +648,26 @@ __global__ __launch_bounds__(256) void k_pad_kernels(const T2 *__restrict__ src,
             const int64_t k = prow / PS;
             const int row = (int)(prow - k * PS);
             if (row < S)
-                v = src[(k * S + row) * S + col];
+                v = p.src[(k * S + row) * S + col];
         }
-        dst[e] = v;
+        p.dst[e] = v;
     }
 }
 
+// Everything a call needs before its sort, in one launch: the first
+// range.blocks workgroups find the floor range, the next pad.blocks build the padded
+// kernel table, the others clear the areas of z.
+template <typename T2>
+__global__ __launch_bounds__(256) void k_wt_prepare(RangeJob range, PadJob<T2> pad, ZeroList z)
+{
+    if (blockIdx.x < range.blocks) {
+        floor_range_block(range);
+    } else if (blockIdx.x < range.blocks + pad.blocks) {
+        pad_kernels_block(pad, blockIdx.x - range.blocks);
+    } else {
+        z.clear(blockIdx.x - range.blocks - pad.blocks, gridDim.x - range.blocks - pad.blocks);
+    }
+}
 
 // Band records in and subgrid bands out are touched once: nontemporal loads
 // and stores keep them from evicting the kernel table, which every band lane
@@ -560,9 +702,9 @@ __device__ inline void store_once2(double2 *d, double2 a, double2 b)
 // ---- record order inside band items -------------------------------------------------------
 // A band lane's cell depends only on the footprint column gx (its row is fixed),
 // so records sorted by gx keep each lane on one cell for long runs and the
-// Romein register sum rarely flushes.  Every band work item (window records
-// src = wstart[key] + (start - prefix[key]) .. + count of the binned array) is
-// counting-sorted by gx + S (bins < n + S <= SORT_BINS) into its own slot
+// Romein register sum rarely flushes.  Every band work item (the records of its
+// part of the key's window, key_start[key - min(b, mk - 1)] + K times the part, in
+// the binned array) is counting-sorted by gx + S (bins < n + S <= SORT_BINS) into its own slot
 // [start, start + count) of the expanded array as band records of its band
 // b = key mod nb (items of <= 32 records by rank in one wavefront); the
 // order inside a bin is arbitrary.  The band pass relies on every item being
@@ -573,20 +715,34 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ in,
                                                     BandRec<T> *__restrict__ out,
                                                     const Item *__restrict__ items,
-                                                    const unsigned long long *__restrict__ stats,
-                                                    const uint32_t *__restrict__ prefix,
-                                                    const uint32_t *__restrict__ wstart, int nbins,
-                                                    int S, int H, int nb)
+                                                    unsigned long long *stats,
+                                                    const uint32_t *__restrict__ key_start,
+                                                    const uint32_t *__restrict__ item_start,
+                                                    uint32_t K, int mk, int nbins, int S, int H,
+                                                    int nb,
+                                                    const uint32_t *__restrict__ bands_part,
+                                                    int nparts)
 {
     __shared__ uint32_t bins[SORT_BINS];
     __shared__ uint32_t wsum[4];
+    if (blockIdx.x == 0) { // the call's count of bands, from the window scan's parts
+        uint32_t t = 0;
+        for (int k = threadIdx.x; k < nparts; k += 256)
+            t += bands_part[k];
+        for (int o = 32; o > 0; o >>= 1)
+            t += (uint32_t)__shfl_xor((int)t, o);
+        if (__lane_id() == 0 && t)
+            atomicAdd(&stats[CNT_BANDS], (unsigned long long)t);
+    }
     constexpr int z = (int)sizeof(typename Vec2<T>::type);
     const uint32_t nitems = (uint32_t)stats[CNT_ITEMS];
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         const Item item = items[it];
-        const Rec<T> *src = in + (item.start - prefix[item.key] + wstart[item.key]);
+        const int b = (int)(item.key & (uint32_t)(nb - 1));
+        const Rec<T> *src = in + key_start[item.key - (uint32_t)min(b, mk - 1)] +
+                            (size_t)(it - item_start[item.key]) * K;
         BandRec<T> *dst = out + item.start;
-        const int Hb = H * (int)(item.key % (uint32_t)nb);
+        const int Hb = H * b;
         if (item.count <= 32) {
             // rank sort in the first wavefront: lane i counts the records
             // ordered before its own (smaller column, or equal and earlier)
@@ -655,37 +811,59 @@ __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ i
 // ---- band windows ------------------------------------------------------------------------
 // Band b of a task takes the records of keys b - mk + 1 .. b (every footprint
 // that can reach rows [H b, H b + H)); they are contiguous in the binned
-// record array.  Per band key: window length and start.
-// Band windows with records are counted (the bands the pass writes).
-// (grid-stride; the windows with records are counted per workgroup and added
-// with one atomic: one per wavefront on the same word serialised)
-__global__ __launch_bounds__(256) void k_window_len(const uint32_t *__restrict__ key_start,
-                                                    int64_t nkeys, int nb, int mk, uint32_t *len,
-                                                    uint32_t *wstart, unsigned long long *stats)
-{
-    __shared__ uint32_t s_any[4];
-    uint32_t nany = 0;
-    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nkeys;
-         k += (int64_t)gridDim.x * blockDim.x) {
-        const int b = (int)(k % nb);
-        const int64_t k0 = k - min(b, mk - 1);
-        const uint32_t w0 = key_start[k0];
-        const uint32_t l = key_start[k + 1] - w0;
-        len[k] = l;
-        wstart[k] = w0;
-        nany += l > 0 ? 1u : 0u;
+// record array.  The scan of the windows' lengths gives their work items and,
+// per slot, the bands with records: bit b % 32 of word b / 32 of the slot's
+// (nb + 31) / 32 words.  nb is a power of two.
+struct WindowSource {
+    static constexpr int NREP = 1;
+    const uint32_t *key_start;
+    int nb, mk;
+    uint32_t *masks;
+    uint32_t *bands_part; // [scan blocks] windows with records
+
+    template <int PER>
+    __device__ void load(int64_t nkeys, int64_t k0, uint32_t (&c)[1][PER]) const
+    {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int64_t k = k0 + j;
+            c[0][j] = 0;
+            if (k < nkeys)
+                c[0][j] = key_start[k + 1] - key_start[k - min((int)(k & (nb - 1)), mk - 1)];
+        }
     }
-    for (int o = 32; o > 0; o >>= 1)
-        nany += (uint32_t)__shfl_xor((int)nany, o);
-    if (__lane_id() == 0)
-        s_any[threadIdx.x / 64] = nany;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t tot = s_any[0] + s_any[1] + s_any[2] + s_any[3];
-        if (tot)
-            atomicAdd(&stats[CNT_BANDS], (unsigned long long)tot);
+    template <int PER>
+    __device__ void store(int64_t nkeys, int64_t k0, const uint32_t (&)[PER],
+                          const uint32_t (&)[1][PER], const uint32_t (&tot)[PER]) const
+    {
+        __shared__ uint32_t s_any[SCAN_BLOCK / 64];
+        uint32_t bits = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            bits |= (tot[j] ? 1u : 0u) << j;
+        uint32_t any = __popc(bits);
+        // a word's bits lie in W / PER consecutive lanes
+        const int W = min(nb, 32), lane = __lane_id(), g = max(W / PER, 1);
+        uint32_t word = bits << (PER * (lane & (g - 1)));
+        for (int o = 1; o < g; o <<= 1)
+            word |= (uint32_t)__shfl_xor((int)word, o);
+        if (k0 < nkeys && (lane & (g - 1)) == 0)
+            masks[k0 / W] = word;
+        for (int o = 32; o > 0; o >>= 1)
+            any += (uint32_t)__shfl_xor((int)any, o);
+        if (lane == 0)
+            s_any[threadIdx.x / 64] = any;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t t = 0;
+            for (int k = 0; k < SCAN_BLOCK / 64; ++k)
+                t += s_any[k];
+            // (added up by the column sort: atomics on one word serialise)
+            bands_part[blockIdx.x] = t;
+        }
     }
-}
+    __device__ void finish(int64_t, uint32_t, unsigned long long *) const {}
+};
 
 // ---- batched band pass -------------------------------------------------------------------
 // One workgroup per work item: up to K band records of the window of band b of
@@ -1109,8 +1287,8 @@ __global__ __launch_bounds__(256) void k_band_combine(const Item *__restrict__ i
 }
 
 // ---- batched column pass -------------------------------------------------------------------
-// Block (cb, c): column block cb of chunk c (up to 32 consecutive tasks of
-// one tower).  For every task the column block of its subgrid is inverse
+// Block (cb, c): column block cb of chunk c (consecutive tasks of one
+// tower).  For every task the column block of its subgrid is inverse
 // FFT'd with the first stage reading straight from HBM (bands without records
 // are zero and are not read) and the last stage's outputs, which stay with
 // their thread, multiplied by E^wp = exp(-2 pi i wp winc base) and
@@ -1185,11 +1363,11 @@ __global__ __launch_bounds__(CB *((1 << LOGN) / 8)) void k_tower_cols(
         for (int k = first; k < last; ++k) {
             const T2 *g = G + (size_t)(k - t0) * n * n + (size_t)blockIdx.x * n * CB + line;
             // band b of the task was written iff it has work items (bit b of
-            // the task's mask; uniform loads)
+            // its slot's mask; uniform loads)
             uint32_t bm[MW];
 #pragma unroll
             for (int q = 0; q < MW; ++q)
-                bm[q] = band_masks[(size_t)k * MW + q];
+                bm[q] = band_masks[(size_t)bref.task_slot[k] * MW + q];
             const int wp = task_wp[k];
             if (run > 0 && (run == SCREEN_RUN || wp != wp_prev + 1)) {
                 close_run(wp_prev);
@@ -1258,51 +1436,134 @@ __global__ __launch_bounds__(256) void k_tower_reduce(const T2 *__restrict__ P, 
     }
 }
 
-// ---- fold ------------------------------------------------------------------------------------
-// Owner computes: each master pixel sums the towers whose window covers it.
-// Channel c's master grid is the c-th N x N grid; its towers have ids
-// (c cc + cy) cc + cx.
+// One batch holds every task: the partial images of rank blockIdx.y's chunks are added
+// as the rows [B blockIdx.x, + B) of its subimage are read for the forward row
+// transform (fft_block, B rows per workgroup, padded lines), so the subimage is
+// written once, transformed, and never cleared.
+template <typename T2, int LOGN, int B>
+__global__ __launch_bounds__(B *((1 << LOGN) / 8)) void k_tower_rows(
+    const T2 *__restrict__ P, T2 *subimg, const T2 *__restrict__ twg,
+    const int32_t *__restrict__ totals, const int32_t *__restrict__ rank_chunk0,
+    const int32_t *__restrict__ rank_nchunk)
+{
+    constexpr int n = 1 << LOGN, NT = B * (n / 8), LS = B + 1;
+    static_assert(n % B == 0, "whole blocks of rows");
+    __shared__ T2 lds[n * LS];
+    __shared__ T2 tw[n];
+    const int r = blockIdx.y;
+    if (r >= totals[1])
+        return;
+    for (int k = threadIdx.x; k < n; k += NT)
+        tw[k] = twg[k];
+    const int c0 = rank_chunk0[r], c1 = min(totals[2], c0 + rank_nchunk[r]);
+    const size_t row0 = (size_t)blockIdx.x * B * n;
+    constexpr int PER = 8; // elements per thread
+    T2 a[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        a[q].x = a[q].y = 0;
+#pragma unroll 4
+    for (int c = c0; c < c1; ++c) {
+        const T2 *p = P + (size_t)c * n * n + row0 + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const T2 v = p[q * NT];
+            a[q].x += v.x;
+            a[q].y += v.y;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = (int)threadIdx.x + q * NT, line = e / n, idx = e % n;
+        lds[idx * LS + line] = a[q];
+    }
+    __syncthreads();
+    fft_block<T2, LOGN, B, LS, false>(lds, tw);
+    T2 *out = subimg + (size_t)r * n * n + row0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = (int)threadIdx.x + q * NT, line = e / n, idx = e % n;
+        out[e] = lds[idx * LS + line];
+    }
+}
+
+template <typename T2, int LOGN>
+static int launch_tower_rows_t(const T2 *P, T2 *subimg, const T2 *tw, const int32_t *totals,
+                               const int32_t *rank_chunk0, const int32_t *rank_nchunk, int ntowers,
+                               hipStream_t s)
+{
+    // one wavefront per workgroup: few towers leave few rows to share out
+    constexpr int n = 1 << LOGN, TPL = n / 8, B = 64 / TPL;
+    hipLaunchKernelGGL((k_tower_rows<T2, LOGN, B>), dim3(n / B, (unsigned)ntowers), dim3(B * TPL), 0,
+                       s, P, subimg, tw, totals, rank_chunk0, rank_nchunk);
+    RG_HIP(hipGetLastError());
+    return RG_OK;
+}
+
 template <typename T2>
-__global__ __launch_bounds__(256) void k_fold(double2 *grid, int N, int64_t total,
+static int launch_tower_rows(int n, const T2 *P, T2 *subimg, const T2 *tw, const int32_t *totals,
+                             const int32_t *rank_chunk0, const int32_t *rank_nchunk, int ntowers,
+                             hipStream_t s)
+{
+    switch (n) {
+    case 64: return launch_tower_rows_t<T2, 6>(P, subimg, tw, totals, rank_chunk0, rank_nchunk, ntowers, s);
+    case 128: return launch_tower_rows_t<T2, 7>(P, subimg, tw, totals, rank_chunk0, rank_nchunk, ntowers, s);
+    case 256: return launch_tower_rows_t<T2, 8>(P, subimg, tw, totals, rank_chunk0, rank_nchunk, ntowers, s);
+    default: return launch_tower_rows_t<T2, 9>(P, subimg, tw, totals, rank_chunk0, rank_nchunk, ntowers, s);
+    }
+}
+
+// ---- fold ------------------------------------------------------------------------------------
+// Owner computes: each master pixel sums the towers whose window covers it and
+// is written, covered or not (the grid needs no clearing).  Channel c's master
+// grid is the c-th N x N grid; its towers have ids (c cc + cy) cc + cx.  n is a
+// power of two, so that 1 / n^2 is exact.  Grid (N / 256 rounded up, rows of all
+// channels): a workgroup's row and its towers' rows are uniform.
+template <typename T2>
+__global__ __launch_bounds__(256) void k_fold(double2 *grid, int N, int64_t rows,
                                               const T2 *subimg, const int32_t *rank_of_tower, int n,
                                               int margin, int chunk, int cc)
 {
-    const int64_t NN = (int64_t)N * N;
-    for (int64_t gidx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; gidx < total;
-         gidx += (int64_t)gridDim.x * blockDim.x) {
-        const int ch = (int)(gidx / NN);
-        const int64_t idx = gidx - (int64_t)ch * NN;
-        const int py = (int)(idx / N), px = (int)(idx - (int64_t)py * N);
-        const int x = px - N / 2, y = py - N / 2;
-        const double norm = (double)n * (double)n;
+    const int px = (int)(blockIdx.x * 256 + threadIdx.x);
+    const double inv = 1.0 / ((double)n * (double)n);
+    const int ax = px + margin / 2, cxh = min(cc - 1, ax / chunk);
+    for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
+        const int ch = (int)(row / N), py = (int)(row - (int64_t)ch * N);
+        const int ay = py + margin / 2, cyh = min(cc - 1, ay / chunk);
+        if (px >= N)
+            continue;
         double re = 0.0, im = 0.0;
-        bool any = false;
-        const int ax = x + N / 2 + margin / 2, ay = y + N / 2 + margin / 2;
-        const int cxh = min(cc - 1, ax / chunk), cyh = min(cc - 1, ay / chunk);
         for (int cy = max(0, cyh - 2); cy <= cyh; ++cy) {
-            const int y0 = chunk * cy - N / 2 - margin / 2;
-            if (y < y0 || y >= y0 + n)
+            const int y = ay - chunk * cy; // row in the tower's window
+            if (y < 0 || y >= n)
                 continue;
             for (int cx = max(0, cxh - 2); cx <= cxh; ++cx) {
-                const int x0 = chunk * cx - N / 2 - margin / 2;
-                if (x < x0 || x >= x0 + n)
+                const int x = ax - chunk * cx;
+                if (x < 0 || x >= n)
                     continue;
                 const int rk = rank_of_tower[(ch * cc + cy) * cc + cx];
                 if (rk < 0)
                     continue;
-                const T2 s = subimg[(size_t)rk * n * n + (size_t)(y - y0) * n + (x - x0)];
-                re += (double)s.x / norm;
-                im += (double)s.y / norm;
-                any = true;
+                const T2 s = subimg[(size_t)rk * n * n + (size_t)y * n + x];
+                re += (double)s.x * inv;
+                im += (double)s.y * inv;
             }
         }
-        if (any) {
-            double2 g = grid[gidx];
-            g.x += re;
-            g.y += im;
-            grid[gidx] = g;
-        }
+        grid[row * N + px] = make_double2(re, im);
     }
+}
+
+template <typename T2>
+static int launch_fold(double2 *grid, int N, int nchan, const T2 *subimg,
+                       const int32_t *rank_of_tower, int n, int margin, int chunk, int cc,
+                       hipStream_t s)
+{
+    const int64_t rows = (int64_t)N * nchan;
+    hipLaunchKernelGGL((k_fold<T2>),
+                       dim3((unsigned)((N + 255) / 256), (unsigned)std::min<int64_t>(rows, 65535)),
+                       dim3(256), 0, s, grid, N, rows, subimg, rank_of_tower, n, margin, chunk, cc);
+    RG_HIP(hipGetLastError());
+    return RG_OK;
 }
 
 // ---- plain-mode kernels ---------------------------------------------------------------------
@@ -1538,6 +1799,11 @@ struct WtGeom {
     int64_t ntw; // tower ids: nchan cc^2
 };
 
+// Sort counters of a W-towers call in all: (task, band) keys get 4 counter
+// replicas at the reference's workload (the scans read every replica; 16 were
+// slower).
+constexpr int64_t WT_COUNTERS = (int64_t)1 << 20;
+
 static WtGeom wt_geom(const rg_grid_params *p, const rg_wkern *wk, int nchan, int H)
 {
     WtGeom g;
@@ -1585,21 +1851,36 @@ static TowerKeyer wt_keyer(const rg_grid_params *p, const rg_flat_vis *vis, cons
     return kf;
 }
 
-// Floor range of the call into d_range[0..1] (on the device).
-static int floor_range(const rg_grid_params *p, const rg_flat_vis *vis, const WtGeom &g,
-                       int *d_range, hipStream_t s)
+// The launch that finds the floor range into d_range[0..1] (d_range: RANGE_BYTES, the
+// range, then the workgroups' parts), builds the padded kernel table (pad NULL: none) and
+// clears the areas of zero.
+template <typename T2>
+static int wt_prepare(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis,
+                      const WtGeom &g, int *d_range, const PadJob<T2> *pad, ZeroList &zero,
+                      hipStream_t s)
 {
-    // d_range: RANGE_BYTES (the range, then the workgroups' parts)
-    int2 *part = reinterpret_cast<int2 *>(reinterpret_cast<char *>(d_range) + 256);
-    int64_t blocks = (vis->n + 256 * RANGE_VPT - 1) / (256 * RANGE_VPT);
-    if (blocks > RANGE_BLOCKS)
-        blocks = RANGE_BLOCKS;
-    if (blocks > 0)
-        hipLaunchKernelGGL(k_floor_range, dim3((unsigned)blocks), dim3(256), 0, s, vis->u, vis->v,
-                           vis->w, vis->n, p->theta, g.N, g.chunk, g.cc, p->winc, part);
-    hipLaunchKernelGGL(k_range_finish, dim3(1), dim3(1024), 0, s, (const int2 *)part,
-                       (int)blocks, d_range);
+    RangeJob r;
+    r.u = vis->u;
+    r.v = vis->v;
+    r.w = vis->w;
+    r.n = vis->n;
+    r.theta = p->theta;
+    r.winc = p->winc;
+    r.N = g.N;
+    r.chunk = g.chunk;
+    r.cc = g.cc;
+    r.range = d_range;
+    r.part = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(d_range) + 256);
+    RG_TRY(range_done_counter(ctx, &r.done, s));
+    r.blocks = (unsigned)std::max<int64_t>(
+        1, std::min<int64_t>((vis->n + 256 * RANGE_VPT - 1) / (256 * RANGE_VPT), RANGE_BLOCKS));
+    PadJob<T2> pj{};
+    if (pad)
+        pj = *pad;
+    hipLaunchKernelGGL((k_wt_prepare<T2>), dim3(r.blocks + pj.blocks + zero.blocks()), dim3(256), 0,
+                       s, r, pj, zero);
     RG_HIP(hipGetLastError());
+    zero.n = 0;
     return RG_OK;
 }
 
@@ -1632,12 +1913,13 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
 {
     const WtGeom g = wt_geom(p, wk, 1, 0);
     const int N = g.N, n = g.n, M = g.M, S = g.S, cc = g.cc;
-    RG_TRY(zero_fill(grid, sizeof(double2) * (size_t)N * N, s));
+    ZeroList zero;
+    RG_TRY(zero.add(grid, sizeof(double2) * (size_t)N * N));
     if (vis->n == 0)
-        return RG_OK;
+        return zero.launch(s);
     RG_TRY(ctx->scratch[8].ensure(RANGE_BYTES));
     int *d_range = ctx->scratch[8].as<int>();
-    RG_TRY(floor_range(p, vis, g, d_range, s));
+    RG_TRY(wt_prepare<double2>(ctx, p, vis, g, d_range, nullptr, zero, s));
     int wp_min = 0, nwp = 0;
     bool empty = false;
     RG_TRY(read_range(ctx, d_range, wp_min, nwp, empty, s));
@@ -1651,7 +1933,6 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
     const TowerKeyer kf = wt_keyer(p, vis, wk, g, d_range, nwp, nullptr);
     const int64_t nslots = (int64_t)cc * cc * nwp;
     BinResult br;
-    ZeroList zero;
     RG_TRY((bin_visibilities<TowerKeyer, double>(ctx, kf, vis->n, nslots, 0x40000000u, zero, s, br,
                                                  (int64_t)1 << 20)));
     RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (2 * nslots + 1)));
@@ -1742,12 +2023,7 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
         RG_TRY(fft2d(ctx, img, RG_C128, n, 1, -1, s));
     }
     KernelTimer kt_finish(ctx, RG_TIMER_TOWER_FINISH, s);
-    const int64_t npx = (int64_t)N * N;
-    hipLaunchKernelGGL((k_fold<double2>), dim3((unsigned)std::min<int64_t>((npx + 255) / 256, 65536)),
-                       dim3(256), 0, s, (double2 *)grid, N, npx, (const double2 *)subimg,
-                       (const int32_t *)d_rot, n, M, g.chunk, cc);
-    RG_HIP(hipGetLastError());
-    return RG_OK;
+    return launch_fold<double2>((double2 *)grid, N, 1, subimg, d_rot, n, M, g.chunk, cc, s);
 }
 
 // ---- batched mode ----------------------------------------------------------------------------
@@ -1760,21 +2036,55 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
 // stream never reads back: it needs a plan from an eager call of its shape,
 // and an overrun is reported by rg_context_stats.
 
+// Records per band work item when the caller leaves it open: items of 1024 up
+// to about half a million visibilities, where the longest item decides, 4096
+// from 2 M, where every split costs a spilled band and its sum (band pass and
+// sum of spilled parts: 520 k FP32 204 us at 2048, 180 at 1024, 179 at 512;
+// FP64 343 / 346 / 361; 8.4 M FP32 2025 us at 2048, 1952 at 4096).
+static uint32_t default_band_item(int64_t nvis)
+{
+    return nvis < (1 << 20) ? 1024u : nvis < (1 << 21) ? 2048u : 4096u;
+}
+
 static bool plan_fits(const WtPlan &pl, const rg_grid_params *p, const rg_flat_vis *vis,
                       const rg_wkern *wk, int nchan, int H, int type)
 {
     return pl.valid && pl.N == p->grid_size && pl.n == p->subgrid_size &&
            pl.M == p->subgrid_margin && pl.S == wk->size && pl.R == wk->oversampling &&
            pl.P == wk->plane_count && pl.H == H && pl.type == type && pl.nchan == nchan &&
-           pl.K == (p->vis_per_item > 0 ? p->vis_per_item : 2048) &&
+           (p->vis_per_item > 0 ? !pl.k_auto && pl.K == (uint32_t)p->vis_per_item : pl.k_auto) &&
            pl.floor_batch == p->floor_batch && pl.theta == p->theta && pl.winc == p->winc &&
            pl.w_min == wk->w_min && pl.w_step == wk->w_step && vis->n <= pl.nvis;
 }
 
+// Table layout (int32): 6 per-tower arrays, 2 per-task, 2 per-chunk, one per
+// slot, totals, the batches' spill counters.
+struct TableLayout {
+    size_t o_tn, o_to, o_co, o_rot, o_rc0, o_rnc, o_ts, o_twp, o_cf, o_cn, o_ros, o_tot, o_spill,
+        end;
+    TableLayout(int64_t ntw, int64_t nslots, int64_t ntasks, int64_t nchunks, int64_t nbatch)
+    {
+        o_tn = 0;
+        o_to = o_tn + ntw;
+        o_co = o_to + ntw;
+        o_rot = o_co + ntw;
+        o_rc0 = o_rot + ntw;
+        o_rnc = o_rc0 + ntw;
+        o_ts = o_rnc + ntw;
+        o_twp = o_ts + ntasks;
+        o_cf = o_twp + ntasks;
+        o_cn = o_cf + nchunks;
+        o_ros = o_cn + nchunks;
+        o_tot = o_ros + nslots;
+        o_spill = (o_tot + 16 + 3) / 4 * 4; // 16-byte aligned: cleared per call
+        end = o_spill + nbatch;
+    }
+};
+
 template <typename T>
 static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis,
                              const int64_t *d_off, int nchan, const rg_wkern *wk, void *grid,
-                             hipStream_t s, bool capturing, bool measure)
+                             hipStream_t s, bool measure)
 {
     using T2 = typename Vec2<T>::type;
     const int H = band_height_of(p, sizeof(T) == 4);
@@ -1782,19 +2092,74 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     const int n = g.n, S = g.S, NB = g.NB;
     const size_t nn = (size_t)n * n;
     const int type = sizeof(T) == 4 ? RG_C64 : RG_C128;
-    const uint32_t K = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item : 2048u;
     WtPlan &pl = ctx->wt_plan;
+    const uint32_t K = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item
+                       : measure           ? default_band_item(vis->n)
+                                           : pl.K;
     auto *stats = ctx->counters.as<unsigned long long>();
+    const size_t grid_bytes = sizeof(double2) * (size_t)g.N * g.N * nchan;
+    ZeroList zero;
+    RG_TRY(zero.add(stats, sizeof(unsigned long long) * CNT__N));
+    if (vis->n == 0) {
+        RG_TRY(zero.add(grid, grid_bytes));
+        return zero.launch(s);
+    }
 
-    RG_TRY(zero_fill(grid, sizeof(double2) * (size_t)g.N * g.N * nchan, s));
-    if (vis->n == 0)
-        return RG_OK;
+    // the FP32 band pass reads the table with zero rows after every sub-kernel;
+    // taps are addressed by 32-bit byte offsets
+    const int64_t nsub = (int64_t)wk->plane_count * wk->oversampling * wk->oversampling;
+    const int64_t krows = padded_taps<T>() ? (int64_t)H + nsub * padded_rows(S, H) : nsub * S;
+    const int64_t kbytes = krows * S * (int64_t)sizeof(T2);
+    PadJob<T2> pad{};
+    if (padded_taps<T>() && kbytes < ((int64_t)1 << 31)) {
+        RG_TRY(ctx->scratch[12].ensure((size_t)kbytes));
+        pad.src = (const T2 *)wk->data;
+        pad.dst = ctx->scratch[12].as<T2>();
+        pad.nsub = nsub;
+        pad.S = S;
+        pad.H = H;
+        pad.blocks = (unsigned)std::min<int64_t>((krows * S + 255) / 256, 4096);
+    }
 
-    // floor range (device); the plan fixes the floors per tower slot
+    // Capacities: tables by the slot count, buffers by the plan (or, measuring,
+    // by the counts read back below).  With a plan everything a call clears
+    // is known before its first launch.
+    const int ntw = (int)g.ntw;
+    constexpr size_t BATCH_BYTES = (size_t)16 << 30;
+    const int q_fit = (int)std::max<size_t>(1, BATCH_BYTES / (sizeof(T2) * nn));
+    auto batch_tasks_of = [&](int ntasks) { // tasks per batch: all while they fit 16 GiB
+        return std::max(1, std::min(ntasks, p->floor_batch > 0 ? p->floor_batch : q_fit));
+    };
+    int nwp_cap = pl.nwp_cap, ntasks_cap = pl.ntasks_cap, nchunks_cap = pl.nchunks_cap,
+        ntowers_cap = pl.ntowers_cap, nitems_cap = pl.nitems_cap;
     RG_TRY(ctx->scratch[8].ensure(RANGE_BYTES));
     int *d_range = ctx->scratch[8].as<int>();
-    RG_TRY(floor_range(p, vis, g, d_range, s));
-    int nwp_cap;
+    T2 *subimg = nullptr;
+    auto clear_subimages = [&](int nbatch, uint32_t *spill_ctr) {
+        RG_TRY(ctx->scratch[10].ensure(sizeof(T2) * nn * ntowers_cap));
+        subimg = ctx->scratch[10].as<T2>();
+        if (nbatch > 1) // one batch writes them
+            RG_TRY(zero.add(subimg, sizeof(T2) * nn * ntowers_cap));
+        return zero.add(spill_ctr, sizeof(uint32_t) * nbatch);
+    };
+    auto table_layout = [&]() {
+        const int q = batch_tasks_of(ntasks_cap);
+        return TableLayout(ntw, g.ntw * nwp_cap, ntasks_cap, nchunks_cap,
+                           (ntasks_cap + q - 1) / q);
+    };
+    const BinPlan *ready = nullptr;
+    BinPlan bin;
+    if (!measure) {
+        const TableLayout tl = table_layout();
+        RG_TRY(ctx->scratch[18].ensure(sizeof(int32_t) * tl.end));
+        const int q = batch_tasks_of(ntasks_cap);
+        RG_TRY(clear_subimages((ntasks_cap + q - 1) / q,
+                               ctx->scratch[18].as<uint32_t>() + tl.o_spill));
+        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, 0x40000000u, WT_COUNTERS, zero,
+                               bin)));
+        ready = &bin;
+    }
+    RG_TRY(wt_prepare<T2>(ctx, p, vis, g, d_range, &pad, zero, s));
     if (measure) {
         int wp_min = 0, nwp = 0;
         bool empty = false;
@@ -1804,11 +2169,9 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
             cnt[CNT_DROPPED] = (unsigned long long)vis->n;
             RG_HIP(hipMemcpyAsync(ctx->counters.p, cnt, sizeof(cnt), hipMemcpyHostToDevice, s));
             RG_HIP(hipStreamSynchronize(s));
-            return RG_OK;
+            return zero_fill(grid, grid_bytes, s);
         }
         nwp_cap = nwp + nwp / 8 + 4;
-    } else {
-        nwp_cap = pl.nwp_cap;
     }
     const int64_t nslots = g.ntw * nwp_cap;
     const int64_t nkeys = nslots * NB;
@@ -1828,80 +2191,74 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     RG_TRY(ctx->scratch[4].ensure(sizeof(Item) * std::max<int64_t>(nkeys + 1, max_items_w)));
     const TowerKeyer kf = wt_keyer(p, vis, wk, g, d_range, nwp_cap, d_off);
     BinResult br;
-    // (task, band) keys: 4 counter replicas at the reference's workload (the
-    // scans read every replica; 16 were slower, 1 << 20 counters in all)
-    ZeroList zero;
+    RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (nslots + 1)));
+    uint32_t *slot_start = ctx->scratch[9].as<uint32_t>();
+    br.group_start = slot_start;
+    br.group_keys = NB;
     RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, 0x40000000u, zero, s, br,
-                                            (int64_t)1 << 20)));
+                                            WT_COUNTERS, ready)));
 
-    // capacities: tables by the slot count, buffers by the plan (or, measuring,
-    // by the counts read back below)
-    const int ntw = (int)g.ntw;
-    const int64_t nchunks_bound = nslots / TASKS_PER_CHUNK + g.ntw;
-    int ntasks_cap, nchunks_cap, ntowers_cap, nitems_cap;
     if (measure) {
         ntasks_cap = (int)std::min<int64_t>(nslots, 0x7fffffff);
-        nchunks_cap = (int)std::min<int64_t>(nchunks_bound, 0x7fffffff);
+        // (enough for the shortest chunks, so that no later call needs larger tables)
+        nchunks_cap =
+            (int)std::min<int64_t>(nslots / TASKS_PER_CHUNK_MIN + g.ntw, 0x7fffffff);
         ntowers_cap = ntw;
         nitems_cap = (int)std::min<int64_t>(max_items_w, 0x7fffffff);
-    } else {
-        ntasks_cap = pl.ntasks_cap;
-        nchunks_cap = pl.nchunks_cap;
-        ntowers_cap = pl.ntowers_cap;
-        nitems_cap = pl.nitems_cap;
     }
-    // table layout (int32): 7 per-tower arrays, 3 per-task, 2 per-chunk, one
-    // per slot, totals
-    const size_t o_tn = 0, o_to = o_tn + ntw, o_co = o_to + ntw, o_rot = o_co + ntw,
-                 o_tor = o_rot + ntw, o_rc0 = o_tor + ntw, o_rnc = o_rc0 + ntw,
-                 o_ts = o_rnc + ntw, o_twp = o_ts + ntasks_cap, o_trk = o_twp + ntasks_cap,
-                 o_cf = o_trk + ntasks_cap, o_cn = o_cf + nchunks_cap, o_ros = o_cn + nchunks_cap,
-                 o_tot = o_ros + nslots, o_end = o_tot + 16;
-    RG_TRY(ctx->scratch[18].ensure(sizeof(int32_t) * o_end));
+    const TableLayout tl = table_layout();
+    RG_TRY(ctx->scratch[18].ensure(sizeof(int32_t) * tl.end));
     int32_t *tab = ctx->scratch[18].as<int32_t>();
     TaskTables tt;
-    tt.tower_ntasks = tab + o_tn;
-    tt.tower_task_off = tab + o_to;
-    tt.tower_chunk_off = tab + o_co;
-    tt.rank_of_tower = tab + o_rot;
-    tt.tower_of_rank = tab + o_tor;
-    tt.rank_chunk0 = tab + o_rc0;
-    tt.rank_nchunk = tab + o_rnc;
-    tt.task_slot = tab + o_ts;
-    tt.task_wp = tab + o_twp;
-    tt.task_rank = tab + o_trk;
-    tt.chunk_first = tab + o_cf;
-    tt.chunk_count = tab + o_cn;
-    tt.rank_of_slot = tab + o_ros;
-    tt.totals = tab + o_tot;
+    tt.tower_ntasks = tab + tl.o_tn;
+    tt.tower_task_off = tab + tl.o_to;
+    tt.tower_chunk_off = tab + tl.o_co;
+    tt.rank_of_tower = tab + tl.o_rot;
+    tt.rank_chunk0 = tab + tl.o_rc0;
+    tt.rank_nchunk = tab + tl.o_rnc;
+    tt.task_slot = tab + tl.o_ts;
+    tt.task_wp = tab + tl.o_twp;
+    tt.chunk_first = tab + tl.o_cf;
+    tt.chunk_count = tab + tl.o_cn;
+    tt.rank_of_slot = tab + tl.o_ros;
+    tt.totals = tab + tl.o_tot;
+    uint32_t *spill_ctr = reinterpret_cast<uint32_t *>(tab + tl.o_spill);
     tt.ntw = ntw;
     tt.nwp = nwp_cap;
-    tt.nk = NB;
+    tt.tpc = measure ? TASKS_PER_CHUNK_MAX : pl.tpc;
     tt.ntasks_cap = ntasks_cap;
     tt.nchunks_cap = nchunks_cap;
     tt.ntowers_cap = ntowers_cap;
-    hipLaunchKernelGGL(k_tower_count, dim3(ntw), dim3(256), 0, s, (const uint32_t *)br.vis_start,
-                       tt);
-    hipLaunchKernelGGL(k_tower_scan, dim3(1), dim3(1024), 0, s, tt, stats);
-    hipLaunchKernelGGL(k_tower_tasks, dim3(ntw), dim3(256), 0, s, (const uint32_t *)br.vis_start,
-                       tt, (const int *)d_range);
+    if (ntw <= TABLE_TOWERS && nslots <= TABLE_SLOTS) {
+        hipLaunchKernelGGL(k_tower_tables, dim3(1), dim3(1024), 0, s, slot_start, tt, (int)nslots, 
+                           (const int *)d_range, stats);
+    } else {
+        hipLaunchKernelGGL(k_tower_count, dim3(ntw), dim3(256), 0, s,
+                           (const uint32_t *)slot_start, tt);
+        hipLaunchKernelGGL(k_tower_scan, dim3(1), dim3(1024), 0, s, tt, stats);
+        hipLaunchKernelGGL(k_tower_tasks, dim3(ntw), dim3(256), 0, s,
+                           (const uint32_t *)slot_start, tt, (const int *)d_range);
+    }
     RG_HIP(hipGetLastError());
 
-    // band window work items (in the binning's item_start slot; window lengths
-    // and prefix in the count / cursor slots)
-    RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (nkeys + 1)));
-    uint32_t *d_wstart = ctx->scratch[9].as<uint32_t>();
-    uint32_t *item_start_w = br.item_start;
+    // band window work items (their starts in the sort's cursor slot) and the
+    // slots' written bands
+    const int mw = (NB + 31) / 32;
+    RG_TRY(ctx->scratch[19].ensure(sizeof(uint32_t) * ((size_t)nslots * mw + scan_blocks(nkeys))));
+    uint32_t *band_masks = ctx->scratch[19].as<uint32_t>();
+    uint32_t *bands_part = band_masks + (size_t)nslots * mw;
+    uint32_t *item_start_w = ctx->scratch[3].as<uint32_t>();
     Item *items_w = br.items;
-    uint32_t *prefix = ctx->scratch[3].as<uint32_t>();
     {
         KernelTimer kt(ctx, RG_TIMER_BINNING, s);
-        uint32_t *len = ctx->scratch[0].as<uint32_t>();
-        const unsigned wblocks = (unsigned)std::min<int64_t>((nkeys + 255) / 256, 1024);
-        hipLaunchKernelGGL(k_window_len, dim3(wblocks), dim3(256), 0, s,
-                           (const uint32_t *)br.vis_start, nkeys, NB, g.mk, len, d_wstart, stats);
-        RG_HIP(hipGetLastError());
-        RG_TRY(items_from_lengths(ctx, len, nkeys, K, prefix, item_start_w, items_w, s));
+        WindowSource win;
+        win.key_start = br.vis_start;
+        win.nb = NB;
+        win.mk = g.mk;
+        win.masks = band_masks;
+        win.bands_part = bands_part;
+        RG_TRY(scan_source(win, nkeys, K, ctx->scratch[6].as<uint2>(), item_start_w, items_w,
+                           stats, s));
     }
 
     if (measure) {
@@ -1922,6 +2279,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         pl.type = type;
         pl.nchan = nchan;
         pl.K = K;
+        pl.k_auto = p->vis_per_item <= 0;
         pl.floor_batch = p->floor_batch;
         pl.theta = p->theta;
         pl.winc = p->winc;
@@ -1930,11 +2288,17 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         pl.nvis = vis->n;
         pl.nwp_cap = nwp_cap;
         pl.ntasks_cap = (int)std::min<int64_t>(ntasks_cap, nt + nt / 8 + 16);
-        pl.nchunks_cap = (int)std::min<int64_t>(nchunks_cap, nch + nch / 8 + 16);
+        // later calls cut the towers' tasks into shorter chunks: at most one
+        // partial chunk per tower beside the whole ones
+        pl.tpc = tasks_per_chunk(nt, n);
+        const int64_t nch_later =
+            pl.tpc == TASKS_PER_CHUNK_MAX ? nch : nt / pl.tpc + std::min<int64_t>(ntow, nt);
+        pl.nchunks_cap = (int)std::min<int64_t>(nslots / pl.tpc + g.ntw,
+                                                std::max(nch, nch_later) + nch_later / 8 + 16);
         pl.ntowers_cap = (int)std::min<int64_t>(ntw, ntow + ntow / 8 + 4);
         pl.nitems_cap = (int)std::min<int64_t>(max_items_w, nit + nit / 8 + 64);
         if (nt == 0)
-            return RG_OK;
+            return zero_fill(grid, grid_bytes, s);
         // this call's buffers use the plan's capacities (the tables above were
         // built with the slot-count bounds, which hold every index)
         ntasks_cap = pl.ntasks_cap;
@@ -1944,19 +2308,20 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         pl.valid = true;
     }
 
-    // subimages (one per active tower, by rank)
-    RG_TRY(ctx->scratch[10].ensure(sizeof(T2) * nn * ntowers_cap));
-    T2 *subimg = ctx->scratch[10].as<T2>();
-    RG_TRY(zero_fill(subimg, sizeof(T2) * nn * ntowers_cap, s));
-    const void *tw_inv = nullptr, *tw_stage = nullptr;
+    const void *tw_inv = nullptr, *tw_fwd = nullptr, *tw_stage = nullptr;
     RG_TRY(get_twiddles(ctx, n, type, +1, &tw_inv));
+    RG_TRY(get_twiddles(ctx, n, type, -1, &tw_fwd));
     RG_TRY(get_stage_twiddles(ctx, n, type, +1, &tw_stage));
 
-    // batches of Q tasks (by default every task while the subgrids fit 16 GiB)
-    constexpr size_t BATCH_BYTES = (size_t)16 << 30;
-    const int q_fit = (int)std::max<size_t>(1, BATCH_BYTES / (sizeof(T2) * nn));
-    const int Q = std::max(1, std::min(ntasks_cap, p->floor_batch > 0 ? p->floor_batch : q_fit));
+    // batches of Q tasks
+    const int Q = batch_tasks_of(ntasks_cap);
     const int nbatch = (ntasks_cap + Q - 1) / Q;
+    if (measure) {
+        // the slot-count table layout holds a spill counter for every batch of
+        // the plan's (fewer) tasks
+        RG_TRY(clear_subimages(nbatch, spill_ctr));
+        RG_TRY(zero.launch(s));
+    }
     // spill slots (parts of split keys: at most 2 R / K for R records), per batch
     const uint64_t max_spill = 2 * ((uint64_t)g.mk * vis->n) / K + 1;
     const size_t band_bytes = sizeof(T2) * (size_t)H * n;
@@ -1964,20 +2329,15 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     const size_t p_bytes = sizeof(T2) * nn * (size_t)nchunks_cap;
     const size_t sp_bytes = band_bytes * max_spill;
     const size_t is_bytes = (sizeof(uint32_t) * (size_t)max_items_w + 255) / 256 * 256;
-    const size_t ctr_bytes = (sizeof(uint32_t) * nbatch + 255) / 256 * 256;
     const size_t si_bytes = sizeof(uint32_t) * (size_t)max_spill;
-    RG_TRY(ctx->scratch[7].ensure(g_bytes + p_bytes + sp_bytes + is_bytes + ctr_bytes +
-                                  si_bytes));
+    RG_TRY(ctx->scratch[7].ensure(g_bytes + p_bytes + sp_bytes + is_bytes + si_bytes));
     char *base7 = ctx->scratch[7].as<char>();
     T2 *G = reinterpret_cast<T2 *>(base7);
     T2 *Pp = reinterpret_cast<T2 *>(base7 + g_bytes);
     T2 *spill = reinterpret_cast<T2 *>(base7 + g_bytes + p_bytes);
     uint32_t *item_spill = reinterpret_cast<uint32_t *>(base7 + g_bytes + p_bytes + sp_bytes);
-    uint32_t *spill_ctr =
+    uint32_t *spill_item =
         reinterpret_cast<uint32_t *>(base7 + g_bytes + p_bytes + sp_bytes + is_bytes);
-    uint32_t *spill_item = reinterpret_cast<uint32_t *>(base7 + g_bytes + p_bytes + sp_bytes +
-                                                        is_bytes + ctr_bytes);
-    RG_TRY(zero_fill(spill_ctr, sizeof(uint32_t) * nbatch, s));
 
     // every work item's records sorted by footprint column into the expanded
     // array (window records laid out item after item)
@@ -1987,9 +2347,11 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     {
         KernelTimer kt(ctx, RG_TIMER_BINNING, s);
         hipLaunchKernelGGL((k_sort_items<T>),
-                           dim3((unsigned)std::min<int64_t>(max_items_w, 8192)), dim3(256), 0, s,
-                           (const Rec<T> *)br.recs, sorted, (const Item *)items_w, stats,
-                           (const uint32_t *)prefix, (const uint32_t *)d_wstart, n + S, S, H, NB);
+                           dim3((unsigned)std::min<int64_t>(std::max(nitems_cap, 1), 8192)),
+                           dim3(256), 0, s, (const Rec<T> *)br.recs, sorted, (const Item *)items_w,
+                           stats, (const uint32_t *)br.vis_start, (const uint32_t *)item_start_w, K,
+                           g.mk, n + S, S, H, NB, (const uint32_t *)bands_part,
+                           (int)scan_blocks(nkeys));
         RG_HIP(hipGetLastError());
     }
 
@@ -2003,27 +2365,11 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     bl.bref.totals = tt.totals;
     bl.bref.Q = Q;
     bl.rank_of_slot = tt.rank_of_slot;
-    {
-        // the FP32 band pass reads the table with zero rows after every
-        // sub-kernel; taps are addressed by 32-bit byte offsets
-        const int64_t nsub = (int64_t)wk->plane_count * wk->oversampling * wk->oversampling;
-        const int64_t rows = padded_taps<T>() ? (int64_t)H + nsub * padded_rows(S, H) : nsub * S;
-        const int64_t kb = rows * S * (int64_t)sizeof(T2);
-        if (kb >= ((int64_t)1 << 31))
-            return fail(RG_ERR_UNSUPPORTED, "batched W-towers kernel table too large (%lld bytes)",
-                        (long long)kb);
-        bl.kern = wk->data;
-        if (padded_taps<T>()) {
-            RG_TRY(ctx->scratch[12].ensure((size_t)kb));
-            T2 *padded = ctx->scratch[12].as<T2>();
-            hipLaunchKernelGGL(k_pad_kernels<T2>,
-                               dim3((unsigned)std::min<int64_t>((rows * S + 255) / 256, 65536)),
-                               dim3(256), 0, s, (const T2 *)wk->data, padded, nsub, S, H);
-            RG_HIP(hipGetLastError());
-            bl.kern = padded;
-        }
-        bl.kern_bytes = (uint32_t)kb;
-    }
+    if (kbytes >= ((int64_t)1 << 31))
+        return fail(RG_ERR_UNSUPPORTED, "batched W-towers kernel table too large (%lld bytes)",
+                    (long long)kbytes);
+    bl.kern = padded_taps<T>() ? (const void *)pad.dst : wk->data;
+    bl.kern_bytes = (uint32_t)kbytes;
     bl.tw = tw_stage;
     bl.G = G;
     bl.spill = spill;
@@ -2034,17 +2380,6 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     // one band-pass workgroup per work item (the plan's item capacity; a
     // batch with more items reports an overrun)
     bl.blocks = (uint32_t)std::max(1, nitems_cap);
-    // per task: which bands were written
-    const int mw = (NB + 31) / 32;
-    RG_TRY(ctx->scratch[19].ensure(sizeof(uint32_t) * (size_t)std::max(ntasks_cap, 1) * mw));
-    uint32_t *band_masks = ctx->scratch[19].as<uint32_t>();
-    {
-        const int64_t ne = (int64_t)ntasks_cap * mw;
-        hipLaunchKernelGGL(k_band_masks, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s,
-                           (const uint32_t *)item_start_w, (const int32_t *)tt.task_slot,
-                           (const int32_t *)tt.totals, NB, mw, band_masks);
-        RG_HIP(hipGetLastError());
-    }
     ColsLaunch cl;
     cl.G = G;
     cl.band_masks = band_masks;
@@ -2074,8 +2409,11 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
             KernelTimer kt(ctx, RG_TIMER_TOWER_COLS, s);
             RG_TRY(launch_cols<T>(n, H, cl, s));
         }
-        {
-            KernelTimer kt(ctx, RG_TIMER_TOWER_REDUCE, s);
+        KernelTimer kt(ctx, RG_TIMER_TOWER_REDUCE, s);
+        if (nbatch == 1) {
+            RG_TRY(launch_tower_rows<T2>(n, Pp, subimg, (const T2 *)tw_fwd, tt.totals,
+                                         tt.rank_chunk0, tt.rank_nchunk, ntowers_cap, s));
+        } else {
             hipLaunchKernelGGL((k_tower_reduce<T2>), dim3((unsigned)rgx, rgy), dim3(256), 0, s,
                                (const T2 *)Pp, subimg, (int64_t)nn, bl.bref, b,
                                (const int32_t *)tt.rank_chunk0, (const int32_t *)tt.rank_nchunk,
@@ -2085,14 +2423,11 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     }
 
     KernelTimer kt_finish(ctx, RG_TIMER_TOWER_FINISH, s);
-    RG_TRY(fft2d(ctx, subimg, type, n, ntowers_cap, -1, s, nullptr, tt.totals + 1));
-    const int64_t npx = (int64_t)g.N * g.N * nchan;
-    hipLaunchKernelGGL((k_fold<T2>), dim3((unsigned)std::min<int64_t>((npx + 255) / 256, 1 << 20)),
-                       dim3(256), 0, s, (double2 *)grid, g.N, npx, (const T2 *)subimg,
-                       (const int32_t *)tt.rank_of_tower, n, g.M, g.chunk, g.cc);
-    RG_HIP(hipGetLastError());
-    (void)capturing;
-    return RG_OK;
+    if (nbatch > 1)
+        RG_TRY(fft_rows(ctx, subimg, type, n, (int64_t)n * ntowers_cap, -1, s, tt.totals + 1));
+    RG_TRY(fft_cols(ctx, subimg, type, n, ntowers_cap, -1, s, tt.totals + 1));
+    return launch_fold<T2>((double2 *)grid, g.N, nchan, subimg, tt.rank_of_tower, n, g.M, g.chunk,
+                           g.cc, s);
 }
 
 template <typename T>
@@ -2109,21 +2444,21 @@ static int wtowers_batched(rg_context *ctx, const rg_grid_params *p, const rg_fl
                         "a W-towers call on a capturing stream needs an earlier eager call of the "
                         "same shape (grid, subgrid, kernels, parameters, no more visibilities) on "
                         "this context");
-        return wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, true, false);
+        return wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, false);
     }
     if (fits) {
-        RG_TRY((wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, false, false)));
-        unsigned long long over = 0;
-        RG_HIP(hipMemcpyAsync(&over, ctx->counters.as<unsigned long long>() + CNT_OVERFLOW,
-                              sizeof(over), hipMemcpyDeviceToHost, s));
+        RG_TRY((wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, false)));
+        // into pinned memory: a copy to pageable memory goes through a staging buffer
+        auto *over = static_cast<unsigned long long *>(ctx->counters_host.p);
+        RG_HIP(hipMemcpyAsync(over, ctx->counters.as<unsigned long long>() + CNT_OVERFLOW,
+                              sizeof(*over), hipMemcpyDeviceToHost, s));
         RG_HIP(hipStreamSynchronize(s));
-        if (over == 0)
+        if (*over == 0)
             return RG_OK;
         // a capacity of the plan was too small for this call: measure again
-        RG_TRY(zero_fill(ctx->counters.p, sizeof(unsigned long long) * CNT__N, s));
     }
     ctx->wt_plan.valid = false;
-    return wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, false, true);
+    return wtowers_batched_t<T>(ctx, p, vis, d_off, nchan, wk, grid, s, true);
 }
 
 int wtowers_run(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis,
