@@ -58,3 +58,24 @@ def test_invalid_arguments_are_rejected(ctx):
     grids = torch.zeros((2, 8, 8), dtype=torch.complex64, device="cuda")
     with pytest.raises(rgamd.RGError):
         ctx.epic_grid(f, xy, xy, il, grids)  # support 0
+
+
+@pytest.mark.parametrize("g,S,nb,na,spread", [
+    (5, 1, 3, 40, 7), (33, 2, 2, 257, 40), (64, 2, 1, 300, 1), (64, 8, 3, 512, 70),
+    (91, 3, 2, 300, 95), (200, 5, 2, 64, 210), (256, 8, 1, 300, 3), (400, 16, 1, 20, 420),
+    (128, 4, 2, 5000, 130)])
+def test_bands_footprints_and_collisions(ctx, g, S, nb, na, spread):
+    """Every kernel form: supports 1, 2, 3 and run-time ones, one and several
+    bands, odd grids, antennas that all stand on a few cells, and the global
+    atomics taken with many antennas.  FP32 sums of at most na S^2 terms a
+    cell: each is off by at most terms 2^-23 of the sum of their moduli."""
+    rng = np.random.default_rng(g + S)
+    f = fields(rng, nb, na)
+    x = rng.integers(-S, spread - S + 1, nb * na)
+    y = rng.integers(-S, spread - S + 1, nb * na)
+    il = (rng.standard_normal((S, S)) + 1j * rng.standard_normal((S, S))).astype(np.complex64)
+    got = run(ctx, f, x, y, il, g)
+    ref = orc.epic_grid(f.astype(np.complex128), x, y, il.astype(np.complex128), g)
+    mod = orc.epic_grid(np.abs(f).astype(np.complex128), x, y, np.abs(il).astype(np.complex128), g)
+    hits = orc.epic_grid(np.ones_like(f, np.complex128), x, y, np.ones((S, S), np.complex128), g)
+    assert (np.abs(got - ref) <= (hits.real + 4) * 2.0 ** -23 * mod.real + 1e-30).all()
