@@ -7,6 +7,10 @@
 //   store(nkeys, k0, start, c, tot)  start[j] first record of the key, c[r][j] start of
 //                                    part r, tot[j] its records (whole wavefronts call)
 //   finish(nkeys, total, stats)      once, by one thread
+// and may choose the records per work item of a key of c records, and see each
+// item put:
+//   item_size(c, per_item)
+//   item_put(index, size, per_item)
 #pragma once
 
 #include "binning.hpp"
@@ -17,6 +21,11 @@ __device__ inline uint32_t items_of(uint32_t c, uint32_t per_item)
 {
     return (c + per_item - 1) / per_item;
 }
+
+struct FixedItems {
+    __device__ static uint32_t item_size(uint32_t, uint32_t per_item) { return per_item; }
+    __device__ static void item_put(uint32_t, uint32_t, uint32_t) {}
+};
 
 // Exclusive scan over the SCAN_BLOCK threads of (x, y) pairs: wavefront scans
 // by shuffles, then the wavefronts' totals through LDS (two barriers).
@@ -99,7 +108,7 @@ __device__ inline void store_keys(uint32_t *dst, int64_t nkeys, int64_t k0,
     }
 }
 
-template <int NREPS> struct CountSource {
+template <int NREPS, typename Items = FixedItems> struct CountSource : Items {
     static constexpr int NREP = NREPS;
     const uint32_t *count; // NREP replicas, stride apart
     int64_t stride;
@@ -153,7 +162,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(Src src, int64_t nke
         for (int r = 0; r < NREP; ++r)
             t += c[r][j];
         acc.x += t;
-        acc.y += items_of(t, per_item);
+        acc.y += items_of(t, src.item_size(t, per_item));
     }
     uint2 total;
     scan_block(acc, total, wtot);
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(
         for (int r = 0; r < NREP; ++r)
             tot[j] += c[r][j];
         acc.x += tot[j];
-        acc.y += items_of(tot[j], per_item);
+        acc.y += items_of(tot[j], src.item_size(tot[j], per_item));
     }
     uint2 total;
     uint2 run = scan_block(acc, total, wtot);
@@ -209,7 +218,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(
         vs[j] = run.x;
         is[j] = run.y;
         run.x += tot[j];
-        run.y += items_of(tot[j], per_item);
+        run.y += items_of(tot[j], src.item_size(tot[j], per_item));
         // counts to the replicas' cursors
         uint32_t cur = vs[j];
 #pragma unroll
@@ -223,24 +232,27 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(
     src.store(nkeys, k0, vs, c, tot);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-        const uint32_t ni = items_of(tot[j], per_item);
+        const uint32_t ni = items_of(tot[j], src.item_size(tot[j], per_item));
         auto put = [&](uint32_t key, uint32_t start, uint32_t cnt, uint32_t i0, uint32_t q) {
+            const uint32_t size = src.item_size(cnt, per_item);
             Item it;
             it.key = key;
-            it.start = start + q * per_item;
-            it.count = min(per_item, cnt - q * per_item);
+            it.start = start + q * size;
+            it.count = min(size, cnt - q * size);
             items[i0 + q] = it;
+            src.item_put(i0 + q, size, per_item);
         };
         if (ni <= 2)
             for (uint32_t q = 0; q < ni; ++q)
                 put((uint32_t)(k0 + j), vs[j], tot[j], is[j], q);
         for (unsigned long long m = __ballot(ni > 2); m; m &= m - 1) {
-            const int src = __ffsll((long long)m) - 1;
-            const uint32_t key = (uint32_t)(k0 + j) + (uint32_t)(src - __lane_id()) * PER;
-            const uint32_t st = (uint32_t)__shfl((int)vs[j], src);
-            const uint32_t cn = (uint32_t)__shfl((int)tot[j], src);
-            const uint32_t i0 = (uint32_t)__shfl((int)is[j], src);
-            for (uint32_t q = __lane_id(); q < items_of(cn, per_item); q += 64)
+            const int from = __ffsll((long long)m) - 1;
+            const uint32_t key = (uint32_t)(k0 + j) + (uint32_t)(from - __lane_id()) * PER;
+            const uint32_t st = (uint32_t)__shfl((int)vs[j], from);
+            const uint32_t cn = (uint32_t)__shfl((int)tot[j], from);
+            const uint32_t i0 = (uint32_t)__shfl((int)is[j], from);
+            const uint32_t nq = items_of(cn, src.item_size(cn, per_item));
+            for (uint32_t q = __lane_id(); q < nq; q += 64)
                 put(key, st, cn, i0, q);
         }
     }

@@ -11,11 +11,12 @@
 // value per source: a few sources are transformed along their rows and then
 // summed directly over the columns, more sources by one batched 2-D FFT.
 //
-// Degridding: visibilities counting-sorted by uv tile, one wavefront per
-// visibility with lanes spread over the kernel's taps so that each load
-// instruction reads whole stack rows, each wavefront walking a contiguous
-// chunk of the sorted order (chunks grouped per XCD); shuffle reduction.
+// Degridding: visibilities counting-sorted by (uv tile, w plane); the reference's
+// 8 x 4 kernels take dense keys cell by cell as FP64 matrix products (16
+// visibilities by the cell's taps), sparse ones with 16 lanes per visibility and
+// the tile's taps in LDS; other kernels one wavefront per visibility.
 #include "binning_impl.hpp"
+#include "scan.hpp"
 
 namespace rg {
 
@@ -353,6 +354,21 @@ __device__ inline double row16_sum(double x)
     return x;
 }
 
+// Sum over the lanes of a DPP row with this lane's parity, in all of them.
+__device__ inline double row8_sum(double x)
+{
+    auto step = [&](auto ctrl) {
+        constexpr int c = decltype(ctrl)::value;
+        const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), c, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), c, 0xf, 0xf, false);
+        x += __hiloint2double(hi, lo);
+    };
+    step(std::integral_constant<int, 0x128>{}); // row_ror:8
+    step(std::integral_constant<int, 0x124>{}); // row_ror:4
+    step(std::integral_constant<int, 0x122>{}); // row_ror:2
+    return x;
+}
+
 // ---- degridding ------------------------------------------------------------------------------
 // deconvolve_visibility_ (wstack_common.h:420-470) over the tile-sorted
 // records.  LV lanes per visibility: tap t = lane % aa_uv along u, pair
@@ -415,6 +431,12 @@ __global__ __launch_bounds__(256) void k_ws_degrid(
     }
 }
 
+// Keys of at least WS_DENSE records (12 per cell) go to k_ws_degrid_cells: whole
+// predictions of 10 M visibilities (6 k on a key) take 1.46 ms so and 1.89 ms by
+// k_ws_degrid_tile; from 2048 on, 3 M (1.8 k on a key) would take 1.02 ms, not 0.96.
+constexpr uint32_t WS_DENSE = 3072;
+constexpr uint32_t WS_ITEM = 1024; // records of a sparse key's work items
+
 // Fixed 8 x 4 support with the stack staged in LDS: one work item (<= K
 // records of one (uv tile, w plane) key) at a time per workgroup; the
 // (16 + 8)^2 cells x 4 planes its taps can reach (36 KiB) are loaded once,
@@ -440,6 +462,8 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     const uint32_t nitems = *nitems_p;
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         const Item item = items[it];
+        if (item.count > WS_ITEM) // k_ws_degrid_cells
+            continue;
         const int ws = (int)(item.key % (uint32_t)wp);
         const int tile = (int)(item.key / (uint32_t)wp);
         const int col0 = (tile % ntx) * T - H, row0 = (tile / ntx) * T - H, pl0 = ws - AW / 2;
@@ -534,6 +558,243 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     }
 }
 
+// Dense keys of the same 8 x 4 support (at least WS_DENSE records on a key's 16
+// x 16 cells): every visibility of a cell has the same 8 x 8 x 4 taps, so a
+// workgroup orders its item's records by cell (indices in LDS) and its wavefronts
+// take a cell's visibilities 16 at a time as a matrix product: (16 visibilities x
+// 32 weights along w and u) times (32 taps x 16 columns, one per row and re or
+// im), eight v_mfma_f64_16x16x4 per batch with the cell's taps held in 16
+// registers; the weight along v and the sum over rows follow on the vector pipe.
+// Loads run ahead: the records of batch q + 2 and the weights of batch q + 1 are
+// in flight during the product of batch q.  The taps come from the tile in LDS:
+// its planes and rows are powers of two apart in HBM, and read from there they
+// queue on few L2 channels (1 M visibilities on 1024^2 planes: 132 us, 92 so).
+// 40 M visibilities over 42 k cells and two planes: 3.83 ms with 16 lanes per
+// visibility, where every visibility reads its 4 KiB from LDS (k_ws_degrid_tile);
+// 4.07 ms with a visibility per lane and the taps as scalar operands (the scalar
+// cache holds half a tile); 3.47 ms with these products but no load ahead; 2.58 ms
+// with it; 2.29 ms with the taps in LDS.  What is left is the 16-byte stores at random
+// places of the stream: in sorted order they take 1.1 ms less, but a pass that brings
+// the results back to stream order takes 0.8 ms and slows streams of a few millions.
+// Items of 8192 records where there are enough of them: 4096 cost 9 % at 40 M, 16384
+// and 32768 5 and 11 %.
+constexpr uint32_t WS_DENSE_MAX = 8192; // records of an item
+constexpr int WS_DENSE_THREADS = 1024;
+
+// records per work item: dense keys in equal parts of at most dense_max, each listed
+// (in any order); down to WS_DENSE / 2 a part holds more than WS_DENSE / 3
+struct WsItems {
+    uint32_t dense_max; // 0: the support has no dense form
+    uint32_t *ndense, *dense;
+    __device__ void item_put(uint32_t index, uint32_t size, uint32_t per_item) const
+    {
+        if (size > per_item)
+            dense[atomicAdd(ndense, 1u)] = index;
+    }
+    __device__ uint32_t item_size(uint32_t c, uint32_t per_item) const
+    {
+        if (!dense_max || c < WS_DENSE)
+            return per_item;
+        const uint32_t parts = (c + dense_max - 1) / dense_max;
+        return (c + parts - 1) / parts;
+    }
+};
+
+// N consecutive doubles at an 8-byte aligned address, 16 bytes per load
+template <int N> __device__ inline void load_row(const double *p, double (&w)[N])
+{
+    struct __attribute__((packed, aligned(8))) Pair {
+        double a, b;
+    };
+#pragma unroll
+    for (int k = 0; k < N; k += 2) {
+        const Pair q = *reinterpret_cast<const Pair *>(p + k);
+        w[k] = q.a;
+        w[k + 1] = q.b;
+    }
+}
+
+template <int AUV, int AW>
+__global__ __launch_bounds__(WS_DENSE_THREADS) void k_ws_degrid_cells(
+    const double2 *__restrict__ stack, int og, int wp, int ntx,
+    const WsRec *__restrict__ recs, const Item *__restrict__ items,
+    const uint32_t *__restrict__ dense, const uint32_t *__restrict__ ndense_p,
+    const double *__restrict__ conv_uv, const double *__restrict__ conv_w,
+    double2 *__restrict__ out)
+{
+    constexpr int SH = WStackKeyer::TILE_SHIFT, T = 1 << SH, CELLS = T * T;
+    static_assert(CELLS <= WS_DENSE_THREADS, "a thread per cell");
+    static_assert(AUV == 8, "a row's taps are two steps of inner length 4");
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    // the taps of the item's tile; rows 8 mod 16 banks apart, so that with odd k
+    // taking its two taps in reverse a half wavefront reads all banks once
+    constexpr int R = T + AUV, PITCH = R + 2;
+    static_assert(PITCH % 4 == 2, "rows 8 (mod 16) LDS banks apart");
+    __shared__ double2 region[AW * R * PITCH];
+    __shared__ uint16_t list[WS_DENSE_MAX];
+    __shared__ uint32_t batch[WS_DENSE_MAX / 16 + CELLS];
+    __shared__ uint32_t cnt[CELLS], nbatch;
+    __shared__ uint2 wsum[CELLS / 64];
+    constexpr uint32_t NWAVES = WS_DENSE_THREADS / 64;
+    static_assert(WS_DENSE_MAX <= 1 << 15 && CELLS <= 1 << 13, "fields of a batch");
+    const int tid = threadIdx.x, lane = tid % 64, k = lane / 16, j = lane % 16;
+    const uint32_t n = *ndense_p;
+    for (uint32_t t = blockIdx.x; t < n; t += gridDim.x) {
+        const Item item = items[dense[t]];
+        const WsRec *r = recs + item.start;
+        auto cell_of = [&](uint32_t i) {
+            const uint32_t c = r[i].cell;
+            return (c & (T - 1)) | (((c >> 16) & (T - 1)) << SH);
+        };
+        const int ws = (int)(item.key % (uint32_t)wp), tile = (int)(item.key / (uint32_t)wp);
+        const int us0 = (tile % ntx) * T - AUV / 2, vs0 = (tile / ntx) * T - AUV / 2;
+        __syncthreads(); // the previous item is done with the list and the taps
+        if (tid < CELLS)
+            cnt[tid] = 0;
+        for (int i = tid; i < AW * R * R; i += WS_DENSE_THREADS) {
+            const int pr = i / R, col = i % R, row = vs0 + pr % R; // pr: plane, row
+            double2 val = make_double2(0.0, 0.0);
+            if (row >= 0 && row < og && us0 + col >= 0 && us0 + col < og)
+                val = stack[((size_t)(ws - AW / 2 + pr / R) * og + row) * og + us0 + col];
+            region[pr * PITCH + col] = val;
+        }
+        __syncthreads();
+        // f(record index, cell) over the item, eight loads in flight
+        auto each = [&](auto &&f) {
+            for (uint32_t i0 = tid; i0 < item.count; i0 += 8 * WS_DENSE_THREADS) {
+                uint32_t c[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    c[q] = cell_of(min(i0 + q * WS_DENSE_THREADS, item.count - 1));
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (i0 + q * WS_DENSE_THREADS < item.count)
+                        f(i0 + q * WS_DENSE_THREADS, c[q]);
+            }
+        };
+        each([&](uint32_t, uint32_t c) { atomicAdd(&cnt[c], 1u); });
+        __syncthreads();
+        // starts of the cells' records and of their batches
+        uint32_t mine = 0, inc = 0, bat = 0, binc = 0;
+        if (tid < CELLS) {
+            mine = inc = cnt[tid];
+            bat = binc = (mine + 15) / 16;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t x = (uint32_t)__shfl_up((int)inc, o);
+                const uint32_t y = (uint32_t)__shfl_up((int)binc, o);
+                if (lane >= o) {
+                    inc += x;
+                    binc += y;
+                }
+            }
+            if (lane == 63)
+                wsum[tid / 64] = make_uint2(inc, binc);
+        }
+        __syncthreads();
+        if (tid < CELLS) {
+            for (int w = 0; w < tid / 64; ++w) {
+                inc += wsum[w].x;
+                binc += wsum[w].y;
+            }
+            const uint32_t s0 = inc - mine;
+            cnt[tid] = s0; // the placement's cursor
+            // a batch: first list entry | visibilities less one << 15 | cell << 19
+            for (uint32_t q = 0; q < bat; ++q)
+                batch[binc - bat + q] =
+                    (s0 + 16 * q) | (min(mine - 16 * q, 16u) - 1) << 15 | (uint32_t)tid << 19;
+            if (tid == CELLS - 1)
+                nbatch = binc;
+        }
+        __syncthreads();
+        each([&](uint32_t i, uint32_t c) { list[atomicAdd(&cnt[c], 1u)] = (uint16_t)i; });
+        __syncthreads();
+        // B of a cell: column j = 2 pv + (0 re, 1 im) of plane pw holds taps 2 k and
+        // 2 k + 1 of row pv (the product's inner index may be taken in any order)
+        const int odd = k & 1;
+        const double *tap0 =
+            reinterpret_cast<const double *>(region + (j >> 1) * PITCH + 2 * k + odd) + (j & 1);
+        const int other = odd ? -2 : 2;
+        double b0[AW], b1[AW];
+        auto taps = [&](uint32_t c) {
+            const double *tap = tap0 + 2 * ((c >> SH) * PITCH + (c & (uint32_t)(T - 1)));
+#pragma unroll
+            for (int pw = 0; pw < AW; ++pw) {
+                b0[pw] = tap[pw * R * PITCH * 2];
+                b1[pw] = tap[pw * R * PITCH * 2 + other];
+            }
+        };
+        // this wavefront's batches, a contiguous share
+        const uint32_t nb = nbatch;
+        const uint32_t q0 = nb * (uint32_t)(tid / 64) / NWAVES;
+        const uint32_t q1 = nb * (uint32_t)(tid / 64 + 1) / NWAVES;
+        struct Rec {
+            uint32_t pos, ovu, hi; // hi: ovv | ovw << 16
+        };
+        struct Weights {
+            double gu[2], gw[AW]; // A: along u (taps 2 k, 2 k + 1) and w, visibility j
+            double gv[4];         // of row j / 2, visibilities k + 4 i
+            uint32_t pos[4];
+        };
+        auto load_rec = [&](uint32_t q) { // visibility j of batch q
+            const uint32_t e = batch[min(q, nb - 1)];
+            const uint32_t n1 = (e >> 15) & 15u; // visibilities less one
+            const WsRec w = r[list[(e & 0x7fffu) + min((uint32_t)j, n1)]];
+            Rec o;
+            o.pos = w.pos;
+            o.ovu = (uint32_t)(w.bits >> 16) & 0xffffu;
+            o.hi = (uint32_t)(w.bits >> 32);
+            return o;
+        };
+        auto load_weights = [&](const Rec &o) {
+            Weights w;
+            load_row<2>(conv_uv + AUV * (int)o.ovu + 2 * k, w.gu);
+            load_row<AW>(conv_w + AW * (int)(o.hi >> 16), w.gw);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t ov = (uint32_t)__shfl((int)o.hi, k + 4 * i);
+                w.gv[i] = conv_uv[AUV * (int)(ov & 0xffffu) + (j >> 1)];
+                w.pos[i] = (uint32_t)__shfl((int)o.pos, k + 4 * i);
+            }
+            return w;
+        };
+        uint32_t cell = 0xffffffffu;
+        Rec r1 = load_rec(q0 + 1);
+        Weights cur = load_weights(load_rec(q0));
+        for (uint32_t q = q0; q < q1; ++q) { // uniform in the wavefront
+            const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)batch[q]);
+            if ((e >> 19) != cell) {
+                cell = e >> 19;
+                taps(cell);
+            }
+            const Rec r2 = load_rec(q + 2);
+            const Weights nxt = load_weights(r1);
+            const double g0 = odd ? cur.gu[1] : cur.gu[0], g1 = odd ? cur.gu[0] : cur.gu[1];
+            v4d d = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int pw = 0; pw < AW; ++pw) {
+                d = __builtin_amdgcn_mfma_f64_16x16x4f64(g0 * cur.gw[pw], b0[pw], d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f64_16x16x4f64(g1 * cur.gw[pw], b1[pw], d, 0, 0, 0);
+            }
+            // this lane holds column j of visibilities k + 4 i
+            uint32_t pos = 0;
+            double val = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double x = row8_sum(d[i] * cur.gv[i]);
+                if ((j >> 1) == i) { // lanes 2 i, 2 i + 1 store re, im
+                    val = x;
+                    pos = cur.pos[i];
+                }
+            }
+            if (j < 8 && (uint32_t)(k + 4 * (j >> 1)) <= ((e >> 15) & 15u))
+                reinterpret_cast<double *>(out + pos)[j & 1] = val;
+            cur = nxt;
+            r1 = r2;
+        }
+    }
+}
+
 // ---- driver --------------------------------------------------------------------------------------
 
 int wstack_build(rg_context *ctx, const rg_wstack_params *p, const double *l, const double *m,
@@ -618,12 +879,12 @@ int wstack_build(rg_context *ctx, const rg_wstack_params *p, const double *l, co
 // visibility when neighbouring visibilities do not share keys (random order),
 // so degridding sorts in two levels with LDS counters only:
 //   coarse count   : workgroup b counts its chunk of the stream per coarse
-//                    bucket c = key >> fb (at most WS_NC buckets) in LDS; each
-//                    visibility's record and its rank in its workgroup's share
-//                    of c are written; hist[c][b] = the share
-//   bucket scan    : hist[c][.] to exclusive prefixes over the workgroups,
+//                    bucket c = key >> fb (at most WS_NC buckets) in LDS;
+//                    hist[b][c] = the share
+//   bucket scan    : hist[.][c] to exclusive prefixes over the workgroups,
 //                    bucket totals to bucket starts
-//   coarse scatter : record of visibility i to bstart[c] + hist[c][b] + rank
+//   coarse scatter : record of visibility i to bstart[c] + hist[b][c] + its
+//                    rank in the workgroup's share of c
 //   fine rank      : chunks of the bucketed records count their keys in LDS,
 //                    reserve each key's share with one device atomic per
 //                    (chunk, key) and give every record its rank in its key
@@ -632,66 +893,73 @@ int wstack_build(rg_context *ctx, const rg_wstack_params *p, const double *l, co
 //   fine scatter   : record to key start + rank
 // Records of one key end up contiguous in key order, in no particular order
 // inside the key (degridding a visibility does not depend on the others).
+// The records are derived twice (count, scatter), which costs less than writing
+// and reading them in between, and two workgroups of 1024 per CU leave each bucket
+// runs long enough for the L2 to fill lines: 40 M visibilities 1.24 -> 0.66 ms for
+// the two passes.
 constexpr int WS_NC = 4096;       // coarse buckets at most
-constexpr int WS_SORT_BLOCKS = 2048; // workgroups of the coarse passes at most
+constexpr int WS_SORT_BLOCKS = 512; // workgroups of the coarse passes at most (two per CU)
+constexpr int WS_SORT_THREADS = 1024;
 constexpr int WS_FB_MAX = 13;     // keys per bucket at most 2^13 (one fine window)
 
-__global__ __launch_bounds__(256) void k_ws_coarse_count(WStackKeyer kf, int64_t n, int64_t chunk,
-                                                         int nb, int fb, int nc, uint32_t *rank,
-                                                         WsRec *rec, uint32_t *hist,
-                                                         unsigned long long *stats)
+__global__ __launch_bounds__(WS_SORT_THREADS) void k_ws_coarse_count(WStackKeyer kf, int64_t n,
+                                                                     int64_t chunk, int fb, int nc,
+                                                                     uint32_t *hist,
+                                                                     unsigned long long *stats)
 {
     __shared__ uint32_t h[WS_NC];
     __shared__ uint32_t dropped;
-    for (int c = threadIdx.x; c < nc; c += 256)
+    for (int c = threadIdx.x; c < nc; c += WS_SORT_THREADS)
         h[c] = 0;
     if (threadIdx.x == 0)
         dropped = 0;
     __syncthreads();
     const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
     uint32_t nd = 0;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) {
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += WS_SORT_THREADS) {
         WsCell cl;
-        uint32_t rk = KEY_NONE;
-        if (kf.cell(i, cl, true)) {
-            const uint32_t key = WStackKeyer::key_of(cl.us, cl.vs, cl.ws, kf.ntx, kf.wp);
-            rk = atomicAdd(&h[key >> fb], 1u);
-            rec[i] = WStackKeyer::pack(i, cl);
-        } else {
+        if (kf.cell(i, cl, false))
+            atomicAdd(&h[WStackKeyer::key_of(cl.us, cl.vs, cl.ws, kf.ntx, kf.wp) >> fb], 1u);
+        else
             ++nd;
-        }
-        rank[i] = rk;
     }
     if (nd)
         atomicAdd(&dropped, nd);
     __syncthreads();
-    for (int c = threadIdx.x; c < nc; c += 256)
-        hist[(size_t)c * nb + blockIdx.x] = h[c];
+    for (int c = threadIdx.x; c < nc; c += WS_SORT_THREADS)
+        hist[(size_t)blockIdx.x * nc + c] = h[c];
     if (threadIdx.x == 0 && dropped)
         atomicAdd(&stats[CNT_DROPPED], (unsigned long long)dropped);
 }
 
-// workgroup c: hist[c][0..nb) to its exclusive prefix, bucket total to tot[c]
-__global__ __launch_bounds__(256) void k_ws_bucket_scan(uint32_t *hist, int nb, uint32_t *tot)
+// buckets [64 blockIdx.x, + 64): hist[0..nb)[c] to its exclusive prefix over the
+// workgroups, bucket total to tot[c]; 16 threads per bucket, each a run of workgroups
+__global__ __launch_bounds__(1024) void k_ws_bucket_scan(uint32_t *hist, int nb, int nc,
+                                                         uint32_t *tot)
 {
-    __shared__ uint32_t tmp[256];
-    uint32_t *hc = hist + (size_t)blockIdx.x * nb;
-    const int per = (nb + 255) / 256, b0 = (int)threadIdx.x * per;
+    __shared__ uint32_t part[16][64];
+    const int c = (int)(blockIdx.x * 64 + threadIdx.x % 64), seg = threadIdx.x / 64;
+    const int per = (nb + 15) / 16, b0 = seg * per, b1 = min(nb, b0 + per);
     uint32_t sum = 0;
-    for (int j = 0; j < per; ++j)
-        if (b0 + j < nb)
-            sum += hc[b0 + j];
-    uint32_t total;
-    uint32_t run = block_prefix256(sum, total, tmp);
-    for (int j = 0; j < per; ++j) {
-        if (b0 + j < nb) {
-            const uint32_t v = hc[b0 + j];
-            hc[b0 + j] = run;
-            run += v;
-        }
+    if (c < nc)
+#pragma unroll 8
+        for (int b = b0; b < b1; ++b)
+            sum += hist[(size_t)b * nc + c];
+    part[seg][threadIdx.x % 64] = sum;
+    __syncthreads();
+    uint32_t run = 0;
+    for (int k = 0; k < seg; ++k)
+        run += part[k][threadIdx.x % 64];
+    if (c >= nc)
+        return;
+    if (seg == 15)
+        tot[c] = run + sum;
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) {
+        const uint32_t v = hist[(size_t)b * nc + c];
+        hist[(size_t)b * nc + c] = run;
+        run += v;
     }
-    if (threadIdx.x == 0)
-        tot[blockIdx.x] = total;
 }
 
 // one workgroup: tot[0..nc) to bucket starts bstart[0..nc] (in place, nc + 1 entries)
@@ -716,22 +984,25 @@ __global__ __launch_bounds__(256) void k_ws_bucket_starts(uint32_t *bstart, int 
         bstart[nc] = total;
 }
 
-__global__ __launch_bounds__(256) void k_ws_coarse_scatter(int64_t n, int64_t chunk, int nb,
-                                                           int fb, int ntx, int wp,
-                                                           const uint32_t *__restrict__ rank,
-                                                           const WsRec *__restrict__ rec,
-                                                           const uint32_t *__restrict__ hist,
-                                                           const uint32_t *__restrict__ bstart,
-                                                           WsRec *tmp)
+// records of the chunk to their places in the buckets (a visibility without a
+// record is not predicted: 0)
+__global__ __launch_bounds__(WS_SORT_THREADS) void k_ws_coarse_scatter(
+    WStackKeyer kf, int64_t n, int64_t chunk, int fb, int nc, const uint32_t *__restrict__ hist,
+    const uint32_t *__restrict__ bstart, WsRec *__restrict__ tmp, double2 *__restrict__ out)
 {
+    __shared__ uint32_t cur[WS_NC];
+    for (int c = threadIdx.x; c < nc; c += WS_SORT_THREADS)
+        cur[c] = bstart[c] + hist[(size_t)blockIdx.x * nc + c];
+    __syncthreads();
     const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) {
-        const uint32_t rk = rank[i];
-        if (rk == KEY_NONE)
-            continue;
-        const WsRec r = rec[i];
-        const uint32_t c = WStackKeyer::key_of(r, ntx, wp) >> fb;
-        tmp[bstart[c] + hist[(size_t)c * nb + blockIdx.x] + rk] = r;
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += WS_SORT_THREADS) {
+        WsCell cl;
+        if (kf.cell(i, cl, true)) {
+            const uint32_t c = WStackKeyer::key_of(cl.us, cl.vs, cl.ws, kf.ntx, kf.wp) >> fb;
+            tmp[atomicAdd(&cur[c], 1u)] = WStackKeyer::pack(i, cl);
+        } else {
+            out[i] = make_double2(0.0, 0.0);
+        }
     }
 }
 
@@ -787,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_ws_fine_scatter(const WsRec *__restrict
                                                          int ntx, int wp,
                                                          const uint32_t *__restrict__ key_start,
                                                          const uint32_t *__restrict__ rank,
-                                                         WsRec *recs)
+                                                         WsRec *__restrict__ recs)
 {
     const uint32_t total = *total_p;
     for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < total; j += gridDim.x * 256u) {
@@ -797,7 +1068,7 @@ __global__ __launch_bounds__(256) void k_ws_fine_scatter(const WsRec *__restrict
 }
 
 static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nkeys, uint32_t K,
-                   hipStream_t s, BinResult &out)
+                   uint32_t dense_max, double2 *pred, hipStream_t s, BinResult &out)
 {
     if (n >= (int64_t)0x7fffffff)
         return fail(RG_ERR_PARAM, "visibility stream too long for one call (%lld)", (long long)n);
@@ -807,9 +1078,10 @@ static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nk
     if (fb > WS_FB_MAX)
         return fail(RG_ERR_UNSUPPORTED, "W-stack key space too large (%lld)", (long long)nkeys);
     const int nc = (int)((nkeys + (1ll << fb) - 1) >> fb);
-    // chunks of whole 256-visibility rounds, at most WS_SORT_BLOCKS of them
+    // chunks of whole rounds of the workgroup, at most WS_SORT_BLOCKS of them
     int64_t chunk = (n + WS_SORT_BLOCKS - 1) / WS_SORT_BLOCKS;
-    chunk = std::max<int64_t>(1024, (chunk + 255) / 256 * 256);
+    chunk = std::max<int64_t>(2, (chunk + WS_SORT_THREADS - 1) / WS_SORT_THREADS) *
+            WS_SORT_THREADS;
     const int nb = (int)((n + chunk - 1) / chunk);
     const int64_t max_items = nkeys + n / K + 1;
 
@@ -821,32 +1093,42 @@ static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nk
     RG_TRY(ctx->scratch[4].ensure(sizeof(Item) * max_items));                // items
     RG_TRY(ctx->scratch[5].ensure(sizeof(WsRec) * n));                       // records
     RG_TRY(ctx->scratch[7].ensure(sizeof(WsRec) * n));                       // bucketed records
-    RG_TRY(ctx->scratch[8].ensure(sizeof(uint32_t) * nkeys));                // per-key counts
-    RG_TRY(ctx->scratch[15].ensure(sizeof(uint32_t) * n)); // bucket ranks, then key ranks
+    // per-key counts, the dense items' number and list
+    const int64_t max_dense = dense_max ? n / (WS_DENSE / 3) + 1 : 0;
+    RG_TRY(ctx->scratch[8].ensure(sizeof(uint32_t) * (nkeys + 1 + max_dense)));
+    RG_TRY(ctx->scratch[15].ensure(sizeof(uint32_t) * n));                   // key ranks
     KernelTimer kt(ctx, RG_TIMER_BINNING, s);
     uint32_t *hist = ctx->scratch[0].as<uint32_t>(), *bst = ctx->scratch[3].as<uint32_t>();
     auto *stats = ctx->counters.as<unsigned long long>();
-    // the records in stream order go to the final record array (free until
-    // the fine scatter), their bucket ranks to scratch 15
     uint32_t *rank = ctx->scratch[15].as<uint32_t>();
-    WsRec *rec0 = ctx->scratch[5].as<WsRec>();
-    hipLaunchKernelGGL(k_ws_coarse_count, dim3((unsigned)nb), dim3(256), 0, s, kf, n, chunk, nb,
-                       fb, nc, rank, rec0, hist, stats);
-    hipLaunchKernelGGL(k_ws_bucket_scan, dim3((unsigned)nc), dim3(256), 0, s, hist, nb, bst);
+    hipLaunchKernelGGL(k_ws_coarse_count, dim3((unsigned)nb), dim3(WS_SORT_THREADS), 0, s, kf, n,
+                       chunk, fb, nc, hist, stats);
+    hipLaunchKernelGGL(k_ws_bucket_scan, dim3((unsigned)((nc + 63) / 64)), dim3(1024), 0, s, hist,
+                       nb, nc, bst);
     hipLaunchKernelGGL(k_ws_bucket_starts, dim3(1), dim3(256), 0, s, bst, nc);
-    hipLaunchKernelGGL(k_ws_coarse_scatter, dim3((unsigned)nb), dim3(256), 0, s, n, chunk, nb, fb,
-                       kf.ntx, kf.wp, (const uint32_t *)rank, (const WsRec *)rec0,
-                       (const uint32_t *)hist, (const uint32_t *)bst, ctx->scratch[7].as<WsRec>());
+    hipLaunchKernelGGL(k_ws_coarse_scatter, dim3((unsigned)nb), dim3(WS_SORT_THREADS), 0, s, kf, n,
+                       chunk, fb, nc, (const uint32_t *)hist, (const uint32_t *)bst,
+                       ctx->scratch[7].as<WsRec>(), pred);
     uint32_t *cnt_key = ctx->scratch[8].as<uint32_t>();
-    // bucket ranks are no longer read: the key ranks reuse their array
     const WsRec *tmp = ctx->scratch[7].as<WsRec>();
-    RG_TRY(zero_fill(cnt_key, sizeof(uint32_t) * nkeys, s));
+    RG_TRY(zero_fill(cnt_key, sizeof(uint32_t) * (nkeys + 1), s));
     hipLaunchKernelGGL(k_ws_fine_rank, dim3((unsigned)((n + WS_FINE_CHUNK - 1) / WS_FINE_CHUNK)),
                        dim3(256), 0, s, tmp, (const uint32_t *)(bst + nc), kf.ntx, kf.wp, fb,
                        cnt_key, rank);
     RG_HIP(hipGetLastError());
-    RG_TRY(items_from_lengths(ctx, cnt_key, nkeys, K, ctx->scratch[1].as<uint32_t>(),
-                              ctx->scratch[2].as<uint32_t>(), ctx->scratch[4].as<Item>(), s));
+    RG_TRY(ctx->scratch[6].ensure(scan_sums_bytes(nkeys)));
+    CountSource<1, WsItems> src;
+    src.dense_max = dense_max;
+    src.ndense = cnt_key + nkeys;
+    src.dense = src.ndense + 1;
+    src.count = cnt_key;
+    src.stride = nkeys;
+    src.vis_start = ctx->scratch[1].as<uint32_t>();
+    src.cursor = nullptr;
+    src.group_start = nullptr;
+    src.group_keys = 0;
+    RG_TRY(scan_source(src, nkeys, K, ctx->scratch[6].as<uint2>(), ctx->scratch[2].as<uint32_t>(),
+                       ctx->scratch[4].as<Item>(), stats, s));
     hipLaunchKernelGGL(k_ws_fine_scatter,
                        dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)), dim3(256), 0, s,
                        tmp, (const uint32_t *)(bst + nc), kf.ntx, kf.wp,
@@ -877,8 +1159,6 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
     if (nvis == 0)
         return RG_OK;
     const double2 *stack = ctx->scratch[17].as<double2>();
-    // sort by uv tile (dropped visibilities keep the zero written here)
-    RG_TRY(zero_fill(out, sizeof(double2) * (size_t)nvis, s));
     WStackKeyer kf;
     kf.u = u;
     kf.v = v;
@@ -897,8 +1177,14 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         return fail(RG_ERR_UNSUPPORTED, "W-stack indices beyond 16 bits");
     BinResult br;
     const int64_t nkeys = (int64_t)kf.ntx * kf.ntx * wp;
-    constexpr uint32_t K = 1024; // records per work item
-    RG_TRY(ws_sort(ctx, kf, nvis, nkeys, K, s, br));
+    static_assert(WS_ITEM <= WS_DENSE / 3, "items of sparse keys are told apart by their size");
+    if (((uintptr_t)out & 15) != 0)
+        return fail(RG_ERR_PARAM, "predicted visibilities must be 16-byte aligned");
+    // sort by uv tile and plane; dense keys in parts of 1/256 of the stream, so that
+    // every CU has one (300 k on 128^2 planes: 156 us with 8192, 112 so)
+    const bool fixed = p->aa_support_uv == 8 && p->aa_support_w == 4;
+    const uint32_t part = (uint32_t)std::clamp<int64_t>(nvis / 256, WS_DENSE / 2, WS_DENSE_MAX);
+    RG_TRY(ws_sort(ctx, kf, nvis, nkeys, WS_ITEM, fixed ? part : 0, (double2 *)out, s, br));
     const WsRec *recs = reinterpret_cast<const WsRec *>(br.recs);
     const uint32_t *nrec = br.vis_start + nkeys;
     // one wavefront per visibility (the uv support, a power of two <= 64,
@@ -908,7 +1194,17 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         int64_t blocks = std::min<int64_t>((nvis + 16 * per_block - 1) / (16 * per_block), 8192);
         return (blocks + 7) / 8 * 8;
     };
-    if (p->aa_support_uv == 8 && p->aa_support_w == 4) {
+    if (fixed) {
+        const uint32_t *ndense = ctx->scratch[8].as<uint32_t>() + nkeys;
+        // fewer than nvis / WS_ITEM dense items; 2048 workgroups, dispatched as others
+        // finish
+        if (nvis >= (int64_t)WS_DENSE)
+            hipLaunchKernelGGL((k_ws_degrid_cells<8, 4>),
+                               dim3((unsigned)std::min<int64_t>(2048, nvis / WS_ITEM)),
+                               dim3(WS_DENSE_THREADS), 0, s,
+                               stack, og, wp, kf.ntx, recs, (const Item *)br.items,
+                               (const uint32_t *)(ndense + 1), (const uint32_t *)ndense,
+                               conv_uv->data, conv_w->data, (double2 *)out);
         constexpr int LV = 16;
         // persistent workgroups over the work items (nitems read on the device)
         const int64_t blocks = std::min<int64_t>(br.max_items, 4096);

@@ -814,7 +814,7 @@ __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ i
 // record array.  The scan of the windows' lengths gives their work items and,
 // per slot, the bands with records: bit b % 32 of word b / 32 of the slot's
 // (nb + 31) / 32 words.  nb is a power of two.
-struct WindowSource {
+struct WindowSource : FixedItems {
     static constexpr int NREP = 1;
     const uint32_t *key_start;
     int nb, mk;

@@ -272,3 +272,50 @@ def test_dense_sky_with_long_rows(ctx, kernels, lam):
                                  d["n"])
     assert (og, wp) == (stack.shape[1], stack.shape[0])
     assert np.abs(ctx.wstack_stack(og, wp) - stack).max() < 1e-11 * np.abs(stack).max()
+
+
+@pytest.mark.parametrize("per_tile", [1536, 1537, 3071, 3072, 3073, 4609, 8193, 16385])
+def test_dense_keys_at_their_edges(ctx, kernels, per_tile):
+    """Visibilities of one (16 x 16-cell tile, plane) key around the sizes where
+    it becomes dense and where it is split into work items: spread over the
+    tile's cells, with a full batch and a batch of one in two of them, next to a
+    key of a few visibilities, a key of one cell only and visibilities that leave
+    the stack (0), in random order.  Results are sums of 256 products of at most
+    |stack| sum |taps| each, so FP64 agrees far below 1e-10."""
+    theta, lam = 0.1, 640.0
+    h, d = kernels["host"], kernels["desc"]
+    rng = np.random.default_rng(per_tile)
+    du, dw = h["uv"].du, h["w"].dw
+    l, m = card(theta)
+    g = int(np.floor(theta * lam))
+    def at(cell):  # a coordinate whose centre tap is `cell` of the stack
+        return (cell - g - rng.uniform(0.01, 0.99, len(cell))) * du
+
+    base = 64  # a tile's first cell
+    cu, cv = rng.integers(base, base + 16, (2, per_tile))
+    cu[:33], cv[:33] = base + 3, base + 5  # two full batches and more
+    dense = at(cu), at(cv)
+    cu, cv = base + 16 + rng.integers(0, 16, 40), np.full(40, base + 2)
+    sparse = at(cu), at(cv)
+    one = at(np.full(4500, base + 7)), at(np.full(4500, base + 24))
+    gone = np.full(19, 1e7), np.zeros(19)
+    u, v = (np.concatenate([a[k] for a in (dense, sparse, one, gone)]) for k in (0, 1))
+    w = -rng.uniform(0.01, 0.99, len(u)) * dw
+    order = rng.permutation(len(u))
+    u, v, w = u[order], v[order], w[order]
+    stack, _ = orc.wstack_build(theta, lam, l, m, None, du, dw, h["w"].size, h["lm"].x0,
+                                h["lm"].data, h["n"].data)
+    ref, nd = orc.wstack_degrid(stack, g, u, v, w, du, dw, h["uv"].data, h["uv"].size,
+                                h["uv"].oversampling, h["w"].data, h["w"].size,
+                                h["w"].oversampling)
+    assert nd == 19
+    p = params(kernels, theta, lam)
+    ctx.wstack_build(p, dev(l), dev(m), None, d["lm"], d["n"])
+    out = torch.full((len(u),), 5.0, dtype=torch.complex128, device="cuda")
+    ctx.wstack_degrid(p, dev(u), dev(v), dev(w), d["uv"], d["w"], out)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.abs(got - ref).max() < 1e-10 * np.abs(ref).max()
+    assert np.all(got[order >= len(order) - 19] == 0)
+    st = ctx.stats()
+    assert st.n_dropped == 19 and st.n_gridded == len(u) - 19
