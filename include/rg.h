@@ -88,10 +88,12 @@ typedef struct rg_grid_params {
     int32_t subgrid_size;   /* W-towers n (0 = W-projection) */
     int32_t subgrid_margin; /* W-towers margin M */
     double winc;            /* W-towers floor spacing (wavelengths) */
-    int32_t tile;           /* batched W-projection: tile edge in cells (32 or 48, 0 = 32);
+    int32_t tile;           /* batched W-projection: 32, 48 or 0 (all three run the same
+                               tiles of 16 x 16 positions);
                                batched W-towers: band height in rows (4, 8 or 16 (16 in
                                FP32 only), 0 = 8) */
-    int32_t vis_per_item;   /* batched visibilities per work item (0 = default) */
+    int32_t vis_per_item;   /* batched visibilities per work item (0 = default;
+                               W-projection: at most 512) */
     int32_t compensated;    /* batched FP32: 0 plain FP32 sums (default), 1 two-sum
                                compensated sums: W-projection tile sums (worth it only into
                                an RG_C128 grid), W-towers band lanes' register sums */
@@ -191,7 +193,7 @@ int rg_grid_channels(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis
  * serving loops, harnesses that forbid hipMalloc.  Same parameters and result
  * as rg_grid with RG_MODE_BATCHED and subgrid_size 0 (FP32 or FP64 kernels),
  * on the current HIP device, with no context: the sort's working memory is a
- * 64 MiB device array inside librg (one per device, held until the process
+ * 192 MiB device array inside librg (one per device, held until the process
  * ends), enough for about 2.0 M visibilities (FP32 kernels) or 1.4 M (FP64)
  * per call on a 2048^2 grid; a call that needs more returns RG_ERR_PARAM.
  * accumulate = 0 zeroes the grid first (as rg_grid), 1 adds into it, so a

@@ -58,9 +58,13 @@ int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, in
     RG_TRY(ensure_counters(ctx));
     // items and scan sums: room for every call of up to this many visibilities
     // and keys, whatever item size it picks (scratch that a captured graph holds
-    // cannot grow)
-    const int64_t room = nkeys + std::max<int64_t>(n / per_item, std::max<int64_t>(700, n / 512)) + 1;
+    // cannot grow; a shorter stream's smaller items are at most 24 times 512);
+    // counters likewise: fewer keys may take more replicas
+    const int64_t room = nkeys + std::max<int64_t>(n / per_item, std::max<int64_t>(12288, n / 512)) + 1;
     const size_t count_bytes = pl.bytes[BIN_COUNT];
+    const size_t counters = sizeof(uint32_t) * (size_t)std::min<int64_t>(16 * pl.rp.stride, max_counters);
+    for (int k : {BIN_COUNT, BIN_CURSOR})
+        pl.bytes[k] = std::max(pl.bytes[k], counters);
     pl.bytes[BIN_ITEMS] = std::max(pl.bytes[BIN_ITEMS], sizeof(Item) * (size_t)room);
     pl.bytes[BIN_BSUMS] = scan_sums_bytes(nkeys);
     for (int k = 0; k < BIN__N; ++k)

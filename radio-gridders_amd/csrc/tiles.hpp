@@ -1,22 +1,29 @@
 // tiles.hpp -- tiled Romein accumulation kernel of batched W-projection
 // (device code).
 //
-// One workgroup of S*S threads takes one work item: up to K sorted records of
-// one key.  A key is (group, tile): the group selects the target array (a
-// channel grid) and the tile a TILE x TILE block of footprint top-left
-// positions, whose footprints cover (TILE + S - 1)^2 cells held in LDS (rows
-// TILE + S - 1 rounded up to S apart, so that the binning can hand each record
-// its cell and sub-kernel as byte offsets).
-// Thread (myU, myV) handles, for every record, the footprint cell congruent to
-// (myU, myV) modulo S (Romein); it keeps a register sum while that cell stays
-// the same and adds it into LDS when the cell changes.  Two threads never
-// share a cell, so the LDS updates need no atomics, and a thread reads a
-// cell's LDS value when it starts summing into it: leaving the cell is then a
-// store, and the read's latency is hidden behind the records in between.  At the end the tile is
-// added to the target with global atomics (neighbouring tiles and items of
-// the same tile overlap).  Storing per-item partials and summing them per cell
-// instead measured slower at the C2 shape: the atomics overlap with the
-// accumulation of other workgroups.
+// One wavefront takes one work item: up to K sorted records of one key.  A key
+// is (plane group, group, tile): the group selects the target array (a channel grid), the tile a
+// 16 x 16 block of footprint top-left positions, whose footprints cover
+// (S + 15) x (S + 15) cells held in LDS, and the plane group a range of
+// W-planes (items of a group follow one another, so the sub-kernels in use at a time
+// stay in an XCD's L2).
+//
+// The wavefront holds the sums of a whole footprint in registers, S S / 64
+// taps a lane, for as long as consecutive records have the same position,
+// and adds them into LDS when the position changes (a wavefront's LDS region is
+// its own: plain read-modify-write).  Records are therefore ordered by position
+// first: SORT at a time, by counts in LDS.  A record costs a lane its 4 FMAs a tap,
+// three lane reads (first tap as the loads' scalar offset, value) and one or
+// two 16-byte tap loads whose addresses are fixed per lane.  At the end the region is
+// added to the target with global atomics (neighbouring tiles and items of the
+// same tile overlap), a row at a time as consecutive numbers.
+//
+// Bound by VALU issue (31 instructions a record in FP32, 16 of them the FMAs; 62 % busy)
+// beside the tap reads (2 KB a record from L2, 19 TB/s).  With a workgroup of S S threads
+// per item, a tap a lane (every lane of four wavefronts found its own cell and tap
+// address for every record: about 64 instructions) and records of all planes mixed
+// (a 60 MB table read past L2), tiles took, now, us: 8.4 M visibilities FP32 1571 -> 890;
+// 520 k FP64 273 -> 168; 448 FP64 7.3 -> 5.2.
 #pragma once
 
 #include "binning.hpp"
@@ -35,159 +42,288 @@ template <typename T> __device__ inline void two_sum_into(T &hi, T &lo, T b)
 }
 
 struct TileSink {
-    void *base;              // target arrays, group g at base + g * gsize^2 complex elements
-    int gsize;               // edge of a target array (N or n)
-    int ntx;                 // tiles per row
-    int ntiles;              // tiles per group
-    const int32_t *group_map; // optional: group -> rank (slot of the target array)
-    int32_t group_offset;     // rank - offset = target slot
+    void *base; // target arrays, group g at base + g * gsize^2 complex elements
+    int gsize;  // edge of a target array
+    int ntx;    // tiles per row
+    int ntiles; // tiles per group
+    int groups; // target arrays
 };
 
-template <typename T, int S, int TILE, bool COMP, typename GT>
-__global__ __launch_bounds__(S *S) void k_tiles(const Rec<T> *__restrict__ recs,
-                                                const Item *__restrict__ items, uint32_t item0,
-                                                uint32_t item_end,
-                                                const unsigned long long *__restrict__ stats,
-                                                const typename Vec2<T>::type *__restrict__ kern,
-                                                uint32_t kern_bytes, TileSink sink)
+__device__ inline float lane_value(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+__device__ inline double lane_value(double v, int lane)
+{
+    const uint2 b = __builtin_bit_cast(uint2, v);
+    uint2 r;
+    r.x = (uint32_t)__builtin_amdgcn_readlane((int)b.x, lane);
+    r.y = (uint32_t)__builtin_amdgcn_readlane((int)b.y, lane);
+    return __builtin_bit_cast(double, r);
+}
+
+// Complex values per lane and load of a sub-kernel read by one wavefront.
+template <typename T, int S> struct TapSpan {
+    static constexpr int Z = 2 * (int)sizeof(T);
+    static constexpr int BYTES = S * S * Z;
+    static constexpr int LOAD = BYTES / 64 < 16 ? BYTES / 64 : 16; // bytes per lane and load
+    static constexpr int NL = BYTES / (64 * LOAD);                 // loads
+    static constexpr int E = LOAD / Z;                             // taps per load
+};
+
+template <typename T, int E> struct TapLoad;
+template <> struct TapLoad<float, 1> {
+    float2 t[1];
+    __device__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+    {
+        t[0] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+    }
+};
+template <> struct TapLoad<float, 2> {
+    float2 t[2];
+    __device__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+    {
+        const float4 v =
+            __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+        t[0] = make_float2(v.x, v.y);
+        t[1] = make_float2(v.z, v.w);
+    }
+};
+template <> struct TapLoad<double, 1> {
+    double2 t[1];
+    __device__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+    {
+        t[0] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+    }
+};
+
+constexpr int TILE_POS = 16;      // tile edge in footprint positions
+constexpr int TILE_SORT = 512;    // records ordered by position at a time
+constexpr int TILE_UNSORTED = 16; // up to this many are taken as they come
+
+template <typename T, int S, bool COMP, typename GT>
+__global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
+    const Rec<T> *__restrict__ recs, const Item *__restrict__ items,
+    const unsigned long long *__restrict__ stats, const typename Vec2<T>::type *__restrict__ kern,
+    uint32_t kern_bytes, TileSink sink)
 {
     using T2 = typename Vec2<T>::type;
-    constexpr int NT = S * S;
-    constexpr int RT = TILE + S - 1;
-    // cell rows RTP apart (RT rounded up to S): a record's (lx, ly) residues
-    // follow from its byte offsets
-    constexpr int RTP = (RT + S - 1) / S * S;
-    constexpr int CELLS = RT * RTP;
-    constexpr int z = (int)sizeof(T2);
-    static_assert(CELLS * z <= 65536, "cell byte offsets fit 16 bits");
+    using Span = TapSpan<T, S>;
+    constexpr int TW = TILE_POS, TH = TILE_POS;
+    constexpr int RW = TW + S - 1, RH = TH + S - 1;
+    // odd row stride: the rows a wavefront adds to start in different LDS banks
+    constexpr int RS = RW | 1;
+    constexpr int CELLS = RH * RS;
     constexpr int LC = COMP ? CELLS : 1;
+    constexpr int BINS = TW * TH;
+    constexpr int BPL = BINS / 64; // bins per lane
+    static_assert(BINS % 64 == 0 && TILE_SORT % 64 == 0, "whole wavefronts");
     __shared__ T2 s_cell[CELLS]; // (re, im) of every cell of the tile and its halo
     __shared__ T2 s_lo[LC];      // COMP: the two-sum low parts
-    __shared__ Rec<T> s_rec[NT];
+    __shared__ uint32_t s_bin[BINS];
+    __shared__ uint16_t s_order[TILE_SORT];
 
-    const uint32_t end = stats ? (uint32_t)stats[CNT_ITEMS] : item_end;
-    const uint32_t it = item0 + blockIdx.x;
-    if (it >= end)
-        return;
-    const Item item = items[it];
-
-    for (int c = threadIdx.x; c < CELLS; c += NT) {
-        s_cell[c].x = T(0);
-        s_cell[c].y = T(0);
-        if (COMP) {
-            s_lo[c].x = T(0);
-            s_lo[c].y = T(0);
-        }
-    }
-
-    const int myU = threadIdx.x % S, myV = threadIdx.x / S;
-    const int myUz = myU * z, myVSz = myV * S * z;
-    char *cell_b = reinterpret_cast<char *>(s_cell);
-    char *lo_b = reinterpret_cast<char *>(s_lo);
-    auto cellp = [&](int c) { return reinterpret_cast<T2 *>(cell_b + c); };
-    auto lop = [&](int c) { return reinterpret_cast<T2 *>(lo_b + c); };
+    const int lane = threadIdx.x;
     const __amdgpu_buffer_rsrc_t ktab =
         __builtin_amdgcn_make_buffer_rsrc((void *)kern, 0, (int)kern_bytes, BUF_RSRC_W3);
-    int cur = -1;
-    T sr = T(0), si = T(0);
-    T2 pre; // !COMP: the LDS value of cell cur when the thread started it
-    pre.x = T(0);
-    pre.y = T(0);
-    // adds the register sum into cell cur
-    auto flush = [&]() {
-        if (COMP) {
-            two_sum_into(cellp(cur)->x, lop(cur)->x, sr);
-            two_sum_into(cellp(cur)->y, lop(cur)->y, si);
-        } else {
-            T2 o = pre;
-            o.x += sr;
-            o.y += si;
-            *cellp(cur) = o;
-        }
-    };
+    // the lane's first cell of load 0, from the footprint's corner
+    const int lbase = lane * Span::E / S * RS + lane * Span::E % S;
 
-    // Records are staged NT at a time and consumed U at a time: the U tap
-    // loads are issued together, then the U updates run in stream order.  A
-    // partial batch is padded with zero-weight records (tile corner 0).
-    constexpr int U = 8;
-    static_assert(NT % U == 0, "record batch must be a multiple of the unroll");
-    for (uint32_t b = 0; b < item.count; b += NT) {
-        const uint32_t nloc = min((uint32_t)NT, item.count - b);
-        const uint32_t nlocU = (nloc + U - 1) / U * U;
-        __syncthreads();
-        if (threadIdx.x < nloc) {
-            s_rec[threadIdx.x] = recs[item.start + b + threadIdx.x];
-        } else if (threadIdx.x < nlocU) {
-            Rec<T> z;
-            z.pos = 0;
-            z.kidx = 0;
-            z.vis.x = T(0);
-            z.vis.y = T(0);
-            s_rec[threadIdx.x] = z;
-        }
-        __syncthreads();
-        using B = RecBatch<T, U>;
-        auto fetch = [&](uint32_t j, B &bt) {
-#pragma unroll
-            for (int q = 0; q < U; ++q) {
-                // pos = (ly RTP + lx) z | (ly S z) << 16, kidx = sub-kernel byte offset
-                const Rec<T> r = s_rec[j + q];
-                const int cxz = (myUz - (int)r.pos) & ((S - 1) * z);
-                const int cyS = (myVSz - (int)(r.pos >> 16)) & ((S - 1) * S * z);
-                bt.cell[q] = (int)(r.pos & 0xffffu) + cyS * (RTP / S) + cxz;
-                bt.v[q] = r.vis;
-                bt.k[q] = tap_load(ktab, r.kidx + (uint32_t)(cyS + cxz), (T2 *)nullptr);
-            }
-        };
-        auto update = [&](const B &bt) {
-#pragma unroll
-            for (int q = 0; q < U; ++q) {
-                if (bt.cell[q] != cur) {
-                    if (cur >= 0)
-                        flush();
-                    cur = bt.cell[q];
-                    if (!COMP)
-                        pre = *cellp(cur);
-                    sr = T(0);
-                    si = T(0);
-                }
-                // conj(k) * v
-                sr = fma(bt.k[q].x, bt.v[q].x, sr);
-                sr = fma(bt.k[q].y, bt.v[q].y, sr);
-                si = fma(bt.k[q].x, bt.v[q].y, si);
-                si = fma(-bt.k[q].y, bt.v[q].x, si);
-            }
-        };
-        pipelined_records<U, B>(nlocU, fetch, update);
-    }
-    if (cur >= 0)
-        flush();
-    __syncthreads();
-
-    const uint32_t group = item.key / (uint32_t)sink.ntiles;
-    const int tile = (int)(item.key - group * (uint32_t)sink.ntiles);
-    const int tx = tile % sink.ntx, ty = tile / sink.ntx;
-    const int ox = tx * TILE - S, oy = ty * TILE - S;
-    int64_t slot = (int64_t)group;
-    if (sink.group_map)
-        slot = (int64_t)sink.group_map[group] - sink.group_offset;
-    const int G = sink.gsize;
-    GT *g = reinterpret_cast<GT *>(sink.base) + (size_t)slot * G * G * 2;
-    for (int c = threadIdx.x; c < CELLS; c += NT) {
-        const int ry = c / RTP, rx = c - ry * RTP;
-        const int gx = ox + rx, gy = oy + ry;
-        if (rx < RT && (unsigned)gx < (unsigned)G && (unsigned)gy < (unsigned)G) {
-            GT re = (GT)s_cell[c].x, im = (GT)s_cell[c].y;
+    const uint32_t nitems = (uint32_t)stats[CNT_ITEMS];
+    // the grid is no larger than the item list: the first item is read beside its length
+    Item item = items[blockIdx.x];
+    for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
+        if (it != blockIdx.x)
+            item = items[it];
+#pragma unroll 2
+        for (int c = lane; c < CELLS; c += 64) {
+            s_cell[c].x = T(0);
+            s_cell[c].y = T(0);
             if (COMP) {
-                re += (GT)s_lo[c].x;
-                im += (GT)s_lo[c].y;
-            }
-            if (re != GT(0) || im != GT(0)) {
-                GT *dst = g + 2 * ((size_t)gy * G + gx);
-                atomicAdd(dst, re);
-                atomicAdd(dst + 1, im);
+                s_lo[c].x = T(0);
+                s_lo[c].y = T(0);
             }
         }
+        T2 sum[Span::NL][Span::E];
+        int cur = -1; // corner cell of the footprint the sums belong to
+        auto clear = [&]() {
+#pragma unroll
+            for (int l = 0; l < Span::NL; ++l)
+#pragma unroll
+                for (int e = 0; e < Span::E; ++e)
+                    sum[l][e].x = sum[l][e].y = T(0);
+        };
+        auto flush = [&]() {
+            const int c0 = cur + lbase;
+#pragma unroll
+            for (int l = 0; l < Span::NL; ++l)
+#pragma unroll
+                for (int e = 0; e < Span::E; ++e) {
+                    const int c = c0 + l * (64 * Span::E / S) * RS + e;
+                    if (COMP) {
+                        two_sum_into(s_cell[c].x, s_lo[c].x, sum[l][e].x);
+                        two_sum_into(s_cell[c].y, s_lo[c].y, sum[l][e].y);
+                    } else {
+                        s_cell[c].x += sum[l][e].x;
+                        s_cell[c].y += sum[l][e].y;
+                    }
+                }
+        };
+        clear();
+        for (uint32_t b = 0; b < item.count; b += TILE_SORT) {
+            const int n = (int)min((uint32_t)TILE_SORT, item.count - b);
+            const Rec<T> *r0 = recs + item.start + b;
+            // order the n records by position
+            const bool ordered = n > TILE_UNSORTED;
+            if (ordered) {
+                __syncthreads();
+#pragma unroll
+                for (int k = 0; k < BPL; ++k)
+                    s_bin[lane + 64 * k] = 0;
+                __syncthreads();
+                auto bin = [&](int i) {
+                    const uint32_t p = r0[i].pos;
+                    return (p >> 16) * TW + (p & 0xffffu);
+                };
+#pragma unroll 2
+                for (int i = lane; i < n; i += 64)
+                    atomicAdd(&s_bin[bin(i)], 1u);
+                __syncthreads();
+                uint32_t c[BPL], tot = 0;
+#pragma unroll
+                for (int k = 0; k < BPL; ++k) {
+                    c[k] = s_bin[lane * BPL + k];
+                    tot += c[k];
+                }
+                uint32_t inc = tot;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t x = (uint32_t)__shfl_up((int)inc, o);
+                    if (lane >= o)
+                        inc += x;
+                }
+                uint32_t run = inc - tot;
+#pragma unroll
+                for (int k = 0; k < BPL; ++k) {
+                    s_bin[lane * BPL + k] = run;
+                    run += c[k];
+                }
+                __syncthreads();
+#pragma unroll 2
+                for (int i = lane; i < n; i += 64)
+                    s_order[atomicAdd(&s_bin[bin(i)], 1u)] = (uint16_t)i;
+                __syncthreads();
+            }
+
+            auto record = [&](int k) {
+                Rec<T> r;
+                r.pos = 0;
+                r.kidx = 0;
+                r.vis.x = T(0);
+                r.vis.y = T(0);
+                if (k + lane < n)
+                    r = r0[ordered ? (int)s_order[k + lane] : k + lane];
+                return r;
+            };
+            // FP64 taps take twice the registers
+            constexpr int U = Span::NL * Span::LOAD > 32 ? 2 : 4;
+            struct Batch {
+                TapLoad<T, Span::E> t[U][Span::NL];
+            };
+            auto fetch = [&](uint32_t kidx, int j, Batch &bt) {
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    const int off = __builtin_amdgcn_readlane((int)kidx, j + q);
+#pragma unroll
+                    for (int l = 0; l < Span::NL; ++l)
+                        bt.t[q][l].load(ktab, lane * Span::LOAD + l * 64 * Span::LOAD, off);
+                }
+            };
+            // Taps are fetched U records ahead without a condition, so that the wait
+            // for a batch leaves the next one in flight; across a chunk's end from the
+            // next chunk's records (records past the last read the first sub-kernel).
+            Rec<T> next = record(0);
+            Batch ba, bb;
+            fetch(next.kidx, 0, ba);
+            for (int k = 0; k < n; k += 64) {
+                const Rec<T> r = next;
+                next = record(k + 64);
+                const int m = min(64, n - k);
+                const int cell = (int)((r.pos >> 16) * RS + (r.pos & 0xffffu));
+                int prev = __shfl_up(cell, 1);
+                if (lane == 0)
+                    prev = cur;
+                const unsigned long long change = __ballot(cell != prev);
+                auto update = [&](int j, const Batch &bt) {
+#pragma unroll
+                    for (int q = 0; q < U; ++q) {
+                        const int i = j + q;
+                        if (i >= m)
+                            break;
+                        if ((change >> i) & 1ull) {
+                            if (cur >= 0) {
+                                flush();
+                                clear();
+                            }
+                            cur = __builtin_amdgcn_readlane(cell, i);
+                        }
+                        const T vr = lane_value(r.vis.x, i), vi = lane_value(r.vis.y, i);
+#pragma unroll
+                        for (int l = 0; l < Span::NL; ++l)
+#pragma unroll
+                            for (int e = 0; e < Span::E; ++e) {
+                                // conj(tap) * value
+                                const T2 t = bt.t[q][l].t[e];
+                                T2 &s = sum[l][e];
+                                s.x = fma(t.x, vr, s.x);
+                                s.x = fma(t.y, vi, s.x);
+                                s.y = fma(t.x, vi, s.y);
+                                s.y = fma(-t.y, vr, s.y);
+                            }
+                    }
+                };
+                for (int j = 0; j < m; j += 2 * U) {
+                    fetch(r.kidx, j + U, bb);
+                    update(j, ba);
+                    fetch(j + 2 * U < 64 ? r.kidx : next.kidx, (j + 2 * U) & 63, ba);
+                    update(j + U, bb);
+                }
+            }
+        }
+        flush();
+        __syncthreads();
+
+        const uint32_t gt = item.key % (uint32_t)(sink.ntiles * sink.groups);
+        const uint32_t group = gt / (uint32_t)sink.ntiles;
+        const int tile = (int)(gt - group * (uint32_t)sink.ntiles);
+        const int tx = tile % sink.ntx, ty = tile / sink.ntx;
+        const int ox = tx * TW - S, oy = ty * TH - S;
+        const int G = sink.gsize;
+        GT *g = reinterpret_cast<GT *>(sink.base) + (size_t)group * G * G * 2;
+        // a row's cells as 2 RW consecutive numbers: whole 64-byte pieces of the grid's row
+        // in one instruction; FB rows' LDS reads in flight
+        constexpr int FB = 8;
+        const T *cf = reinterpret_cast<const T *>(s_cell), *lf = reinterpret_cast<const T *>(s_lo);
+        for (int f = lane; f < 2 * RW; f += 64) {
+            if ((unsigned)(ox + f / 2) >= (unsigned)G)
+                continue;
+            GT *gf = g + 2 * ((int64_t)oy * G + ox) + f;
+            for (int r0 = 0; r0 < RH; r0 += FB) {
+                GT v[FB];
+#pragma unroll
+                for (int q = 0; q < FB; ++q) {
+                    const int ry = min(r0 + q, RH - 1);
+                    v[q] = (GT)cf[ry * 2 * RS + f];
+                    if (COMP)
+                        v[q] += (GT)lf[ry * 2 * RS + f];
+                }
+#pragma unroll
+                for (int q = 0; q < FB; ++q)
+                    if (r0 + q < RH && (unsigned)(oy + r0 + q) < (unsigned)G && v[q] != GT(0))
+                        atomicAdd(gf + 2 * (int64_t)(r0 + q) * G, v[q]);
+            }
+        }
+        __syncthreads();
     }
 }
 

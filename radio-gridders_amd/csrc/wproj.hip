@@ -7,8 +7,8 @@
 // thread's grid point changes.
 //
 // Batched path: visibilities are counting-sorted by the grid tile of their
-// footprint (binning.hpp), coordinates computed once per visibility during
-// the sort (FP64, same formulas), then accumulated per tile in LDS by the
+// footprint and the group of its W-plane (binning.hpp), coordinates computed once per
+// visibility during the sort (FP64, same formulas), then accumulated per tile in LDS by the
 // Romein kernel of tiles.hpp.
 #include <algorithm>
 #include <mutex>
@@ -137,6 +137,10 @@ int wproj_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis
     return RG_OK;
 }
 
+// Workgroups of the tile kernel: enough that each takes one item of all but the
+// longest calls; they loop beyond that.
+constexpr int64_t TILE_GRID = 65536;
+
 // ---- batched tiled Romein -------------------------------------------------------
 
 struct WprojKeyer {
@@ -145,8 +149,9 @@ struct WprojKeyer {
     int vis_type;
     int N, S, R, P;
     double theta, w_min, w_step;
-    int tile, ntx, ntiles;
-    int zb, rtp; // bytes per kernel tap; cell row stride of a tile (tile + S - 1 rounded up to S)
+    int ntx, ntiles;         // tiles per row and grid
+    int group_planes;        // W-planes per plane group
+    int zb;                  // bytes per kernel tap
     const int64_t *chan_off;
     int nchan;
 
@@ -172,13 +177,11 @@ struct WprojKeyer {
         const int p = w_plane(w[i], w_min, w_step);
         if (p < 0 || p >= P)
             return VIS_BAD_PLANE;
-        const int tx = (gx + S) / tile, ty = (gy + S) / tile;
-        const int lx = gx + S - tx * tile, ly = gy + S - ty * tile;
+        const int tx = (gx + S) / TILE_POS, ty = (gy + S) / TILE_POS;
         const int c = nchan > 1 ? chan_of(i) : 0;
-        key = (uint32_t)(c * ntiles + ty * ntx + tx);
-        // byte offsets as the tile kernel uses them: cell (lx, ly) of the tile's
-        // LDS cells and row ly of a sub-kernel; first tap of the sub-kernel
-        pos = (uint32_t)((ly * rtp + lx) * zb) | ((uint32_t)(ly * S * zb) << 16);
+        key = (uint32_t)((p / group_planes * nchan + c) * ntiles + ty * ntx + tx);
+        // position in the tile; byte offset of the sub-kernel
+        pos = (uint32_t)(gx + S - tx * TILE_POS) | (uint32_t)(gy + S - ty * TILE_POS) << 16;
         kidx = (uint32_t)((p * R + yf) * R + xf) * (uint32_t)(S * S * zb);
         return VIS_OK;
     }
@@ -199,90 +202,92 @@ struct WprojKeyer {
     }
 };
 
-template <typename T, int S, int TILE, bool COMP, typename GT>
-static int launch_tiles(const BinResult &br, rg_context *timer_ctx, unsigned long long *stats,
-                        const rg_wkern *wk, void *grid, int N, int ntx, int ntiles, hipStream_t s)
+// Tile geometry and sort parameters of batched W-projection.
+struct WprojShape {
+    int ntx, ntiles;
+    int group_planes; // W-planes per plane group
+    int64_t nkeys;    // plane groups x grids x tiles
+    uint32_t per_item;
+
+    void one_group(int planes, int n_chan)
+    {
+        group_planes = std::max(planes, 1);
+        nkeys = (int64_t)ntiles * n_chan;
+    }
+};
+constexpr int64_t WPROJ_COUNTERS = (int64_t)1 << 22;
+
+template <typename T, int S, bool COMP, typename GT>
+static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
+                        const unsigned long long *stats, const rg_wkern *wk, void *grid, int N,
+                        int n_chan, const WprojShape &sh, hipStream_t s)
 {
     TileSink sink;
     sink.base = grid;
     sink.gsize = N;
-    sink.ntx = ntx;
-    sink.ntiles = ntiles;
-    sink.group_map = nullptr;
-    sink.group_offset = 0;
+    sink.ntx = sh.ntx;
+    sink.ntiles = sh.ntiles;
+    sink.groups = n_chan;
     KernelTimer kt(timer_ctx, RG_TIMER_WPROJ_TILES, s);
     const uint64_t kbytes = (uint64_t)wk->plane_count * wk->oversampling * wk->oversampling * S *
                             S * sizeof(typename Vec2<T>::type);
     if (kbytes > 0x7fffffffull)
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection kernel tables above 2 GiB");
-    if (br.max_items > 0)
-        hipLaunchKernelGGL((k_tiles<T, S, TILE, COMP, GT>), dim3((unsigned)br.max_items),
-                           dim3(S * S), 0, s, (const Rec<T> *)br.recs, (const Item *)br.items, 0u,
-                           0u, (const unsigned long long *)stats,
+    if (br.max_items > 0) {
+        const int64_t nb = std::min<int64_t>(br.max_items, TILE_GRID);
+        hipLaunchKernelGGL((k_tiles<T, S, COMP, GT>), dim3((unsigned)nb), dim3(64), 0, s,
+                           (const Rec<T> *)br.recs, (const Item *)br.items, stats,
                            (const typename Vec2<T>::type *)wk->data, (uint32_t)kbytes, sink);
+    }
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
 
-template <typename T, int S, int TILE>
+template <typename T, int S>
 static int dispatch_comp_grid(const BinResult &br, rg_context *timer_ctx,
-                              unsigned long long *stats, const rg_wkern *wk, void *grid,
-                              int grid_type, bool comp, int N, int ntx, int ntiles, hipStream_t s)
+                              const unsigned long long *stats, const rg_wkern *wk, void *grid,
+                              int grid_type, bool comp, int N, int n_chan, const WprojShape &sh,
+                              hipStream_t s)
 {
+    auto run = [&](auto c, auto g) {
+        return launch_tiles<T, S, decltype(c)::value, decltype(g)>(
+            br, timer_ctx, stats, wk, grid, N, n_chan, sh, s);
+    };
     if constexpr (std::is_same<T, double>::value) {
         if (grid_type != RG_C128)
             return fail(RG_ERR_PARAM, "FP64 kernels need an RG_C128 grid");
-        return launch_tiles<double, S, TILE, false, double>(br, timer_ctx, stats, wk, grid, N, ntx,
-                                                            ntiles, s);
+        return run(std::false_type{}, double{});
     } else {
         if (grid_type == RG_C128)
-            return comp ? launch_tiles<float, S, TILE, true, double>(br, timer_ctx, stats, wk, grid,
-                                                                      N, ntx, ntiles, s)
-                        : launch_tiles<float, S, TILE, false, double>(br, timer_ctx, stats, wk,
-                                                                       grid, N, ntx, ntiles, s);
-        return comp ? launch_tiles<float, S, TILE, true, float>(br, timer_ctx, stats, wk, grid, N,
-                                                                 ntx, ntiles, s)
-                    : launch_tiles<float, S, TILE, false, float>(br, timer_ctx, stats, wk, grid, N,
-                                                                  ntx, ntiles, s);
+            return comp ? run(std::true_type{}, double{}) : run(std::false_type{}, double{});
+        return comp ? run(std::true_type{}, float{}) : run(std::false_type{}, float{});
     }
 }
 
 template <typename T>
-static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx, unsigned long long *stats,
-                          const rg_wkern *wk, void *grid, int grid_type, bool comp, int N,
-                          int tile, int ntx, int ntiles, hipStream_t s)
+static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx,
+                          const unsigned long long *stats, const rg_wkern *wk, void *grid,
+                          int grid_type, bool comp, int N, int n_chan, const WprojShape &sh,
+                          hipStream_t s)
 {
-    if (wk->size == 16)
-        return tile == 32 ? dispatch_comp_grid<T, 16, 32>(br, timer_ctx, stats, wk, grid,
-                                                          grid_type, comp, N, ntx, ntiles, s)
-                          : dispatch_comp_grid<T, 16, 48>(br, timer_ctx, stats, wk, grid,
-                                                          grid_type, comp, N, ntx, ntiles, s);
-    return tile == 32 ? dispatch_comp_grid<T, 8, 32>(br, timer_ctx, stats, wk, grid, grid_type,
-                                                     comp, N, ntx, ntiles, s)
-                      : dispatch_comp_grid<T, 8, 48>(br, timer_ctx, stats, wk, grid, grid_type,
-                                                     comp, N, ntx, ntiles, s);
+    auto run = [&](auto sz) {
+        return dispatch_comp_grid<T, decltype(sz)::value>(br, timer_ctx, stats, wk, grid, grid_type,
+                                                          comp, N, n_chan, sh, s);
+    };
+    using std::integral_constant;
+    return wk->size == 16 ? run(integral_constant<int, 16>{}) : run(integral_constant<int, 8>{});
 }
 
-// Tile geometry and sort parameters of batched W-projection.
-struct WprojShape {
-    int tile, ntx, ntiles;
-    uint32_t per_item;
-};
-
-// Records per work item when the caller leaves it open.  A workgroup walks its
-// item's records one after another (about 0.1 us each), so a stream is cut
-// into about 350 to 700 items, which fills the CUs without flushing a tile for a
-// handful of records; long streams take larger items, up to the size at which
-// the longest item still hides behind the others.  Tile time, FP64, 32-cell tiles:
-// 448 visibilities 32 us in items of 2048, 10 us in items of 32; 90 k 167 -> 53
-// us (2048 -> 256; 64: 61); 520 k, FP32, 186 -> 117 us (2048 -> 1024; 256: 135);
-// 64 channels, 4.2 M: 907 -> 845 us (2048 -> 512; 256: 968); 48-cell tiles, 8.4 M: 1539
-// us at 2048, 1689 at 1024.
-static uint32_t default_item(int64_t nvis, int n_chan, int tile)
+// Records per work item when the caller leaves it open.  A wavefront walks its
+// item's records one after another, and every item adds its tile to the grid, so both the
+// records of an item and the items grow with the stream: the largest power of two from 4 to
+// 512 with 12 K^2 <= records.  Tile kernel or call, us, at half / this / twice the size:
+// 448 records FP64 - / 5.2 / 6.7; 16 k FP64 on 2000^2 60 / 54 / 57; 150 k FP32 69 / 65
+// / -; 520 k FP64 225 / 204 / 237; 8.4 M FP32 1032 / 1042 / 1161.
+static uint32_t default_item(int64_t nvis)
 {
-    const uint32_t cap = n_chan > 1 ? 512 : tile == 48 ? 2048 : 1024;
-    uint32_t k = 32;
-    while (k < cap && (int64_t)k * 700 <= nvis)
+    uint32_t k = 4;
+    while (k < TILE_SORT && 12 * (int64_t)(2 * k) * (2 * k) <= nvis)
         k *= 2;
     return k;
 }
@@ -291,15 +296,30 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
                        WprojShape &sh)
 {
     const int S = wk->size;
-    sh.tile = p->tile > 0 ? p->tile : 32;
-    if (sh.tile != 32 && sh.tile != 48)
-        return fail(RG_ERR_UNSUPPORTED, "batched tile must be 32 or 48 (got %d)", sh.tile);
+    // both values of the parameter run the same tiles
+    const int tile = p->tile > 0 ? p->tile : 32;
+    if (tile != 32 && tile != 48)
+        return fail(RG_ERR_UNSUPPORTED, "batched tile must be 32 or 48 (got %d)", tile);
     if (S != 8 && S != 16)
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection supports kernel sizes 8 and 16 (got %d)", S);
-    sh.ntx = (p->grid_size + S + sh.tile - 1) / sh.tile;
+    sh.ntx = (p->grid_size + S + TILE_POS - 1) / TILE_POS;
     sh.ntiles = sh.ntx * sh.ntx;
-    sh.per_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item
-                                      : default_item(nvis, n_chan, sh.tile);
+    // Plane groups of 2^18 taps (2 MB in FP32, 4 MB in FP64, an XCD's L2) where a tile
+    // has at least 64 records: 8.4 M FP32 1730 us in one group, 1120 in groups of twice the size,
+    // 1040; 520 k FP64 275, 222, 204.  Sparser streams pay more for the extra items than they save:
+    // 16 k on 2000^2 57 us in one group, 93 in groups; 64 channels (16 a tile) 1120, 1415.
+    const int64_t plane_taps = (int64_t)wk->oversampling * wk->oversampling * S * S;
+    const int64_t planes = std::max<int64_t>(wk->plane_count, 1);
+    const int64_t group = std::max<int64_t>({1, ((int64_t)1 << 18) / std::max<int64_t>(plane_taps, 1),
+                                             (planes + 63) / 64});
+    const int64_t one = (int64_t)sh.ntiles * n_chan, all = (planes + group - 1) / group;
+    sh.one_group(wk->plane_count, n_chan);
+    if (nvis >= 64 * one && all > 1) {
+        sh.group_planes = (int)group;
+        sh.nkeys = one * all;
+    }
+    sh.per_item = p->vis_per_item > 0 ? std::min<uint32_t>((uint32_t)p->vis_per_item, TILE_SORT)
+                                      : default_item(nvis);
     return RG_OK;
 }
 
@@ -319,11 +339,10 @@ static WprojKeyer wproj_keyer(const rg_grid_params *p, const rg_flat_vis *vis, c
     kf.theta = p->theta;
     kf.w_min = wk->w_min;
     kf.w_step = wk->w_step;
-    kf.tile = sh.tile;
     kf.ntx = sh.ntx;
     kf.ntiles = sh.ntiles;
+    kf.group_planes = sh.group_planes;
     kf.zb = zb;
-    kf.rtp = (sh.tile + wk->size - 1 + wk->size - 1) / wk->size * wk->size;
     kf.chan_off = d_off;
     kf.nchan = n_chan;
     return kf;
@@ -343,14 +362,23 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     ZeroList zero;
     RG_TRY(zero.add(ctx->counters.p, sizeof(unsigned long long) * CNT__N));
     RG_TRY(zero.add(grid, gbytes));
+    BinPlan pl;
+    int rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
+    if (rc != RG_OK && sh.nkeys != (int64_t)sh.ntiles * n_chan) {
+        // no room for the plane groups (a captured graph holds the scratch): without them
+        sh.one_group(wk->plane_count, n_chan);
+        rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
+    }
+    if (rc != RG_OK)
+        return rc;
 
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
-    RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, (int64_t)sh.ntiles * n_chan,
-                                            sh.per_item, zero, s, br)));
+    RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, sh.nkeys,
+                                            sh.per_item, zero, s, br, WPROJ_COUNTERS, &pl)));
     return dispatch_tiles<T>(br, ctx, ctx->counters.as<unsigned long long>(), wk, grid, grid_type,
-                             p->compensated != 0, N, sh.tile, sh.ntx, sh.ntiles, s);
+                             p->compensated != 0, N, n_chan, sh, s);
 }
 
 int wproj_batched(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis,
@@ -369,7 +397,10 @@ int wproj_batched(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *v
 // device address on the current device comes from hipGetSymbolAddress, looked
 // up once per device and kept.  Calls on one device share the array, so calls
 // that overlap in time on one device (several streams or host threads) race.
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
+// NOALLOC_LIMIT_BYTES bounds the stream (about 2.0 M visibilities with FP32 kernels,
+// 1.4 M with FP64 at 2048^2); the rest is room for the finer tiles' keys up to 36 000^2 grids.
+constexpr size_t NOALLOC_LIMIT_BYTES = (size_t)64 << 20;
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)192 << 20;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -395,7 +426,7 @@ static int noalloc_scratch(void **out)
     return RG_OK;
 }
 
-size_t noalloc_scratch_bytes() { return NOALLOC_SCRATCH_BYTES; }
+size_t noalloc_scratch_bytes() { return NOALLOC_LIMIT_BYTES; }
 
 template <typename T>
 static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk,
@@ -404,35 +435,47 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     const int N = p->grid_size;
     WprojShape sh;
     RG_TRY(wproj_shape(p, vis->n, 1, wk, sh));
-    BinPlan pl;
-    RG_TRY(bin_plan(vis->n, sh.ntiles, sh.per_item, (int64_t)1 << 22, sizeof(Rec<T>), pl));
-    // Carve the arrays from the static scratch, 256-byte aligned.  The scatter
-    // cursors take the place of the counters they are made from; the space this leaves
-    // covers the shorter default work items and scan blocks of small calls, so
-    // the limit on the stream is that of separate cursors, items of 2048
-    // records and scan blocks of 1024 keys.
     auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t head = aligned(sizeof(unsigned long long) * CNT__N); // call counters first
-    const int64_t limit_item = p->vis_per_item > 0 ? p->vis_per_item : 2048;
+    // The limit on the stream is that of a sort by tiles of the parameter's 32 or 48
+    // cells with separate cursors, items of 2048 records and scan blocks of 1024 keys in
+    // NOALLOC_LIMIT_BYTES.
+    BinPlan pl;
+    const uint32_t limit_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item : 2048u;
+    const int64_t lt = p->tile > 0 ? p->tile : 32, ln = (N + wk->size + lt - 1) / lt, lk = ln * ln;
+    RG_TRY(bin_plan(vis->n, lk, limit_item, WPROJ_COUNTERS, sizeof(Rec<T>), pl));
+    size_t want = head;
+    for (int k = 0; k < BIN__N; ++k)
+        want += aligned(k == BIN_BSUMS ? sizeof(uint2) * (size_t)((lk + 1023) / 1024 + 1)
+                                       : pl.bytes[k]);
+    // Carve the arrays from the static scratch, 256-byte aligned.  The scatter
+    // cursors take the place of the counters they are made from.
     size_t off[BIN__N];
-    size_t at = head, want = head;
-    for (int k = 0; k < BIN__N; ++k) {
-        if (k == BIN_CURSOR) {
-            off[k] = off[BIN_COUNT];
-        } else {
-            off[k] = at;
-            at += aligned(pl.bytes[k]);
+    size_t at = 0;
+    auto carve = [&](int64_t max_counters) {
+        RG_TRY(bin_plan(vis->n, sh.nkeys, sh.per_item, max_counters, sizeof(Rec<T>), pl));
+        at = head;
+        for (int k = 0; k < BIN__N; ++k) {
+            if (k == BIN_CURSOR) {
+                off[k] = off[BIN_COUNT];
+            } else {
+                off[k] = at;
+                at += aligned(pl.bytes[k]);
+            }
         }
-        want += aligned(
-            k == BIN_ITEMS ? sizeof(Item) * (size_t)(sh.ntiles + vis->n / limit_item + 1)
-            : k == BIN_BSUMS ? sizeof(uint2) * (size_t)((sh.ntiles + 1023) / 1024 + 1)
-                             : pl.bytes[k]);
+        return (int)RG_OK;
+    };
+    RG_TRY(carve(WPROJ_COUNTERS));
+    if (at > NOALLOC_SCRATCH_BYTES) { // leaner: no plane groups, larger items, one replica
+        sh.one_group(wk->plane_count, 1);
+        sh.per_item = std::max(sh.per_item, limit_item);
+        RG_TRY(carve(1));
     }
-    if (want > NOALLOC_SCRATCH_BYTES || at > NOALLOC_SCRATCH_BYTES)
+    if (want > NOALLOC_LIMIT_BYTES || at > NOALLOC_SCRATCH_BYTES)
         return fail(RG_ERR_PARAM,
                     "rg_grid_noalloc: %lld visibilities on a %d^2 grid need %zu bytes of scratch; "
                     "the static scratch holds %zu: split the stream over calls with accumulate = 1",
-                    (long long)vis->n, N, want, NOALLOC_SCRATCH_BYTES);
+                    (long long)vis->n, N, want, NOALLOC_LIMIT_BYTES);
     void *base = nullptr;
     RG_TRY(noalloc_scratch(&base));
     char *b0 = static_cast<char *>(base);
@@ -456,10 +499,10 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
-    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.ntiles, sh.per_item, pl, b, zero, false, nullptr,
+    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.nkeys, sh.per_item, pl, b, zero, false, nullptr,
                                    s, br)));
-    return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N,
-                             sh.tile, sh.ntx, sh.ntiles, s);
+    return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N, 1,
+                             sh, s);
 }
 
 int wproj_noalloc(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk, void *grid,

@@ -122,3 +122,51 @@ def test_short_call_on_a_frozen_context(table):
         assert float((g - want).abs().max()) <= 1e-12 * float(want.abs().max())
     del graph
     c.close()
+
+
+def crowd(n, N, s, planes, seed):
+    """n visibilities: half in one 16 x 16 tile of positions (several a position), half over
+    the grid and its edges; planes of the whole table."""
+    rng = np.random.default_rng(seed)
+    half = N / THETA / 2
+    k = n // 2
+    u = np.concatenate([rng.uniform(-60.0, 60.0, k), rng.uniform(-1.1 * half, 1.1 * half, n - k)])
+    v = np.concatenate([rng.uniform(-60.0, 60.0, k), rng.uniform(-1.1 * half, 1.1 * half, n - k)])
+    w = rng.uniform(-0.5, planes - 0.6, n)
+    order = rng.permutation(n)
+    return (u[order], v[order], w[order], rng.standard_normal(n) + 1j * rng.standard_normal(n))
+
+
+@pytest.mark.parametrize("s,planes", [(16, 35), (8, 140)])
+@pytest.mark.parametrize("n,per_item", [(15, 16), (16, 16), (17, 17), (65, 512), (129, 512),
+                                        (1599, 0), (1600, 0), (1601, 513), (6000, 512)])
+@pytest.mark.parametrize("dt,gdt,comp", [(torch.complex128, torch.complex128, 0),
+                                         (torch.complex64, torch.complex64, 0),
+                                         (torch.complex64, torch.complex128, 1)])
+def test_wprojection_item_edges(ctx, s, planes, n, per_item, dt, gdt, comp):
+    """Items up to and above the 16 records that are taken unordered, one and more chunks of 64,
+    whole items of 512; streams below and above 64 records a tile (25 tiles at S = 16, 25 at
+    S = 8), where planes come in groups (16 and 64 planes, the last one partial).  Every cell is
+    a sum of at most n products, and a product takes four roundings: an error of
+    (n + 4) eps sum |k| |v|, with the sum gridded from the absolute values."""
+    N, r = 64, 8
+    rng = np.random.default_rng(s)
+    table = (rng.standard_normal((planes, r, r, s, s)) +
+             1j * rng.standard_normal((planes, r, r, s, s)))
+    u, v, w, vis = crowd(n, N, s, planes, n)
+    np_dt = np.complex64 if dt == torch.complex64 else np.complex128
+    table, vis = table.astype(np_dt).astype(np.complex128), vis.astype(np_dt).astype(np.complex128)
+    ref, _, bad = orc.grid_wprojection(N, THETA, u, v, w, vis, table, 0.0, 1.0)
+    mag, _, _ = orc.grid_wprojection(N, THETA, u, v, w, np.abs(vis) + 0j, np.abs(table) + 0j, 0.0,
+                                     1.0)
+    _, fv = stage(u, v, w, vis, dt)
+    _, wk = kern(table, 0.0, 1.0, dt)
+    g = torch.empty((N, N), dtype=gdt, device="cuda")
+    ctx.grid(rgamd.params(N, THETA, vis_per_item=per_item, compensated=comp), fv, wk, g)
+    st = ctx.stats()
+    assert st.n_bad_plane == bad
+    eps = 2.0 ** -24 if dt == torch.complex64 else 2.0 ** -53
+    # the oracle's own sums, too, in FP64
+    bound = (n + 4) * (eps + 2.0 ** -53) * mag.real
+    err = np.abs(g.cpu().numpy().astype(np.complex128) - ref)
+    assert (err <= bound).all(), float((err / np.maximum(bound, 1e-300)).max())
