@@ -286,7 +286,7 @@ static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx,
 // / -; 520 k FP64 225 / 204 / 237; 8.4 M FP32 1032 / 1042 / 1161.
 static uint32_t default_item(int64_t nvis)
 {
-    uint32_t k = 4;
+    uint32_t k = 8;
     while (k < TILE_SORT && 12 * (int64_t)(2 * k) * (2 * k) <= nvis)
         k *= 2;
     return k;
