@@ -607,7 +607,7 @@ __host__ __device__ constexpr int padded_rows(int S, int H) { return S + H; }
 constexpr int BAND_LEAD = 16;
 
 template <typename T>
-__device__ inline BandRec<T> band_record(const Rec<T> &r, int S, int H, int Hb, int z)
+__device__ inline BandRec<T> band_record(const Rec<T> &r, int S, int H, int Hb, int z, int tz)
 {
     const int gx = (int)(r.pos & 0xffffu) - S, gy = (int)(r.pos >> 16) - S;
     const int cy0 = Hb - gy; // >= 1 - H for every record of band Hb / H's window
@@ -617,9 +617,9 @@ __device__ inline BandRec<T> band_record(const Rec<T> &r, int S, int H, int Hb, 
     else
         o.xy = (uint32_t)((gx + BAND_LEAD) * z) | ((uint32_t)cy0 << 16);
     if constexpr (padded_taps<T>())
-        o.kb = ((H + (int32_t)r.kidx * padded_rows(S, H) + min(cy0, S)) * S) * z;
+        o.kb = ((H + (int32_t)r.kidx * padded_rows(S, H) + min(cy0, S)) * S) * tz;
     else
-        o.kb = ((int32_t)r.kidx * S * S + cy0 * S) * z;
+        o.kb = ((int32_t)r.kidx * S * S + cy0 * S) * tz;
     o.vis = r.vis;
     return o;
 }
@@ -631,6 +631,7 @@ template <typename T2> struct PadJob {
     T2 *dst;
     int64_t nsub;
     int S, H;
+    int pair; // every entry followed by the one H / 2 rows below it
     unsigned blocks;
 };
 
@@ -639,18 +640,25 @@ template <typename T2> __device__ inline void pad_kernels_block(const PadJob<T2>
     const int S = p.S, H = p.H, PS = padded_rows(S, H);
     const int64_t total = ((int64_t)H + p.nsub * PS) * S;
     for (int64_t e = (int64_t)b * 256 + threadIdx.x; e < total; e += (int64_t)p.blocks * 256) {
-        const int64_t prow = e / S - H; // row counted from the first sub-kernel
         const int col = (int)(e % S);
-        T2 v;
-        v.x = 0;
-        v.y = 0;
-        if (prow >= 0) {
-            const int64_t k = prow / PS;
-            const int row = (int)(prow - k * PS);
-            if (row < S)
-                v = p.src[(k * S + row) * S + col];
+        auto tap = [&](int64_t prow) { // row counted from the first sub-kernel
+            T2 v;
+            v.x = 0;
+            v.y = 0;
+            if (prow >= 0 && prow < p.nsub * PS) {
+                const int64_t k = prow / PS;
+                const int row = (int)(prow - k * PS);
+                if (row < S)
+                    v = p.src[(k * S + row) * S + col];
+            }
+            return v;
+        };
+        if (p.pair) {
+            p.dst[2 * e] = tap(e / S - H);
+            p.dst[2 * e + 1] = tap(e / S - H + H / 2);
+        } else {
+            p.dst[e] = tap(e / S - H);
         }
-        p.dst[e] = v;
     }
 }
 
@@ -719,7 +727,7 @@ __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ i
                                                     const uint32_t *__restrict__ key_start,
                                                     const uint32_t *__restrict__ item_start,
                                                     uint32_t K, int mk, int nbins, int S, int H,
-                                                    int nb,
+                                                    int tz, int nb,
                                                     const uint32_t *__restrict__ bands_part,
                                                     int nparts)
 {
@@ -761,7 +769,7 @@ __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ i
                     rank += (kj < key || (kj == key && j < (int)threadIdx.x)) ? 1u : 0u;
                 }
                 if (have)
-                    dst[rank] = band_record(r, S, H, Hb, z);
+                    dst[rank] = band_record(r, S, H, Hb, z, tz);
             }
             continue;
         }
@@ -803,7 +811,7 @@ __global__ __launch_bounds__(256) void k_sort_items(const Rec<T> *__restrict__ i
         for (uint32_t i = threadIdx.x; i < item.count; i += 256) {
             const Rec<T> r = src[i];
             const uint32_t d = atomicAdd(&bins[min(r.pos & 0xffffu, (uint32_t)nbins - 1)], 1u);
-            dst[d] = band_record(r, S, H, Hb, z);
+            dst[d] = band_record(r, S, H, Hb, z, tz);
         }
     }
 }
@@ -881,8 +889,16 @@ struct WindowSource : FixedItems {
 // stores the band straight into the task's subgrid; a key split over several
 // items stores each part in a spill slot and k_band_combine sums the parts in
 // item order.
-template <typename T, int S, int H, int LOGN, int GRP, bool COMP>
-__global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
+//
+// Bound by the vector cache's data return: a tap load takes it 16 to 20 cycles whether its
+// lanes read 8 or 16 bytes, and with one row a lane it was 93 % busy.  PAIR: a lane
+// owns rows myV and myV + H / 2 of its columns and reads both taps at once from
+// a table that holds every tap beside the one H / 2 rows below it, which halves the
+// loads and shares cell and tap addresses, half as many wavefronts a workgroup.  8.4 M
+// visibilities, 512^2 subgrids, FP32, S = 16: 2072 -> 1860 us (62 % VALU busy).  In FP64 a
+// tap is 16 bytes already, and at S = 8 a pair would leave a wavefront half empty.
+template <typename T, int S, int H, int LOGN, int GRP, bool COMP, bool PAIR>
+__global__ __launch_bounds__(S *H *GRP / (PAIR ? 2 : 1)) void k_tower_band_items(
     const BandRec<T> *__restrict__ recs, const Item *__restrict__ items,
     const uint32_t *__restrict__ item_start, BatchRef bref, int batch,
     const int32_t *__restrict__ rank_of_slot,
@@ -893,7 +909,8 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
 {
     using T2 = typename Vec2<T>::type;
     constexpr int n = 1 << LOGN;
-    constexpr int NL = S * H;
+    constexpr int RPL = PAIR ? 2 : 1; // band rows per lane
+    constexpr int NL = S * H / RPL;
     constexpr int NT = NL * GRP;
     constexpr int NB = n / H;
     constexpr int z = (int)sizeof(T2);
@@ -901,7 +918,8 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
     // the twiddles, which keeps the FP32 8-row band at four workgroups per CU
     constexpr int RS = 256;
     constexpr int RG = RS / GRP;
-    static_assert(RS % GRP == 0 && RS <= NT, "record staging");
+    constexpr int RPT = RS > NT ? RS / NT : 1; // records a thread stages
+    static_assert(RS % GRP == 0 && (RS <= NT || RS % NT == 0), "record staging");
     // row l of the band at logical [BAND_LEAD + l LS, + n) (pad16 after the
     // first IFFT stage, so the buffer holds the padded extent); the
     // S - 1 columns either side of a row fall in the gaps
@@ -953,9 +971,9 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
         // thread t < RG stages record t of each RS-record stage if t < split,
         // thread RG + u record split + u; the next stage's record is loaded
         // while the current stage is processed
-        auto stage_rec = [&](uint32_t base) {
+        auto stage_rec = [&](uint32_t base, int t) {
             BandRec<T> r;
-            const int t = (int)threadIdx.x, h = split(base);
+            const int h = split(base);
             const uint32_t nl = min((uint32_t)RS, item.count - base);
             const uint32_t i = GRP != 2 ? (uint32_t)t : t < RG ? (t < h ? (uint32_t)t : nl)
                                                             : (uint32_t)(h + t - RG);
@@ -972,9 +990,11 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
             }
             return r;
         };
-        BandRec<T> next;
-        if (threadIdx.x < RS)
-            next = stage_rec(0);
+        BandRec<T> next[RPT];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (threadIdx.x < RS)
+                next[q] = stage_rec(0, (int)threadIdx.x + q * NT);
         {
             // zero the band, 16 bytes per store
             float4 *b4 = reinterpret_cast<float4 *>(band);
@@ -991,38 +1011,57 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
         const int lane = threadIdx.x % NL, grp = threadIdx.x / NL;
         const int myU = lane % S, myV = lane / S;
         // per lane, in bytes: column residue, tap row, cell row
-        const int uz = myU * z, tap_row = myV * S * z, cell_row = myV * LS * z;
+        const int uz = myU * z, tap_row = myV * S * z * RPL, cell_row = myV * LS * z;
+        constexpr int PAIR_ROWS = H / 2 * LS * z; // from a lane's cell to its second row's
         char *band_b = reinterpret_cast<char *>(band);
         // cells are byte offsets in the logical (unpadded) layout
         int cur = -1, carry = -1; // carry: the kept cell of the unpadded form
-        T sr = T(0), si = T(0);
+        T sr[RPL] = {}, si[RPL] = {};
         // COMP: two-sum (Knuth) compensation of the register sums; cr, ci hold
         // the rounding errors, folded into sr, si before a sum leaves the lane
-        T cr = T(0), ci = T(0);
+        T cr[RPL] = {}, ci[RPL] = {};
         auto two_sum = [](T &s, T &c, T x) {
             const T t = s + x;
             const T bp = t - s;
             c += (s - (t - bp)) + (x - bp);
             s = t;
         };
-        auto mac = [&](const T2 &k, const T2 &v) { // sr + i si += conj(k) v
-            if constexpr (COMP) {
-                two_sum(sr, cr, fma(k.x, v.x, k.y * v.y));
-                two_sum(si, ci, fma(k.x, v.y, -(k.y * v.x)));
-            } else {
-                sr = fma(k.x, v.x, sr);
-                sr = fma(k.y, v.y, sr);
-                si = fma(k.x, v.y, si);
-                si = fma(-k.y, v.x, si);
+        auto mac = [&](const TapLoad<T, RPL> &tap, const T2 &v) { // sr + i si += conj(k) v
+#pragma unroll
+            for (int e = 0; e < RPL; ++e) {
+                const T2 k = tap.t[e];
+                if constexpr (COMP) {
+                    two_sum(sr[e], cr[e], fma(k.x, v.x, k.y * v.y));
+                    two_sum(si[e], ci[e], fma(k.x, v.y, -(k.y * v.x)));
+                } else {
+                    sr[e] = fma(k.x, v.x, sr[e]);
+                    sr[e] = fma(k.y, v.y, sr[e]);
+                    si[e] = fma(k.x, v.y, si[e]);
+                    si[e] = fma(-k.y, v.x, si[e]);
+                }
             }
         };
         auto fold = [&]() {
-            if constexpr (COMP) {
-                sr += cr;
-                si += ci;
-                cr = T(0);
-                ci = T(0);
-            }
+            if constexpr (COMP)
+#pragma unroll
+                for (int e = 0; e < RPL; ++e) {
+                    sr[e] += cr[e];
+                    si[e] += ci[e];
+                    cr[e] = T(0);
+                    ci[e] = T(0);
+                }
+        };
+        auto zero_sums = [&]() {
+#pragma unroll
+            for (int e = 0; e < RPL; ++e)
+                sr[e] = si[e] = T(0);
+        };
+        auto any_sum = [&]() {
+            bool any = false;
+#pragma unroll
+            for (int e = 0; e < RPL; ++e)
+                any = any || sr[e] != T(0) || si[e] != T(0);
+            return any;
         };
         // The groups take contiguous, column-sorted runs of each record stage,
         // so the cells of two groups can meet only within one footprint width
@@ -1038,30 +1077,31 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
         int safe_a = INT_MIN, safe_b = INT_MAX;
         // a cell of the row's gap: flushes into it are discarded
         const int gap_cell = cell_row + (n + BAND_LEAD) * z;
+        auto cellp = [&](int cl, int e) {
+            return reinterpret_cast<T2 *>(band_b + cl + e * PAIR_ROWS);
+        };
         auto flush = [&]() {
             fold();
-            T *c = reinterpret_cast<T *>(band_b + cur);
             const int col = cur - cell_row;
-            if (!REV && GRP > 1 && (col < safe_a || col >= safe_b)) {
-                atomicAdd(c, sr);
-                atomicAdd(c + 1, si);
-            } else {
-                T2 *c2 = reinterpret_cast<T2 *>(c);
-                T2 o = *c2;
-                o.x += sr;
-                o.y += si;
-                *c2 = o;
+            const bool shared = !REV && GRP > 1 && (col < safe_a || col >= safe_b);
+#pragma unroll
+            for (int e = 0; e < RPL; ++e) {
+                T2 *c2 = cellp(cur, e);
+                if (shared) {
+                    atomicAdd(&c2->x, sr[e]);
+                    atomicAdd(&c2->y, si[e]);
+                } else {
+                    T2 o = *c2;
+                    o.x += sr[e];
+                    o.y += si[e];
+                    *c2 = o;
+                }
             }
         };
         // with two groups a lane reads a cell's LDS value when it starts
         // summing into it (no other lane writes that cell before the lane's
         // flush), so the flush is a store
-        T2 pre;
-        pre.x = T(0);
-        pre.y = T(0);
-        auto cellp = [&](int cl) {
-            return reinterpret_cast<T2 *>(band_b + cl);
-        };
+        T2 pre[RPL] = {};
         if (REV) {
             cur = gap_cell;
             carry = gap_cell;
@@ -1069,13 +1109,15 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
         for (uint32_t base = 0; base < item.count; base += RS) {
             const uint32_t nloc = min((uint32_t)RS, item.count - base);
             __syncthreads();
-            if (threadIdx.x < RS) {
-                // the second group's half backwards (its walk descends)
-                const int t = (int)threadIdx.x;
-                s_rec[REV && t >= RG ? 3 * RG - 1 - t : t] = next;
-                if (base + RS < item.count)
-                    next = stage_rec(base + RS);
-            }
+#pragma unroll
+            for (int q = 0; q < RPT; ++q)
+                if (threadIdx.x < RS) {
+                    // the second group's half backwards (its walk descends)
+                    const int t = (int)threadIdx.x + q * NT;
+                    s_rec[REV && t >= RG ? 3 * RG - 1 - t : t] = next[q];
+                    if (base + RS < item.count)
+                        next[q] = stage_rec(base + RS, t);
+                }
             __syncthreads();
             const int h = split(base);
             const int ng = REV ? (grp == 0 ? h : max(0, (int)nloc - h))
@@ -1090,7 +1132,11 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
                 safe_a = grp > 0 ? (int)(s_rec[grp * RG - 1].xy & 0xffffu) + S * z : INT_MIN;
                 safe_b = grp < GRP - 1 ? (int)(s_rec[(grp + 1) * RG].xy & 0xffffu) : INT_MAX;
             }
-            using Bt = RecBatch<T, U>;
+            struct Bt {
+                int cell[U];
+                TapLoad<T, RPL> k[U];
+                T2 v[U];
+            };
             // A lane whose row the footprint misses reads a zero tap: from the
             // padding of the record's sub-kernel (its cell then follows the
             // footprint column like every other lane's, so it changes cell with
@@ -1105,14 +1151,13 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
                     bt.v[q] = r.vis;
                     if constexpr (padded_taps<T>()) {
                         bt.cell[q] = cell_row + gz + cxz;
-                        bt.k[q] = tap_load(ktab, (uint32_t)(r.kb + tap_row + cxz), (T2 *)nullptr);
+                        bt.k[q].load(ktab, r.kb + tap_row + cxz * RPL, 0);
                     } else {
                         const int cy = ((int)r.xy >> 16) + myV;
                         const bool in = (unsigned)cy < (unsigned)S;
                         carry = in ? cell_row + gz + cxz : carry;
                         bt.cell[q] = carry;
-                        bt.k[q] = tap_load(ktab, in ? (uint32_t)(r.kb + tap_row + cxz) : TAP_NONE,
-                                           (T2 *)nullptr);
+                        bt.k[q].load(ktab, in ? r.kb + tap_row + cxz : (int)TAP_NONE, 0);
                     }
                 }
             };
@@ -1132,24 +1177,28 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
                     if (bt.cell[q] != cur) {
                         fold();
                         if (REV) {
-                            T2 o = pre;
-                            o.x += sr;
-                            o.y += si;
-                            *cellp(cur) = o;
+#pragma unroll
+                            for (int e = 0; e < RPL; ++e) {
+                                T2 o = pre[e];
+                                o.x += sr[e];
+                                o.y += si[e];
+                                *cellp(cur, e) = o;
+                            }
                             cur = bt.cell[q];
-                            pre = *cellp(cur);
+#pragma unroll
+                            for (int e = 0; e < RPL; ++e)
+                                pre[e] = *cellp(cur, e);
                         } else {
                             if (cur >= 0)
                                 flush();
                             cur = bt.cell[q];
                         }
-                        sr = T(0);
-                        si = T(0);
+                        zero_sums();
                     }
                     mac(bt.k[q], bt.v[q]);
                 }
             };
-            pipelined_records<U, Bt>((uint32_t)nbu, fetch, update);
+            pipelined_records<U, PAIR, Bt>((uint32_t)nbu, fetch, update);
             if (REV) {
                 // last cells: the first group's, then (after a barrier) the
                 // second's, which may be the same cells
@@ -1160,21 +1209,19 @@ __global__ __launch_bounds__(S *H *GRP) void k_tower_band_items(
                     flush();
                 cur = gap_cell;
                 carry = gap_cell;
-                sr = T(0);
-                si = T(0);
+                zero_sums();
             } else if (GRP > 1) {
                 // the next stage's runs start elsewhere: nothing stays in flight
                 fold();
-                if (cur >= 0 && (sr != T(0) || si != T(0)))
+                if (cur >= 0 && any_sum())
                     flush();
                 cur = -1;
                 carry = -1;
-                sr = T(0);
-                si = T(0);
+                zero_sums();
             }
         }
         fold();
-        if (GRP == 1 && cur >= 0 && (sr != T(0) || si != T(0)))
+        if (GRP == 1 && cur >= 0 && any_sum())
             flush();
 
         // destination: the task's subgrid band (column blocks), or a spill slot
@@ -1674,16 +1721,18 @@ struct BandLaunch {
     uint32_t blocks; // workgroups (each loops over the batch's items)
     rg_context *timer_ctx;
     bool comp;       // FP32: two-sum compensated register sums
+    bool pair;       // kernel table of row pairs
 };
 
-template <typename T, int S, int H, int LOGN, bool COMP>
+template <typename T, int S, int H, int LOGN, bool COMP, bool PAIR = false>
 static int launch_band_items(const BandLaunch &a, hipStream_t s)
 {
     using T2 = typename Vec2<T>::type;
     constexpr int GRP = S * H >= 256 ? 1 : 256 / (S * H);
+    constexpr int NT = S * H * GRP / (PAIR ? 2 : 1);
     KernelTimer kt(a.timer_ctx, RG_TIMER_TOWER_TILES, s);
-    hipLaunchKernelGGL((k_tower_band_items<T, S, H, LOGN, GRP, COMP>), dim3(a.blocks),
-                       dim3(S * H * GRP), 0, s, (const BandRec<T> *)a.recs, a.items,
+    hipLaunchKernelGGL((k_tower_band_items<T, S, H, LOGN, GRP, COMP, PAIR>), dim3(a.blocks),
+                       dim3(NT), 0, s, (const BandRec<T> *)a.recs, a.items,
                        a.item_start, a.bref, a.batch, a.rank_of_slot, (const T2 *)a.kern,
                        a.kern_bytes, (const T2 *)a.tw, (T2 *)a.G, (T2 *)a.spill, a.spill_cap,
                        a.spill_ctr, a.item_spill, a.spill_item, a.stats);
@@ -1696,10 +1745,14 @@ static int launch_bands_h(const BandLaunch &a, hipStream_t s)
 {
     using T2 = typename Vec2<T>::type;
     if constexpr (sizeof(T) == 4) {
-        if (a.comp)
-            RG_TRY((launch_band_items<T, S, H, LOGN, true>(a, s)));
+        auto run = [&](auto pair) {
+            return a.comp ? launch_band_items<T, S, H, LOGN, true, decltype(pair)::value>(a, s)
+                          : launch_band_items<T, S, H, LOGN, false, decltype(pair)::value>(a, s);
+        };
+        if constexpr (S == 16 && H == 8)
+            RG_TRY(a.pair ? run(std::true_type{}) : run(std::false_type{}));
         else
-            RG_TRY((launch_band_items<T, S, H, LOGN, false>(a, s)));
+            RG_TRY(run(std::false_type{}));
     } else {
         RG_TRY((launch_band_items<T, S, H, LOGN, false>(a, s)));
     }
@@ -2109,7 +2162,12 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     // taps are addressed by 32-bit byte offsets
     const int64_t nsub = (int64_t)wk->plane_count * wk->oversampling * wk->oversampling;
     const int64_t krows = padded_taps<T>() ? (int64_t)H + nsub * padded_rows(S, H) : nsub * S;
-    const int64_t kbytes = krows * S * (int64_t)sizeof(T2);
+    // two band rows per lane (k_tower_band_items): S = 16 and 8-row bands, while
+    // the table of pairs stays below the 2 GiB that offsets reach
+    const bool pair = padded_taps<T>() && S == 16 && H == 8 &&
+                      2 * krows * S * (int64_t)sizeof(T2) < ((int64_t)1 << 31);
+    const int tap_bytes = (int)sizeof(T2) * (pair ? 2 : 1);
+    const int64_t kbytes = krows * S * (int64_t)tap_bytes;
     PadJob<T2> pad{};
     if (padded_taps<T>() && kbytes < ((int64_t)1 << 31)) {
         RG_TRY(ctx->scratch[12].ensure((size_t)kbytes));
@@ -2118,6 +2176,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         pad.nsub = nsub;
         pad.S = S;
         pad.H = H;
+        pad.pair = pair;
         pad.blocks = (unsigned)std::min<int64_t>((krows * S + 255) / 256, 4096);
     }
 
@@ -2350,7 +2409,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
                            dim3((unsigned)std::min<int64_t>(std::max(nitems_cap, 1), 8192)),
                            dim3(256), 0, s, (const Rec<T> *)br.recs, sorted, (const Item *)items_w,
                            stats, (const uint32_t *)br.vis_start, (const uint32_t *)item_start_w, K,
-                           g.mk, n + S, S, H, NB, (const uint32_t *)bands_part,
+                           g.mk, n + S, S, H, tap_bytes, NB,
+                           (const uint32_t *)bands_part,
                            (int)scan_blocks(nkeys));
         RG_HIP(hipGetLastError());
     }
@@ -2358,6 +2418,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     BandLaunch bl;
     bl.timer_ctx = ctx;
     bl.comp = p->compensated != 0;
+    bl.pair = pair;
     bl.recs = sorted;
     bl.items = items_w;
     bl.item_start = item_start_w;

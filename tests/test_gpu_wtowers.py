@@ -136,3 +136,28 @@ def test_other_shapes_match_oracle(ctx, sub, margin, S, radix):
         torch.cuda.synchronize()
         assert rel_max(g.cpu().numpy(), ref) < tol, (dt, sub, S)
         assert st.n_gridded == obs.n_vis
+
+
+@pytest.mark.parametrize("sub", [64, 128, 256, 512])
+@pytest.mark.parametrize("n,spread", [(1, 1.0), (9, 20.0), (129, 30.0), (257, 200.0), (600, 3.0)])
+def test_batched_fp32_row_pairs(ctx, sub, n, spread):
+    """Support-16 tables in 8-row bands, where a lane takes two rows: single records, batches of
+    8 and one more, stages of 256 records, one column and many (the wavefronts' runs meet in
+    one footprint), every subgrid size.  FP32 against the oracle in FP64, the image to the 1e-5 of
+    the other FP32 tests."""
+    N, theta = sub, 0.1
+    rng = np.random.default_rng(sub + n)
+    u = 40.0 + rng.uniform(-spread, spread, n)
+    v = -30.0 + rng.uniform(-spread, spread, n)
+    w = rng.uniform(-14.0, 14.0, n)
+    vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    table = rgamd.make_wkernels(11, 4, 16, theta, -5.0, 1.0)
+    ref, _, bad = orc.grid_wtowers(N, theta, u, v, w, vis, table, -5.0, 1.0, sub, MARGIN, WINC)
+    assert bad == 0
+    _, fv = stage(u, v, w, vis, torch.complex64)
+    _, wk = kern(table, -5.0, 1.0, torch.complex64)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    ctx.grid(rgamd.params(N, theta, subgrid=sub, margin=MARGIN, winc=WINC), fv, wk, g)
+    assert ctx.stats().n_gridded == n
+    img, img_ref = orc.grid_to_image(g.cpu().numpy()), orc.grid_to_image(ref)
+    assert rel_max(img, img_ref) < 1e-5 and rel_rms(img, img_ref) < 1e-5
