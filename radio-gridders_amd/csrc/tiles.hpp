@@ -22,8 +22,8 @@
 // beside the tap reads (2 KB a record from L2, 19 TB/s).  With a workgroup of S S threads
 // per item, a tap a lane (every lane of four wavefronts found its own cell and tap
 // address for every record: about 64 instructions) and records of all planes mixed
-// (a 60 MB table read past L2), tiles took, now, us: 8.4 M visibilities FP32 1571 -> 890;
-// 520 k FP64 273 -> 168; 448 FP64 7.3 -> 5.2.
+// (a 60 MB table read past L2), tiles took, now, us: 8.4 M visibilities FP32 1571 -> 950;
+// 520 k FP64 273 -> 168; 448 FP64 7.3 -> 6.6.
 #pragma once
 
 #include "binning.hpp"
@@ -41,12 +41,37 @@ template <typename T> __device__ inline void two_sum_into(T &hi, T &lo, T b)
     lo += e;
 }
 
+constexpr int TILE_POS = 16; // tile edge in footprint positions
+
 struct TileSink {
     void *base; // target arrays, group g at base + g * gsize^2 complex elements
     int gsize;  // edge of a target array
     int ntx;    // tiles per row
     int ntiles; // tiles per group
     int groups; // target arrays
+    // FP32 arrays: keys of at least hot_min records (0: none) add their items up in FP64
+    // slots of tile_slot() numbers, which k_hot_tiles then adds to the arrays
+    uint32_t hot_min;
+    const uint32_t *key_start; // first record of every key
+    double *hot;
+    uint32_t *hot_key; // key + 1 of every slot in use
+};
+
+// Numbers of a tile and its halo.
+constexpr int tile_slot(int S) { return 2 * (TILE_POS + S - 1) * (TILE_POS + S - 1); }
+
+// Tile of a key: its array and the cell of its corner.
+struct TilePlace {
+    uint32_t group;
+    int ox, oy;
+    __device__ TilePlace(const TileSink &sink, uint32_t key, int S)
+    {
+        const uint32_t gt = key % (uint32_t)(sink.ntiles * sink.groups);
+        group = gt / (uint32_t)sink.ntiles;
+        const int tile = (int)(gt - group * (uint32_t)sink.ntiles);
+        ox = tile % sink.ntx * TILE_POS - S;
+        oy = tile / sink.ntx * TILE_POS - S;
+    }
 };
 
 __device__ inline float lane_value(float v, int lane)
@@ -97,7 +122,6 @@ template <> struct TapLoad<double, 1> {
     }
 };
 
-constexpr int TILE_POS = 16;      // tile edge in footprint positions
 constexpr int TILE_SORT = 512;    // records ordered by position at a time
 constexpr int TILE_UNSORTED = 16; // up to this many are taken as they come
 
@@ -135,6 +159,17 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         if (it != blockIdx.x)
             item = items[it];
+        double *slot = nullptr; // of a hot key
+        if (sizeof(GT) == 4 && sink.hot_min) {
+            const uint32_t k0 = sink.key_start[item.key];
+            if (sink.key_start[item.key + 1] - k0 >= sink.hot_min) {
+                // hot keys start at least hot_min records apart
+                const uint32_t h = k0 / sink.hot_min;
+                slot = sink.hot + (size_t)h * tile_slot(S);
+                if (item.start == k0 && lane == 0)
+                    sink.hot_key[h] = item.key + 1;
+            }
+        }
 #pragma unroll 2
         for (int c = lane; c < CELLS; c += 64) {
             s_cell[c].x = T(0);
@@ -293,19 +328,16 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
         flush();
         __syncthreads();
 
-        const uint32_t gt = item.key % (uint32_t)(sink.ntiles * sink.groups);
-        const uint32_t group = gt / (uint32_t)sink.ntiles;
-        const int tile = (int)(gt - group * (uint32_t)sink.ntiles);
-        const int tx = tile % sink.ntx, ty = tile / sink.ntx;
-        const int ox = tx * TW - S, oy = ty * TH - S;
+        const TilePlace at(sink, item.key, S);
+        const int ox = at.ox, oy = at.oy;
         const int G = sink.gsize;
-        GT *g = reinterpret_cast<GT *>(sink.base) + (size_t)group * G * G * 2;
+        GT *g = reinterpret_cast<GT *>(sink.base) + (size_t)at.group * G * G * 2;
         // a row's cells as 2 RW consecutive numbers: whole 64-byte pieces of the grid's row
         // in one instruction; FB rows' LDS reads in flight
         constexpr int FB = 8;
         const T *cf = reinterpret_cast<const T *>(s_cell), *lf = reinterpret_cast<const T *>(s_lo);
         for (int f = lane; f < 2 * RW; f += 64) {
-            if ((unsigned)(ox + f / 2) >= (unsigned)G)
+            if (!slot && (unsigned)(ox + f / 2) >= (unsigned)G)
                 continue;
             GT *gf = g + 2 * ((int64_t)oy * G + ox) + f;
             for (int r0 = 0; r0 < RH; r0 += FB) {
@@ -318,12 +350,39 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
                         v[q] += (GT)lf[ry * 2 * RS + f];
                 }
 #pragma unroll
-                for (int q = 0; q < FB; ++q)
-                    if (r0 + q < RH && (unsigned)(oy + r0 + q) < (unsigned)G && v[q] != GT(0))
+                for (int q = 0; q < FB; ++q) {
+                    if (r0 + q >= RH || v[q] == GT(0))
+                        continue;
+                    if (slot)
+                        atomicAdd(slot + (r0 + q) * 2 * RW + f, (double)v[q]);
+                    else if ((unsigned)(oy + r0 + q) < (unsigned)G)
                         atomicAdd(gf + 2 * (int64_t)(r0 + q) * G, v[q]);
+                }
             }
         }
         __syncthreads();
+    }
+}
+
+// Adds the hot keys' FP64 sums to their arrays: one workgroup per slot.  A dense tile has
+// hundreds of items, and adding each to an FP32 array directly rounds at the size of the whole sum every
+// time: 400 k visibilities on 462^2 3.7e-7 from the exact grid (items of 2048 records 1.5e-7).
+template <int S>
+__global__ __launch_bounds__(256) void k_hot_tiles(TileSink sink)
+{
+    const uint32_t key = sink.hot_key[blockIdx.x];
+    if (key == 0)
+        return;
+    constexpr int RW = TILE_POS + S - 1;
+    const TilePlace at(sink, key - 1, S);
+    const int G = sink.gsize;
+    float *g = reinterpret_cast<float *>(sink.base) + (size_t)at.group * G * G * 2;
+    const double *slot = sink.hot + (size_t)blockIdx.x * tile_slot(S);
+    for (int e = threadIdx.x; e < tile_slot(S); e += 256) {
+        const int ry = e / (2 * RW), f = e - ry * 2 * RW;
+        const float v = (float)slot[e];
+        if ((unsigned)(at.oy + ry) < (unsigned)G && (unsigned)(at.ox + f / 2) < (unsigned)G && v != 0.0f)
+            atomicAdd(g + 2 * ((int64_t)(at.oy + ry) * G + at.ox) + f, v);
     }
 }
 

@@ -208,7 +208,15 @@ struct WprojShape {
     int group_planes; // W-planes per plane group
     int64_t nkeys;    // plane groups x grids x tiles
     uint32_t per_item;
+    // FP32 grids: records of a key whose items add up in FP64 first (0: no key),
+    // slots for such keys of this stream, and of any shorter one too
+    uint32_t hot_min;
+    int64_t hot_slots, hot_room;
 
+    size_t hot_bytes(int S, int64_t slots) const
+    {
+        return slots * sizeof(double) * (size_t)tile_slot(S);
+    }
     void one_group(int planes, int n_chan)
     {
         group_planes = std::max(planes, 1);
@@ -217,12 +225,21 @@ struct WprojShape {
 };
 constexpr int64_t WPROJ_COUNTERS = (int64_t)1 << 22;
 
+struct HotSlots {
+    double *sums;
+    uint32_t *key;
+};
+
 template <typename T, int S, bool COMP, typename GT>
 static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
                         const unsigned long long *stats, const rg_wkern *wk, void *grid, int N,
-                        int n_chan, const WprojShape &sh, hipStream_t s)
+                        int n_chan, const WprojShape &sh, const HotSlots &hot, hipStream_t s)
 {
     TileSink sink;
+    sink.hot_min = sizeof(GT) == 4 ? sh.hot_min : 0;
+    sink.key_start = br.vis_start;
+    sink.hot = hot.sums;
+    sink.hot_key = hot.key;
     sink.base = grid;
     sink.gsize = N;
     sink.ntx = sh.ntx;
@@ -238,6 +255,9 @@ static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
         hipLaunchKernelGGL((k_tiles<T, S, COMP, GT>), dim3((unsigned)nb), dim3(64), 0, s,
                            (const Rec<T> *)br.recs, (const Item *)br.items, stats,
                            (const typename Vec2<T>::type *)wk->data, (uint32_t)kbytes, sink);
+        if (sink.hot_min)
+            hipLaunchKernelGGL((k_hot_tiles<S>), dim3((unsigned)sh.hot_slots), dim3(256), 0, s,
+                               sink);
     }
     RG_HIP(hipGetLastError());
     return RG_OK;
@@ -247,11 +267,11 @@ template <typename T, int S>
 static int dispatch_comp_grid(const BinResult &br, rg_context *timer_ctx,
                               const unsigned long long *stats, const rg_wkern *wk, void *grid,
                               int grid_type, bool comp, int N, int n_chan, const WprojShape &sh,
-                              hipStream_t s)
+                              const HotSlots &hot, hipStream_t s)
 {
     auto run = [&](auto c, auto g) {
         return launch_tiles<T, S, decltype(c)::value, decltype(g)>(
-            br, timer_ctx, stats, wk, grid, N, n_chan, sh, s);
+            br, timer_ctx, stats, wk, grid, N, n_chan, sh, hot, s);
     };
     if constexpr (std::is_same<T, double>::value) {
         if (grid_type != RG_C128)
@@ -268,11 +288,11 @@ template <typename T>
 static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx,
                           const unsigned long long *stats, const rg_wkern *wk, void *grid,
                           int grid_type, bool comp, int N, int n_chan, const WprojShape &sh,
-                          hipStream_t s)
+                          const HotSlots &hot, hipStream_t s)
 {
     auto run = [&](auto sz) {
         return dispatch_comp_grid<T, decltype(sz)::value>(br, timer_ctx, stats, wk, grid, grid_type,
-                                                          comp, N, n_chan, sh, s);
+                                                          comp, N, n_chan, sh, hot, s);
     };
     using std::integral_constant;
     return wk->size == 16 ? run(integral_constant<int, 16>{}) : run(integral_constant<int, 8>{});
@@ -280,9 +300,9 @@ static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx,
 
 // Records per work item when the caller leaves it open.  A wavefront walks its
 // item's records one after another, and every item adds its tile to the grid, so both the
-// records of an item and the items grow with the stream: the largest power of two from 4 to
+// records of an item and the items grow with the stream: the largest power of two from 8 to
 // 512 with 12 K^2 <= records.  Tile kernel or call, us, at half / this / twice the size:
-// 448 records FP64 - / 5.2 / 6.7; 16 k FP64 on 2000^2 60 / 54 / 57; 150 k FP32 69 / 65
+// 448 records FP64 5.2 / 6.7 / 8.1 (the call is shortest at 8); 16 k FP64 on 2000^2 60 / 54 / 57; 150 k FP32 69 / 65
 // / -; 520 k FP64 225 / 204 / 237; 8.4 M FP32 1032 / 1042 / 1161.
 static uint32_t default_item(int64_t nvis)
 {
@@ -318,6 +338,11 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
         sh.group_planes = (int)group;
         sh.nkeys = one * all;
     }
+    // a key of eight default items or more (the shortest streams have too few items for
+    // it to matter); the next shorter item size needs at most twice the slots
+    sh.hot_min = nvis >= 1024 ? 8 * default_item(nvis) : 0;
+    sh.hot_slots = sh.hot_min ? nvis / sh.hot_min + 1 : 0;
+    sh.hot_room = 2 * sh.hot_slots;
     sh.per_item = p->vis_per_item > 0 ? std::min<uint32_t>((uint32_t)p->vis_per_item, TILE_SORT)
                                       : default_item(nvis);
     return RG_OK;
@@ -371,6 +396,15 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     }
     if (rc != RG_OK)
         return rc;
+    HotSlots hot{};
+    if (grid_type == RG_C64 && sh.hot_min) {
+        const size_t kb = (sizeof(uint32_t) * (size_t)sh.hot_room + 255) / 256 * 256;
+        RG_TRY(ctx->scratch[20].ensure(kb + sh.hot_bytes(wk->size, sh.hot_room)));
+        hot.key = ctx->scratch[20].as<uint32_t>();
+        hot.sums = reinterpret_cast<double *>(ctx->scratch[20].as<char>() + kb);
+        RG_TRY(zero.add(hot.key, kb));
+        RG_TRY(zero.add(hot.sums, sh.hot_bytes(wk->size, sh.hot_slots)));
+    }
 
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));
@@ -378,7 +412,7 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, sh.nkeys,
                                             sh.per_item, zero, s, br, WPROJ_COUNTERS, &pl)));
     return dispatch_tiles<T>(br, ctx, ctx->counters.as<unsigned long long>(), wk, grid, grid_type,
-                             p->compensated != 0, N, n_chan, sh, s);
+                             p->compensated != 0, N, n_chan, sh, hot, s);
 }
 
 int wproj_batched(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *vis,
@@ -471,6 +505,16 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
         sh.per_item = std::max(sh.per_item, limit_item);
         RG_TRY(carve(1));
     }
+    HotSlots hot{};
+    size_t hot_at = at, hot_keys = 0;
+    if (grid_type == RG_C64 && sh.hot_min) {
+        hot_keys = aligned(sizeof(uint32_t) * (size_t)sh.hot_slots);
+        at += hot_keys + aligned(sh.hot_bytes(wk->size, sh.hot_slots));
+        if (at > NOALLOC_SCRATCH_BYTES) { // no room beside the keys of a very large grid
+            at = hot_at;
+            sh.hot_min = 0;
+        }
+    }
     if (want > NOALLOC_LIMIT_BYTES || at > NOALLOC_SCRATCH_BYTES)
         return fail(RG_ERR_PARAM,
                     "rg_grid_noalloc: %lld visibilities on a %d^2 grid need %zu bytes of scratch; "
@@ -492,6 +536,11 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     // the previous call's counters are still there: start from zero
     ZeroList zero;
     RG_TRY(zero.add(b.stats, sizeof(unsigned long long) * CNT__N));
+    if (grid_type == RG_C64 && sh.hot_min) {
+        hot.key = reinterpret_cast<uint32_t *>(b0 + hot_at);
+        hot.sums = reinterpret_cast<double *>(b0 + hot_at + hot_keys);
+        RG_TRY(zero.add(hot.key, hot_keys + sh.hot_bytes(wk->size, sh.hot_slots)));
+    }
     if (!accumulate)
         RG_TRY(zero.add(grid, (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N));
     if (vis->n == 0)
@@ -502,7 +551,7 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.nkeys, sh.per_item, pl, b, zero, false, nullptr,
                                    s, br)));
     return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N, 1,
-                             sh, s);
+                             sh, hot, s);
 }
 
 int wproj_noalloc(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk, void *grid,
