@@ -1852,10 +1852,15 @@ struct WtGeom {
     int64_t ntw; // tower ids: nchan cc^2
 };
 
-// Sort counters of a W-towers call in all: (task, band) keys get 4 counter
-// replicas at the reference's workload (the scans read every replica; 16 were
-// slower).
-constexpr int64_t WT_COUNTERS = (int64_t)1 << 20;
+// Sort counters of a W-towers call in all ((task, band) keys times replicas).
+// Long streams spread their hot keys' returning atomics over more replicas: 8.4 M
+// visibilities, 762 k keys: count 417 us with one replica, 358 with two, 328 with four, and
+// the clears and scans that read them 3 us more; 520 k: 33 -> 25 us and 4 us more.  Short ones
+// only pay for reading them (22 k: 1 us).
+static int64_t wt_counters(int64_t nvis)
+{
+    return (int64_t)1 << (nvis >= ((int64_t)1 << 18) ? 22 : 20);
+}
 
 static WtGeom wt_geom(const rg_grid_params *p, const rg_wkern *wk, int nchan, int H)
 {
@@ -2214,8 +2219,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         const int q = batch_tasks_of(ntasks_cap);
         RG_TRY(clear_subimages((ntasks_cap + q - 1) / q,
                                ctx->scratch[18].as<uint32_t>() + tl.o_spill));
-        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, 0x40000000u, WT_COUNTERS, zero,
-                               bin)));
+        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, 0x40000000u,
+                               wt_counters(vis->n), zero, bin)));
         ready = &bin;
     }
     RG_TRY(wt_prepare<T2>(ctx, p, vis, g, d_range, &pad, zero, s));
@@ -2255,7 +2260,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     br.group_start = slot_start;
     br.group_keys = NB;
     RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, 0x40000000u, zero, s, br,
-                                            WT_COUNTERS, ready)));
+                                            wt_counters(vis->n), ready)));
 
     if (measure) {
         ntasks_cap = (int)std::min<int64_t>(nslots, 0x7fffffff);
