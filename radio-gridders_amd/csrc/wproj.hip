@@ -387,6 +387,9 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     ZeroList zero;
     RG_TRY(zero.add(ctx->counters.p, sizeof(unsigned long long) * CNT__N));
     RG_TRY(zero.add(grid, gbytes));
+    // a context's first call: the grids are cleared while the host allocates
+    if (!ctx->scratch[5].p)
+        RG_TRY(zero.launch(s));
     BinPlan pl;
     int rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
     if (rc != RG_OK && sh.nkeys != (int64_t)sh.ntiles * n_chan) {
