@@ -896,7 +896,9 @@ struct WindowSource : FixedItems {
 // a table that holds every tap beside the one H / 2 rows below it, which halves the
 // loads and shares cell and tap addresses, half as many wavefronts a workgroup.  8.4 M
 // visibilities, 512^2 subgrids, FP32, S = 16: 2072 -> 1860 us (62 % VALU busy).  In FP64 a
-// tap is 16 bytes already, and at S = 8 a pair would leave a wavefront half empty.
+// tap is 16 bytes already, and at S = 8 a pair would leave a wavefront half empty.  Sparser
+// items (188 records of 7.8 M visibilities) gain less, 2321 -> 2269 us: their rows' FFTs
+// run on half the wavefronts.
 template <typename T, int S, int H, int LOGN, int GRP, bool COMP, bool PAIR>
 __global__ __launch_bounds__(S *H *GRP / (PAIR ? 2 : 1)) void k_tower_band_items(
     const BandRec<T> *__restrict__ recs, const Item *__restrict__ items,
@@ -1745,14 +1747,13 @@ static int launch_bands_h(const BandLaunch &a, hipStream_t s)
 {
     using T2 = typename Vec2<T>::type;
     if constexpr (sizeof(T) == 4) {
-        auto run = [&](auto pair) {
-            return a.comp ? launch_band_items<T, S, H, LOGN, true, decltype(pair)::value>(a, s)
-                          : launch_band_items<T, S, H, LOGN, false, decltype(pair)::value>(a, s);
-        };
-        if constexpr (S == 16 && H == 8)
-            RG_TRY(a.pair ? run(std::true_type{}) : run(std::false_type{}));
+        constexpr bool PAIRS = S == 16 && H == 8;
+        if (a.comp)
+            RG_TRY((launch_band_items<T, S, H, LOGN, true>(a, s)));
+        else if (PAIRS && a.pair)
+            RG_TRY((launch_band_items<T, S, H, LOGN, false, PAIRS>(a, s)));
         else
-            RG_TRY(run(std::false_type{}));
+            RG_TRY((launch_band_items<T, S, H, LOGN, false>(a, s)));
     } else {
         RG_TRY((launch_band_items<T, S, H, LOGN, false>(a, s)));
     }
@@ -2168,14 +2169,18 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     const int64_t nsub = (int64_t)wk->plane_count * wk->oversampling * wk->oversampling;
     const int64_t krows = padded_taps<T>() ? (int64_t)H + nsub * padded_rows(S, H) : nsub * S;
     // two band rows per lane (k_tower_band_items): S = 16 and 8-row bands, while
-    // the table of pairs stays below the 2 GiB that offsets reach
-    const bool pair = padded_taps<T>() && S == 16 && H == 8 &&
-                      2 * krows * S * (int64_t)sizeof(T2) < ((int64_t)1 << 31);
+    // the table of pairs stays below the 2 GiB that offsets reach; compensated sums
+    // do four times the arithmetic a tap, which half the wavefronts hide worse (7.8 M
+    // visibilities 2623 us a row a lane, 2885 us in pairs; uncompensated 2321 and 2269)
+    const bool pairs_fit = padded_taps<T>() && S == 16 && H == 8 &&
+                           2 * krows * S * (int64_t)sizeof(T2) < ((int64_t)1 << 31);
+    const bool pair = pairs_fit && !p->compensated;
     const int tap_bytes = (int)sizeof(T2) * (pair ? 2 : 1);
     const int64_t kbytes = krows * S * (int64_t)tap_bytes;
     PadJob<T2> pad{};
     if (padded_taps<T>() && kbytes < ((int64_t)1 << 31)) {
-        RG_TRY(ctx->scratch[12].ensure((size_t)kbytes));
+        // (room for a table of pairs beside a captured compensated call)
+        RG_TRY(ctx->scratch[12].ensure((size_t)kbytes * (pairs_fit && !pair ? 2 : 1)));
         pad.src = (const T2 *)wk->data;
         pad.dst = ctx->scratch[12].as<T2>();
         pad.nsub = nsub;
