@@ -3,8 +3,8 @@
 //
 // One wavefront takes one work item: up to K sorted records of one key.  A key
 // is (plane group, group, tile): the group selects the target array (a channel grid), the tile a
-// 16 x 16 block of footprint top-left positions, whose footprints cover
-// (S + 15) x (S + 15) cells held in LDS, and the plane group a range of
+// TW x 16 block of footprint top-left positions, whose footprints cover
+// (S + TW - 1) x (S + 15) cells held in LDS, and the plane group a range of
 // W-planes (items of a group follow one another, so the sub-kernels in use at a time
 // stay in an XCD's L2).
 //
@@ -41,12 +41,13 @@ template <typename T> __device__ inline void two_sum_into(T &hi, T &lo, T b)
     lo += e;
 }
 
-constexpr int TILE_POS = 16; // tile edge in footprint positions
+constexpr int TILE_POS = 16; // rows of footprint positions of a tile; columns: 16 or 32
 
 struct TileSink {
     void *base; // target arrays, group g at base + g * gsize^2 complex elements
     int gsize;  // edge of a target array
     int ntx;    // tiles per row
+    int tw;     // columns of positions of a tile
     int ntiles; // tiles per group
     int groups; // target arrays
     // FP32 arrays: keys of at least hot_min records (0: none) add their items up in FP64
@@ -58,7 +59,7 @@ struct TileSink {
 };
 
 // Numbers of a tile and its halo.
-constexpr int tile_slot(int S) { return 2 * (TILE_POS + S - 1) * (TILE_POS + S - 1); }
+constexpr int tile_slot(int S, int TW) { return 2 * (TILE_POS + S - 1) * (TW + S - 1); }
 
 // Tile of a key: its array and the cell of its corner.
 struct TilePlace {
@@ -69,7 +70,7 @@ struct TilePlace {
         const uint32_t gt = key % (uint32_t)(sink.ntiles * sink.groups);
         group = gt / (uint32_t)sink.ntiles;
         const int tile = (int)(gt - group * (uint32_t)sink.ntiles);
-        ox = tile % sink.ntx * TILE_POS - S;
+        ox = tile % sink.ntx * sink.tw - S;
         oy = tile / sink.ntx * TILE_POS - S;
     }
 };
@@ -125,15 +126,15 @@ template <> struct TapLoad<double, 1> {
 constexpr int TILE_SORT = 512;    // records ordered by position at a time
 constexpr int TILE_UNSORTED = 16; // up to this many are taken as they come
 
-template <typename T, int S, bool COMP, typename GT>
-__global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
+template <typename T, int S, int TW, bool COMP, typename GT>
+__global__ __launch_bounds__(64, TW > 16 ? 2 : sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
     const Rec<T> *__restrict__ recs, const Item *__restrict__ items,
     const unsigned long long *__restrict__ stats, const typename Vec2<T>::type *__restrict__ kern,
     uint32_t kern_bytes, TileSink sink)
 {
     using T2 = typename Vec2<T>::type;
     using Span = TapSpan<T, S>;
-    constexpr int TW = TILE_POS, TH = TILE_POS;
+    constexpr int TH = TILE_POS;
     constexpr int RW = TW + S - 1, RH = TH + S - 1;
     // odd row stride: the rows a wavefront adds to start in different LDS banks
     constexpr int RS = RW | 1;
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
             if (sink.key_start[item.key + 1] - k0 >= sink.hot_min) {
                 // hot keys start at least hot_min records apart
                 const uint32_t h = k0 / sink.hot_min;
-                slot = sink.hot + (size_t)h * tile_slot(S);
+                slot = sink.hot + (size_t)h * tile_slot(S, TW);
                 if (item.start == k0 && lane == 0)
                     sink.hot_key[h] = item.key + 1;
             }
@@ -367,18 +368,18 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 && !COMP ? 4 : 3) void k_tiles(
 // Adds the hot keys' FP64 sums to their arrays: one workgroup per slot.  A dense tile has
 // hundreds of items, and adding each to an FP32 array directly rounds at the size of the whole sum every
 // time: 400 k visibilities on 462^2 3.7e-7 from the exact grid (items of 2048 records 1.5e-7).
-template <int S>
+template <int S, int TW>
 __global__ __launch_bounds__(256) void k_hot_tiles(TileSink sink)
 {
     const uint32_t key = sink.hot_key[blockIdx.x];
     if (key == 0)
         return;
-    constexpr int RW = TILE_POS + S - 1;
+    constexpr int RW = TW + S - 1;
     const TilePlace at(sink, key - 1, S);
     const int G = sink.gsize;
     float *g = reinterpret_cast<float *>(sink.base) + (size_t)at.group * G * G * 2;
-    const double *slot = sink.hot + (size_t)blockIdx.x * tile_slot(S);
-    for (int e = threadIdx.x; e < tile_slot(S); e += 256) {
+    const double *slot = sink.hot + (size_t)blockIdx.x * tile_slot(S, TW);
+    for (int e = threadIdx.x; e < tile_slot(S, TW); e += 256) {
         const int ry = e / (2 * RW), f = e - ry * 2 * RW;
         const float v = (float)slot[e];
         if ((unsigned)(at.oy + ry) < (unsigned)G && (unsigned)(at.ox + f / 2) < (unsigned)G && v != 0.0f)

@@ -149,7 +149,7 @@ struct WprojKeyer {
     int vis_type;
     int N, S, R, P;
     double theta, w_min, w_step;
-    int ntx, ntiles;         // tiles per row and grid
+    int tw, ntx, ntiles;     // columns of positions of a tile; tiles per row and grid
     int group_planes;        // W-planes per plane group
     int zb;                  // bytes per kernel tap
     const int64_t *chan_off;
@@ -177,11 +177,11 @@ struct WprojKeyer {
         const int p = w_plane(w[i], w_min, w_step);
         if (p < 0 || p >= P)
             return VIS_BAD_PLANE;
-        const int tx = (gx + S) / TILE_POS, ty = (gy + S) / TILE_POS;
+        const int tx = (gx + S) / tw, ty = (gy + S) / TILE_POS;
         const int c = nchan > 1 ? chan_of(i) : 0;
         key = (uint32_t)((p / group_planes * nchan + c) * ntiles + ty * ntx + tx);
         // position in the tile; byte offset of the sub-kernel
-        pos = (uint32_t)(gx + S - tx * TILE_POS) | (uint32_t)(gy + S - ty * TILE_POS) << 16;
+        pos = (uint32_t)(gx + S - tx * tw) | (uint32_t)(gy + S - ty * TILE_POS) << 16;
         kidx = (uint32_t)((p * R + yf) * R + xf) * (uint32_t)(S * S * zb);
         return VIS_OK;
     }
@@ -204,7 +204,7 @@ struct WprojKeyer {
 
 // Tile geometry and sort parameters of batched W-projection.
 struct WprojShape {
-    int ntx, ntiles;
+    int tw, ntx, ntiles;
     int group_planes; // W-planes per plane group
     int64_t nkeys;    // plane groups x grids x tiles
     uint32_t per_item;
@@ -215,7 +215,7 @@ struct WprojShape {
 
     size_t hot_bytes(int S, int64_t slots) const
     {
-        return slots * sizeof(double) * (size_t)tile_slot(S);
+        return slots * sizeof(double) * (size_t)tile_slot(S, tw);
     }
     void one_group(int planes, int n_chan)
     {
@@ -230,7 +230,7 @@ struct HotSlots {
     uint32_t *key;
 };
 
-template <typename T, int S, bool COMP, typename GT>
+template <typename T, int S, int TW, bool COMP, typename GT>
 static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
                         const unsigned long long *stats, const rg_wkern *wk, void *grid, int N,
                         int n_chan, const WprojShape &sh, const HotSlots &hot, hipStream_t s)
@@ -243,6 +243,7 @@ static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
     sink.base = grid;
     sink.gsize = N;
     sink.ntx = sh.ntx;
+    sink.tw = TW;
     sink.ntiles = sh.ntiles;
     sink.groups = n_chan;
     KernelTimer kt(timer_ctx, RG_TIMER_WPROJ_TILES, s);
@@ -252,25 +253,25 @@ static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection kernel tables above 2 GiB");
     if (br.max_items > 0) {
         const int64_t nb = std::min<int64_t>(br.max_items, TILE_GRID);
-        hipLaunchKernelGGL((k_tiles<T, S, COMP, GT>), dim3((unsigned)nb), dim3(64), 0, s,
+        hipLaunchKernelGGL((k_tiles<T, S, TW, COMP, GT>), dim3((unsigned)nb), dim3(64), 0, s,
                            (const Rec<T> *)br.recs, (const Item *)br.items, stats,
                            (const typename Vec2<T>::type *)wk->data, (uint32_t)kbytes, sink);
         if (sink.hot_min)
-            hipLaunchKernelGGL((k_hot_tiles<S>), dim3((unsigned)sh.hot_slots), dim3(256), 0, s,
+            hipLaunchKernelGGL((k_hot_tiles<S, TW>), dim3((unsigned)sh.hot_slots), dim3(256), 0, s,
                                sink);
     }
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
 
-template <typename T, int S>
+template <typename T, int S, int TW>
 static int dispatch_comp_grid(const BinResult &br, rg_context *timer_ctx,
                               const unsigned long long *stats, const rg_wkern *wk, void *grid,
                               int grid_type, bool comp, int N, int n_chan, const WprojShape &sh,
                               const HotSlots &hot, hipStream_t s)
 {
     auto run = [&](auto c, auto g) {
-        return launch_tiles<T, S, decltype(c)::value, decltype(g)>(
+        return launch_tiles<T, S, TW, decltype(c)::value, decltype(g)>(
             br, timer_ctx, stats, wk, grid, N, n_chan, sh, hot, s);
     };
     if constexpr (std::is_same<T, double>::value) {
@@ -291,7 +292,10 @@ static int dispatch_tiles(const BinResult &br, rg_context *timer_ctx,
                           const HotSlots &hot, hipStream_t s)
 {
     auto run = [&](auto sz) {
-        return dispatch_comp_grid<T, decltype(sz)::value>(br, timer_ctx, stats, wk, grid, grid_type,
+        if (sh.tw == 32)
+            return dispatch_comp_grid<T, decltype(sz)::value, 32>(
+                br, timer_ctx, stats, wk, grid, grid_type, comp, N, n_chan, sh, hot, s);
+        return dispatch_comp_grid<T, decltype(sz)::value, 16>(br, timer_ctx, stats, wk, grid, grid_type,
                                                           comp, N, n_chan, sh, hot, s);
     };
     using std::integral_constant;
@@ -322,6 +326,7 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
         return fail(RG_ERR_UNSUPPORTED, "batched tile must be 32 or 48 (got %d)", tile);
     if (S != 8 && S != 16)
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection supports kernel sizes 8 and 16 (got %d)", S);
+    sh.tw = TILE_POS;
     sh.ntx = (p->grid_size + S + TILE_POS - 1) / TILE_POS;
     sh.ntiles = sh.ntx * sh.ntx;
     // Plane groups of 2^18 taps (2 MB in FP32, 4 MB in FP64, an XCD's L2) where a tile
@@ -337,6 +342,21 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
     if (nvis >= 64 * one && all > 1) {
         sh.group_planes = (int)group;
         sh.nkeys = one * all;
+    } else if (n_chan > 1 && nvis >= 8 * one) {
+        // many channels of 8 to 64 records a tile: tiles twice as wide, so that the items
+        // stay few (256 channels 5.26 -> 5.15 ms), and, while the counters leave room for two
+        // replicas, groups of four times the planes (64 channels 1125 -> 1057 us; 256 channels, whose
+        // 5.5 M keys leave one replica, 5.50 ms)
+        sh.tw = 2 * TILE_POS;
+        const int64_t ntx = (p->grid_size + S + sh.tw - 1) / sh.tw;
+        sh.ntiles = (int)(ntx * sh.ntx);
+        sh.ntx = (int)ntx;
+        sh.one_group(wk->plane_count, n_chan);
+        const int64_t wide = (planes + 4 * group - 1) / (4 * group);
+        if (2 * sh.nkeys * wide <= WPROJ_COUNTERS) {
+            sh.group_planes = (int)std::min<int64_t>(4 * group, planes);
+            sh.nkeys *= wide;
+        }
     }
     // a key of eight default items or more (the shortest streams have too few items for
     // it to matter); the next shorter item size needs at most twice the slots
@@ -364,6 +384,7 @@ static WprojKeyer wproj_keyer(const rg_grid_params *p, const rg_flat_vis *vis, c
     kf.theta = p->theta;
     kf.w_min = wk->w_min;
     kf.w_step = wk->w_step;
+    kf.tw = sh.tw;
     kf.ntx = sh.ntx;
     kf.ntiles = sh.ntiles;
     kf.group_planes = sh.group_planes;

@@ -170,3 +170,36 @@ def test_wprojection_item_edges(ctx, s, planes, n, per_item, dt, gdt, comp):
     bound = (n + 4) * (eps + 2.0 ** -53) * mag.real
     err = np.abs(g.cpu().numpy().astype(np.complex128) - ref)
     assert (err <= bound).all(), float((err / np.maximum(bound, 1e-300)).max())
+
+
+@pytest.mark.parametrize("planes", [35, 140])
+@pytest.mark.parametrize("n", [599, 600, 601, 4799, 4800, 9000])
+@pytest.mark.parametrize("dt,gdt,comp", [(torch.complex128, torch.complex128, 0),
+                                         (torch.complex64, torch.complex64, 0),
+                                         (torch.complex64, torch.complex128, 1)])
+def test_channels_wide_tiles(ctx, planes, n, dt, gdt, comp):
+    """Three channels around 8 and 64 records a tile (3 x 25 tiles), between which tiles are twice
+    as wide, with one group of planes (35) and with groups of 64 (140).  The bound of the item test."""
+    N, r, s = 64, 8, 16
+    rng = np.random.default_rng(planes)
+    table = (rng.standard_normal((planes, r, r, s, s)) +
+             1j * rng.standard_normal((planes, r, r, s, s)))
+    u, v, w, vis = crowd(n, N, s, planes, n)
+    np_dt = np.complex64 if dt == torch.complex64 else np.complex128
+    table, vis = table.astype(np_dt).astype(np.complex128), vis.astype(np_dt).astype(np.complex128)
+    off = np.array([0, n // 5, n // 5, n], dtype=np.int64)  # the second channel is empty
+    _, fv = stage(u, v, w, vis, dt)
+    _, wk = kern(table, 0.0, 1.0, dt)
+    g = torch.empty((3, N, N), dtype=gdt, device="cuda")
+    ctx.grid_channels(rgamd.params(N, THETA, compensated=comp), fv, off, wk, g)
+    eps = (2.0 ** -24 if dt == torch.complex64 else 2.0 ** -53) + 2.0 ** -53
+    for c in range(3):
+        sl = slice(off[c], off[c + 1])
+        got = g[c].cpu().numpy().astype(np.complex128)
+        if off[c] == off[c + 1]:
+            assert not got.any()
+            continue
+        ref, _, _ = orc.grid_wprojection(N, THETA, u[sl], v[sl], w[sl], vis[sl], table, 0.0, 1.0)
+        mag, _, _ = orc.grid_wprojection(N, THETA, u[sl], v[sl], w[sl], np.abs(vis[sl]) + 0j,
+                                         np.abs(table) + 0j, 0.0, 1.0)
+        assert (np.abs(got - ref) <= (n + 4) * eps * mag.real).all(), c
