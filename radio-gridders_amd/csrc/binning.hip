@@ -136,20 +136,4 @@ int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, 
     return RG_OK;
 }
 
-int items_from_lengths(rg_context *ctx, const uint32_t *len, int64_t nkeys, uint32_t per_item,
-                       uint32_t *prefix, uint32_t *item_start, Item *items, hipStream_t s)
-{
-    const int64_t nblocks_scan = nkeys > 0 ? scan_blocks(nkeys) : 0;
-    if (nkeys <= 0 || nblocks_scan > 1024 * 256)
-        return fail(RG_ERR_PARAM, "invalid key space %lld", (long long)nkeys);
-    RG_TRY(ensure_counters(ctx));
-    RG_TRY(ctx->scratch[6].ensure(scan_sums_bytes(nkeys)));
-    Replicas one;
-    one.mask = 0;
-    one.stride = nkeys + 1;
-    // one replica: its cursors would be the prefix again
-    return scan_keys(len, one, nkeys, per_item, ctx->scratch[6].as<uint2>(), prefix, item_start,
-                     nullptr, items, ctx->counters.as<unsigned long long>(), s);
-}
-
 } // namespace rg
