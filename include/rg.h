@@ -139,7 +139,10 @@ int rg_context_stats(rg_context *ctx, rg_grid_stats *out);
  * scratch memory or other channel offsets fails with RG_ERR_PARAM instead of
  * reallocating or rewriting what the graph reads.  rg_context_thaw declares
  * that no graph captured from this context will be replayed again and lifts
- * the restriction (no counterpart in the reference, which has no graphs). */
+ * the restriction (no counterpart in the reference, which has no graphs).  A
+ * direct DFT on a capturing stream allocates nothing; the graph holds its
+ * partial sums, so until the thaw later DFTs on the context leave that memory
+ * in place too, taking fewer partial sums where it is too small. */
 int rg_context_thaw(rg_context *ctx);
 
 /* Kernel timers: when enabled, librg records HIP events on the launch stream

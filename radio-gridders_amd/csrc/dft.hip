@@ -225,13 +225,29 @@ __global__ __launch_bounds__(256) void k_dft_sum(const double2 *__restrict__ par
     out[p] = a;
 }
 
-// ranges of the visibility stream: partial sums in scratch when there are several
-static int dft_ranges(rg_context *ctx, int64_t nr, int64_t npix, double2 *out, double2 **dst)
+// Ranges the partial sums of which the context's scratch can take: as many as wanted,
+// but a call that is being captured allocates nothing and none takes the scratch away
+// from a captured one, so these make do with the ranges that fit it (one needs none).
+static int dft_fit(rg_context *ctx, int64_t &nr, int64_t npix, bool &capturing, hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    RG_HIP(hipStreamIsCapturing(s, &cap));
+    capturing = cap != hipStreamCaptureStatusNone;
+    if (capturing || ctx->frozen || ctx->dft_captured)
+        nr = std::max<int64_t>(
+            1, std::min<int64_t>(nr, (int64_t)(ctx->scratch[14].bytes / sizeof(double2)) / npix));
+    return RG_OK;
+}
+
+// partial sums of nr ranges (fitted) in scratch when there are several
+static int dft_ranges(rg_context *ctx, int64_t nr, int64_t npix, bool capturing, double2 *out,
+                      double2 **dst)
 {
     *dst = out;
     if (nr > 1) {
         RG_TRY(ctx->scratch[14].ensure(sizeof(double2) * (size_t)(nr * npix)));
         *dst = ctx->scratch[14].as<double2>();
+        ctx->dft_captured = ctx->dft_captured || capturing;
     }
     return RG_OK;
 }
@@ -262,9 +278,11 @@ static int launch_mixed(rg_context *ctx, const rg_flat_vis *vis, const int32_t *
                         hipStream_t s)
 {
     const int64_t blocks = (npix + DFT_THREADS - 1) / DFT_THREADS;
-    const int64_t nr = long_ranges(vis->n, npix);
+    int64_t nr = long_ranges(vis->n, npix);
+    bool capturing;
+    RG_TRY(dft_fit(ctx, nr, npix, capturing, s));
     double2 *dst;
-    RG_TRY(dft_ranges(ctx, nr, npix, out, &dst));
+    RG_TRY(dft_ranges(ctx, nr, npix, capturing, out, &dst));
     hipLaunchKernelGGL((k_dft_mixed<LIST, VT>), dim3((unsigned)blocks, (unsigned)nr),
                        dim3(DFT_THREADS), 0, s, vis->u, vis->v, vis->w, (const VT *)vis->vis,
                        vis->n, px, py, npix, N, lambda, dst);
@@ -284,16 +302,12 @@ static int launch_fp64(rg_context *ctx, const rg_flat_vis *vis, const int32_t *p
     // partial sums stay below a few percent), at most 1024
     int64_t nr = std::min<int64_t>(1024, (4096 + blocks - 1) / blocks);
     nr = std::max<int64_t>(1, std::min<int64_t>(nr, vis->n / 256));
-    // scratch that may not grow (a graph being captured, or one that holds the
-    // context's scratch): the long ranges, which need none for short streams
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    RG_HIP(hipStreamIsCapturing(s, &cap));
-    if (ctx->frozen || cap != hipStreamCaptureStatusNone)
-        nr = long_ranges(vis->n, npix);
+    bool capturing;
+    RG_TRY(dft_fit(ctx, nr, npix, capturing, s));
     const int64_t per = ((vis->n + nr - 1) / nr + 15) / 16 * 16;
     nr = std::max<int64_t>(1, (vis->n + per - 1) / std::max<int64_t>(per, 1));
     double2 *dst;
-    RG_TRY(dft_ranges(ctx, nr, npix, out, &dst));
+    RG_TRY(dft_ranges(ctx, nr, npix, capturing, out, &dst));
     hipLaunchKernelGGL((k_dft_fp64<LIST, VT, PT>), dim3((unsigned)blocks, (unsigned)nr),
                        dim3(DFT_THREADS), 0, s, vis->u, vis->v, vis->w, (const VT *)vis->vis,
                        vis->n, per, px, py, npix, N, lambda, dst);

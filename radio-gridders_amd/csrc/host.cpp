@@ -365,6 +365,7 @@ int rg_context_thaw(rg_context *ctx)
     if (!ctx)
         return fail(RG_ERR_PARAM, "ctx is NULL");
     ctx->frozen = false;
+    ctx->dft_captured = false;
     return RG_OK;
 }
 

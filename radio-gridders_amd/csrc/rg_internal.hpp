@@ -150,6 +150,9 @@ struct rg_context {
     // so no slot may be reallocated and the offsets not rewritten until
     // rg_context_thaw
     bool frozen = false;
+    // set by a DFT with partial sums on a capturing stream (the graph holds scratch[14]),
+    // until rg_context_thaw
+    bool dft_captured = false;
     // batched W-towers capacities of the last shape
     rg::WtPlan wt_plan;
     std::map<rg::TwKey, rg::DevBuf> twiddles;

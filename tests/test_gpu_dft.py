@@ -104,3 +104,46 @@ def test_dft_tile_remainders(ctx, npix, nvis, vdt):
     ctx.dft(fv, dev(px), dev(py), N, lam, out)
     torch.cuda.synchronize()
     assert np.abs(out.cpu().numpy() - ref).max() < 1e-12 * np.abs(vis).sum()
+
+
+@pytest.mark.parametrize("mode,tol", [(rgamd.RG_DFT_FP64, 1e-11), (rgamd.RG_DFT_MIXED, 2e-5)])
+@pytest.mark.parametrize("warm", [0, 40, 400])
+def test_dft_capture_keeps_its_partial_sums(mode, tol, warm):
+    """A captured DFT takes no more partial sums than the scratch of the calls before it holds
+    (none, some, all of what it would like), and later calls on the context, which would like more
+    of it, leave it in place: they are right, and so is every replay after them."""
+    rng = np.random.default_rng(5)
+    N, lam = 2048, 20480.0
+    c = rgamd.Context(0)
+
+    def stream(n, npix):
+        u, v = rng.uniform(-5000, 5000, (2, n))
+        w = rng.uniform(-300, 300, n)
+        vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+        px, py = rng.integers(0, N, (2, npix)).astype(np.int32)
+        keep, fv = stage(u, v, w, vis)
+        return (keep, fv, dev(px), dev(py), torch.empty(npix, dtype=torch.complex128, device="cuda"),
+                orc.dft(px, py, N, lam, u, v, w, vis))
+
+    a, b = stream(140_000, 400), stream(200_000, 500)
+    if warm:
+        c.dft(a[1], a[2][:warm].clone(), a[3][:warm].clone(), N, lam, a[4][:warm].clone(), mode)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.dft(a[1], a[2], a[3], N, lam, a[4], mode,
+              stream=torch.cuda.current_stream().cuda_stream)
+    for rep in range(3):
+        c.dft(b[1], b[2], b[3], N, lam, b[4], mode)
+        a[4].zero_()
+        torch.cuda.synchronize()
+        assert rel_max(b[4].cpu().numpy(), b[5]) < tol
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_max(a[4].cpu().numpy(), a[5]) < tol, rep
+    del graph
+    c.thaw()
+    c.dft(b[1], b[2], b[3], N, lam, b[4], mode)
+    torch.cuda.synchronize()
+    assert rel_max(b[4].cpu().numpy(), b[5]) < tol
+    c.close()
