@@ -209,13 +209,23 @@ struct WprojShape {
     int64_t nkeys;    // plane groups x grids x tiles
     uint32_t per_item;
     // FP32 grids: records of a key whose items add up in FP64 first (0: no key),
-    // slots for such keys of this stream, and of any shorter one too
+    // slots for such keys of this stream, and for any shorter one too
     uint32_t hot_min;
     int64_t hot_slots, hot_room;
+    // records per work item of a call without such slots, whose items are added up in FP32:
+    // with 512 a dense tile's sum would be rounded four times as often
+    static constexpr uint32_t COLD_ITEM = 2048;
 
     size_t hot_bytes(int S, int64_t slots) const
     {
         return slots * sizeof(double) * (size_t)tile_slot(S, tw);
+    }
+    // no room for the slots
+    void cold()
+    {
+        hot_min = 0;
+        hot_slots = hot_room = 0;
+        per_item = std::max(per_item, COLD_ITEM);
     }
     void one_group(int planes, int n_chan)
     {
@@ -359,10 +369,12 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
         }
     }
     // a key of eight default items or more (the shortest streams have too few items for
-    // it to matter); the next shorter item size needs at most twice the slots
-    sh.hot_min = nvis >= 1024 ? 8 * default_item(nvis) : 0;
+    // it to matter)
+    const int64_t k = default_item(nvis);
+    sh.hot_min = nvis >= 1024 ? (uint32_t)(8 * k) : 0;
     sh.hot_slots = sh.hot_min ? nvis / sh.hot_min + 1 : 0;
-    sh.hot_room = 2 * sh.hot_slots;
+    // of the shorter streams the longest with items of k / 2, 12 k^2 - 1 records, takes most
+    sh.hot_room = std::max<int64_t>(sh.hot_slots, sh.hot_min && k > 8 ? 3 * k : 0);
     sh.per_item = p->vis_per_item > 0 ? std::min<uint32_t>((uint32_t)p->vis_per_item, TILE_SORT)
                                       : default_item(nvis);
     return RG_OK;
@@ -411,6 +423,20 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     // a context's first call: the grids are cleared while the host allocates
     if (!ctx->scratch[5].p)
         RG_TRY(zero.launch(s));
+    HotSlots hot{};
+    if (grid_type == RG_C64 && sh.hot_min) {
+        const size_t kb = (sizeof(uint32_t) * (size_t)sh.hot_room + 255) / 256 * 256;
+        DevBuf &buf = ctx->scratch[20];
+        // (scratch that a captured graph holds, of another kind of call perhaps, may not do)
+        if (buf.ensure(kb + sh.hot_bytes(wk->size, sh.hot_room)) == RG_OK) {
+            hot.key = buf.as<uint32_t>();
+            hot.sums = reinterpret_cast<double *>(buf.as<char>() + kb);
+            RG_TRY(zero.add(hot.key, kb));
+            RG_TRY(zero.add(hot.sums, sh.hot_bytes(wk->size, sh.hot_slots)));
+        } else {
+            sh.cold();
+        }
+    }
     BinPlan pl;
     int rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
     if (rc != RG_OK && sh.nkeys != (int64_t)sh.ntiles * n_chan) {
@@ -420,15 +446,6 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     }
     if (rc != RG_OK)
         return rc;
-    HotSlots hot{};
-    if (grid_type == RG_C64 && sh.hot_min) {
-        const size_t kb = (sizeof(uint32_t) * (size_t)sh.hot_room + 255) / 256 * 256;
-        RG_TRY(ctx->scratch[20].ensure(kb + sh.hot_bytes(wk->size, sh.hot_room)));
-        hot.key = ctx->scratch[20].as<uint32_t>();
-        hot.sums = reinterpret_cast<double *>(ctx->scratch[20].as<char>() + kb);
-        RG_TRY(zero.add(hot.key, kb));
-        RG_TRY(zero.add(hot.sums, sh.hot_bytes(wk->size, sh.hot_slots)));
-    }
 
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));

@@ -124,6 +124,57 @@ def test_short_call_on_a_frozen_context(table):
     c.close()
 
 
+@pytest.mark.parametrize("first,sizes", [
+    (("c64", 60_000), (49_151, 12_287, 1_025, 60_000)), (("c64", 200_000), (196_607, 190_000)),
+    (("c128", 60_000), (60_000, 49_151, 1_025)), (("towers", 60_000), (60_000, 49_151, 1_025))])
+def test_single_precision_calls_on_a_frozen_context(table, first, sizes):
+    """FP32 calls with an FP32 grid on a context whose scratch a captured graph holds: of a longer
+    call of that kind, of one with an FP64 grid and of a W-towers one, neither of which has sums
+    of dense tiles; at the lengths where the item size halves.  A cell is a sum of at most n products of four
+    roundings each."""
+    N, kind, n0 = 128, *first
+    c, plain = rgamd.Context(0), rgamd.Context(0)
+    _, wk = kern(table, -5.0, 1.0, torch.complex64)
+    t64 = table.astype(np.complex64).astype(np.complex128)
+    _, wk64 = kern(t64, -5.0, 1.0)
+    _, wkabs = kern(np.abs(t64) + 0j, -5.0, 1.0)
+    u, v, w, vis = stream(n0, 60.0, 4.0, 3)
+    vis = vis.astype(np.complex64)
+    g32 = torch.empty((N, N), dtype=torch.complex64, device="cuda")
+    g128 = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    p = rgamd.params(N, THETA)
+    keep, fv = stage(u, v, w, vis, torch.complex64)
+    call = {"c64": (p, fv, wk, g32), "c128": (p, fv, wk, g128),
+            "towers": (rgamd.params(N, THETA, subgrid=64, margin=16, winc=10.0), fv, wk, g128)}[kind]
+    for _ in range(2):
+        c.grid(*call)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.grid(*call)
+    want = call[3].clone()
+    for n in sizes:
+        k, f = stage(u[:n], v[:n], w[:n], vis[:n], torch.complex64)
+        got = torch.empty_like(g32)
+        c.grid(p, f, wk, got)
+        _, f64 = stage(u[:n], v[:n], w[:n], vis[:n].astype(np.complex128))
+        _, fabs = stage(u[:n], v[:n], w[:n], np.abs(vis[:n].astype(np.complex128)) + 0j)
+        ref, mag = torch.empty_like(g128), torch.empty_like(g128)
+        pp = rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN)
+        plain.grid(pp, f64, wk64, ref)
+        plain.grid(pp, fabs, wkabs, mag)
+        torch.cuda.synchronize()
+        assert ((got.to(torch.complex128) - ref).abs() <= (n + 4) * 2.0 ** -24 * mag.real).all(), n
+    for _ in range(3):
+        call[3].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((call[3] - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    del graph
+    c.close()
+    plain.close()
+
+
 def crowd(n, N, s, planes, seed):
     """n visibilities: half in one 16 x 16 tile of positions (several a position), half over
     the grid and its edges; planes of the whole table."""
