@@ -119,7 +119,7 @@ int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, 
     // counter replicas: up to 16, at most max_counters counters in all
     // (replicas spread the atomics of hot keys; a stream without hot keys
     // is better served by fewer counters that stay in cache)
-    pl.rp.stride = (nkeys + 1 + 63) / 64 * 64;
+    pl.rp.stride = bin_stride(nkeys);
     uint32_t nrep = 16;
     while (nrep > 1 && (int64_t)nrep * pl.rp.stride > max_counters)
         nrep >>= 1;

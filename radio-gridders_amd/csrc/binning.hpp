@@ -92,6 +92,9 @@ __device__ inline uint32_t wave_agg_add(uint32_t *counters, uint32_t key, bool a
     return want ? wave_agg_rank(base, my_head) : 0u;
 }
 
+// counters of a sort in all, at most (unless its keys are more)
+constexpr int64_t BIN_MAX_COUNTERS = (int64_t)1 << 22;
+
 // Counter replicas: NREP arrays of `stride` entries (stride >= nkeys + 1).
 struct Replicas {
     uint32_t mask;   // NREP - 1, NREP a power of two
@@ -364,6 +367,8 @@ struct BinBufs {
     unsigned long long *stats; // CNT__N call counters
 };
 
+// counters of one replica
+inline int64_t bin_stride(int64_t nkeys) { return (nkeys + 1 + 63) / 64 * 64; }
 // Validates the sort's sizes and fills the plan (no device work).
 int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, size_t rec_bytes,
              BinPlan &pl);
@@ -375,16 +380,25 @@ template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
             const BinBufs &b, ZeroList &zero, bool cleared, rg_context *timer_ctx,
             hipStream_t s, BinResult &out);
-// Plan and scratch (the context's slots 0-6 and 15) of a sort, and what it needs
-// cleared added to `zero`: for a caller that clears more in the same launch.
+// Plan and scratch (the context's slots 0-6 and 15, with room for key_room keys) of a
+// sort, and what it needs cleared added to `zero`: for a caller that clears more in the same
+// launch.
 template <typename T>
-int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters,
-                ZeroList &zero, BinPlan &pl);
+int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uint32_t per_item,
+                int64_t max_counters, ZeroList &zero, BinPlan &pl);
+// Keys of a W-projection of n_chan N^2 grids by the narrowest tiles, in one plane group: every
+// gridding call makes room for them, so that a context whose scratch a captured graph
+// of any gridder holds takes a W-projection of its grids.
+inline int64_t wproj_key_room(int N, int n_chan)
+{
+    const int64_t nt = (N + 16 + 15) / 16;
+    return nt * nt * n_chan;
+}
 // bin_run into the context's scratch; ready: the plan of a bin_prepare whose
 // areas have been cleared (NULL: none).
 template <typename Keyer, typename T>
-int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
-                     ZeroList &zero, hipStream_t s, BinResult &out,
-                     int64_t max_counters = (int64_t)1 << 22, const BinPlan *ready = nullptr);
+int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, int64_t key_room,
+                     uint32_t per_item, ZeroList &zero, hipStream_t s, BinResult &out,
+                     int64_t max_counters, const BinPlan *ready = nullptr);
 
 } // namespace rg

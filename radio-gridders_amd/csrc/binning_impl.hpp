@@ -51,22 +51,26 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
 static const int bin_slot[BIN__N] = {0, 1, 2, 3, 4, 5, 6, 15};
 
 template <typename T>
-int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters,
-                ZeroList &zero, BinPlan &pl)
+int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uint32_t per_item,
+                int64_t max_counters, ZeroList &zero, BinPlan &pl)
 {
     RG_TRY(bin_plan(n, nkeys, per_item, max_counters, sizeof(Rec<T>), pl));
     RG_TRY(ensure_counters(ctx));
     // items and scan sums: room for every call of up to this many visibilities
     // and keys, whatever item size it picks (scratch that a captured graph holds
     // cannot grow; a shorter stream's smaller items are at most 24 times 512);
-    // counters likewise: fewer keys may take more replicas
-    const int64_t room = nkeys + std::max<int64_t>(n / per_item, std::max<int64_t>(12288, n / 512)) + 1;
+    // counters likewise: fewer keys, or another gridder's, may take more replicas
+    key_room = std::max(key_room, nkeys);
+    const int64_t stride = bin_stride(key_room);
+    const int64_t items = key_room + std::max<int64_t>({n / per_item, 12288, n / 512}) + 1;
     const size_t count_bytes = pl.bytes[BIN_COUNT];
-    const size_t counters = sizeof(uint32_t) * (size_t)std::min<int64_t>(16 * pl.rp.stride, max_counters);
     for (int k : {BIN_COUNT, BIN_CURSOR})
-        pl.bytes[k] = std::max(pl.bytes[k], counters);
-    pl.bytes[BIN_ITEMS] = std::max(pl.bytes[BIN_ITEMS], sizeof(Item) * (size_t)room);
-    pl.bytes[BIN_BSUMS] = scan_sums_bytes(nkeys);
+        pl.bytes[k] = sizeof(uint32_t) *
+                      (size_t)std::max(stride, std::min(16 * stride, BIN_MAX_COUNTERS));
+    for (int k : {BIN_VIS_START, BIN_ITEM_START})
+        pl.bytes[k] = sizeof(uint32_t) * (size_t)(key_room + 1);
+    pl.bytes[BIN_ITEMS] = sizeof(Item) * (size_t)items;
+    pl.bytes[BIN_BSUMS] = scan_sums_bytes(key_room);
     for (int k = 0; k < BIN__N; ++k)
         RG_TRY(ctx->scratch[bin_slot[k]].ensure(pl.bytes[k]));
     if (!bin_small(n, nkeys))
@@ -75,15 +79,15 @@ int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, uint32_t per_item, in
 }
 
 template <typename Keyer, typename T>
-int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item,
-                     ZeroList &zero, hipStream_t s, BinResult &out, int64_t max_counters,
-                     const BinPlan *ready)
+int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys, int64_t key_room,
+                     uint32_t per_item, ZeroList &zero, hipStream_t s, BinResult &out,
+                     int64_t max_counters, const BinPlan *ready)
 {
     BinPlan pl;
     if (ready)
         pl = *ready;
     else
-        RG_TRY(bin_prepare<T>(ctx, n, nkeys, per_item, max_counters, zero, pl));
+        RG_TRY(bin_prepare<T>(ctx, n, nkeys, key_room, per_item, max_counters, zero, pl));
     const int *slot = bin_slot;
     BinBufs b;
     b.count = ctx->scratch[slot[BIN_COUNT]].as<uint32_t>();

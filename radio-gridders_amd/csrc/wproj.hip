@@ -233,7 +233,6 @@ struct WprojShape {
         nkeys = (int64_t)ntiles * n_chan;
     }
 };
-constexpr int64_t WPROJ_COUNTERS = (int64_t)1 << 22;
 
 struct HotSlots {
     double *sums;
@@ -363,7 +362,7 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
         sh.ntx = (int)ntx;
         sh.one_group(wk->plane_count, n_chan);
         const int64_t wide = (planes + 4 * group - 1) / (4 * group);
-        if (2 * sh.nkeys * wide <= WPROJ_COUNTERS) {
+        if (2 * sh.nkeys * wide <= BIN_MAX_COUNTERS) {
             sh.group_planes = (int)std::min<int64_t>(4 * group, planes);
             sh.nkeys *= wide;
         }
@@ -437,12 +436,13 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
             sh.cold();
         }
     }
+    const int64_t room = wproj_key_room(N, n_chan);
     BinPlan pl;
-    int rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
+    int rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, room, sh.per_item, BIN_MAX_COUNTERS, zero, pl);
     if (rc != RG_OK && sh.nkeys != (int64_t)sh.ntiles * n_chan) {
         // no room for the plane groups (a captured graph holds the scratch): without them
         sh.one_group(wk->plane_count, n_chan);
-        rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, sh.per_item, WPROJ_COUNTERS, zero, pl);
+        rc = bin_prepare<T>(ctx, vis->n, sh.nkeys, room, sh.per_item, BIN_MAX_COUNTERS, zero, pl);
     }
     if (rc != RG_OK)
         return rc;
@@ -450,8 +450,8 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));
     BinResult br;
-    RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, sh.nkeys,
-                                            sh.per_item, zero, s, br, WPROJ_COUNTERS, &pl)));
+    RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, sh.nkeys, room, sh.per_item,
+                                            zero, s, br, BIN_MAX_COUNTERS, &pl)));
     return dispatch_tiles<T>(br, ctx, ctx->counters.as<unsigned long long>(), wk, grid, grid_type,
                              p->compensated != 0, N, n_chan, sh, hot, s);
 }
@@ -518,7 +518,7 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     BinPlan pl;
     const uint32_t limit_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item : 2048u;
     const int64_t lt = p->tile > 0 ? p->tile : 32, ln = (N + wk->size + lt - 1) / lt, lk = ln * ln;
-    RG_TRY(bin_plan(vis->n, lk, limit_item, WPROJ_COUNTERS, sizeof(Rec<T>), pl));
+    RG_TRY(bin_plan(vis->n, lk, limit_item, BIN_MAX_COUNTERS, sizeof(Rec<T>), pl));
     size_t want = head;
     for (int k = 0; k < BIN__N; ++k)
         want += aligned(k == BIN_BSUMS ? sizeof(uint2) * (size_t)((lk + 1023) / 1024 + 1)
@@ -540,7 +540,7 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
         }
         return (int)RG_OK;
     };
-    RG_TRY(carve(WPROJ_COUNTERS));
+    RG_TRY(carve(BIN_MAX_COUNTERS));
     if (at > NOALLOC_SCRATCH_BYTES) { // leaner: no plane groups, larger items, one replica
         sh.one_group(wk->plane_count, 1);
         sh.per_item = std::max(sh.per_item, limit_item);

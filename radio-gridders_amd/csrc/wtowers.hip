@@ -1992,8 +1992,8 @@ static int wtowers_plain(rg_context *ctx, const rg_grid_params *p, const rg_flat
     const TowerKeyer kf = wt_keyer(p, vis, wk, g, d_range, nwp, nullptr);
     const int64_t nslots = (int64_t)cc * cc * nwp;
     BinResult br;
-    RG_TRY((bin_visibilities<TowerKeyer, double>(ctx, kf, vis->n, nslots, 0x40000000u, zero, s, br,
-                                                 (int64_t)1 << 20)));
+    RG_TRY((bin_visibilities<TowerKeyer, double>(ctx, kf, vis->n, nslots, wproj_key_room(N, 1),
+                                                 0x40000000u, zero, s, br, (int64_t)1 << 20)));
     RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (2 * nslots + 1)));
     uint32_t *d_nvis = ctx->scratch[9].as<uint32_t>();
     uint32_t *d_item0 = d_nvis + nslots;
@@ -2216,6 +2216,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         return TableLayout(ntw, g.ntw * nwp_cap, ntasks_cap, nchunks_cap,
                            (ntasks_cap + q - 1) / q);
     };
+    const int64_t key_room = wproj_key_room(g.N, nchan);
     const BinPlan *ready = nullptr;
     BinPlan bin;
     if (!measure) {
@@ -2224,7 +2225,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         const int q = batch_tasks_of(ntasks_cap);
         RG_TRY(clear_subimages((ntasks_cap + q - 1) / q,
                                ctx->scratch[18].as<uint32_t>() + tl.o_spill));
-        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, 0x40000000u,
+        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, key_room, 0x40000000u,
                                wt_counters(vis->n), zero, bin)));
         ready = &bin;
     }
@@ -2264,8 +2265,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     uint32_t *slot_start = ctx->scratch[9].as<uint32_t>();
     br.group_start = slot_start;
     br.group_keys = NB;
-    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, 0x40000000u, zero, s, br,
-                                            wt_counters(vis->n), ready)));
+    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, key_room, 0x40000000u, zero, s,
+                                            br, wt_counters(vis->n), ready)));
 
     if (measure) {
         ntasks_cap = (int)std::min<int64_t>(nslots, 0x7fffffff);

@@ -175,6 +175,49 @@ def test_single_precision_calls_on_a_frozen_context(table, first, sizes):
     plain.close()
 
 
+@pytest.mark.parametrize("captured", ["towers", "two channels"])
+def test_more_keys_than_the_captured_call(table, captured):
+    """On a context whose scratch a captured graph holds, W-projections of the same stream with more keys:
+    after a W-towers call of few towers and one floor (2880 keys), after two sparse channels, whose
+    tiles are wide (1024^2 grids, 4225 keys, and 1216^2, of about as many cells as the two channels have)."""
+    N, n = 1024, 70_000
+    c, plain = rgamd.Context(0), rgamd.Context(0)
+    _, wk = kern(table, -5.0, 1.0)
+    u, v, w, vis = stream(n, 4500.0, 4.0, 8)
+    _, fv = stage(u, v, w, vis)
+    off = np.array([0, n // 3, n], dtype=np.int64)
+    if captured == "towers":
+        p = rgamd.params(N, THETA, subgrid=512, margin=16, winc=10.0)
+        g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+        call = lambda: c.grid(p, fv, wk, g)  # noqa: E731
+    else:
+        p = rgamd.params(N, THETA)
+        g = torch.empty((2, N, N), dtype=torch.complex128, device="cuda")
+        call = lambda: c.grid_channels(p, fv, off, wk, g)  # noqa: E731
+    for _ in range(2):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    want = g.clone()
+    for size in (N, 1216) if captured != "towers" else (N,):
+        got = torch.empty((size, size), dtype=torch.complex128, device="cuda")
+        ref = torch.empty_like(got)
+        c.grid(rgamd.params(size, THETA), fv, wk, got)
+        plain.grid(rgamd.params(size, THETA, mode=rgamd.RG_MODE_PLAIN), fv, wk, ref)
+        torch.cuda.synchronize()
+        assert float((got - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
+    for _ in range(3):
+        g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((g - want).abs().max()) <= 1e-12 * float(want.abs().max())
+    del graph
+    c.close()
+    plain.close()
+
+
 def crowd(n, N, s, planes, seed):
     """n visibilities: half in one 16 x 16 tile of positions (several a position), half over
     the grid and its edges; planes of the whole table."""
