@@ -1086,7 +1086,11 @@ static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nk
     const int64_t max_items = nkeys + n / K + 1;
 
     RG_TRY(ensure_counters(ctx));
-    RG_TRY(ctx->scratch[0].ensure(sizeof(uint32_t) * (size_t)nc * nb));      // hist
+    // hist: of a shorter stream's workgroups too, which may be more (scratch that a captured
+    // graph holds cannot grow)
+    const int64_t nb_room = std::min<int64_t>(WS_SORT_BLOCKS, (n + 2 * WS_SORT_THREADS - 1) /
+                                                                  (2 * WS_SORT_THREADS));
+    RG_TRY(ctx->scratch[0].ensure(sizeof(uint32_t) * (size_t)nc * nb_room));
     RG_TRY(ctx->scratch[1].ensure(sizeof(uint32_t) * (nkeys + 1)));          // vis_start
     RG_TRY(ctx->scratch[2].ensure(sizeof(uint32_t) * (nkeys + 1)));          // item_start
     RG_TRY(ctx->scratch[3].ensure(sizeof(uint32_t) * (nc + 1)));             // bucket starts

@@ -319,3 +319,36 @@ def test_dense_keys_at_their_edges(ctx, kernels, per_tile):
     assert np.all(got[order >= len(order) - 19] == 0)
     st = ctx.stats()
     assert st.n_dropped == 19 and st.n_gridded == len(u) - 19
+
+
+def test_shorter_prediction_on_a_frozen_context(kernels):
+    """A prediction sized the scratch, a captured gridding call holds it: shorter predictions, one of
+    which the sort cuts into more workgroups (1 090 000 into 355, 1 040 000 into 508)."""
+    theta, lam = 0.1, 640.0
+    h, d = kernels["host"], kernels["desc"]
+    rng = np.random.default_rng(3)
+    c = rgamd.Context(0)
+    p = params(kernels, theta, lam)
+    l, m = card(theta)
+    c.wstack_build(p, dev(l), dev(m), None, d["lm"], d["n"])
+    n = 1_090_000
+    u, v, w = (dev(a) for a in uvw(rng, theta, lam, h["w"].dw, n))
+    out = torch.empty(n, dtype=torch.complex128, device="cuda")
+    c.wstack_degrid(p, u, v, w, d["uv"], d["w"], out)
+    want = out.clone()
+    k = torch.randn((1, 4, 4, 8, 8), dtype=torch.complex128, device="cuda")
+    g = torch.empty((128, 128), dtype=torch.complex128, device="cuda")
+    fv = rgamd.flat_vis(u[:5000], v[:5000], w[:5000], want[:5000])
+    for _ in range(2):
+        c.grid(rgamd.params(128, theta), fv, rgamd.wkern_desc(k, 0.0, 1e9), g)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.grid(rgamd.params(128, theta), fv, rgamd.wkern_desc(k, 0.0, 1e9), g)
+    for n1 in (1_040_000, n, 3000):
+        out.zero_()
+        c.wstack_degrid(p, u[:n1], v[:n1], w[:n1], d["uv"], d["w"], out[:n1])
+        torch.cuda.synchronize()
+        assert float((out[:n1] - want[:n1]).abs().max()) <= 1e-12 * float(want.abs().max()), n1
+    del graph
+    c.close()
