@@ -448,8 +448,8 @@ template <int AUV, int AW, int LV>
 __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     const double2 *__restrict__ stack, int og, int wp, int ntx,
     const WsRec *__restrict__ recs, const Item *__restrict__ items,
-    const uint32_t *__restrict__ nitems_p, const double *__restrict__ conv_uv,
-    const double *__restrict__ conv_w, double2 *out)
+    const uint32_t *__restrict__ nitems_p, const uint32_t *__restrict__ key_start,
+    const double *__restrict__ conv_uv, const double *__restrict__ conv_w, double2 *out)
 {
 #pragma clang fp contract(off)
     constexpr int T = 1 << WStackKeyer::TILE_SHIFT, H = AUV / 2, R = T + AUV, P = AW;
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     const uint32_t nitems = *nitems_p;
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         const Item item = items[it];
-        if (item.count > WS_ITEM) // k_ws_degrid_cells
+        if (key_start[item.key + 1] - key_start[item.key] >= WS_DENSE) // k_ws_degrid_cells
             continue;
         const int ws = (int)(item.key % (uint32_t)wp);
         const int tile = (int)(item.key / (uint32_t)wp);
@@ -581,8 +581,9 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
 constexpr uint32_t WS_DENSE_MAX = 8192; // records of an item
 constexpr int WS_DENSE_THREADS = 1024;
 
-// records per work item: dense keys in equal parts of at most dense_max, each listed
-// (in any order); down to WS_DENSE / 2 a part holds more than WS_DENSE / 3
+// records per work item: dense keys in parts of at most dense_max, each listed (in any
+// order).  Down to a dense_max of WS_DENSE / 2 the size of a dense key's parts (the last one
+// has what is left) is above WS_DENSE / 3, and so above per_item.
 struct WsItems {
     uint32_t dense_max; // 0: the support has no dense form
     uint32_t *ndense, *dense;
@@ -1181,7 +1182,7 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         return fail(RG_ERR_UNSUPPORTED, "W-stack indices beyond 16 bits");
     BinResult br;
     const int64_t nkeys = (int64_t)kf.ntx * kf.ntx * wp;
-    static_assert(WS_ITEM <= WS_DENSE / 3, "items of sparse keys are told apart by their size");
+    static_assert(WS_ITEM <= WS_DENSE / 3, "a dense key's item size is told apart by its value");
     if (((uintptr_t)out & 15) != 0)
         return fail(RG_ERR_PARAM, "predicted visibilities must be 16-byte aligned");
     // sort by uv tile and plane; dense keys in parts of 1/256 of the stream, so that
@@ -1214,7 +1215,8 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         const int64_t blocks = std::min<int64_t>(br.max_items, 4096);
         hipLaunchKernelGGL((k_ws_degrid_tile<8, 4, LV>), dim3((unsigned)blocks), dim3(256), 0, s,
                            stack, og, wp, kf.ntx, recs, (const Item *)br.items,
-                           (const uint32_t *)(br.item_start + nkeys), conv_uv->data, conv_w->data,
+                           (const uint32_t *)(br.item_start + nkeys),
+                           (const uint32_t *)br.vis_start, conv_uv->data, conv_w->data,
                            (double2 *)out);
     } else {
         constexpr int LV = 64;

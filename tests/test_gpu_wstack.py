@@ -352,3 +352,30 @@ def test_shorter_prediction_on_a_frozen_context(kernels):
         assert float((out[:n1] - want[:n1]).abs().max()) <= 1e-12 * float(want.abs().max()), n1
     del graph
     c.close()
+
+
+@pytest.mark.parametrize("copies", [3071, 3073, 4609, 6145])
+def test_every_part_of_a_dense_key_is_predicted_once(ctx, kernels, copies):
+    """Copies of one visibility, a key whose last part is shorter than the others (3073: 1025, 1025
+    and 1023 records; 3071 is sparse).  The weights along u are scaled by 1e180, those along v and w by 1e-180:
+    the sparse keys' kernel multiplies by v and w first, which underflows to 0, the dense ones' by u
+    and w, which does not, so that a part that both have computed shows the last one's 0."""
+    theta, lam = 0.1, 640.0
+    h, d = kernels["host"], kernels["desc"]
+    rng = np.random.default_rng(11)
+    l = rng.uniform(-0.45 * theta, 0.45 * theta, 40)
+    m = rng.uniform(-0.45 * theta, 0.45 * theta, 40)
+    p = params(kernels, theta, lam)
+    ctx.wstack_build(p, dev(l), dev(m), None, d["lm"], d["n"])
+    uv, kw = kernels["dev"]["uv"].clone().reshape(-1), kernels["dev"]["w"] * 1e-180
+    half = h["uv"].size * (h["uv"].oversampling // 2)
+    uv[:half] *= 1e180
+    uv[half:] *= 1e-180
+    du = h["uv"].du
+    u, v, w = (np.full(copies, x) for x in (2.75 * du, 2.25 * du, 0.3 * h["w"].dw))
+    out = torch.empty(copies, dtype=torch.complex128, device="cuda")
+    ctx.wstack_degrid(p, dev(u), dev(v), dev(w),
+                      rgamd.sep_kern_desc(uv, h["uv"].size, h["uv"].oversampling),
+                      rgamd.sep_kern_desc(kw, h["w"].size, h["w"].oversampling), out)
+    torch.cuda.synchronize()
+    assert float((out - out[0]).abs().max()) <= 1e-13 * float(out[0].abs())
