@@ -435,7 +435,21 @@ __global__ __launch_bounds__(256) void k_ws_degrid(
 // predictions of 10 M visibilities (6 k on a key) take 1.46 ms so and 1.89 ms by
 // k_ws_degrid_tile; from 2048 on, 3 M (1.8 k on a key) would take 1.02 ms, not 0.96.
 constexpr uint32_t WS_DENSE = 3072;
-constexpr uint32_t WS_ITEM = 1024; // records of a sparse key's work items
+// Only in streams of at least WS_DENSE_STREAM: shorter ones have too few dense items to fill the
+// chip, and the two kernels, one after the other, each take as long as their longest item.
+// Degridding with dense keys, without, us: 100 k on 512^2 planes 129 / 66, 600 k on 1024^2
+// 179 / 134, 300 k on 128^2 79 / 89; 1 M 205 / 189 and 155 / 177; 4 M 398 / 478 and 327 / 461.
+constexpr int64_t WS_DENSE_STREAM = (int64_t)1 << 20;
+// Records of a sparse key's work items: 1024, fewer where that leaves less than the
+// 1024 workgroups that fit the chip (30 k on 128^2 planes: 82 us with 1024, 52 so).
+constexpr uint32_t WS_ITEM = 1024, WS_ITEM_MIN = 128;
+static uint32_t ws_item(int64_t nvis)
+{
+    return (uint32_t)std::clamp<int64_t>(nvis / 1024, WS_ITEM_MIN, WS_ITEM);
+}
+// items of sparse keys beyond one a key, of any stream up to this one (n / ws_item(n) is no
+// more than 1032 below 1 M)
+static int64_t ws_item_room(int64_t nvis) { return std::max<int64_t>(nvis / WS_ITEM, 1032); }
 
 // Fixed 8 x 4 support with the stack staged in LDS: one work item (<= K
 // records of one (uv tile, w plane) key) at a time per workgroup; the
@@ -449,7 +463,8 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     const double2 *__restrict__ stack, int og, int wp, int ntx,
     const WsRec *__restrict__ recs, const Item *__restrict__ items,
     const uint32_t *__restrict__ nitems_p, const uint32_t *__restrict__ key_start,
-    const double *__restrict__ conv_uv, const double *__restrict__ conv_w, double2 *out)
+    uint32_t dense_from, const double *__restrict__ conv_uv, const double *__restrict__ conv_w,
+    double2 *out)
 {
 #pragma clang fp contract(off)
     constexpr int T = 1 << WStackKeyer::TILE_SHIFT, H = AUV / 2, R = T + AUV, P = AW;
@@ -462,7 +477,7 @@ __global__ __launch_bounds__(256) void k_ws_degrid_tile(
     const uint32_t nitems = *nitems_p;
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         const Item item = items[it];
-        if (key_start[item.key + 1] - key_start[item.key] >= WS_DENSE) // k_ws_degrid_cells
+        if (key_start[item.key + 1] - key_start[item.key] >= dense_from) // k_ws_degrid_cells
             continue;
         const int ws = (int)(item.key % (uint32_t)wp);
         const int tile = (int)(item.key / (uint32_t)wp);
@@ -582,8 +597,7 @@ constexpr uint32_t WS_DENSE_MAX = 8192; // records of an item
 constexpr int WS_DENSE_THREADS = 1024;
 
 // records per work item: dense keys in parts of at most dense_max, each listed (in any
-// order).  Down to a dense_max of WS_DENSE / 2 the size of a dense key's parts (the last one
-// has what is left) is above WS_DENSE / 3, and so above per_item.
+// order).  The size of a dense key's parts (the last one has what is left) is above per_item.
 struct WsItems {
     uint32_t dense_max; // 0: the support has no dense form
     uint32_t *ndense, *dense;
@@ -1084,7 +1098,7 @@ static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nk
     chunk = std::max<int64_t>(2, (chunk + WS_SORT_THREADS - 1) / WS_SORT_THREADS) *
             WS_SORT_THREADS;
     const int nb = (int)((n + chunk - 1) / chunk);
-    const int64_t max_items = nkeys + n / K + 1;
+    const int64_t max_items = nkeys + ws_item_room(n) + 1;
 
     RG_TRY(ensure_counters(ctx));
     // hist: of a shorter stream's workgroups too, which may be more (scratch that a captured
@@ -1099,7 +1113,7 @@ static int ws_sort(rg_context *ctx, const WStackKeyer &kf, int64_t n, int64_t nk
     RG_TRY(ctx->scratch[5].ensure(sizeof(WsRec) * n));                       // records
     RG_TRY(ctx->scratch[7].ensure(sizeof(WsRec) * n));                       // bucketed records
     // per-key counts, the dense items' number and list
-    const int64_t max_dense = dense_max ? n / (WS_DENSE / 3) + 1 : 0;
+    const int64_t max_dense = dense_max ? n / WS_ITEM + 1 : 0;
     RG_TRY(ctx->scratch[8].ensure(sizeof(uint32_t) * (nkeys + 1 + max_dense)));
     RG_TRY(ctx->scratch[15].ensure(sizeof(uint32_t) * n));                   // key ranks
     KernelTimer kt(ctx, RG_TIMER_BINNING, s);
@@ -1182,14 +1196,16 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         return fail(RG_ERR_UNSUPPORTED, "W-stack indices beyond 16 bits");
     BinResult br;
     const int64_t nkeys = (int64_t)kf.ntx * kf.ntx * wp;
-    static_assert(WS_ITEM <= WS_DENSE / 3, "a dense key's item size is told apart by its value");
     if (((uintptr_t)out & 15) != 0)
         return fail(RG_ERR_PARAM, "predicted visibilities must be 16-byte aligned");
     // sort by uv tile and plane; dense keys in parts of 1/256 of the stream, so that
-    // every CU has one (300 k on 128^2 planes: 156 us with 8192, 112 so)
+    // every CU has one.  Half a part is above WS_ITEM: a dense key's item size is told apart
+    // from the sparse ones' by its value, and there are at most nvis / WS_ITEM dense items.
+    static_assert(WS_DENSE_STREAM / 256 > 2 * WS_ITEM && WS_DENSE > WS_ITEM, "size of parts");
     const bool fixed = p->aa_support_uv == 8 && p->aa_support_w == 4;
-    const uint32_t part = (uint32_t)std::clamp<int64_t>(nvis / 256, WS_DENSE / 2, WS_DENSE_MAX);
-    RG_TRY(ws_sort(ctx, kf, nvis, nkeys, WS_ITEM, fixed ? part : 0, (double2 *)out, s, br));
+    const bool dense = fixed && nvis >= WS_DENSE_STREAM;
+    const uint32_t part = (uint32_t)std::min<int64_t>(nvis / 256, WS_DENSE_MAX);
+    RG_TRY(ws_sort(ctx, kf, nvis, nkeys, ws_item(nvis), dense ? part : 0, (double2 *)out, s, br));
     const WsRec *recs = reinterpret_cast<const WsRec *>(br.recs);
     const uint32_t *nrec = br.vis_start + nkeys;
     // one wavefront per visibility (the uv support, a power of two <= 64,
@@ -1201,9 +1217,8 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
     };
     if (fixed) {
         const uint32_t *ndense = ctx->scratch[8].as<uint32_t>() + nkeys;
-        // fewer than nvis / WS_ITEM dense items; 2048 workgroups, dispatched as others
-        // finish
-        if (nvis >= (int64_t)WS_DENSE)
+        // 2048 workgroups, dispatched as others finish
+        if (dense)
             hipLaunchKernelGGL((k_ws_degrid_cells<8, 4>),
                                dim3((unsigned)std::min<int64_t>(2048, nvis / WS_ITEM)),
                                dim3(WS_DENSE_THREADS), 0, s,
@@ -1216,8 +1231,8 @@ int wstack_degrid(rg_context *ctx, const rg_wstack_params *p, const double *u, c
         hipLaunchKernelGGL((k_ws_degrid_tile<8, 4, LV>), dim3((unsigned)blocks), dim3(256), 0, s,
                            stack, og, wp, kf.ntx, recs, (const Item *)br.items,
                            (const uint32_t *)(br.item_start + nkeys),
-                           (const uint32_t *)br.vis_start, conv_uv->data, conv_w->data,
-                           (double2 *)out);
+                           (const uint32_t *)br.vis_start, dense ? WS_DENSE : 0xffffffffu,
+                           conv_uv->data, conv_w->data, (double2 *)out);
     } else {
         constexpr int LV = 64;
         hipLaunchKernelGGL(k_ws_degrid<LV>, dim3((unsigned)nblocks(256 / LV)), dim3(256), 0, s,

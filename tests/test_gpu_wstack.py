@@ -354,12 +354,25 @@ def test_shorter_prediction_on_a_frozen_context(kernels):
     c.close()
 
 
-@pytest.mark.parametrize("copies", [3071, 3073, 4609, 6145])
-def test_every_part_of_a_dense_key_is_predicted_once(ctx, kernels, copies):
-    """Copies of one visibility, a key whose last part is shorter than the others (3073: 1025, 1025
-    and 1023 records; 3071 is sparse).  The weights along u are scaled by 1e180, those along v and w by 1e-180:
-    the sparse keys' kernel multiplies by v and w first, which underflows to 0, the dense ones' by u
-    and w, which does not, so that a part that both have computed shows the last one's 0."""
+# visibilities beside a test's own, on another plane, so that the stream is long enough for
+# kernels of dense keys (2^20)
+LONG = 1 << 20
+
+
+def with_filler(rng, theta, lam, dw, u, v, w):
+    k = LONG - len(u)
+    fu, fv, _ = uvw(rng, theta, lam, dw, k)
+    return (np.concatenate([u, fu]), np.concatenate([v, fv]),
+            np.concatenate([w, rng.uniform(0.01, 0.99, k) * dw]))
+
+
+@pytest.mark.parametrize("copies,long", [(3073, False), (6145, False), (3071, True), (3072, True),
+                                         (4097, True), (20_481, True)])
+def test_every_part_of_a_dense_key_is_predicted_once(ctx, kernels, copies, long):
+    """Copies of one visibility: one kernel takes every part of its key.  The weights along u are
+    scaled by 1e180, those along v and w by 1e-180: the sparse keys' kernel multiplies by v and w
+    first, which underflows to 0, the dense ones' by u and w, which does not, so that a part
+    that both have computed shows the last one's 0."""
     theta, lam = 0.1, 640.0
     h, d = kernels["host"], kernels["desc"]
     rng = np.random.default_rng(11)
@@ -372,10 +385,52 @@ def test_every_part_of_a_dense_key_is_predicted_once(ctx, kernels, copies):
     uv[:half] *= 1e180
     uv[half:] *= 1e-180
     du = h["uv"].du
-    u, v, w = (np.full(copies, x) for x in (2.75 * du, 2.25 * du, 0.3 * h["w"].dw))
-    out = torch.empty(copies, dtype=torch.complex128, device="cuda")
+    u, v, w = (np.full(copies, x) for x in (2.75 * du, 2.25 * du, -0.3 * h["w"].dw))
+    if long:
+        u, v, w = with_filler(rng, theta, lam, h["w"].dw, u, v, w)
+    out = torch.empty(len(u), dtype=torch.complex128, device="cuda")
     ctx.wstack_degrid(p, dev(u), dev(v), dev(w),
                       rgamd.sep_kern_desc(uv, h["uv"].size, h["uv"].oversampling),
                       rgamd.sep_kern_desc(kw, h["w"].size, h["w"].oversampling), out)
     torch.cuda.synchronize()
+    out = out[:copies]
+    assert bool(out[0]) == (long and copies >= 3072)
     assert float((out - out[0]).abs().max()) <= 1e-13 * float(out[0].abs())
+
+
+@pytest.mark.parametrize("per_tile", [3071, 3072, 4095, 4097, 8191, 8193, 20_481])
+def test_dense_keys_of_a_long_stream(ctx, kernels, per_tile):
+    """One (16 x 16-cell tile, plane) key around the sizes where it becomes dense and where it is
+    split into parts (4096 records, a 256th of the stream), with two full batches and one visibility more in one
+    of its cells, and a key of one cell only; the rest of the stream on the next plane, about
+    3 k to 16 k a key.  Sums of 256 products of at most |stack| sum |taps| each."""
+    theta, lam = 0.1, 640.0
+    h, d = kernels["host"], kernels["desc"]
+    rng = np.random.default_rng(per_tile)
+    du, dw = h["uv"].du, h["w"].dw
+    l, m = card(theta)
+    g = int(np.floor(theta * lam))
+
+    def at(cell):  # a coordinate whose centre tap is `cell` of the stack
+        return (cell - g - rng.uniform(0.01, 0.99, len(cell))) * du
+
+    cu, cv = 64 + rng.integers(0, 16, (2, per_tile))
+    cu[:33], cv[:33] = 67, 69
+    u = np.concatenate([at(cu), at(np.full(4500, 71))])
+    v = np.concatenate([at(cv), at(np.full(4500, 88))])
+    w = -rng.uniform(0.01, 0.99, len(u)) * dw
+    u, v, w = with_filler(rng, theta, lam, dw, u, v, w)
+    order = rng.permutation(len(u))
+    u, v, w = u[order], v[order], w[order]
+    stack, _ = orc.wstack_build(theta, lam, l, m, None, du, dw, h["w"].size, h["lm"].x0,
+                                h["lm"].data, h["n"].data)
+    ref, _ = orc.wstack_degrid(stack, g, u, v, w, du, dw, h["uv"].data, h["uv"].size,
+                               h["uv"].oversampling, h["w"].data, h["w"].size,
+                               h["w"].oversampling)
+    p = params(kernels, theta, lam)
+    ctx.wstack_build(p, dev(l), dev(m), None, d["lm"], d["n"])
+    out = torch.full((len(u),), 5.0, dtype=torch.complex128, device="cuda")
+    ctx.wstack_degrid(p, dev(u), dev(v), dev(w), d["uv"], d["w"], out)
+    torch.cuda.synchronize()
+    assert np.abs(out.cpu().numpy() - ref).max() < 1e-10 * np.abs(ref).max()
+    assert ctx.stats().n_dropped == 0
