@@ -79,17 +79,17 @@ __global__ __launch_bounds__(DFT_THREADS) void k_dft_mixed(
 }
 
 // sin and cos of pi t, t given in half turns.  t = q + r with q the nearest
-// integer (adding and taking off 1.5 * 2^52 rounds t, |t| < 2^51, and leaves q
-// in the low mantissa bits) and r exact; both series are Chebyshev fits in r^2
-// over |r| <= 1/2 with 9 terms (error 7e-19 and 4e-18, below the rounding of
-// the result), and q mod 2 is the common sign.  Against libm's sincos of the
-// angle in radians (argument reduction with pi, branches, about 75 instructions)
-// this is 25 instructions without a branch.
+// integer and r exact; both series are Chebyshev fits in r^2 over |r| <= 1/2
+// with 9 terms (errors 7e-19 and 4e-18; 3.1e-17 and 9.8e-17 with the
+// coefficients rounded to FP64), and q mod 2 is the common sign: adding 1.5 * 2^52
+// leaves q in the low mantissa bits for |t| < 2^51.  (From there on t has no digits
+// left below half a turn: any sign will do, but r has to stay the remainder.)  Against
+// libm's sincos of the angle in radians (argument reduction with pi, branches, about 75
+// instructions) this is 25 instructions without a branch.
 __device__ inline void half_turn_sincos(double t, double &s, double &c)
 {
-    constexpr double MAGIC = 6755399441055744.0; // 1.5 * 2^52
-    const double qm = t + MAGIC;
-    const double r = t - (qm - MAGIC);
+    const double qm = t + 6755399441055744.0; // 1.5 * 2^52
+    const double r = t - rint(t);
     const double z = r * r;
     double ps = 7.697826768224191e-07, pc = 4.149564353942586e-06;
     ps = fma(ps, z, -2.1903497074626018e-05);

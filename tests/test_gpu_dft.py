@@ -147,3 +147,31 @@ def test_dft_capture_keeps_its_partial_sums(mode, tol, warm):
     torch.cuda.synchronize()
     assert rel_max(b[4].cpu().numpy(), b[5]) < tol
     c.close()
+
+
+@pytest.mark.parametrize("vdt", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("npix", [300, 5000])
+def test_dft_flagged_samples_far_away(ctx, vdt, npix):
+    """Samples at coordinates far outside any array, whose phases have no digits left below a turn,
+    add nothing if their value is 0 and at most its modulus otherwise.  The bound of the tile test
+    on the rest."""
+    rng = np.random.default_rng(npix)
+    n, N, lam = 2000, 2048, 20480.0
+    u, v = rng.uniform(-3000, 3000, (2, n))
+    w = rng.uniform(-300, 300, n)
+    vis = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(np.complex64).astype(complex)
+    px, py = rng.integers(0, N, (2, npix)).astype(np.int32)
+    far = rng.permutation(n)[:400]
+    vis[far] = 0
+    ref = orc.dft(px, py, N, lam, u, v, w, vis)
+    bound = 1e-12 * np.abs(vis).sum()
+    u[far[:300]] = 10.0 ** rng.uniform(14, 24, 300)
+    v[far[100:]] = -10.0 ** rng.uniform(14, 24, 300)
+    w[far[300:]], u[far[:3]] = 1e22, 1e300
+    for value in (0.0, 1.0):
+        vis[far] = value
+        _, fv = stage(u, v, w, vis, vdt)
+        out = torch.empty(npix, dtype=torch.complex128, device="cuda")
+        ctx.dft(fv, dev(px), dev(py), N, lam, out)
+        torch.cuda.synchronize()
+        assert (np.abs(out.cpu().numpy() - ref) <= bound + value * 400 * (1 + 1e-12)).all()
