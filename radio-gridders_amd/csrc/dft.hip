@@ -46,9 +46,8 @@ __global__ __launch_bounds__(DFT_THREADS) void k_dft_mixed(
     __shared__ double su[DFT_THREADS], sv[DFT_THREADS], sw[DFT_THREADS];
     __shared__ double2 svis[DFT_THREADS];
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double l = 0.0, m = 0.0, nn = 0.0;
-    if (p < npix)
-        dft_pixel<LIST>(px, py, p, N, lambda, l, m, nn);
+    double l, m, nn;
+    dft_pixel<LIST>(px, py, min(p, npix - 1), N, lambda, l, m, nn);
     double re = 0.0, im = 0.0;
     for (int64_t base = v0; base < v1; base += DFT_THREADS) {
         const int nloc = (int)min((int64_t)DFT_THREADS, v1 - base);
