@@ -79,3 +79,36 @@ def test_bands_footprints_and_collisions(ctx, g, S, nb, na, spread):
     mod = orc.epic_grid(np.abs(f).astype(np.complex128), x, y, np.abs(il).astype(np.complex128), g)
     hits = orc.epic_grid(np.ones_like(f, np.complex128), x, y, np.ones((S, S), np.complex128), g)
     assert (np.abs(got - ref) <= (hits.real + 4) * 2.0 ** -23 * mod.real + 1e-30).all()
+
+
+@pytest.mark.parametrize("na", [1, 255, 256, 257, 513])
+@pytest.mark.parametrize("g,S,nb,spread", [(64, 2, 5, 2), (64, 4, 3, 20), (100, 7, 2, 100),
+                                           (70, 64, 1, 30), (300, 2, 2, 310)])
+def test_lists_of_antennas_on_shared_cells(ctx, g, S, nb, na, spread):
+    """Antennas around the 256 that a workgroup lists at a time, within 4 x 4 cells, close together
+    and spread over the grid, footprints up to the largest.  The bound of the test above."""
+    rng = np.random.default_rng(na + S)
+    f = fields(rng, nb, na)
+    x, y = rng.integers(-S, spread - S + 1, (2, nb * na)) + min(S, g // 4)
+    il = (rng.standard_normal((S, S)) + 1j * rng.standard_normal((S, S))).astype(np.complex64)
+    got = run(ctx, f, x, y, il, g)
+    ref = orc.epic_grid(f.astype(np.complex128), x, y, il.astype(np.complex128), g)
+    mod = orc.epic_grid(np.abs(f).astype(np.complex128), x, y, np.abs(il).astype(np.complex128), g)
+    hits = orc.epic_grid(np.ones_like(f, np.complex128), x, y, np.ones((S, S), np.complex128), g)
+    assert (np.abs(got - ref) <= (hits.real + 4) * 2.0 ** -23 * mod.real + 1e-30).all()
+
+
+@pytest.mark.parametrize("g,S,nb,na", [(64, 2, 1, 60_000), (91, 3, 1, 40_001), (256, 1, 2, 90_000),
+                                       (64, 2, 40, 6000), (8, 1, 2, 100)])
+def test_many_antennas_by_bands_and_by_atomics(ctx, g, S, nb, na):
+    """One or two grids of very many antennas (global atomics) and more of them (bands, many lists
+    each).  The bound of the tests above."""
+    rng = np.random.default_rng(na)
+    f = fields(rng, nb, na)
+    x, y = rng.integers(-S, g + 1, (2, nb * na))
+    il = (rng.standard_normal((S, S)) + 1j * rng.standard_normal((S, S))).astype(np.complex64)
+    got = run(ctx, f, x, y, il, g)
+    ref = orc.epic_grid(f.astype(np.complex128), x, y, il.astype(np.complex128), g)
+    mod = orc.epic_grid(np.abs(f).astype(np.complex128), x, y, np.abs(il).astype(np.complex128), g)
+    hits = orc.epic_grid(np.ones_like(f, np.complex128), x, y, np.ones((S, S), np.complex128), g)
+    assert (np.abs(got - ref) <= (hits.real + 4) * 2.0 ** -23 * mod.real + 1e-30).all()
