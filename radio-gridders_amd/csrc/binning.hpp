@@ -373,13 +373,11 @@ inline int64_t bin_stride(int64_t nkeys) { return (nkeys + 1 + 63) / 64 * 64; }
 int bin_plan(int64_t n, int64_t nkeys, uint32_t per_item, int64_t max_counters, size_t rec_bytes,
              BinPlan &pl);
 // The sort into caller-provided arrays of the plan's sizes; timer_ctx (may be
-// NULL) receives the RG_TIMER_BINNING events.  The areas of `zero` are cleared
-// before the sort, in one launch with the counters it needs cleared (`cleared`:
-// those are clear already).
+// NULL) receives the RG_TIMER_BINNING events.  The areas of `zero` are cleared before the
+// sort; the sort's counters (unless bin_small) are among them, or clear already.
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, ZeroList &zero, bool cleared, rg_context *timer_ctx,
-            hipStream_t s, BinResult &out);
+            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s, BinResult &out);
 // Plan and scratch (the context's slots 0-6 and 15, with room for key_room keys) of a
 // sort, and what it needs cleared added to `zero`: for a caller that clears more in the same
 // launch.

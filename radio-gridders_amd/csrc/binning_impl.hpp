@@ -10,8 +10,7 @@ namespace rg {
 
 template <typename Keyer, typename T>
 int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const BinPlan &pl,
-            const BinBufs &b, ZeroList &zero, bool cleared, rg_context *timer_ctx,
-            hipStream_t s, BinResult &out)
+            const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s, BinResult &out)
 {
     const Replicas rp = pl.rp;
     out.vis_start = b.vis_start;
@@ -20,8 +19,6 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
     out.recs = b.recs;
     out.max_items = pl.max_items;
     const bool small = bin_small(n, nkeys);
-    if (!small && !cleared)
-        RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
     RG_TRY(zero.launch(s));
     KernelTimer kt(timer_ctx, RG_TIMER_BINNING, s);
     if (small) {
@@ -49,6 +46,7 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
 
 // context scratch slots of the sort (rg_internal.hpp)
 static const int bin_slot[BIN__N] = {0, 1, 2, 3, 4, 5, 6, 15};
+inline void *bin_buffer(rg_context *ctx, BinArray k) { return ctx->scratch[bin_slot[k]].p; }
 
 template <typename T>
 int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uint32_t per_item,
@@ -99,7 +97,7 @@ int bin_visibilities(rg_context *ctx, const Keyer &kf, int64_t n, int64_t nkeys,
     b.bsums = ctx->scratch[slot[BIN_BSUMS]].as<uint2>();
     b.krp = ctx->scratch[slot[BIN_KRP]].as<uint4>();
     b.stats = ctx->counters.as<unsigned long long>();
-    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, zero, true, ctx, s, out);
+    return bin_run<Keyer, T>(kf, n, nkeys, per_item, pl, b, zero, ctx, s, out);
 }
 
 } // namespace rg

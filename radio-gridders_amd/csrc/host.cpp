@@ -102,7 +102,10 @@ int range_done_counter(rg_context *ctx, uint32_t **done, hipStream_t s)
     *done = reinterpret_cast<uint32_t *>(ctx->counters.as<char>() + COUNTER_BYTES - 64);
     if (!ctx->range_ready) {
         RG_TRY(zero_fill(*done, 64, s));
-        ctx->range_ready = true;
+        // (captured, the clear has not run yet)
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        RG_HIP(hipStreamIsCapturing(s, &cap));
+        ctx->range_ready = cap == hipStreamCaptureStatusNone;
     }
     return RG_OK;
 }

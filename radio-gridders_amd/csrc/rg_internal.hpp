@@ -179,9 +179,10 @@ enum Counter {
     CNT__N = 11
 };
 
-// the counters and, in the last 64 bytes, the word of range_done_counter
-constexpr size_t COUNTER_BYTES = 256;
-static_assert(sizeof(unsigned long long) * CNT__N <= COUNTER_BYTES - 64, "counter space");
+// the counters, the word of a W-projection's planes per group and, 64 bytes on, that of
+// range_done_counter
+constexpr size_t COUNTER_BYTES = 256, COUNTER_PLANES = COUNTER_BYTES - 128;
+static_assert(sizeof(unsigned long long) * CNT__N <= COUNTER_PLANES, "counter space");
 int ensure_counters(rg_context *ctx);
 // a device word that is 0 between launches (behind the counters; cleared on s
 // the first time)

@@ -150,7 +150,8 @@ struct WprojKeyer {
     int N, S, R, P;
     double theta, w_min, w_step;
     int tw, ntx, ntiles;     // columns of positions of a tile; tiles per row and grid
-    int group_planes;        // W-planes per plane group
+    const uint32_t *group_planes; // device: W-planes per plane group; NULL: one group
+    int min_planes;          // of the finest groups, which the keys have room for
     int zb;                  // bytes per kernel tap
     const int64_t *chan_off;
     int nchan;
@@ -168,20 +169,35 @@ struct WprojKeyer {
         return lo;
     }
 
+    // tile of visibility i (at ui, vi) over all grids, its position there; false: off the grid
+    __device__ bool place(int64_t i, double ui, double vi, uint32_t &tile, uint32_t &pos, int &xf,
+                          int &yf) const
+    {
+        int gx, gy;
+        frac_coord(N, S, R, theta, ui, vi, 0.0, 0.0, gx, gy, xf, yf);
+        if (gx <= -S || gx >= N || gy <= -S || gy >= N)
+            return false;
+        const int tx = (gx + S) / tw, ty = (gy + S) / TILE_POS;
+        const int c = nchan > 1 ? chan_of(i) : 0;
+        tile = (uint32_t)(c * ntiles + ty * ntx + tx);
+        pos = (uint32_t)(gx + S - tx * tw) | (uint32_t)(gy + S - ty * TILE_POS) << 16;
+        return true;
+    }
+
     __device__ int classify(int64_t i, uint32_t &key, uint32_t &pos, uint32_t &kidx) const
     {
-        int gx, gy, xf, yf;
-        frac_coord(N, S, R, theta, u[i], v[i], 0.0, 0.0, gx, gy, xf, yf);
-        if (gx <= -S || gx >= N || gy <= -S || gy >= N)
+        int xf, yf;
+        uint32_t tile;
+        if (!place(i, u[i], v[i], tile, pos, xf, yf))
             return VIS_DROPPED;
         const int p = w_plane(w[i], w_min, w_step);
         if (p < 0 || p >= P)
             return VIS_BAD_PLANE;
-        const int tx = (gx + S) / tw, ty = (gy + S) / TILE_POS;
-        const int c = nchan > 1 ? chan_of(i) : 0;
-        key = (uint32_t)((p / group_planes * nchan + c) * ntiles + ty * ntx + tx);
-        // position in the tile; byte offset of the sub-kernel
-        pos = (uint32_t)(gx + S - tx * tw) | (uint32_t)(gy + S - ty * TILE_POS) << 16;
+        key = tile;
+        if (group_planes)
+            key += (uint32_t)p / max(*group_planes, (uint32_t)min_planes) *
+                   (uint32_t)(nchan * ntiles);
+        // byte offset of the sub-kernel
         kidx = (uint32_t)((p * R + yf) * R + xf) * (uint32_t)(S * S * zb);
         return VIS_OK;
     }
@@ -202,11 +218,108 @@ struct WprojKeyer {
     }
 };
 
+// Plane groups.  Sub-kernels are read fastest while the planes in use at a time fit an
+// XCD's L2, so items are ordered by groups of W-planes; but every item adds the cells its
+// records touch to the grid, so a tile whose few records fall into many groups costs more
+// than it saves.  How many records share a tile depends on the stream: tracks crowd the
+// centre (520 k visibilities on 4225 tiles: 123 a tile, 4020 on a record's own), even
+// coverage does not.  A sample of the stream tells, while the call's memory is
+// cleared: pairs of samples on one tile, D records on a record's tile.  As many groups as
+// leave a key 80 of them, an even number (the planes around w = 0, which tracks
+// crowd, lie at a group's end then), at most max_groups, of which each has min_planes planes.
+// Calls, us, in one group / the finest groups / these: 8.4 M tracks, 2048^2, FP32 1694 / 1110 / 1123; 520 k,
+// 1024^2, FP64 248 / 213 / 217; even coverage of 1024^2, 320 planes, FP32, 66 a tile 134 / 354 / 141, 260
+// 407 / 530 / 374, 520 753 / 648 / 529; of 4096^2, 70 a tile 1641 / 5340 / 1660.
+struct PlaneGroups {
+    uint32_t *planes;      // device: the choice, planes per group
+    uint32_t *done;        // device: 0 between launches
+    uint32_t *bin;         // device: [samples]
+    int min_planes;        // of the finest groups
+    int max_groups;
+    int samples;           // 0: one group
+};
+constexpr int SAMPLE_THREADS = 256, SAMPLE_BINS = 8192;
+constexpr double GROUP_RECORDS = 80.0;
+
+__device__ inline uint32_t sample_bin(uint32_t tile)
+{
+    tile = (tile ^ tile >> 16) * 0x9e3779b1u;
+    tile = (tile ^ tile >> 13) * 0x85ebca77u;
+    return (tile ^ tile >> 16) % SAMPLE_BINS;
+}
+
+constexpr uint32_t NO_BIN = 0xffffffffu;
+
+// The first samples / SAMPLE_THREADS workgroups look at a sample a thread (one workgroup's
+// misses alone would take 30 us for 4096) and the last of them to finish chooses the plane groups; the
+// other workgroups clear the areas of z.
+__global__ __launch_bounds__(SAMPLE_THREADS) void k_clear_and_sample(ZeroList z, WprojKeyer kf,
+                                                                     int64_t n, PlaneGroups pg)
+{
+    const unsigned nsb = (unsigned)pg.samples / SAMPLE_THREADS;
+    if (blockIdx.x >= nsb) {
+        z.clear(blockIdx.x - nsb, gridDim.x - nsb);
+        return;
+    }
+    __shared__ __align__(16) uint32_t bins[SAMPLE_BINS];
+    __shared__ double wsum[SAMPLE_THREADS / 64];
+    __shared__ uint32_t s_last;
+    {
+        const int k = (int)(blockIdx.x * SAMPLE_THREADS + threadIdx.x);
+        const int64_t i = (int64_t)(k * ((double)n / pg.samples));
+        uint32_t tile, pos;
+        int xf, yf;
+        const uint32_t bin =
+            kf.place(i, kf.u[i], kf.v[i], tile, pos, xf, yf) ? sample_bin(tile) : NO_BIN;
+        // device-scope exchange; its result is awaited before the workgroup is counted
+        const uint32_t old = __hip_atomic_exchange(&pg.bin[k], bin, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" : : "v"(old) : "memory");
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(pg.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 nsb - 1;
+    for (int k = threadIdx.x; k < SAMPLE_BINS / 4; k += SAMPLE_THREADS)
+        reinterpret_cast<uint4 *>(bins)[k] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    if (!s_last)
+        return;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < pg.samples; k += SAMPLE_THREADS) {
+        const uint32_t bin =
+            __hip_atomic_load(&pg.bin[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (bin < SAMPLE_BINS)
+            atomicAdd(&bins[bin], 1u);
+    }
+    __syncthreads();
+    double pairs = 0.0;
+    for (int k = threadIdx.x; k < SAMPLE_BINS; k += SAMPLE_THREADS)
+        pairs += (double)bins[k] * ((double)bins[k] - 1.0);
+    for (int o = 32; o > 0; o >>= 1)
+        pairs += __shfl_xor(pairs, o);
+    if (__lane_id() == 0)
+        wsum[threadIdx.x / 64] = pairs;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        pairs = 0.0;
+        for (int k = 0; k < SAMPLE_THREADS / 64; ++k)
+            pairs += wsum[k];
+        // less the pairs that only share a bin
+        const double m = pg.samples;
+        const double d = (double)n * (pairs / (m * (m - 1.0)) - 1.0 / SAMPLE_BINS);
+        const int g = d < 2 * GROUP_RECORDS ? 1 : (int)fmin(d / GROUP_RECORDS, 65536.0) / 2 * 2;
+        *pg.planes = (uint32_t)(g >= pg.max_groups ? pg.min_planes : max((kf.P + g - 1) / g, 1));
+        *pg.done = 0;
+    }
+}
+
 // Tile geometry and sort parameters of batched W-projection.
 struct WprojShape {
     int tw, ntx, ntiles;
-    int group_planes; // W-planes per plane group
-    int64_t nkeys;    // plane groups x grids x tiles
+    int min_planes;   // W-planes per plane group at least
+    int max_groups;   // plane groups at most
+    int64_t nkeys;    // max_groups x grids x tiles
     uint32_t per_item;
     // FP32 grids: records of a key whose items add up in FP64 first (0: no key),
     // slots for such keys of this stream, and for any shorter one too
@@ -229,10 +342,39 @@ struct WprojShape {
     }
     void one_group(int planes, int n_chan)
     {
-        group_planes = std::max(planes, 1);
+        min_planes = std::max(planes, 1);
+        max_groups = 1;
         nkeys = (int64_t)ntiles * n_chan;
     }
+    // The choice of plane groups, with words: the word of the planes per group and, 64 bytes
+    // on, the one of finished workgroups; room: space for 16 bytes a record, in use later.  1024 samples up
+    // to 256 k records, 4096 from 1 M (D is then known to 4e-6 n).
+    PlaneGroups groups(char *words, void *room, int64_t nvis) const
+    {
+        PlaneGroups pg{};
+        if (max_groups > 1 && nvis >= SAMPLE_THREADS) {
+            pg.planes = reinterpret_cast<uint32_t *>(words);
+            pg.done = reinterpret_cast<uint32_t *>(words + 64);
+            pg.bin = static_cast<uint32_t *>(room);
+            pg.min_planes = min_planes;
+            pg.max_groups = max_groups;
+            pg.samples = (int)std::min<int64_t>(nvis, std::clamp<int64_t>(nvis / 256, 1024, 4096)) /
+                         SAMPLE_THREADS * SAMPLE_THREADS;
+        }
+        return pg;
+    }
 };
+
+// The call's clears (emptying the list) and the choice of plane groups.
+static int clear_and_sample(ZeroList &zero, const WprojKeyer &kf, int64_t n, const PlaneGroups &pg,
+                            hipStream_t s)
+{
+    const unsigned nb = zero.blocks();
+    hipLaunchKernelGGL(k_clear_and_sample, dim3((unsigned)pg.samples / SAMPLE_THREADS + nb), dim3(SAMPLE_THREADS), 0, s, zero, kf, n, pg);
+    RG_HIP(hipGetLastError());
+    zero.n = 0;
+    return RG_OK;
+}
 
 struct HotSlots {
     double *sums;
@@ -336,36 +478,35 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
     if (S != 8 && S != 16)
         return fail(RG_ERR_UNSUPPORTED, "batched W-projection supports kernel sizes 8 and 16 (got %d)", S);
     sh.tw = TILE_POS;
-    sh.ntx = (p->grid_size + S + TILE_POS - 1) / TILE_POS;
-    sh.ntiles = sh.ntx * sh.ntx;
-    // Plane groups of 2^18 taps (2 MB in FP32, 4 MB in FP64, an XCD's L2) where a tile
-    // has at least 64 records: 8.4 M FP32 1730 us in one group, 1120 in groups of twice the size,
-    // 1040; 520 k FP64 275, 222, 204.  Sparser streams pay more for the extra items than they save:
-    // 16 k on 2000^2 57 us in one group, 93 in groups; 64 channels (16 a tile) 1120, 1415.
+    const int nty = (p->grid_size + S + TILE_POS - 1) / TILE_POS;
+    sh.ntx = nty;
+    sh.ntiles = nty * nty;
+    // The finest plane groups hold 2^18 taps (2 MB in FP32, 4 MB in FP64), of up to 64 groups.
+    // Streams of fewer than 64 records a tile take at most four groups and, on grids beyond 64 MB, whose
+    // cells are no longer added to in L2, tiles twice as wide (S = 8: only these streams; 16 channels of 1024^2, even
+    // coverage, 9 / 30 / 150 records a tile, S = 16: 428 / 775 / 3354 us, wide 375 / 751 / 3148).
     const int64_t plane_taps = (int64_t)wk->oversampling * wk->oversampling * S * S;
     const int64_t planes = std::max<int64_t>(wk->plane_count, 1);
-    const int64_t group = std::max<int64_t>({1, ((int64_t)1 << 18) / std::max<int64_t>(plane_taps, 1),
-                                             (planes + 63) / 64});
-    const int64_t one = (int64_t)sh.ntiles * n_chan, all = (planes + group - 1) / group;
-    sh.one_group(wk->plane_count, n_chan);
-    if (nvis >= 64 * one && all > 1) {
-        sh.group_planes = (int)group;
-        sh.nkeys = one * all;
-    } else if (n_chan > 1 && nvis >= 8 * one) {
-        // many channels of 8 to 64 records a tile: tiles twice as wide, so that the items
-        // stay few (256 channels 5.26 -> 5.15 ms), and, while the counters leave room for two
-        // replicas, groups of four times the planes (64 channels 1125 -> 1057 us; 256 channels, whose
-        // 5.5 M keys leave one replica, 5.50 ms)
+    int64_t group = std::max<int64_t>({1, ((int64_t)1 << 18) / std::max<int64_t>(plane_taps, 1),
+                                       (planes + 63) / 64});
+    int64_t one = (int64_t)sh.ntiles * n_chan;
+    const bool dense = nvis >= 64 * one, sparse = nvis < 8 * one;
+    const bool large = (int64_t)p->grid_size * p->grid_size * n_chan *
+                           (wk->type == RG_C128 ? 16 : 8) > (int64_t)64 << 20;
+    if (large && !sparse && (S == 16 || !dense)) {
         sh.tw = 2 * TILE_POS;
-        const int64_t ntx = (p->grid_size + S + sh.tw - 1) / sh.tw;
-        sh.ntiles = (int)(ntx * sh.ntx);
-        sh.ntx = (int)ntx;
-        sh.one_group(wk->plane_count, n_chan);
-        const int64_t wide = (planes + 4 * group - 1) / (4 * group);
-        if (2 * sh.nkeys * wide <= BIN_MAX_COUNTERS) {
-            sh.group_planes = (int)std::min<int64_t>(4 * group, planes);
-            sh.nkeys *= wide;
-        }
+        sh.ntx = (p->grid_size + S + sh.tw - 1) / sh.tw;
+        sh.ntiles = sh.ntx * nty;
+        one = (int64_t)sh.ntiles * n_chan;
+    }
+    sh.one_group(wk->plane_count, n_chan);
+    if (!dense)
+        group = std::max(group, (planes + 3) / 4);
+    const int64_t all = (planes + group - 1) / group;
+    if (!sparse && all > 1 && (dense || 2 * one * all <= BIN_MAX_COUNTERS)) {
+        sh.min_planes = (int)group;
+        sh.max_groups = (int)all;
+        sh.nkeys = one * all;
     }
     // a key of eight default items or more (the shortest streams have too few items for
     // it to matter)
@@ -380,7 +521,8 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
 }
 
 static WprojKeyer wproj_keyer(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk,
-                              const WprojShape &sh, const int64_t *d_off, int n_chan, int zb)
+                              const WprojShape &sh, const int64_t *d_off, int n_chan, int zb,
+                              const PlaneGroups &pg)
 {
     WprojKeyer kf;
     kf.u = vis->u;
@@ -398,7 +540,8 @@ static WprojKeyer wproj_keyer(const rg_grid_params *p, const rg_flat_vis *vis, c
     kf.tw = sh.tw;
     kf.ntx = sh.ntx;
     kf.ntiles = sh.ntiles;
-    kf.group_planes = sh.group_planes;
+    kf.group_planes = pg.samples ? pg.planes : nullptr;
+    kf.min_planes = pg.min_planes;
     kf.zb = zb;
     kf.chan_off = d_off;
     kf.nchan = n_chan;
@@ -447,8 +590,16 @@ static int wproj_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_fl
     if (rc != RG_OK)
         return rc;
 
-    const WprojKeyer kf =
-        wproj_keyer(p, vis, wk, sh, d_off, n_chan, (int)sizeof(typename Vec2<T>::type));
+    if (sh.max_groups > 1) {
+        uint32_t *done; // the word after COUNTER_PLANES'
+        RG_TRY(range_done_counter(ctx, &done, s));
+    }
+    const PlaneGroups pg = sh.groups(ctx->counters.as<char>() + COUNTER_PLANES,
+                                     bin_buffer(ctx, BIN_KRP), vis->n);
+    const WprojKeyer kf = wproj_keyer(p, vis, wk, sh, d_off, n_chan,
+                                      (int)sizeof(typename Vec2<T>::type), pg);
+    if (pg.samples)
+        RG_TRY(clear_and_sample(zero, kf, vis->n, pg, s));
     BinResult br;
     RG_TRY((bin_visibilities<WprojKeyer, T>(ctx, kf, vis->n, sh.nkeys, room, sh.per_item,
                                             zero, s, br, BIN_MAX_COUNTERS, &pl)));
@@ -511,7 +662,7 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     WprojShape sh;
     RG_TRY(wproj_shape(p, vis->n, 1, wk, sh));
     auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t head = aligned(sizeof(unsigned long long) * CNT__N); // call counters first
+    const size_t head = aligned(COUNTER_BYTES); // call counters first
     // The limit on the stream is that of a sort by tiles of the parameter's 32 or 48
     // cells with separate cursors, items of 2048 records and scan blocks of 1024 keys in
     // NOALLOC_LIMIT_BYTES.
@@ -586,10 +737,15 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
         RG_TRY(zero.add(grid, (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N));
     if (vis->n == 0)
         return zero.launch(s);
+    if (!bin_small(vis->n, sh.nkeys))
+        RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
+    const PlaneGroups pg = sh.groups(b0 + COUNTER_PLANES, b.krp, vis->n);
     const WprojKeyer kf =
-        wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type));
+        wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type), pg);
+    if (pg.samples)
+        RG_TRY(clear_and_sample(zero, kf, vis->n, pg, s));
     BinResult br;
-    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.nkeys, sh.per_item, pl, b, zero, false, nullptr,
+    RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.nkeys, sh.per_item, pl, b, zero, nullptr,
                                    s, br)));
     return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N, 1,
                              sh, hot, s);

@@ -218,6 +218,63 @@ def test_more_keys_than_the_captured_call(table, captured):
     plain.close()
 
 
+def spread(n, N, planes, seed, even):
+    """n visibilities over the grid and past its edges: evenly, or crowded as tracks are (the
+    density falling by e every twentieth of the grid)."""
+    rng = np.random.default_rng(seed)
+    half = N / THETA / 2
+    if even:
+        u, v = rng.uniform(-1.02 * half, 1.02 * half, (2, n))
+    else:
+        r, t = rng.exponential(half / 10, n), rng.uniform(0, 2 * np.pi, n)
+        u, v = r * np.cos(t), r * np.sin(t)
+    return (u, v, rng.uniform(-0.5, planes - 0.4, n),
+            rng.standard_normal(n) + 1j * rng.standard_normal(n))
+
+
+@pytest.mark.parametrize("N,s,per", [(256, 16, 63.9), (256, 16, 64.1), (256, 16, 400), (256, 8, 400),
+                                     (2100, 16, 7.9), (2100, 16, 8.1), (2100, 8, 20), (2100, 16, 64.1),
+                                     (2100, 8, 64.1)])
+def test_plane_groups_by_sample(N, s, per):
+    """Streams of even coverage and crowded ones around 8 and 64 records a tile, grids below and
+    above 64 MB: the number of plane groups comes from a sample of the stream, in the call, so that a
+    captured call serves either.  FP64 sums against the plain form's: at most n products a cell."""
+    planes, r = 300, 8
+    one = ((N + s + 15) // 16) ** 2
+    n = int(per * one)
+    table = torch.randn((planes, r, r, s, s), dtype=torch.complex128, device="cuda")
+    wk = rgamd.wkern_desc(table, 0.0, 1.0)
+    c, plain = rgamd.Context(0), rgamd.Context(0)
+    p, pp = rgamd.params(N, THETA), rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    ref = torch.empty_like(g)
+    streams = [stage(*spread(n, N, planes, 5, even)) for even in (True, False)]
+    (du, dv, dw, dvis), fv = stage(*spread(n, N, planes, 6, True))
+    for keep, f in streams:
+        plain.grid(pp, f, wk, ref)
+        c.grid(p, f, wk, g)
+        assert float((g - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
+        if n <= 700_000:
+            rgamd.grid_noalloc(p, f, wk, g)
+            assert float((g - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        c.grid(p, fv, wk, g)
+    for keep, f in streams * 2:
+        for dst, src in zip((du, dv, dw, dvis), keep):
+            dst.copy_(src)
+        plain.grid(pp, f, wk, ref)
+        g.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((g - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
+    del graph
+    c.close()
+    plain.close()
+
+
 def crowd(n, N, s, planes, seed):
     """n visibilities: half in one 16 x 16 tile of positions (several a position), half over
     the grid and its edges; planes of the whole table."""
