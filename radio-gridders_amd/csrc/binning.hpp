@@ -53,43 +53,75 @@ enum VisStatus { VIS_OK = 0, VIS_DROPPED = 1, VIS_BAD_PLANE = 2, VIS_OVERFLOW = 
 // atomic.  All runs of the wavefront issue their atomics in one instruction
 // and the results are gathered once, so a wavefront costs one atomic round
 // trip whatever its keys (visibility streams are baseline-track ordered, so
-// neighbouring lanes often share keys).  wave_agg_issue returns the atomic's
-// old value (meaningful on head lanes) and the lane's head; wave_agg_rank
-// turns them into the lane's rank.  Splitting the two lets a thread keep
-// several atomics in flight.  Must be called by the whole wavefront in
+// neighbouring lanes often share keys).  Where the runs are short, lanes of one key wherever
+// they stand are gathered first, a few keys at a time: a crowded tile's records that alternate
+// between plane groups or tiles would otherwise meet on a few counters one by one (3 M records
+// of 4 tiles and 2 groups in random order: a call of 1104 us with runs alone, 527 us so; from the first
+// key of a single lane on the rest stays as it is, so that streams of many keys pay for one look).
+// wave_agg_issue returns the atomic's old value (meaningful on head lanes), the lane's head and
+// its place among the head's; wave_agg_rank turns them into the lane's rank.  Splitting the
+// two lets a thread keep several atomics in flight.  Must be called by the whole wavefront in
 // uniform control flow.
+struct AggPlace {
+    int head, off;
+};
+constexpr int AGG_RUNS = 16; // runs of a wavefront that are short
+constexpr int AGG_SAME = 2;  // lanes of one key worth gathering
+
 __device__ inline uint32_t wave_agg_issue(uint32_t *counters, uint32_t key, bool active,
-                                          int &my_head)
+                                          AggPlace &place)
 {
     const int lane = __lane_id();
-    const unsigned long long act = __ballot(active);
+    const unsigned long long below = (1ull << lane) - 1ull;
     const uint32_t prev = (uint32_t)__shfl_up((int)key, 1);
-    const bool head = active && (lane == 0 || !((act >> (lane - 1)) & 1ull) || prev != key);
-    const unsigned long long heads = __ballot(head);
-    const unsigned long long ends = heads | ~act; // a run stops at the next head or idle lane
+    unsigned long long act = __ballot(active);
+    auto run_heads = [&]() {
+        return __ballot(((act >> lane) & 1ull) &&
+                        (lane == 0 || !((act >> (lane - 1)) & 1ull) || prev != key));
+    };
+    unsigned long long heads = run_heads();
+    unsigned long long mine = 0; // gathered: the lanes of this lane's key
+    if (__popcll(heads) > AGG_RUNS) {
+        for (unsigned long long left = act; left;) {
+            const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)key, __ffsll((long long)left) - 1);
+            const unsigned long long same = __ballot(key == k) & left;
+            if (__popcll(same) < AGG_SAME)
+                break;
+            if (key == k)
+                mine = same;
+            left &= ~same;
+            act &= ~same;
+        }
+        mine = active ? mine : 0;
+        heads = run_heads();
+    }
     uint32_t base = 0;
-    if (head) {
+    const bool leader = mine && !(mine & below);
+    if (leader || ((heads >> lane) & 1ull)) {
+        const unsigned long long ends = heads | ~act; // a run stops at the next head or idle lane
         const unsigned long long nxt = lane == 63 ? 0ull : (ends >> (lane + 1));
-        const uint32_t len = nxt ? (uint32_t)__ffsll((long long)nxt) : (uint32_t)(64 - lane);
+        const uint32_t len = leader ? (uint32_t)__popcll(mine)
+                             : nxt  ? (uint32_t)__ffsll((long long)nxt)
+                                    : (uint32_t)(64 - lane);
         base = atomicAdd(&counters[key], len);
     }
-    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-    const unsigned long long hm = heads & upto;
-    my_head = hm ? 63 - __clzll((long long)hm) : 0;
+    const unsigned long long hm = heads & (below | 1ull << lane);
+    place.head = mine ? __ffsll((long long)mine) - 1 : hm ? 63 - __clzll((long long)hm) : 0;
+    place.off = mine ? __popcll(mine & below) : lane - place.head;
     return base;
 }
 
-__device__ inline uint32_t wave_agg_rank(uint32_t base, int my_head)
+__device__ inline uint32_t wave_agg_rank(uint32_t base, const AggPlace &place)
 {
-    return (uint32_t)__shfl((int)base, my_head) + (uint32_t)(__lane_id() - my_head);
+    return (uint32_t)__shfl((int)base, place.head) + (uint32_t)place.off;
 }
 
 // Both steps; the rank only when `want` (uniform) is set.
 __device__ inline uint32_t wave_agg_add(uint32_t *counters, uint32_t key, bool active, bool want)
 {
-    int my_head;
-    const uint32_t base = wave_agg_issue(counters, key, active, my_head);
-    return want ? wave_agg_rank(base, my_head) : 0u;
+    AggPlace place;
+    const uint32_t base = wave_agg_issue(counters, key, active, place);
+    return want ? wave_agg_rank(base, place) : 0u;
 }
 
 // counters of a sort in all, at most (unless its keys are more)
@@ -121,7 +153,8 @@ __global__ __launch_bounds__(BIN_TB) void k_bin_count(Keyer kf, int64_t n, uint3
     const int64_t i0 = (int64_t)blockIdx.x * BIN_CHUNK + threadIdx.x;
     uint32_t *cnt = count + (blockIdx.x & rp.mask) * rp.stride;
     uint32_t key[BIN_VPT], pos[BIN_VPT], kidx[BIN_VPT], base[BIN_VPT];
-    int st[BIN_VPT], head[BIN_VPT];
+    int st[BIN_VPT];
+    AggPlace place[BIN_VPT];
 #pragma unroll
     for (int q = 0; q < BIN_VPT; ++q) {
         const int64_t i = i0 + q * BIN_TB;
@@ -131,13 +164,13 @@ __global__ __launch_bounds__(BIN_TB) void k_bin_count(Keyer kf, int64_t n, uint3
     // every atomic in flight before the first result is used
 #pragma unroll
     for (int q = 0; q < BIN_VPT; ++q)
-        base[q] = wave_agg_issue(cnt, key[q], i0 + q * BIN_TB < n && st[q] == VIS_OK, head[q]);
+        base[q] = wave_agg_issue(cnt, key[q], i0 + q * BIN_TB < n && st[q] == VIS_OK, place[q]);
     uint32_t dropped = 0, badp = 0, over = 0;
 #pragma unroll
     for (int q = 0; q < BIN_VPT; ++q) {
         const int64_t i = i0 + q * BIN_TB;
         const bool in = i < n, ok = in && st[q] == VIS_OK;
-        const uint32_t rank = wave_agg_rank(base[q], head[q]);
+        const uint32_t rank = wave_agg_rank(base[q], place[q]);
         if (in)
             krp[i] = make_uint4(ok ? key[q] : KEY_NONE, rank, pos[q], kidx[q]);
         // per-wave status counts

@@ -218,6 +218,32 @@ def test_more_keys_than_the_captured_call(table, captured):
     plain.close()
 
 
+@pytest.mark.parametrize("tiles", [1, 2, 5, 30, 64])
+@pytest.mark.parametrize("n", [5000, 70_001])
+def test_few_keys_in_any_order(ctx, tiles, n):
+    """Records that alternate between a few keys (tiles, and plane groups from 64 a tile on), some
+    dropped, so that the lanes of a key stand apart in their wavefront: keys with one lane, two and many.
+    FP64 against the plain form, W-projection and W-towers."""
+    N, s, planes, r = 256, 8, 140, 8
+    rng = np.random.default_rng(tiles)
+    pick = rng.choice(tiles, n, p=1.0 / np.arange(1, tiles + 1) / (1.0 / np.arange(1, tiles + 1)).sum())
+    place = rng.uniform(-110, 110, (2, tiles))
+    u, v = (place[:, pick] + rng.uniform(0, 4, (2, n))) / THETA
+    u[rng.integers(0, n, n // 50)] = 1e6
+    w = rng.uniform(-0.4, planes - 0.6, n)
+    vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    t = rng.standard_normal((planes, r, r, s, s)) + 1j * rng.standard_normal((planes, r, r, s, s))
+    _, fv = stage(u, v, w, vis)
+    _, wk = kern(t, 0.0, 1.0)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    ref = torch.empty_like(g)
+    for kw in ({}, dict(subgrid=64, margin=16, winc=200.0)):
+        ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN, **kw), fv, wk, ref)
+        for _ in range(2):
+            ctx.grid(rgamd.params(N, THETA, **kw), fv, wk, g)
+            assert float((g - ref).abs().max()) <= 1e-11 * float(ref.abs().max())
+
+
 def spread(n, N, planes, seed, even):
     """n visibilities over the grid and past its edges: evenly, or crowded as tracks are (the
     density falling by e every twentieth of the grid)."""
