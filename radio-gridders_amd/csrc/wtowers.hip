@@ -2168,19 +2168,23 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     // taps are addressed by 32-bit byte offsets
     const int64_t nsub = (int64_t)wk->plane_count * wk->oversampling * wk->oversampling;
     const int64_t krows = padded_taps<T>() ? (int64_t)H + nsub * padded_rows(S, H) : nsub * S;
-    // two band rows per lane (k_tower_band_items): S = 16 and 8-row bands, while
-    // the table of pairs stays below the 2 GiB that offsets reach; compensated sums
-    // do four times the arithmetic a tap, which half the wavefronts hide worse (7.8 M
-    // visibilities 2623 us a row a lane, 2885 us in pairs; uncompensated 2321 and 2269)
-    const bool pairs_fit = padded_taps<T>() && S == 16 && H == 8 &&
-                           2 * krows * S * (int64_t)sizeof(T2) < ((int64_t)1 << 31);
-    const bool pair = pairs_fit && !p->compensated;
-    const int tap_bytes = (int)sizeof(T2) * (pair ? 2 : 1);
-    const int64_t kbytes = krows * S * (int64_t)tap_bytes;
+    // Two band rows per lane (k_tower_band_items): S = 16 and 8-row bands, streams of 4 M and
+    // more, whose calls the band pass decides (2.1 M, 256^2 subgrids: 1730 us a row a lane, 1751 in pairs; 116 k 287 /
+    // 297), and tables of pairs of up to 6 MB: twice the plain table, they outgrow an XCD's L2 sooner (8.4
+    // M, 512^2 subgrids, 4.3 MB of pairs 3509 / 3300 us, 6.3 MB 3463 / 3458, 8.3 MB 3477 / 3780, 17 MB 3828 / 4618).
+    // Compensated sums do four times the arithmetic a tap, which half the wavefronts hide worse
+    // (7.8 M: band pass 2623 us a row a lane, 2885 in pairs).
+    const int64_t plain_bytes = krows * S * (int64_t)sizeof(T2);
+    const bool pairs_fit =
+        padded_taps<T>() && S == 16 && H == 8 && 2 * plain_bytes <= (int64_t)6 << 20;
+    bool pair = pairs_fit && !p->compensated && vis->n >= (int64_t)1 << 22;
     PadJob<T2> pad{};
-    if (padded_taps<T>() && kbytes < ((int64_t)1 << 31)) {
-        // (room for a table of pairs beside a captured compensated call)
-        RG_TRY(ctx->scratch[12].ensure((size_t)kbytes * (pairs_fit && !pair ? 2 : 1)));
+    if (padded_taps<T>() && plain_bytes < ((int64_t)1 << 31)) {
+        // room for pairs beside a captured call without; scratch that a captured graph holds may
+        // have none
+        if (pairs_fit && ctx->scratch[12].ensure((size_t)(2 * plain_bytes)) != RG_OK)
+            pair = false;
+        RG_TRY(ctx->scratch[12].ensure((size_t)(plain_bytes * (pair ? 2 : 1))));
         pad.src = (const T2 *)wk->data;
         pad.dst = ctx->scratch[12].as<T2>();
         pad.nsub = nsub;
@@ -2189,6 +2193,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         pad.pair = pair;
         pad.blocks = (unsigned)std::min<int64_t>((krows * S + 255) / 256, 4096);
     }
+    const int tap_bytes = (int)sizeof(T2) * (pair ? 2 : 1);
+    const int64_t kbytes = krows * S * (int64_t)tap_bytes;
 
     // Capacities: tables by the slot count, buffers by the plan (or, measuring,
     // by the counts read back below).  With a plan everything a call clears

@@ -161,3 +161,65 @@ def test_batched_fp32_row_pairs(ctx, sub, n, spread):
     assert ctx.stats().n_gridded == n
     img, img_ref = orc.grid_to_image(g.cpu().numpy()), orc.grid_to_image(ref)
     assert rel_max(img, img_ref) < 1e-5 and rel_rms(img, img_ref) < 1e-5
+
+
+@pytest.fixture(scope="module")
+def outside():
+    """2^22 visibilities outside every tower: with them a stream is long enough for two band rows a
+    lane."""
+    n = 1 << 22
+    return [torch.full((n,), 1e9, dtype=torch.float64, device="cuda") for _ in range(3)] + [
+        torch.ones(n, dtype=torch.complex64, device="cuda")]
+
+
+@pytest.mark.parametrize("sub", [64, 128, 256, 512])
+@pytest.mark.parametrize("n,spread,planes", [(1, 1.0, 11), (9, 20.0, 11), (129, 30.0, 11), (257, 200.0, 11),
+                                             (600, 3.0, 11), (600, 30.0, 121)])
+def test_long_streams_by_row_pairs(ctx, outside, sub, n, spread, planes):
+    """The streams and the bound of the test above, in calls long enough for row pairs; a table too
+    large for pairs (121 planes at R = 4: 12 MB)."""
+    N, theta = sub, 0.1
+    rng = np.random.default_rng(sub + n)
+    u = 40.0 + rng.uniform(-spread, spread, n)
+    v = -30.0 + rng.uniform(-spread, spread, n)
+    w = rng.uniform(-14.0, 14.0, n)
+    vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    step = 10.0 / (planes - 1)
+    table = rgamd.make_wkernels(planes, 4, 16, theta, -5.0, step)
+    ref, _, bad = orc.grid_wtowers(N, theta, u, v, w, vis, table, -5.0, step, sub, MARGIN, WINC)
+    assert bad == 0
+    few, _ = stage(u, v, w, vis, torch.complex64)
+    keep = [torch.cat([o[:(1 << 21) + 7], f, o[(1 << 21) + 7:]]) for f, o in zip(few, outside)]
+    _, wk = kern(table, -5.0, step, torch.complex64)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    ctx.grid(rgamd.params(N, theta, subgrid=sub, margin=MARGIN, winc=WINC), rgamd.flat_vis(*keep),
+             wk, g)
+    assert ctx.stats().n_gridded == n
+    img, img_ref = orc.grid_to_image(g.cpu().numpy()), orc.grid_to_image(ref)
+    assert rel_max(img, img_ref) < 1e-5 and rel_rms(img, img_ref) < 1e-5
+
+
+def test_row_pairs_and_single_rows_agree(ctx):
+    """A dense stream of 2^22 visibilities (row pairs) and of one less (a row a lane), both in FP32,
+    against FP64: the same products and sums, so neither is further off by more than a half."""
+    N, theta, sub, n = 1024, 0.1, 256, 1 << 22
+    rng = np.random.default_rng(2)
+    u, v = rng.uniform(-4000, 4000, (2, n))
+    w = rng.uniform(-24.0, 24.0, n)
+    vis = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    vis[-1] = 0
+    vis = vis.astype(np.complex64)
+    table = rgamd.make_wkernels(11, 8, 16, theta, -5.0, 1.0).astype(np.complex64)
+    p = rgamd.params(N, theta, subgrid=sub, margin=MARGIN, winc=WINC)
+    keep, f64 = stage(u, v, w, vis.astype(np.complex128))
+    _, k64 = kern(table.astype(np.complex128), -5.0, 1.0)
+    ref = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    ctx.grid(p, f64, k64, ref)
+    _, k32 = kern(table, -5.0, 1.0, torch.complex64)
+    v32 = keep[3].to(torch.complex64)
+    err = []
+    for m in (n, n - 1):
+        g = torch.empty_like(ref)
+        ctx.grid(p, rgamd.flat_vis(keep[0][:m], keep[1][:m], keep[2][:m], v32[:m]), k32, g)
+        err.append(float((g - ref).norm() / ref.norm()))
+    assert err[0] <= 1.5 * err[1] and err[1] <= 1.5 * err[0] and max(err) < 1e-5, err
