@@ -413,10 +413,10 @@ int bin_run(const Keyer &kf, int64_t n, int64_t nkeys, uint32_t per_item, const 
             const BinBufs &b, ZeroList &zero, rg_context *timer_ctx, hipStream_t s, BinResult &out);
 // Plan and scratch (the context's slots 0-6 and 15, with room for key_room keys) of a
 // sort, and what it needs cleared added to `zero`: for a caller that clears more in the same
-// launch.
+// launch, or needs room for min_items items.
 template <typename T>
 int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uint32_t per_item,
-                int64_t max_counters, ZeroList &zero, BinPlan &pl);
+                int64_t max_counters, ZeroList &zero, BinPlan &pl, int64_t min_items = 0);
 // Keys of a W-projection of n_chan N^2 grids by the narrowest tiles, in one plane group: every
 // gridding call makes room for them, so that a context whose scratch a captured graph
 // of any gridder holds takes a W-projection of its grids.

@@ -50,7 +50,7 @@ inline void *bin_buffer(rg_context *ctx, BinArray k) { return ctx->scratch[bin_s
 
 template <typename T>
 int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uint32_t per_item,
-                int64_t max_counters, ZeroList &zero, BinPlan &pl)
+                int64_t max_counters, ZeroList &zero, BinPlan &pl, int64_t min_items)
 {
     RG_TRY(bin_plan(n, nkeys, per_item, max_counters, sizeof(Rec<T>), pl));
     RG_TRY(ensure_counters(ctx));
@@ -58,19 +58,25 @@ int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uin
     // and keys, whatever item size it picks (scratch that a captured graph holds
     // cannot grow; a shorter stream's smaller items are at most 24 times 512);
     // counters likewise: fewer keys, or another gridder's, may take more replicas
-    key_room = std::max(key_room, nkeys);
-    const int64_t stride = bin_stride(key_room);
-    const int64_t items = key_room + std::max<int64_t>({n / per_item, 12288, n / 512}) + 1;
+    auto counters = [](int64_t keys, int64_t most) {
+        const int64_t stride = bin_stride(keys);
+        return sizeof(uint32_t) * (size_t)std::max(stride, std::min(16 * stride, most));
+    };
     const size_t count_bytes = pl.bytes[BIN_COUNT];
     for (int k : {BIN_COUNT, BIN_CURSOR})
-        pl.bytes[k] = sizeof(uint32_t) *
-                      (size_t)std::max(stride, std::min(16 * stride, BIN_MAX_COUNTERS));
+        pl.bytes[k] =
+            std::max(counters(nkeys, max_counters), counters(key_room, BIN_MAX_COUNTERS));
+    key_room = std::max(key_room, nkeys);
+    const int64_t items = std::max(
+        min_items, key_room + std::max<int64_t>({n / per_item, 12288, n / 512}) + 1);
     for (int k : {BIN_VIS_START, BIN_ITEM_START})
         pl.bytes[k] = sizeof(uint32_t) * (size_t)(key_room + 1);
     pl.bytes[BIN_ITEMS] = sizeof(Item) * (size_t)items;
     pl.bytes[BIN_BSUMS] = scan_sums_bytes(key_room);
+    DevBuf *buf[BIN__N];
     for (int k = 0; k < BIN__N; ++k)
-        RG_TRY(ctx->scratch[bin_slot[k]].ensure(pl.bytes[k]));
+        buf[k] = &ctx->scratch[bin_slot[k]];
+    RG_TRY(ensure_together(buf, pl.bytes, BIN__N));
     if (!bin_small(n, nkeys))
         RG_TRY(zero.add(ctx->scratch[bin_slot[BIN_COUNT]].p, count_bytes));
     return RG_OK;

@@ -61,10 +61,46 @@ int DevBuf::ensure(size_t n)
 
 void DevBuf::release()
 {
-    if (p)
+    if (block)
+        block.reset();
+    else if (p)
         (void)hipFree(p);
     p = nullptr;
     bytes = 0;
+}
+
+int ensure_together(DevBuf *const *buf, const size_t *n, int count)
+{
+    auto part = [&](int k) {
+        const bool grows = !buf[k]->p || n[k] > buf[k]->bytes;
+        return grows && n[k] <= TOGETHER_BYTES && !(buf[k]->frozen && *buf[k]->frozen);
+    };
+    auto padded = [&](int k) { return (std::max<size_t>(n[k], 1) + 255) / 256 * 256; };
+    size_t total = 0;
+    for (int k = 0; k < count; ++k)
+        if (part(k)) {
+            buf[k]->release();
+            total += padded(k);
+        }
+    std::shared_ptr<void> block;
+    if (total) {
+        void *p = nullptr;
+        hipError_t e = hipMalloc(&p, total);
+        if (e != hipSuccess)
+            return fail(RG_ERR_NOMEM, "hipMalloc(%zu) failed: %s", total, hipGetErrorString(e));
+        block.reset(p, [](void *q) { (void)hipFree(q); });
+    }
+    char *at = static_cast<char *>(block.get());
+    for (int k = 0; k < count; ++k)
+        if (part(k)) {
+            buf[k]->block = block;
+            buf[k]->p = at;
+            buf[k]->bytes = padded(k);
+            at += padded(k);
+        } else {
+            RG_TRY(buf[k]->ensure(n[k]));
+        }
+    return RG_OK;
 }
 
 int PinnedBuf::ensure(size_t n)

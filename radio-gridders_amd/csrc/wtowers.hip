@@ -2223,7 +2223,7 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
                            (ntasks_cap + q - 1) / q);
     };
     const int64_t key_room = wproj_key_room(g.N, nchan);
-    const BinPlan *ready = nullptr;
+    constexpr uint32_t KEY_ITEM = 0x40000000u;
     BinPlan bin;
     if (!measure) {
         const TableLayout tl = table_layout();
@@ -2231,9 +2231,8 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         const int q = batch_tasks_of(ntasks_cap);
         RG_TRY(clear_subimages((ntasks_cap + q - 1) / q,
                                ctx->scratch[18].as<uint32_t>() + tl.o_spill));
-        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, key_room, 0x40000000u,
+        RG_TRY((bin_prepare<T>(ctx, vis->n, g.ntw * nwp_cap * NB, key_room, KEY_ITEM,
                                wt_counters(vis->n), zero, bin)));
-        ready = &bin;
     }
     RG_TRY(wt_prepare<T2>(ctx, p, vis, g, d_range, &pad, zero, s));
     if (measure) {
@@ -2262,17 +2261,21 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
         return fail(RG_ERR_PARAM, "W-towers key space too large (%lld keys: %lld towers x %d "
                     "floors x %d bands)", (long long)nkeys, (long long)g.ntw, nwp_cap, NB);
     // the sort makes one item per key; band work items of at most K records
-    // per band window are built after it
+    // per band window are built after it, in the same array
     const int64_t max_items_w = nkeys + (int64_t)g.mk * vis->n / K + 1;
-    RG_TRY(ctx->scratch[4].ensure(sizeof(Item) * std::max<int64_t>(nkeys + 1, max_items_w)));
+    if (measure)
+        RG_TRY((bin_prepare<T>(ctx, vis->n, nkeys, key_room, KEY_ITEM, wt_counters(vis->n), zero,
+                               bin, max_items_w)));
+    else
+        RG_TRY(ctx->scratch[4].ensure(sizeof(Item) * max_items_w));
     const TowerKeyer kf = wt_keyer(p, vis, wk, g, d_range, nwp_cap, d_off);
     BinResult br;
     RG_TRY(ctx->scratch[9].ensure(sizeof(uint32_t) * (nslots + 1)));
     uint32_t *slot_start = ctx->scratch[9].as<uint32_t>();
     br.group_start = slot_start;
     br.group_keys = NB;
-    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, key_room, 0x40000000u, zero, s,
-                                            br, wt_counters(vis->n), ready)));
+    RG_TRY((bin_visibilities<TowerKeyer, T>(ctx, kf, vis->n, nkeys, key_room, KEY_ITEM, zero, s, br,
+                                            wt_counters(vis->n), &bin)));
 
     if (measure) {
         ntasks_cap = (int)std::min<int64_t>(nslots, 0x7fffffff);

@@ -222,3 +222,28 @@ def test_channels_graph_replay(own_ctx, channels):
         assert rel_max(got[3], refs[3]) < 1e-11, rep
     del graph
     own_ctx.thaw()
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2, 3), (3, 1, 2, 0), (1, 3, 0, 2)])
+def test_scratch_grows_in_parts(own_ctx, case, order):
+    """Calls of one context whose scratch arrays outgrow each other: some get new memory, others
+    stay in the allocation that they had together."""
+    obs, vis, table, ref = case
+    calls = []
+    for k in (1, 8):  # few and all visibilities, by W-towers and by W-projection
+        m = len(obs.u) // 8 * k
+        u, v, w, d = (x[:m] for x in (obs.u, obs.v, obs.w, vis))
+        wt = ref if k == 8 else orc.grid_wtowers(obs.grid_size, obs.theta, u, v, w, d, table,
+                                                 -5.0, 1.0, SUB, MARGIN, WINC, nthreads=8)[0]
+        calls.append((params(obs), u, v, w, d, wt))
+        wp = orc.grid_wprojection(obs.grid_size, obs.theta, u, v, w, d, table, -5.0, 1.0)[0]
+        calls.append((rgamd.params(obs.grid_size, obs.theta, mode=rgamd.RG_MODE_BATCHED), u, v, w,
+                      d, wp))
+    _, wk = kern(table, -5.0, 1.0)
+    g = torch.empty((obs.grid_size,) * 2, dtype=torch.complex128, device="cuda")
+    for k in order + order:
+        p, u, v, w, d, want = calls[k]
+        _, fv = stage(u, v, w, d)
+        own_ctx.grid(p, fv, wk, g)
+        torch.cuda.synchronize()
+        assert rel_max(g.cpu().numpy(), want) < 1e-11
