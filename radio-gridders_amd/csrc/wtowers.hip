@@ -2105,13 +2105,15 @@ static uint32_t default_band_item(int64_t nvis)
     return nvis < (1 << 20) ? 1024u : nvis < (1 << 21) ? 2048u : 4096u;
 }
 
+// (an item size by number fits the plan that has it, however chosen; an automatic one fits an
+// automatic plan, and in a call that cannot plan anew any)
 static bool plan_fits(const WtPlan &pl, const rg_grid_params *p, const rg_flat_vis *vis,
-                      const rg_wkern *wk, int nchan, int H, int type)
+                      const rg_wkern *wk, int nchan, int H, int type, bool capturing)
 {
     return pl.valid && pl.N == p->grid_size && pl.n == p->subgrid_size &&
            pl.M == p->subgrid_margin && pl.S == wk->size && pl.R == wk->oversampling &&
            pl.P == wk->plane_count && pl.H == H && pl.type == type && pl.nchan == nchan &&
-           (p->vis_per_item > 0 ? !pl.k_auto && pl.K == (uint32_t)p->vis_per_item : pl.k_auto) &&
+           (p->vis_per_item > 0 ? pl.K == (uint32_t)p->vis_per_item : pl.k_auto || capturing) &&
            pl.floor_batch == p->floor_batch && pl.theta == p->theta && pl.winc == p->winc &&
            pl.w_min == wk->w_min && pl.w_step == wk->w_step && vis->n <= pl.nvis;
 }
@@ -2518,7 +2520,7 @@ static int wtowers_batched(rg_context *ctx, const rg_grid_params *p, const rg_fl
 {
     const int H = band_height_of(p, sizeof(T) == 4);
     const int type = sizeof(T) == 4 ? RG_C64 : RG_C128;
-    const bool fits = plan_fits(ctx->wt_plan, p, vis, wk, nchan, H, type);
+    const bool fits = plan_fits(ctx->wt_plan, p, vis, wk, nchan, H, type, capturing);
     if (capturing) {
         if (!fits)
             return fail(RG_ERR_PARAM,

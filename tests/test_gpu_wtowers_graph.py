@@ -247,3 +247,24 @@ def test_scratch_grows_in_parts(own_ctx, case, order):
         own_ctx.grid(p, fv, wk, g)
         torch.cuda.synchronize()
         assert rel_max(g.cpu().numpy(), want) < 1e-11
+
+
+@pytest.mark.parametrize("warm,captured", [(0, 1024), (2048, 0), (500, 0), (500, 500)])
+def test_plans_by_number_and_automatic(own_ctx, case, warm, captured):
+    """A plan made with an automatic item size (1024 for a stream of this length) serves a captured
+    call that asks for that size by number, and a plan by number a captured automatic call."""
+    obs, vis, table, ref = case
+    _, fv = stage(obs.u, obs.v, obs.w, vis)
+    _, wk = kern(table, -5.0, 1.0)
+    g = torch.empty((obs.grid_size,) * 2, dtype=torch.complex128, device="cuda")
+    own_ctx.grid(params(obs, vis_per_item=warm), fv, wk, g)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        own_ctx.grid(params(obs, vis_per_item=captured), fv, wk, g)
+    for _ in range(3):
+        g.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_max(g.cpu().numpy(), ref) < 1e-11
+    del graph
