@@ -196,7 +196,7 @@ int rg_grid_channels(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis
  * serving loops, harnesses that forbid hipMalloc.  Same parameters and result
  * as rg_grid with RG_MODE_BATCHED and subgrid_size 0 (FP32 or FP64 kernels),
  * on the current HIP device, with no context: the sort's working memory is a
- * 192 MiB device array inside librg (one per device, held until the process
+ * 64 MiB device array inside librg (one per device, held until the process
  * ends), enough for about 2.0 M visibilities (FP32 kernels) or 1.4 M (FP64)
  * per call on a 2048^2 grid; a call that needs more returns RG_ERR_PARAM.
  * accumulate = 0 zeroes the grid first (as rg_grid), 1 adds into it, so a

@@ -50,6 +50,7 @@ struct TileSink {
     int tw;     // columns of positions of a tile
     int ntiles; // tiles per group
     int groups; // target arrays
+    uint32_t key0; // tile of key 0
     // FP32 arrays: keys of at least hot_min records (0: none) add their items up in FP64
     // slots of tile_slot() numbers, which k_hot_tiles then adds to the arrays
     uint32_t hot_min;
@@ -67,7 +68,7 @@ struct TilePlace {
     int ox, oy;
     __device__ TilePlace(const TileSink &sink, uint32_t key, int S)
     {
-        const uint32_t gt = key % (uint32_t)(sink.ntiles * sink.groups);
+        const uint32_t gt = (key + sink.key0) % (uint32_t)(sink.ntiles * sink.groups);
         group = gt / (uint32_t)sink.ntiles;
         const int tile = (int)(gt - group * (uint32_t)sink.ntiles);
         ox = tile % sink.ntx * sink.tw - S;

@@ -218,6 +218,20 @@ struct WprojKeyer {
     }
 };
 
+// The keys [key0, key0 + count) of a grid whose keys are too many to sort at once.
+struct StripKeyer : WprojKeyer {
+    uint32_t key0, count;
+
+    __device__ int classify(int64_t i, uint32_t &key, uint32_t &pos, uint32_t &kidx) const
+    {
+        const int r = WprojKeyer::classify(i, key, pos, kidx);
+        if (r != VIS_OK)
+            return r;
+        key -= key0;
+        return key < count ? VIS_OK : VIS_DROPPED;
+    }
+};
+
 // Plane groups.  Sub-kernels are read fastest while the planes in use at a time fit an
 // XCD's L2, so items are ordered by groups of W-planes; but every item adds the cells its
 // records touch to the grid, so a tile whose few records fall into many groups costs more
@@ -320,6 +334,7 @@ struct WprojShape {
     int min_planes;   // W-planes per plane group at least
     int max_groups;   // plane groups at most
     int64_t nkeys;    // max_groups x grids x tiles
+    uint32_t key0 = 0; // tile of the sort's key 0 (strips)
     uint32_t per_item;
     // FP32 grids: records of a key whose items add up in FP64 first (0: no key),
     // slots for such keys of this stream, and for any shorter one too
@@ -332,6 +347,12 @@ struct WprojShape {
     size_t hot_bytes(int S, int64_t slots) const
     {
         return slots * sizeof(double) * (size_t)tile_slot(S, tw);
+    }
+    void wide(int N, int S)
+    {
+        tw = 2 * TILE_POS;
+        ntx = (N + S + tw - 1) / tw;
+        ntiles = ntx * ((N + S + TILE_POS - 1) / TILE_POS);
     }
     // no room for the slots
     void cold()
@@ -388,6 +409,7 @@ static int launch_tiles(const BinResult &br, rg_context *timer_ctx,
 {
     TileSink sink;
     sink.hot_min = sizeof(GT) == 4 ? sh.hot_min : 0;
+    sink.key0 = sh.key0;
     sink.key_start = br.vis_start;
     sink.hot = hot.sums;
     sink.hot_key = hot.key;
@@ -494,9 +516,7 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
     const bool large = (int64_t)p->grid_size * p->grid_size * n_chan *
                            (wk->type == RG_C128 ? 16 : 8) > (int64_t)64 << 20;
     if (large && !sparse && (S == 16 || !dense)) {
-        sh.tw = 2 * TILE_POS;
-        sh.ntx = (p->grid_size + S + sh.tw - 1) / sh.tw;
-        sh.ntiles = sh.ntx * nty;
+        sh.wide(p->grid_size, S);
         one = (int64_t)sh.ntiles * n_chan;
     }
     sh.one_group(wk->plane_count, n_chan);
@@ -623,10 +643,9 @@ int wproj_batched(rg_context *ctx, const rg_grid_params *p, const rg_flat_vis *v
 // device address on the current device comes from hipGetSymbolAddress, looked
 // up once per device and kept.  Calls on one device share the array, so calls
 // that overlap in time on one device (several streams or host threads) race.
-// NOALLOC_LIMIT_BYTES bounds the stream (about 2.0 M visibilities with FP32 kernels,
-// 1.4 M with FP64 at 2048^2); the rest is room for the finer tiles' keys up to 36 000^2 grids.
-constexpr size_t NOALLOC_LIMIT_BYTES = (size_t)64 << 20;
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)192 << 20;
+// (A device array is set up with the library's first kernel, which takes 27 ms with
+// 64 MiB and 78 ms with 192 MiB.)
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -652,7 +671,7 @@ static int noalloc_scratch(void **out)
     return RG_OK;
 }
 
-size_t noalloc_scratch_bytes() { return NOALLOC_LIMIT_BYTES; }
+size_t noalloc_scratch_bytes() { return NOALLOC_SCRATCH_BYTES; }
 
 template <typename T>
 static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk,
@@ -664,8 +683,8 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t head = aligned(COUNTER_BYTES); // call counters first
     // The limit on the stream is that of a sort by tiles of the parameter's 32 or 48
-    // cells with separate cursors, items of 2048 records and scan blocks of 1024 keys in
-    // NOALLOC_LIMIT_BYTES.
+    // cells with separate cursors, items of 2048 records and scan blocks of 1024 keys:
+    // about 2.0 M visibilities with FP32 kernels, 1.4 M with FP64 at 2048^2.
     BinPlan pl;
     const uint32_t limit_item = p->vis_per_item > 0 ? (uint32_t)p->vis_per_item : 2048u;
     const int64_t lt = p->tile > 0 ? p->tile : 32, ln = (N + wk->size + lt - 1) / lt, lk = ln * ln;
@@ -674,13 +693,21 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     for (int k = 0; k < BIN__N; ++k)
         want += aligned(k == BIN_BSUMS ? sizeof(uint2) * (size_t)((lk + 1023) / 1024 + 1)
                                        : pl.bytes[k]);
+    if (want > NOALLOC_SCRATCH_BYTES)
+        return fail(RG_ERR_PARAM,
+                    "rg_grid_noalloc: %lld visibilities on a %d^2 grid need %zu bytes of scratch; "
+                    "the static scratch holds %zu: split the stream over calls with accumulate = 1",
+                    (long long)vis->n, N, want, NOALLOC_SCRATCH_BYTES);
+    if (grid_type != RG_C64) {
+        sh.hot_min = 0;
+        sh.hot_slots = 0;
+    }
     // Carve the arrays from the static scratch, 256-byte aligned.  The scatter
     // cursors take the place of the counters they are made from.
-    size_t off[BIN__N];
-    size_t at = 0;
+    size_t off[BIN__N], hot_at = 0, hot_keys = 0;
     auto carve = [&](int64_t max_counters) {
         RG_TRY(bin_plan(vis->n, sh.nkeys, sh.per_item, max_counters, sizeof(Rec<T>), pl));
-        at = head;
+        size_t at = head;
         for (int k = 0; k < BIN__N; ++k) {
             if (k == BIN_CURSOR) {
                 off[k] = off[BIN_COUNT];
@@ -689,29 +716,62 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
                 at += aligned(pl.bytes[k]);
             }
         }
-        return (int)RG_OK;
-    };
-    RG_TRY(carve(BIN_MAX_COUNTERS));
-    if (at > NOALLOC_SCRATCH_BYTES) { // leaner: no plane groups, larger items, one replica
-        sh.one_group(wk->plane_count, 1);
-        sh.per_item = std::max(sh.per_item, limit_item);
-        RG_TRY(carve(1));
-    }
-    HotSlots hot{};
-    size_t hot_at = at, hot_keys = 0;
-    if (grid_type == RG_C64 && sh.hot_min) {
+        hot_at = at;
         hot_keys = aligned(sizeof(uint32_t) * (size_t)sh.hot_slots);
         at += hot_keys + aligned(sh.hot_bytes(wk->size, sh.hot_slots));
-        if (at > NOALLOC_SCRATCH_BYTES) { // no room beside the keys of a very large grid
-            at = hot_at;
-            sh.hot_min = 0;
-        }
+        return at <= NOALLOC_SCRATCH_BYTES ? RG_OK : RG_ERR_NOMEM;
+    };
+    // as many counters a key as there is room for
+    auto carve_any = [&](int64_t least) {
+        int rc = RG_ERR_NOMEM;
+        for (int64_t c = 16; c >= least && rc == RG_ERR_NOMEM; c /= 2)
+            rc = carve(std::min(BIN_MAX_COUNTERS, c * bin_stride(sh.nkeys)));
+        return rc;
+    };
+    // The longest streams' records take almost all of the array.  Such a call does without the
+    // plane groups; a stream whose FP64 sums of items find no room then (the last tenth below
+    // the limit) is gridded in two halves (2.1 M, FP32, tracks on 1024^2: 501 us, without the sums
+    // and with the items of 2048 records that keep the error 622); without such sums
+    // wider tiles have half the keys; and a very large grid is sorted by one strip of
+    // tile rows after another.
+    int rc = carve_any(2);
+    if (rc == RG_ERR_NOMEM && sh.max_groups > 1) {
+        sh.one_group(wk->plane_count, 1);
+        rc = carve_any(2);
     }
-    if (want > NOALLOC_LIMIT_BYTES || at > NOALLOC_SCRATCH_BYTES)
-        return fail(RG_ERR_PARAM,
-                    "rg_grid_noalloc: %lld visibilities on a %d^2 grid need %zu bytes of scratch; "
-                    "the static scratch holds %zu: split the stream over calls with accumulate = 1",
-                    (long long)vis->n, N, want, NOALLOC_LIMIT_BYTES);
+    if (rc == RG_ERR_NOMEM && sh.hot_min && vis->n >= (1 << 16) &&
+        pl.bytes[BIN_VIS_START] <= NOALLOC_SCRATCH_BYTES / 16) {
+        rg_flat_vis half = *vis;
+        half.n = vis->n / 128 * 64;
+        RG_TRY(wproj_noalloc_t<T>(p, &half, wk, grid, grid_type, accumulate, s));
+        const size_t vsz = vis->vis_type == RG_C128 ? 16 : 8;
+        half.u += half.n;
+        half.v += half.n;
+        half.w += half.n;
+        half.vis = (const char *)half.vis + vsz * (size_t)half.n;
+        half.n = vis->n - half.n;
+        return wproj_noalloc_t<T>(p, &half, wk, grid, grid_type, 1, s);
+    }
+    if (rc == RG_ERR_NOMEM) {
+        sh.wide(N, wk->size);
+        sh.one_group(wk->plane_count, 1);
+        rc = carve_any(1);
+    }
+    if (rc == RG_ERR_NOMEM) {
+        if (grid_type == RG_C64)
+            sh.cold();
+        sh.per_item = std::max(sh.per_item, limit_item);
+        rc = carve_any(1);
+    }
+    const int64_t tiles = sh.nkeys;
+    for (int64_t rows = tiles / sh.ntx; rc == RG_ERR_NOMEM && rows > 1;) {
+        rows = (rows + 1) / 2;
+        sh.nkeys = rows * sh.ntx;
+        rc = carve(1);
+    }
+    if (rc == RG_ERR_NOMEM)
+        return fail(RG_ERR_PARAM, "rg_grid_noalloc: no room for a row of tiles");
+    RG_TRY(rc);
     void *base = nullptr;
     RG_TRY(noalloc_scratch(&base));
     char *b0 = static_cast<char *>(base);
@@ -728,7 +788,8 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
     // the previous call's counters are still there: start from zero
     ZeroList zero;
     RG_TRY(zero.add(b.stats, sizeof(unsigned long long) * CNT__N));
-    if (grid_type == RG_C64 && sh.hot_min) {
+    HotSlots hot{};
+    if (sh.hot_min) {
         hot.key = reinterpret_cast<uint32_t *>(b0 + hot_at);
         hot.sums = reinterpret_cast<double *>(b0 + hot_at + hot_keys);
         RG_TRY(zero.add(hot.key, hot_keys + sh.hot_bytes(wk->size, sh.hot_slots)));
@@ -737,18 +798,38 @@ static int wproj_noalloc_t(const rg_grid_params *p, const rg_flat_vis *vis, cons
         RG_TRY(zero.add(grid, (size_t)(grid_type == RG_C128 ? 16 : 8) * N * N));
     if (vis->n == 0)
         return zero.launch(s);
-    if (!bin_small(vis->n, sh.nkeys))
-        RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
     const PlaneGroups pg = sh.groups(b0 + COUNTER_PLANES, b.krp, vis->n);
     const WprojKeyer kf =
         wproj_keyer(p, vis, wk, sh, nullptr, 1, (int)sizeof(typename Vec2<T>::type), pg);
+    auto tiles_of = [&](const BinResult &br) {
+        return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N, 1,
+                                 sh, hot, s);
+    };
+    if (sh.nkeys < tiles) {
+        for (int64_t k = 0; k < tiles; k += sh.nkeys) {
+            sh.key0 = (uint32_t)k;
+            StripKeyer sk;
+            static_cast<WprojKeyer &>(sk) = kf;
+            sk.key0 = sh.key0;
+            sk.count = (uint32_t)sh.nkeys;
+            if (k > 0)
+                RG_TRY(zero.add(b.stats, sizeof(unsigned long long) * CNT__N));
+            RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
+            BinResult br;
+            RG_TRY((bin_run<StripKeyer, T>(sk, vis->n, sh.nkeys, sh.per_item, pl, b, zero, nullptr,
+                                           s, br)));
+            RG_TRY(tiles_of(br));
+        }
+        return RG_OK;
+    }
+    if (!bin_small(vis->n, sh.nkeys))
+        RG_TRY(zero.add(b.count, pl.bytes[BIN_COUNT]));
     if (pg.samples)
         RG_TRY(clear_and_sample(zero, kf, vis->n, pg, s));
     BinResult br;
     RG_TRY((bin_run<WprojKeyer, T>(kf, vis->n, sh.nkeys, sh.per_item, pl, b, zero, nullptr,
                                    s, br)));
-    return dispatch_tiles<T>(br, nullptr, b.stats, wk, grid, grid_type, p->compensated != 0, N, 1,
-                             sh, hot, s);
+    return tiles_of(br);
 }
 
 int wproj_noalloc(const rg_grid_params *p, const rg_flat_vis *vis, const rg_wkern *wk, void *grid,

@@ -78,3 +78,42 @@ def test_split_stream_accumulates(ctx, c1):
     rgamd.grid_noalloc(p, fv_b, wk, g, accumulate=True)
     torch.cuda.synchronize()
     assert rel_max(g.cpu().numpy(), g_ref.cpu().numpy()) < 1e-12
+
+
+def whole_numbers(N, n, theta, S, seed):
+    """A stream all over the grid and past its edges, in and out of the table's planes, and
+    a table, of small whole numbers: sums are exact in FP32, in any order."""
+    rng = np.random.default_rng(seed)
+    u, v = (1.04 * (rng.random((2, n)) - 0.5)) * N / theta
+    w = rng.integers(-4, 4, n).astype(float)
+    cpx = lambda *s: rng.integers(-4, 5, s) + 1j * rng.integers(-4, 5, s)
+    return (u, v, w, cpx(n)), cpx(6, 2, 2, S, S)
+
+
+# (N, visibilities, kernel size, tile, types): records that leave no room for FP64 sums of items
+# (two halves), for narrow tiles' keys, and grids of more tiles than are sorted at once
+@pytest.mark.parametrize("N,n,S,tile,dt,gdt", [
+    (1024, 2_080_000, 8, 0, torch.complex64, torch.complex64),
+    (1000, 2_060_001, 16, 32, torch.complex64, torch.complex64),
+    (2048, 1_390_000, 8, 48, torch.complex128, torch.complex128),
+    (2048, 1_980_000, 16, 48, torch.complex64, torch.complex128),
+    (52000, 600_000, 8, 48, torch.complex64, torch.complex64),
+    (36880, 1000, 16, 32, torch.complex64, torch.complex64),
+])
+def test_close_to_the_limit(ctx, N, n, S, tile, dt, gdt):
+    theta = 0.1
+    data, table = whole_numbers(N, n, theta, S, N + n)
+    _, fv = stage(*data, dt)
+    _, wk = kern(table, -2.0, 1.0, dt)
+    p = rgamd.params(N, theta, mode=rgamd.RG_MODE_BATCHED, tile=tile)
+    want = torch.empty((N, N), dtype=gdt, device="cuda")
+    ctx.grid(p, fv, wk, want)
+    got = torch.full((N, N), 7.0 + 3.0j, dtype=gdt, device="cuda")
+    for k in range(2):
+        rgamd.grid_noalloc(p, fv, wk, got, accumulate=k == 1)
+        torch.cuda.synchronize()
+        # (real parts and imaginary parts as numbers: +0 and -0 are equal)
+        same = [bool((a == (k + 1) * b).all()) for a, b in
+                zip(torch.view_as_real(got).split(4096), torch.view_as_real(want).split(4096))]
+        assert all(same)
+    assert want.abs().max().item() > 0 if N < 4096 else True
