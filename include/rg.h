@@ -93,7 +93,7 @@ typedef struct rg_grid_params {
                                batched W-towers: band height in rows (4, 8 or 16 (16 in
                                FP32 only), 0 = 8) */
     int32_t vis_per_item;   /* batched visibilities per work item (0 = default;
-                               W-projection: at most 512) */
+                               W-projection: at most 512, larger values are as 0) */
     int32_t compensated;    /* batched FP32: 0 plain FP32 sums (default), 1 two-sum
                                compensated sums: W-projection tile sums (worth it only into
                                an RG_C128 grid), W-towers band lanes' register sums */

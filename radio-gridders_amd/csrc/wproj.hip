@@ -535,8 +535,11 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
     sh.hot_slots = sh.hot_min ? nvis / sh.hot_min + 1 : 0;
     // of the shorter streams the longest with items of k / 2, 12 k^2 - 1 records, takes most
     sh.hot_room = std::max<int64_t>(sh.hot_slots, sh.hot_min && k > 8 ? 3 * k : 0);
-    sh.per_item = p->vis_per_item > 0 ? std::min<uint32_t>((uint32_t)p->vis_per_item, TILE_SORT)
-                                      : default_item(nvis);
+    // (items beyond what a wavefront sorts, 1024 to 4096 in parameters that were tuned for
+    // workgroups, leave the choice open too: a call of 150 k FP32 records takes 97 us, with 512
+    // of them an item 109; of 1 M 226, 259)
+    sh.per_item = p->vis_per_item > 0 && p->vis_per_item <= TILE_SORT ? (uint32_t)p->vis_per_item
+                                                                      : default_item(nvis);
     return RG_OK;
 }
 

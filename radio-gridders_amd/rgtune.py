@@ -2,7 +2,7 @@
 
 The batched paths have a few knobs that change speed but not results:
   W-projection (subgrid_size 0): tile edge (32, 48) and visibilities per work
-      item (vis_per_item);
+      item (vis_per_item), which its present kernel has one best choice of;
   W-towers (subgrid_size n > 0): band height (tile: 4, 8, 16 in FP32),
       vis_per_item, tasks per batch (floor_batch) and the radix of the column
       pass's FFT stages (fft_radix: 8 or 4).
@@ -61,7 +61,9 @@ def search_space(p: rgamd.GridParams, fv: rgamd.FlatVis, n_tasks: int = 0) -> di
     """Candidate values per knob (the first value of each is the default)."""
     fp32 = fv.vis_type == rgamd.RG_C64
     if p.subgrid_size == 0:
-        return {"tile": [32, 48], "vis_per_item": [2048, 1024, 4096]}
+        # (both tiles run the same kernel, and items of more than 512 records are chosen by
+        # the stream's length)
+        return {"tile": [32, 48], "vis_per_item": [2048]}
     space = {"tile": [8, 4] + ([16] if fp32 else []),
              "vis_per_item": [2048, 1024, 4096],
              "fft_radix": [8, 4]}

@@ -380,3 +380,21 @@ def test_channels_wide_tiles(ctx, planes, n, dt, gdt, comp):
         mag, _, _ = orc.grid_wprojection(N, THETA, u[sl], v[sl], w[sl], np.abs(vis[sl]) + 0j,
                                          np.abs(table) + 0j, 0.0, 1.0)
         assert (np.abs(got - ref) <= (n + 4) * eps * mag.real).all(), c
+
+
+@pytest.mark.parametrize("per_item", [513, 1024, 2048, 4096])
+def test_large_items_are_the_stream_s_choice(ctx, per_item):
+    """Items of more records than a wavefront sorts are chosen by the stream's length, as 0 is:
+    the same number of items; 512 is taken as it stands."""
+    rng = np.random.default_rng(4)
+    n, N = 30000, 512
+    u, v = (rng.random((2, n)) - 0.5) * 40 / THETA
+    _, fv = stage(u, v, np.zeros(n), np.ones(n, complex))
+    _, wk = kern(np.ones((1, 2, 2, 8, 8), complex), 0.0, 1.0)
+    g = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    items = []
+    for k in (0, per_item, 512):
+        ctx.grid(rgamd.params(N, THETA, vis_per_item=k), fv, wk, g)
+        items.append(ctx.stats().n_items)
+    # 12 32^2 <= n < 12 64^2
+    assert items[0] == items[1] >= n // 32 > 4 * items[2]
