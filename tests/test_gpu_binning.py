@@ -398,3 +398,27 @@ def test_large_items_are_the_stream_s_choice(ctx, per_item):
         items.append(ctx.stats().n_items)
     # 12 32^2 <= n < 12 64^2
     assert items[0] == items[1] >= n // 32 > 4 * items[2]
+
+
+@pytest.mark.parametrize("nchan", [15, 16])
+def test_channels_by_scan_threads_of_one_and_four_keys(ctx, table, nchan):
+    """4225 tiles of 16 x 16 cells per channel (65^2): 63 375 keys, the last number of channels at
+    which a scan thread takes one of them, and 67 600, where it takes four.  FP64 sums of at most
+    5000 terms against the plain form's."""
+    N = 1024
+    counts = np.random.default_rng(nchan).integers(0, 300, nchan)
+    counts[1], counts[2] = 0, 5000
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    u, v, w, vis = stream(off[-1], 4500.0, 5.0, 9)
+    (du, dv, dw, dvis), fv = stage(u, v, w, vis)
+    _, wk = kern(table, -5.0, 1.0)
+    g = torch.empty((nchan, N, N), dtype=torch.complex128, device="cuda")
+    ctx.grid_channels(rgamd.params(N, THETA), fv, off, wk, g)
+    assert ctx.stats().n_gridded == off[-1]
+    one = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    for c in range(nchan):
+        a, b = off[c], off[c + 1]
+        fc = rgamd.flat_vis(du[a:b].clone(), dv[a:b].clone(), dw[a:b].clone(), dvis[a:b].clone())
+        ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN), fc, wk, one)
+        torch.cuda.synchronize()
+        assert float((g[c] - one).abs().max()) <= 1e-12 * max(float(one.abs().max()), 1e-300)
