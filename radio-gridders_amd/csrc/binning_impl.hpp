@@ -76,7 +76,7 @@ int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uin
     DevBuf *buf[BIN__N];
     for (int k = 0; k < BIN__N; ++k)
         buf[k] = &ctx->scratch[bin_slot[k]];
-    RG_TRY(ensure_together(buf, pl.bytes, BIN__N));
+    RG_TRY(ensure_together(buf, pl.bytes, BIN__N, (size_t)16 << 20));
     if (!bin_small(n, nkeys))
         RG_TRY(zero.add(ctx->scratch[bin_slot[BIN_COUNT]].p, count_bytes));
     return RG_OK;

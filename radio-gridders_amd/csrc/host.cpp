@@ -69,11 +69,11 @@ void DevBuf::release()
     bytes = 0;
 }
 
-int ensure_together(DevBuf *const *buf, const size_t *n, int count)
+int ensure_together(DevBuf *const *buf, const size_t *n, int count, size_t most)
 {
     auto part = [&](int k) {
         const bool grows = !buf[k]->p || n[k] > buf[k]->bytes;
-        return grows && n[k] <= TOGETHER_BYTES && !(buf[k]->frozen && *buf[k]->frozen);
+        return grows && n[k] <= most && !(buf[k]->frozen && *buf[k]->frozen);
     };
     auto padded = [&](int k) { return (std::max<size_t>(n[k], 1) + 255) / 256 * 256; };
     size_t total = 0;
@@ -84,6 +84,11 @@ int ensure_together(DevBuf *const *buf, const size_t *n, int count)
         }
     std::shared_ptr<void> block;
     if (total) {
+        // (an allocation of another size than one that was freed is slow half the time, 340 us:
+        // sizes of a few steps)
+        constexpr size_t STEP = (size_t)16 << 20;
+        if (total >= (size_t)2 << 20)
+            total = (total + STEP - 1) / STEP * STEP;
         void *p = nullptr;
         hipError_t e = hipMalloc(&p, total);
         if (e != hipSuccess)

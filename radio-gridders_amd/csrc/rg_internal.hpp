@@ -95,11 +95,10 @@ struct DevBuf {
     template <typename T> T *as() const { return reinterpret_cast<T *>(p); }
 };
 
-// buf[i]->ensure(n[i]) for all of them, those of up to TOGETHER_BYTES that have to grow from one
-// allocation: an allocation of more than 2 MB takes up to 350 us.  (Larger ones stay
+// buf[i]->ensure(n[i]) for all of them, those of up to `most` bytes that have to grow from one
+// allocation: an allocation of 2 MB and more takes up to 350 us.  (Larger ones stay
 // by themselves: their memory goes back when they grow.)
-constexpr size_t TOGETHER_BYTES = (size_t)16 << 20;
-int ensure_together(DevBuf *const *buf, const size_t *n, int count);
+int ensure_together(DevBuf *const *buf, const size_t *n, int count, size_t most);
 
 struct PinnedBuf {
     void *p = nullptr;

@@ -2397,12 +2397,6 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     // batches of Q tasks
     const int Q = batch_tasks_of(ntasks_cap);
     const int nbatch = (ntasks_cap + Q - 1) / Q;
-    if (measure) {
-        // the slot-count table layout holds a spill counter for every batch of
-        // the plan's (fewer) tasks
-        RG_TRY(clear_subimages(nbatch, spill_ctr));
-        RG_TRY(zero.launch(s));
-    }
     // spill slots (parts of split keys: at most 2 R / K for R records), per batch
     const uint64_t max_spill = 2 * ((uint64_t)g.mk * vis->n) / K + 1;
     const size_t band_bytes = sizeof(T2) * (size_t)H * n;
@@ -2411,7 +2405,22 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     const size_t sp_bytes = band_bytes * max_spill;
     const size_t is_bytes = (sizeof(uint32_t) * (size_t)max_items_w + 255) / 256 * 256;
     const size_t si_bytes = sizeof(uint32_t) * (size_t)max_spill;
-    RG_TRY(ctx->scratch[7].ensure(g_bytes + p_bytes + sp_bytes + is_bytes + si_bytes));
+    // every work item's records sorted by footprint column into the expanded
+    // array (window records laid out item after item)
+    const int64_t nexp = (int64_t)g.mk * vis->n;
+    {
+        DevBuf *buf[] = {&ctx->scratch[7], &ctx->scratch[10], &ctx->scratch[11]};
+        const size_t need[] = {g_bytes + p_bytes + sp_bytes + is_bytes + si_bytes,
+                               sizeof(T2) * nn * ntowers_cap,
+                               sizeof(BandRec<T>) * (size_t)std::max<int64_t>(nexp, 1)};
+        RG_TRY(ensure_together(buf, need, 3, (size_t)256 << 20));
+    }
+    if (measure) {
+        // the slot-count table layout holds a spill counter for every batch of
+        // the plan's (fewer) tasks
+        RG_TRY(clear_subimages(nbatch, spill_ctr));
+        RG_TRY(zero.launch(s));
+    }
     char *base7 = ctx->scratch[7].as<char>();
     T2 *G = reinterpret_cast<T2 *>(base7);
     T2 *Pp = reinterpret_cast<T2 *>(base7 + g_bytes);
@@ -2420,10 +2429,6 @@ static int wtowers_batched_t(rg_context *ctx, const rg_grid_params *p, const rg_
     uint32_t *spill_item =
         reinterpret_cast<uint32_t *>(base7 + g_bytes + p_bytes + sp_bytes + is_bytes);
 
-    // every work item's records sorted by footprint column into the expanded
-    // array (window records laid out item after item)
-    const int64_t nexp = (int64_t)g.mk * vis->n;
-    RG_TRY(ctx->scratch[11].ensure(sizeof(BandRec<T>) * (size_t)std::max<int64_t>(nexp, 1)));
     BandRec<T> *sorted = ctx->scratch[11].as<BandRec<T>>();
     {
         KernelTimer kt(ctx, RG_TIMER_BINNING, s);
