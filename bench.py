@@ -684,7 +684,7 @@ def bench_epic(ctx, steps, warmup, skip_cpu):
     r = {"timestamps": nb, "antennas": na, "grid": g, "support": S, "ms": ms,
          "timestamps_per_s": nb / (ms * 1e-3), "samples_per_s": nb * na / (ms * 1e-3),
          "max_rel_err_vs_oracle": float(np.abs(got - ref).max() / np.abs(ref).max()),
-         "roofline": {"kernel": "k_epic_grid", "bound": "hbm", "achieved": ach,
+         "roofline": {"kernel": "k_epic_band", "bound": "hbm", "achieved": ach,
                       "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                       "bytes_per_unit": {"timestamp": per_ts}}}
     if not skip_cpu:
