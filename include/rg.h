@@ -89,7 +89,7 @@ typedef struct rg_grid_params {
     int32_t subgrid_margin; /* W-towers margin M */
     double winc;            /* W-towers floor spacing (wavelengths) */
     int32_t tile;           /* batched W-projection: 32, 48 or 0 (all three run the same
-                               tiles of 16 x 16 positions);
+                               tiles of 16 x 16 positions, or 32 x 16 on large grids);
                                batched W-towers: band height in rows (4, 8 or 16 (16 in
                                FP32 only), 0 = 8) */
     int32_t vis_per_item;   /* batched visibilities per work item (0 = default;

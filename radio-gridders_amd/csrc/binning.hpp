@@ -40,7 +40,7 @@ template <> struct Vec2<double> { using type = double2; };
 
 template <typename T> struct Rec {
     uint32_t pos;  // tile-local footprint top-left: lx | ly << 16
-    uint32_t kidx; // (plane * R + yf) * R + xf
+    uint32_t kidx; // sub-kernel (plane * R + yf) * R + xf; W-projection: its byte offset
     typename Vec2<T>::type vis;
 };
 

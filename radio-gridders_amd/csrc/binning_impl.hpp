@@ -56,7 +56,7 @@ int bin_prepare(rg_context *ctx, int64_t n, int64_t nkeys, int64_t key_room, uin
     RG_TRY(ensure_counters(ctx));
     // items and scan sums: room for every call of up to this many visibilities
     // and keys, whatever item size it picks (scratch that a captured graph holds
-    // cannot grow; a shorter stream's smaller items are at most 24 times 512);
+    // cannot grow; a shorter stream, below 12 512^2, has at most 48 K items, K up to 256);
     // counters likewise: fewer keys, or another gridder's, may take more replicas
     auto counters = [](int64_t keys, int64_t most) {
         const int64_t stride = bin_stride(keys);

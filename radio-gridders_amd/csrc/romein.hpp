@@ -1,4 +1,5 @@
-// romein.hpp -- software-pipelined record loop shared by the Romein kernels.
+// romein.hpp -- software-pipelined record loop of the W-towers band kernel, and the tap
+// reads' buffer resource, which the W-projection tiles use too.
 //
 // Records are consumed in batches of U: `fetch(j, batch)` reads records
 // [j, j + U) from LDS, computes each lane's footprint cell and issues the U

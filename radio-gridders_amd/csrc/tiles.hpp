@@ -18,8 +18,9 @@
 // added to the target with global atomics (neighbouring tiles and items of the
 // same tile overlap), a row at a time as consecutive numbers.
 //
-// Bound by VALU issue (31 instructions a record in FP32, 16 of them the FMAs; 62 % busy)
-// beside the tap reads (2 KB a record from L2, 19 TB/s).  With a workgroup of S S threads
+// Bound by the tap reads: the vector cache's data return is 94 % busy (2 KB a record in FP32,
+// 18 TB/s, of which 4.4 come from beyond L2), VALU issue 59 % (31 instructions a record, 16
+// of them the FMAs).  With a workgroup of S S threads
 // per item, a tap a lane (every lane of four wavefronts found its own cell and tap
 // address for every record: about 64 instructions) and records of all planes mixed
 // (a 60 MB table read past L2), tiles took, now, us: 8.4 M visibilities FP32 1571 -> 950;
