@@ -452,7 +452,7 @@ def bench_c1(ctx, steps, warmup, skip_cpu, npix):
     import rgamd
     import synth
     sys.path.insert(0, os.path.join(REPO, "oracle"))
-    import pyoracle as orc  # the checker: reference image and CPU timing only
+    import pyoracle as orc  # the oracle: reference image and CPU timing only
 
     obs = synth.config_c1()
     N, theta, nv = obs.grid_size, obs.theta, obs.n_vis
@@ -537,7 +537,7 @@ def bench_wstack(ctx, steps, warmup, skip_cpu, cpu_seconds):
 
     import rgamd
     sys.path.insert(0, os.path.join(REPO, "oracle"))
-    import pyoracle as orc  # the checker: accuracy sample and CPU baseline only
+    import pyoracle as orc  # the oracle: accuracy sample and CPU baseline only
 
     sze = os.path.join(REPO, "tests", "golden", "sze")
     ku = rgamd.load_sep_kern(os.path.join(sze, "sepkern_uv_transpose.hdf5"), True)
@@ -653,7 +653,7 @@ def bench_epic(ctx, steps, warmup, skip_cpu):
 
     import rgamd
     sys.path.insert(0, os.path.join(REPO, "oracle"))
-    import pyoracle as orc  # the checker: accuracy and CPU baseline only
+    import pyoracle as orc  # the oracle: accuracy and CPU baseline only
 
     g, S, nb, na = 64, 2, 1000, 256
     rng = np.random.default_rng(9)

@@ -1,7 +1,7 @@
 /*
  * oracle.c -- CPU FP64 restatement of the Radio-Gridders gridding hot path.
  *
- * TEST INFRASTRUCTURE ONLY (the checker).  Loaded by tests/, smoke() and the
+ * TEST INFRASTRUCTURE ONLY (the oracle).  Loaded by tests/, smoke() and the
  * cpu_baseline leg of bench.py; never by the product library.
  *
  * Built without fast-math and with -ffp-contract=off so the coordinate and

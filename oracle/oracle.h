@@ -1,7 +1,7 @@
 /*
  * oracle.h -- CPU FP64 restatement of the Radio-Gridders gridding hot path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker: it may be loaded by
+ * TEST INFRASTRUCTURE ONLY.  This library is the oracle: it may be loaded by
  * tests/, by __graft_entry__.smoke() and by the cpu_baseline leg of bench.py,
  * and by nothing else.  The product library (radio-gridders_amd) never links,
  * loads or calls it.

@@ -1,6 +1,6 @@
 """ctypes wrapper of the oracle (liboracle.so) -- TEST INFRASTRUCTURE ONLY.
 
-The oracle is the checker: only tests/, __graft_entry__.smoke() and the
+The oracle is for checks: only tests/, __graft_entry__.smoke() and the
 cpu_baseline leg of bench.py use it.  Arrays are numpy, complex values
 complex128.
 """
@@ -25,7 +25,7 @@ _L = C.c_int64
 
 
 def lib(fast: bool = False):
-    """liboracle.so (checker) or liboracle_fast.so (CPU-baseline timing build)."""
+    """liboracle.so (oracle) or liboracle_fast.so (CPU-baseline timing build)."""
     name = "liboracle_fast.so" if fast else "liboracle.so"
     if name not in _libs:
         path = os.path.join(HERE, name)
