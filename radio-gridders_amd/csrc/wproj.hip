@@ -525,7 +525,13 @@ static int wproj_shape(const rg_grid_params *p, int64_t nvis, int n_chan, const 
     if (!dense)
         group = std::max(group, (planes + 3) / 4);
     const int64_t all = (planes + group - 1) / group;
-    if (!sparse && all > 1 && (dense || 2 * one * all <= BIN_MAX_COUNTERS)) {
+    // Sub-kernels of 512 bytes (S = 8, FP32) are read fast enough from a table of up to 48 MB
+    // anyhow (15 MB, 8.4 M tracks, 2048^2: one group 529 us, grouped 540; 20 MB, 32 channels of
+    // 1024^2, 154 a tile 1477 / 1669; 61 MB, 2048^2: 678 / 618).
+    const int64_t sub_bytes = (int64_t)S * S * (wk->type == RG_C128 ? 16 : 8);
+    const bool ungrouped =
+        sub_bytes <= 512 && planes * wk->oversampling * wk->oversampling * sub_bytes <= (48 << 20);
+    if (!sparse && !ungrouped && all > 1 && (dense || 2 * one * all <= BIN_MAX_COUNTERS)) {
         sh.min_planes = (int)group;
         sh.max_groups = (int)all;
         sh.nkeys = one * all;

@@ -422,3 +422,33 @@ def test_channels_by_scan_threads_of_one_and_four_keys(ctx, table, nchan):
         ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN), fc, wk, one)
         torch.cuda.synchronize()
         assert float((g[c] - one).abs().max()) <= 1e-12 * max(float(one.abs().max()), 1e-300)
+
+
+@pytest.mark.parametrize("planes", [1536, 1537])
+def test_plane_groups_by_the_size_of_the_table(ctx, planes):
+    """FP32 sub-kernels of 8 x 8 taps: one plane group up to tables of 48 MB (1536 planes), as many as
+    the stream asks for beyond.  Small whole numbers: FP32 sums are exact in any order, and equal
+    to the plain form's."""
+    N, n, r, s = 128, 200_000, 8, 8
+    gen = torch.Generator(device="cuda").manual_seed(planes)
+    small = lambda *sh: torch.randint(-2, 3, (*sh, 2), generator=gen, device="cuda",  # noqa: E731
+                                      dtype=torch.int32).double()
+    table = torch.view_as_complex(small(planes, r, r, s, s))
+    u, v, _, _ = spread(n, N, planes, 3, True)
+    w = np.random.default_rng(2).integers(0, planes, n).astype(float)
+    vis = torch.view_as_complex(small(n)).cpu().numpy()
+    got = torch.empty((N, N), dtype=torch.complex64, device="cuda")
+    want = torch.empty((N, N), dtype=torch.complex128, device="cuda")
+    keep, f = stage(u, v, w, vis)
+    ctx.grid(rgamd.params(N, THETA, mode=rgamd.RG_MODE_PLAIN), f, rgamd.wkern_desc(table, 0.0, 1.0),
+             want)
+    torch.cuda.synchronize()
+    assert float(want.abs().max()) > 0
+    t32 = table.to(torch.complex64)
+    keep32, f32 = stage(u, v, w, vis, torch.complex64)
+    wk = rgamd.wkern_desc(t32, 0.0, 1.0)
+    for call in (ctx.grid, rgamd.grid_noalloc):
+        got.fill_(1)
+        call(rgamd.params(N, THETA), f32, wk, got)
+        torch.cuda.synchronize()
+        assert bool((torch.view_as_real(got.to(torch.complex128)) == torch.view_as_real(want)).all())
